@@ -4,8 +4,9 @@ range gives the bytes of the staged kernels."""
 import numpy as np
 import pytest
 
-from ufsm_amd import lib
+from ufsm_amd import lib, LP, DevBuf, shape5, gnp_t, split_t
 import orc
+from gpuutil import to_mx, mx_bytes
 from test_gpu_conv import exact_case, rand_case, gpu_conv
 
 pytestmark = pytest.mark.gpu
@@ -60,3 +61,77 @@ def test_border_rows_stay_out_of_other_planes(gpu):
     bad = ~np.isfinite(got.reshape(N, Co, D, H, W))
     exp = np.zeros((N, Co, D, H, W), bool); exp[0, :, D - 2:, H - 2:, W - 2:] = True
     assert np.array_equal(bad, exp)
+
+
+def conv_in_slabs(bits, N, Ci, Co, D, H, W, slab, up=0):
+    """One conv over the whole tensor and slab by slab into the planes of a second one (stored statistics): [(MX bytes, sums, kernel of the last call)]."""
+    rng = np.random.default_rng(Ci + Co + D * 3 + W)
+    S, G, dt = D * H * W, 8, 3 if bits == 8 else 4
+    Cu = Ci // 2 if up else 0
+    w = (rng.standard_normal((Co, Ci, 27)) * np.sqrt(2.0 / (Ci * 27))).astype(np.float32)
+    dw, db = DevBuf.from_numpy(w), DevBuf.from_numpy((rng.standard_normal(Co) * 0.1).astype(np.float32))
+    sp = split_t()
+    if up:
+        dx = to_mx(bits, rng.standard_normal((N, Cu, S // 8)).astype(np.float32)); dx2 = to_mx(bits, rng.standard_normal((N, Ci - Cu, S)).astype(np.float32))
+        sp.x2, sp.c_split, sp.up = dx2.ptr, Cu, 1
+    else:
+        dx = to_mx(bits, rng.standard_normal((N, Ci, S)).astype(np.float32))
+    sp.stored_stats = 1
+    f, res = (lib.lp_conv_fwd_f8 if bits == 8 else lib.lp_conv_fwd_f4), []
+    for planes in (D, slab):
+        y, sums, out = DevBuf(mx_bytes(bits, N, Co, S)), DevBuf(N * G * 2 * 24), DevBuf(N * G * 2 * 8)
+        lib.mi_gn_sums_zero(sums.ptr, 2 * N * G)
+        for z0 in range(0, D, planes):
+            sk = min(planes, D - z0)
+            if planes < D:
+                sp.zi0, sp.Di, sp.yzo, sp.yD = z0, D, z0, D
+            assert f(dx.ptr, dt, shape5(N, Ci, sk, H, W), dw.ptr, db.ptr, Co, y.ptr, dt, gnp_t(), sums.ptr, G, sp) == 0
+        lib.mi_gn_sums_get(sums.ptr, 2 * N * G, out.ptr)
+        LP.check()
+        res.append((y.to_numpy(np.uint8), out.to_numpy(np.float64), lib.mi_last_kernel().decode()))
+    return res
+
+
+# whole tensors past the kernel's range whose slabs are inside it, and whole tensors inside it on planes of an odd voxel count and of one that is no
+# multiple of 32 voxels in four planes
+@pytest.mark.parametrize("bits,N,Ci,Co,D,H,W,slab,up,thin", [(8, 1, 192, 64, 32, 32, 32, 4, 0, False), (8, 1, 192, 64, 32, 32, 32, 8, 1, False), (8, 2, 192, 64, 24, 24, 24, 4, 0, False),
+                                                             (4, 1, 96, 96, 24, 24, 24, 4, 0, False), (8, 1, 64, 64, 12, 5, 7, 4, 0, True), (8, 2, 64, 128, 12, 10, 6, 4, 1, True),
+                                                             (8, 1, 256, 64, 10, 9, 5, 4, 0, True), (4, 1, 96, 64, 16, 6, 7, 8, 0, True)])
+def test_slabs_equal_whole(gpu, bits, N, Ci, Co, D, H, W, slab, up, thin):
+    """A conv run in z-slabs takes the kernel of the whole tensor's conv and its statistics over the same voxels: the same bytes, and sums that differ
+    only by the order in which doubles are added."""
+    (y, s, k), (yz, sz, kz) = conv_in_slabs(bits, N, Ci, Co, D, H, W, slab, up)
+    assert ("conv3_thin_k" in k) == thin and ("conv3_thin_k" in kz) == thin, (k, kz)
+    assert np.array_equal(y, yz)
+    assert np.allclose(s, sz, rtol=1e-12, atol=1e-9)
+
+
+@pytest.mark.parametrize("bits,dims,slab", [(8, (64, 64, 64), 8), (8, (24, 20, 12), 4), (4, (32, 20, 28), 4)])
+def test_network_in_slabs(gpu, bits, dims, slab):
+    """Three levels, one window: level 1 of 64^3 is past the kernel's range and its slabs would be inside it; the other windows' levels are inside it on
+    planes of 60 and 70 voxels. Logits and every statistic are those of the forward over whole tensors."""
+    from ufsm_amd.unet import UNet, make_cfg, load_host
+    host = load_host()
+    S = dims[0] * dims[1] * dims[2]
+    net = UNet(make_cfg(4, [32, 64, 128], G=8, head_out=3, act_dt=bits), 1, *dims, seed=3)
+    dx = to_mx(bits, np.random.default_rng(1).standard_normal((1, 4, S)).astype(np.float32))
+    got = []
+    for planes in (0, slab):
+        host.unet_set_infer_slab(planes)
+        try:
+            out = DevBuf(3 * S * 4)
+            assert net.forward_x(dx.ptr, out.ptr) == 0
+            LP.check()
+            st = []
+            for k, (name, _, _) in enumerate(net.layer_outs()):
+                g, mp, rp = net.layer_stats(k)
+                for p in (mp, rp) if g else ():
+                    a = np.empty(g, np.float32); lib.mi_d2h(a.ctypes.data, p, a.nbytes); st.append((name, a))
+            got.append((out.to_numpy(np.float32), st))
+        finally:
+            host.unet_set_infer_slab(0)
+    net.close()
+    assert np.array_equal(got[0][0], got[1][0])
+    assert [n for n, _ in got[0][1]] == [n for n, _ in got[1][1]]
+    for (name, a), (_, b) in zip(got[0][1], got[1][1]):
+        assert np.array_equal(a, b), name

@@ -378,6 +378,7 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
         return conv_stem(who, x, xbf, xs, w, b, cout, y, ybf, gp, osum, Go, sp, true);
     const int N = xs.n, D = sp.Di ? sp.Di : xs.d, H = xs.h, W = xs.w;           // D: the inputs' depth
     const int Do = stride == 2 ? (D - 1) / 2 + 1 : xs.d, Ho = stride == 2 ? (H - 1) / 2 + 1 : H, Wo = stride == 2 ? (W - 1) / 2 + 1 : W;   // src/nn_bwd.cu:132-135
+    const int Dr = stride == 1 ? D : Do;                                        // output planes of the whole tensor, of which a z-range computes Do
     const size_t S = (size_t)D * H * W;
     const int zlo = sp.Di ? (sp.zi0 > 0 ? sp.zi0 - 1 : 0) : 0, zhi = sp.Di ? (sp.zi0 + xs.d + 1 < D ? sp.zi0 + xs.d + 1 : D) : D;      // input planes this launch reads
     const int fdt = fmt == 8 ? 3 : 4;
@@ -543,12 +544,13 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     // tiles); 256 -> 256 35 / 37 / 38 against 16.7 / 29.0 / 48.5 (1024 tiles); 384 -> 128 47 / 48 / 50 against 18.3 / 20.2 / 33.0 (512 tiles). Hence
     // 256 tiles, 512 in e4m3 from eight input blocks on; e2m1 of one or two blocks against the coarse form is even (64 -> 128 at 1 x 11 x 13^2: 11.7 and
     // 12.1 us) and keeps that from 64 tiles on. The row
-    // kernels' and the one-block, one-tile kernel's launches stay theirs
+    // kernels' and the one-block, one-tile kernel's launches stay theirs. The tiles counted are the whole tensor's (Dr planes), not a z-range's: a slab
+    // adds in the order of the whole tensor's conv and takes its statistics over the same runs, so that inference in slabs gives its bytes
     static int thin_env = -1;
     if (thin_env < 0) thin_env = getenv("MI_CONV_THIN") ? atoi(getenv("MI_CONV_THIN")) : 256;      // tuning knob: that tile count (0: never)
     const size_t thin_max = fmt == 8 && a.nbt >= 8 ? 2 * (size_t)thin_env : fmt == 4 && coarse && a.nbt <= 2 ? (size_t)thin_env / 4 : (size_t)thin_env;
     a.thin = thin_env > 0 && !a.row && !a.areg && !s2d && !act && a.wide && cout > 16 && !(osum && (cout / Go) % 4) && !sp.zlo && !sp.zhi && g_split < 0 && g_s2d < 0 && N <= 65535 &&
-             (size_t)D * H * W * 32 < ((size_t)1 << 31) && ((size_t)Do * Ho * Wo + 63) / 64 * (size_t)nmt_all * N <= thin_max;
+             (size_t)D * H * W * 32 < ((size_t)1 << 31) && mi_thin_tiles(Dr, Ho, Wo) * nmt_all * N <= thin_max;
     if (a.thin) { big = false; MT = 1; NT = 2; a.CB = a.nbt; }
     size_t smem = a.thin ? MI_THIN_LDS : a.row1 ? (size_t)10 * 352 * (RB + 4) : a.row ? (size_t)2 * 2048 * (RB + 4) : a.areg ? (size_t)2 * ((TT + 63) / 64 * 64) * (RB + 4) : big ? (size_t)4 * MT * (WTILE + 256) + (size_t)3 * ((TT + 63) / 64 * 64) * (RB + 4) + (size_t)(((27 * a.nbt + 1) >> 1) + 2) * 32 : lds_bytes(a.CB);
     if (s2d) smem = 0;
@@ -580,7 +582,7 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     a.nmt_all = nmt_all; a.ncs = nmt_all / MT;
     a.ntx = a.row ? (Wo + 31) / 32 : (Wo + 15) / 16; a.nty = (Ho + 7) / 8; a.ntz = (Do + TZ - 1) / TZ;      // (the row kernel: 4 x 8 x 32 voxels per tile)
     a.ntiles = (unsigned)((size_t)a.ntx * a.nty * a.ntz * a.ncs * N);
-    if (a.thin) a.ntiles = (unsigned)(((size_t)Do * Ho * Wo + 63) / 64 * 2 * nmt_all * N);      // (a statistics record per run of 32 voxels and channel tile)
+    if (a.thin) { a.ntx = (MI_THIN_ZG * Ho * Wo + 63) / 64; a.ntiles = (unsigned)(mi_thin_tiles(Do, Ho, Wo) * 2 * nmt_all * N); }      // (a statistics record per run of 32 voxels and channel tile)
     // ---- weights ----
     int npairs_all = 0;
     for (int b0 = 0; b0 < a.nbt; b0 += a.CB) npairs_all += (27 * (a.nbt - b0 < a.CB ? a.nbt - b0 : a.CB) + 1) >> 1;
