@@ -378,7 +378,9 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
         return conv_stem(who, x, xbf, xs, w, b, cout, y, ybf, gp, osum, Go, sp, true);
     const int N = xs.n, D = sp.Di ? sp.Di : xs.d, H = xs.h, W = xs.w;           // D: the inputs' depth
     const int Do = stride == 2 ? (D - 1) / 2 + 1 : xs.d, Ho = stride == 2 ? (H - 1) / 2 + 1 : H, Wo = stride == 2 ? (W - 1) / 2 + 1 : W;   // src/nn_bwd.cu:132-135
-    const int Dr = stride == 1 ? D : Do;                                        // output planes of the whole tensor, of which a z-range computes Do
+    // output planes of the whole tensor, of which a z-range computes Do: whatever decides in which order a conv adds, and over which voxels its statistics
+    // records run, is chosen by these, so that a slab gives the whole tensor's bytes
+    const int Dr = stride == 1 ? D : Do;
     const size_t S = (size_t)D * H * W;
     const int zlo = sp.Di ? (sp.zi0 > 0 ? sp.zi0 - 1 : 0) : 0, zhi = sp.Di ? (sp.zi0 + xs.d + 1 < D ? sp.zi0 + xs.d + 1 : D) : D;      // input planes this launch reads
     const int fdt = fmt == 8 ? 3 : 4;
@@ -431,10 +433,10 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
         static int split_env = -1;
         if (split_env < 0) split_env = getenv("MI_CONV_SPLIT") ? atoi(getenv("MI_CONV_SPLIT")) : 192;    // tuning knob: tile count below which the slices are halved (0: never)
         const int split = g_split >= 0 ? g_split : split_env;
-        if (stride == 1 && MT == 4 && nmt_all % 4 == 0 && Do >= 3 &&
+        if (stride == 1 && MT == 4 && nmt_all % 4 == 0 && Dr >= 3 &&
             (size_t)((Wo + 15) / 16) * ((Ho + 7) / 8) * ((Do + 3) / 4) * (nmt_all / 4) * N < (size_t)split) { MT = 2; halved = true; }
     }
-    int NT = (stride == 1 && MT <= 2 && Do >= 4) ? 4 : 2;
+    int NT = (stride == 1 && MT <= 2 && Dr >= 4) ? 4 : 2;
     // ... and when even the slices of 64 give fewer than 128 workgroups (256 -> 256 at 2 x 16^3: 64): one channel tile and two planes per workgroup
     // on the general kernel, four times the workgroups (measured in the 32/64/128/256 forward: 128 -> 256 0.032 -> 0.026 ms, 256 -> 256
     // 0.050 -> 0.038 ms; from 256 slices of 64 on, the wide kernel is the faster one: 128 -> 128 at 2 x 32^3 0.034 against 0.052 ms)
@@ -442,7 +444,7 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     {
         static int ce = -1;
         if (ce < 0) ce = getenv("MI_CONV_COARSE") ? atoi(getenv("MI_CONV_COARSE")) : 1;      // tuning knob: 0 keeps the wide kernel's slices of 64 there (as does a split forced through mi_conv_split)
-        if (ce && halved && g_split < 0 && (size_t)((Wo + 15) / 16) * ((Ho + 7) / 8) * ((Do + 3) / 4) * (nmt_all / 2) * N < 128) { coarse = true; NT = 2; MT = 1; halved = false; }
+        if (ce && halved && g_split < 0 && (size_t)((Wo + 15) / 16) * ((Ho + 7) / 8) * ((Dr + 3) / 4) * (nmt_all / 2) * N < 128) { coarse = true; NT = 2; MT = 1; halved = false; }
     }
     // stride 2 with few tiles (the coarse levels): one-plane tiles double the workgroups; with enough tiles the two-plane tile is faster
     // (measured: 128 -> 128 at 32^3 -> 16^3, N 2: 32 tiles 0.072 ms, 64 tiles 0.042 ms; 32 -> 32 at 128^3: 0.090 vs 0.120 ms)
@@ -478,9 +480,9 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     if (rowcs4_env < 0) rowcs4_env = getenv("MI_CONV_ROW_CS4") ? atoi(getenv("MI_CONV_ROW_CS4")) : 1;      // tuning knob: input blocks up to which 65 .. 128 output channels run the row kernels as three or four slices (0: never).
     // Measured: 32 -> 128 at 2 x 64^3 0.079 -> 0.064 ms on the one-block kernel; from two blocks on the wide kernel is as fast (64 -> 128 and 128 -> 128 at 2 x 32^3)
     // or faster (e2m1 at 32 x 32^3: 0.151 against 0.164 ms), hence 1
-    const bool row_cs4 = rowcs4_env > 0 && g_split < 0 && (nmt_all == 3 || nmt_all == 4) && a.nbt <= rowcs4_env && stride == 1 && !coarse && a.wide && Wo > 16 && Do >= 4 && !(osum && (cout / Go) % 4);
+    const bool row_cs4 = rowcs4_env > 0 && g_split < 0 && (nmt_all == 3 || nmt_all == 4) && a.nbt <= rowcs4_env && stride == 1 && !coarse && a.wide && Wo > 16 && Dr >= 4 && !(osum && (cout / Go) % 4);
     if (row_cs4) { MT = 1; NT = 4; halved = false; }
-    bool big = !row_cs4 && !coarse && big_env && stride == 1 && (MT == 4 || (MT == 2 && (big_env > 1 || a.nbt >= 4 || halved))) && Do >= 3 && a.wide && a.nbt <= 12;            // (its per-tile pair table must fit LDS)
+    bool big = !row_cs4 && !coarse && big_env && stride == 1 && (MT == 4 || (MT == 2 && (big_env > 1 || a.nbt >= 4 || halved))) && Dr >= 3 && a.wide && a.nbt <= 12;            // (its per-tile pair table must fit LDS)
     if (big) {
         // The wide kernel streams input block b >= 2 of a tile into LDS while the tile's earlier blocks are multiplied, one copy round per
         // stage of two pairs, NRND rounds per block, a block starting once block b - 3 has been read for the last time (pair (27 (b - 3) + 26) / 2).
@@ -701,7 +703,8 @@ static size_t conv_scratch_bound(int fmt, const void *x2, int xbf, int ybf, shap
     if (fmt == 4 && Ci <= 8) fmt = 8;
     const size_t S = (size_t)D * xs.h * xs.w, So = (size_t)xs.d * xs.h * xs.w;
     const int nmt_all = (cout + 31) / 32, fdt = fmt == 8 ? 3 : 4;
-    const size_t tiles = (size_t)((xs.w + 15) / 16) * ((xs.h + 7) / 8) * xs.d * nmt_all * N;           // one-plane tiles of one channel tile: no launch has more
+    // one-plane tiles of one channel tile: no launch has more (a z-range of one plane may still run the one-block row kernel: 512 bytes per tile of 32 voxels along x)
+    const size_t tiles = (size_t)((xs.w + 15) / 16) * ((xs.h + 7) / 8) * (sp.Di && xs.d < 2 ? 2 : xs.d) * nmt_all * N;
     size_t need = 256;                                              // the constant page
     if (Ci <= 16 && !x2 && fmt == 8) need += al((size_t)9 * nmt_all * 2048) + al((size_t)9 * nmt_all * 256);      // the tap-packed kernels' weights
     const int nbt = (Cx + 31) / 32 + (x2 ? (C2 + 31) / 32 : 0);
