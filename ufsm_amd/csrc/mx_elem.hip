@@ -53,37 +53,49 @@ static dim3 rows_grid(int N, int nb, size_t S) {
 constexpr int CVT_BW = 16;         // widest block of the two-voxel form
 static bool cvt_pairs(int C, size_t S) { return mx_bw(C) <= CVT_BW && S >= (size_t)1 << 17; }
 static bool cvt_stream(const void *planes, int N, int C, size_t S) { return S % 32 == 0 && !((uintptr_t)planes & 127) && (size_t)N * C * S * 4 >= (size_t)256 << 20; }
-template <typename TI, int V> struct plane_v { typedef TI t __attribute__((ext_vector_type(V), aligned(alignof(TI)))); };      // V neighbouring voxels of a plane (any element's address)
-template <int B, typename TI, int V = 1, bool STREAM = false>
+typedef float plane2_t __attribute__((ext_vector_type(2), aligned(4)));      // two neighbouring voxels of a plane (any element's address)
+template <int B, typename TI, bool STREAM = false>
 __global__ void __launch_bounds__(256) f32_to_mx_k(const TI *x, uint8_t *y, int N, int C, size_t S) {
     const int bw = mx_bw(C), nb = mx_nb(C);
-    size_t v = (blockIdx.x * (size_t)blockDim.x + threadIdx.x) * V;       // grid: x over the voxels, y = n nb + blk (uniform: no per-thread divisions)
+    const size_t v = blockIdx.x * (size_t)blockDim.x + threadIdx.x;       // grid: x over the voxels, y = n nb + blk (uniform: no per-thread divisions)
     if (v >= S) return;
-    if (V > 1 && v + V > S) v = S - V;                                    // (S >= V; the last thread's voxels overlap its neighbour's: the same bytes twice)
     const int blk = (int)(blockIdx.y % (unsigned)nb), n = (int)(blockIdx.y / (unsigned)nb);
     const size_t i = (size_t)blockIdx.y * S + v;
-    float r[V][32];
+    float r[32];
+    // (the loads are written as a conditional value, not as a branch around a pointer: in that form the e2m1 kernel takes 74 registers for 71, a wavefront
+    // per SIMD less, and conversions of 32 channels and more lose 2 - 10 %, of 16-bit planes 5 - 20 %)
 #pragma unroll
     for (int k = 0; k < 32; k++) {
         const int c = blk * bw + k;
-        const bool on = (V == 1 || k < CVT_BW) && k < bw && c < C;
-        const TI *p = x + ((size_t)n * C + c) * S + v;
-        if constexpr (V > 1) {
-            typename plane_v<TI, V>::t q = {};
-            if (on) q = *(const typename plane_v<TI, V>::t *)p;
+        if constexpr (STREAM) r[k] = k < bw && c < C ? __builtin_nontemporal_load(x + (((size_t)n * C + c) * S + v)) : 0.f;
+        else r[k] = k < bw && c < C ? ldx(x, ((size_t)n * C + c) * S + v) : 0.f;
+    }
+    store_row<B, true>(y, mx_scp<B>(y, N, C, S), i, bw, r);
+}
+template <int B>
+__global__ void __launch_bounds__(256) f32_to_mx_pairs_k(const float *x, uint8_t *y, int N, int C, size_t S) {
+    const int bw = min(mx_bw(C), CVT_BW), nb = mx_nb(C);
+    size_t v = (blockIdx.x * (size_t)blockDim.x + threadIdx.x) * 2;
+    if (v >= S) return;
+    if (v + 2 > S) v = S - 2;                                             // (S >= 2; the last thread's voxels overlap its neighbour's: the same bytes twice)
+    const int blk = (int)(blockIdx.y % (unsigned)nb), n = (int)(blockIdx.y / (unsigned)nb);
+    const size_t i = (size_t)blockIdx.y * S + v;
+    float r[2][32];
 #pragma unroll
-            for (int j = 0; j < V; j++) r[j][k] = q[j];
-        } else if constexpr (STREAM) r[0][k] = on ? __builtin_nontemporal_load(p) : 0.f;
-        else r[0][k] = on ? ldx(p, 0) : 0.f;
+    for (int k = 0; k < 32; k++) {
+        const int c = blk * bw + k;
+        plane2_t q = {};
+        if (k < CVT_BW && k < bw && c < C) q = *(const plane2_t *)(x + ((size_t)n * C + c) * S + v);
+        r[0][k] = q[0]; r[1][k] = q[1];
     }
 #pragma unroll
-    for (int j = 0; j < V; j++) store_row<B, true>(y, mx_scp<B>(y, N, C, S), i + j, V > 1 ? min(bw, CVT_BW) : bw, r[j]);
+    for (int j = 0; j < 2; j++) store_row<B, true>(y, mx_scp<B>(y, N, C, S), i + j, bw, r[j]);
 }
 template <int B> static void f32_to_mx(const float *x, int N, int C, size_t S, void *y) {
     const size_t n = (size_t)N * mx_nb(C) * S;
     if (!n) return;
-    if (cvt_pairs(C, S)) f32_to_mx_k<B, float, 2><<<rows_grid(N, mx_nb(C), (S + 1) / 2), 256>>>(x, (uint8_t *)y, N, C, S);
-    else if (cvt_stream(x, N, C, S)) f32_to_mx_k<B, float, 1, true><<<rows_grid(N, mx_nb(C), S), 256>>>(x, (uint8_t *)y, N, C, S);
+    if (cvt_pairs(C, S)) f32_to_mx_pairs_k<B><<<rows_grid(N, mx_nb(C), (S + 1) / 2), 256>>>(x, (uint8_t *)y, N, C, S);
+    else if (cvt_stream(x, N, C, S)) f32_to_mx_k<B, float, true><<<rows_grid(N, mx_nb(C), S), 256>>>(x, (uint8_t *)y, N, C, S);
     else f32_to_mx_k<B, float><<<rows_grid(N, mx_nb(C), S), 256>>>(x, (uint8_t *)y, N, C, S);
     MICK();
 }
@@ -101,35 +113,45 @@ extern "C" void lp_h16_to_mx8(const void *x, int dt, int N, int C, size_t S, voi
 extern "C" void lp_h16_to_mx4(const void *x, int dt, int N, int C, size_t S, void *y) { h16_to_mx<4>(x, dt, N, C, S, y); }
 
 // ---- MX -> fp32 planes (src/lp_mx_cvt.cu:429-447) ----
-template <int B, int V = 1, bool STREAM = false>
+template <int B, bool STREAM = false>
 __global__ void __launch_bounds__(256) mx_to_f32_k(const uint8_t *x, float *y, int N, int C, size_t S) {
     const int bw = mx_bw(C), nb = mx_nb(C);
-    size_t v = (blockIdx.x * (size_t)blockDim.x + threadIdx.x) * V;       // grid: x over the voxels, y = n nb + blk (uniform: no per-thread divisions)
+    const size_t v = blockIdx.x * (size_t)blockDim.x + threadIdx.x;       // grid: x over the voxels, y = n nb + blk (uniform: no per-thread divisions)
     if (v >= S) return;
-    if (V > 1 && v + V > S) v = S - V;                                    // (as f32_to_mx_k)
     const int blk = (int)(blockIdx.y % (unsigned)nb), n = (int)(blockIdx.y / (unsigned)nb);
     const size_t i = (size_t)blockIdx.y * S + v;
-    float r[V][32];
-#pragma unroll
-    for (int j = 0; j < V; j++) load_row<B>(x, mx_scp<B>(x, N, C, S), i + j, V > 1 ? min(bw, CVT_BW) : bw, r[j]);
+    float r[32];
+    load_row<B>(x, mx_scp<B>(x, N, C, S), i, bw, r);
 #pragma unroll
     for (int k = 0; k < 32; k++) {
         const int c = blk * bw + k;
-        if ((V > 1 && k >= CVT_BW) || k >= bw || c >= C) continue;
-        float *p = y + ((size_t)n * C + c) * S + v;
-        if constexpr (V > 1) {
-            typename plane_v<float, V>::t q;
+        if (k < bw && c < C) {
+            if constexpr (STREAM) __builtin_nontemporal_store(r[k], y + (((size_t)n * C + c) * S + v));
+            else y[((size_t)n * C + c) * S + v] = r[k];
+        }
+    }
+}
+template <int B>
+__global__ void __launch_bounds__(256) mx_to_f32_pairs_k(const uint8_t *x, float *y, int N, int C, size_t S) {
+    const int bw = min(mx_bw(C), CVT_BW), nb = mx_nb(C);
+    size_t v = (blockIdx.x * (size_t)blockDim.x + threadIdx.x) * 2;
+    if (v >= S) return;
+    if (v + 2 > S) v = S - 2;                                             // (as f32_to_mx_pairs_k)
+    const int blk = (int)(blockIdx.y % (unsigned)nb), n = (int)(blockIdx.y / (unsigned)nb);
+    const size_t i = (size_t)blockIdx.y * S + v;
+    float r[2][32];
 #pragma unroll
-            for (int j = 0; j < V; j++) q[j] = r[j][k];
-            *(typename plane_v<float, V>::t *)p = q;
-        } else if constexpr (STREAM) __builtin_nontemporal_store(r[0][k], p);
-        else *p = r[0][k];
+    for (int j = 0; j < 2; j++) load_row<B>(x, mx_scp<B>(x, N, C, S), i + j, bw, r[j]);
+#pragma unroll
+    for (int k = 0; k < CVT_BW; k++) {
+        const int c = blk * bw + k;
+        if (k < bw && c < C) { const plane2_t q = {r[0][k], r[1][k]}; *(plane2_t *)(y + ((size_t)n * C + c) * S + v) = q; }
     }
 }
 template <int B> static void mx_to_f32(const void *x, int N, int C, size_t S, float *y) {
     const size_t n = (size_t)N * mx_nb(C) * S; if (!n) return;
-    if (cvt_pairs(C, S)) mx_to_f32_k<B, 2><<<rows_grid(N, mx_nb(C), (S + 1) / 2), 256>>>((const uint8_t *)x, y, N, C, S);
-    else if (cvt_stream(y, N, C, S)) mx_to_f32_k<B, 1, true><<<rows_grid(N, mx_nb(C), S), 256>>>((const uint8_t *)x, y, N, C, S);
+    if (cvt_pairs(C, S)) mx_to_f32_pairs_k<B><<<rows_grid(N, mx_nb(C), (S + 1) / 2), 256>>>((const uint8_t *)x, y, N, C, S);
+    else if (cvt_stream(y, N, C, S)) mx_to_f32_k<B, true><<<rows_grid(N, mx_nb(C), S), 256>>>((const uint8_t *)x, y, N, C, S);
     else mx_to_f32_k<B><<<rows_grid(N, mx_nb(C), S), 256>>>((const uint8_t *)x, y, N, C, S);
     MICK();
 }
