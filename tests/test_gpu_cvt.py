@@ -398,3 +398,17 @@ def test_converters_planes_past_the_cache(gpu, bits, S):
     dz = DevBuf(x.nbytes)
     (lib.lp_mx8_to_f32 if bits == 8 else lib.lp_mx4_to_f32)(dq.ptr, 1, 32, S, dz.ptr)
     assert np.array_equal(dz.to_numpy(np.uint32, x.shape), orc.mx_to_f32(bits, want, 1, 32, S).view(np.uint32))
+
+
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("Cc,S", [(16, 1 << 22), (16, (1 << 22) - 32), (12, 5592416)])
+def test_converters_narrow_planes_past_the_cache(gpu, bits, Cc, S):
+    """Blocks of 16 channels: 256 MB of planes take the streamed form, a line less the two-voxel one: codes, scales and decoded values are the oracle's."""
+    rng = np.random.default_rng(bits + Cc)
+    x = np.resize(wild(rng, (1, 16, 65537)).reshape(-1), Cc * S).reshape(1, Cc, S)
+    dq = to_mx(bits, x)
+    got, want = dq.to_numpy(np.uint8), orc.f32_to_mx(bits, x, 1, Cc, S)
+    assert np.array_equal(got, want)
+    dz = DevBuf(x.nbytes)
+    (lib.lp_mx8_to_f32 if bits == 8 else lib.lp_mx4_to_f32)(dq.ptr, 1, Cc, S, dz.ptr)
+    assert np.array_equal(dz.to_numpy(np.uint32, x.shape), orc.mx_to_f32(bits, want, 1, Cc, S).view(np.uint32))

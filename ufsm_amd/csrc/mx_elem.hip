@@ -41,18 +41,22 @@ static dim3 rows_grid(int N, int nb, size_t S) {
 }
 // ---- fp32 / 16-bit planes [n][C][S] -> MX (src/lp_mx_cvt.cu:9-19) ----
 // The converters are bound by the rate at which a wavefront's many plane streams reach memory. Two forms beside the plain one (a voxel per thread,
-// cached accesses), both with its bytes; measured e4m3, to MX / from MX, each entry us:
-// * V 2, blocks of at most 16 channels: a thread has few values in flight, so it takes two neighbouring voxels (8-byte accesses at any 4-byte address).
-//   4 channels, 3 x 2000003: 48 / 43 -> 33 / 31; 2 x 96^3: 16.7 / 15.3 -> 12.3 / 11.5; 8 channels, 10000003: 94 / 106 -> 76 / 90; 16 channels, 64^3:
-//   5.9 / 6.3 -> 4.9 / 5.7, 2 x 999999: 26.7 / 27.9 -> 25.3 / 27.6. At 32^3 (4 channels) 3.0 / 2.6 and 3.2 / 2.7, hence from 2^17 voxels. Blocks of 32 channels
-//   have 32 streams already and lose (32 channels, 2 x 128^3: 132 / 142 -> 149 / 140), and four voxels are no faster than two.
-// * STREAM: planes past the 256 MB of the last-level cache are read and written past it where a wavefront's accesses are whole 128-byte lines (S a multiple of
-//   32, aligned planes): 32 channels, 2 x 128^3: 132 / 142 -> 122 / 115 (a large copy reaches 5.3 TB/s, these 5.5 / 5.9). Lines shared by two
-//   wavefronts lose their meeting in the cache (64 channels, 999999: 54 / 71 -> 61 / 101), and planes that fit the cache are found there (64 channels, 96^3
-//   to MX: 41 -> 47).
-constexpr int CVT_BW = 16;         // widest block of the two-voxel form
+// cached accesses), both with its bytes. Figures: us to MX / from MX, plain -> the form, e4m3 and e2m1.
+// * Pairs, blocks of at most 16 channels: a thread has few values in flight, so it takes two neighbouring voxels (8-byte accesses at any 4-byte address).
+//   4 channels, 2 x 96^3: 16.5 / 15.5 -> 9.1 / 9.1 and 15.1 / 15.5 -> 7.9 / 8.5; 3 x 2000003: 47 / 44 -> 26 / 25 and 45 / 43 -> 22 / 22; 8 channels, 10000003:
+//   104 / 98 -> 73 / 90 and 83 / 107 -> 66 / 85; 16 channels, 64^3: 5.7 / 6.4 -> 4.6 / 5.5 and 5.7 / 6.4 -> 4.8 / 5.6; 2 x 999999: 26.5 / 28.7 -> 24.9 / 27.4 and
+//   23.8 / 25.6 -> 23.6 / 24.4. With 16 channels and planes of 128 MB and more the two are within 6 % of each other, either way. At 32^3 both are a launch
+//   (4 channels: 4.1 / 3.9 and 4.1 / 4.0), hence from 2^17 voxels. Blocks of 32 channels have 32 streams already and lose (2 x 128^3, e4m3: 132 / 142 -> 149 / 140),
+//   and four voxels are no faster than two.
+// * STREAM, blocks of 16 and 32 channels: planes past the 256 MB of the last-level cache are read and written past it where a wavefront's accesses are
+//   whole 128-byte lines (S a multiple of 32, aligned planes). 32 channels, 2 x 128^3: 135 / 146 -> 123 / 116 and 123 / 126 -> 112 / 111 (a large copy reaches
+//   5.3 TB/s, these 5.5 / 5.9); to MX and back 294 -> 240 and 270 -> 222; 1 x 128^3, the smallest: 151 -> 122 and 142 -> 111; 16 channels, 2 x 128^3: 153 -> 124 and
+//   146 -> 119 (pairs: 160 and 142). Blocks of 8 channels stay pairs (305 MB, to MX and back: 161 and 158, streamed 172 and 165). Lines shared by two
+//   wavefronts lose their meeting in the cache (64 channels, 999999: 53 / 68 -> 61 / 100 and 48 / 59 -> 55 / 98), and planes that fit the cache are found there (64
+//   channels, 96^3 to MX: 43 -> 46 and 39 -> 44).
+constexpr int CVT_BW = 16;         // widest block of the pairs
 static bool cvt_pairs(int C, size_t S) { return mx_bw(C) <= CVT_BW && S >= (size_t)1 << 17; }
-static bool cvt_stream(const void *planes, int N, int C, size_t S) { return S % 32 == 0 && !((uintptr_t)planes & 127) && (size_t)N * C * S * 4 >= (size_t)256 << 20; }
+static bool cvt_stream(const void *planes, int N, int C, size_t S) { return mx_bw(C) > 8 && S % 32 == 0 && !((uintptr_t)planes & 127) && (size_t)N * C * S * 4 >= (size_t)256 << 20; }
 typedef float plane2_t __attribute__((ext_vector_type(2), aligned(4)));      // two neighbouring voxels of a plane (any element's address)
 template <int B, typename TI, bool STREAM = false>
 __global__ void __launch_bounds__(256) f32_to_mx_k(const TI *x, uint8_t *y, int N, int C, size_t S) {
@@ -94,8 +98,8 @@ __global__ void __launch_bounds__(256) f32_to_mx_pairs_k(const float *x, uint8_t
 template <int B> static void f32_to_mx(const float *x, int N, int C, size_t S, void *y) {
     const size_t n = (size_t)N * mx_nb(C) * S;
     if (!n) return;
-    if (cvt_pairs(C, S)) f32_to_mx_pairs_k<B><<<rows_grid(N, mx_nb(C), (S + 1) / 2), 256>>>(x, (uint8_t *)y, N, C, S);
-    else if (cvt_stream(x, N, C, S)) f32_to_mx_k<B, float, true><<<rows_grid(N, mx_nb(C), S), 256>>>(x, (uint8_t *)y, N, C, S);
+    if (cvt_stream(x, N, C, S)) f32_to_mx_k<B, float, true><<<rows_grid(N, mx_nb(C), S), 256>>>(x, (uint8_t *)y, N, C, S);
+    else if (cvt_pairs(C, S)) f32_to_mx_pairs_k<B><<<rows_grid(N, mx_nb(C), (S + 1) / 2), 256>>>(x, (uint8_t *)y, N, C, S);
     else f32_to_mx_k<B, float><<<rows_grid(N, mx_nb(C), S), 256>>>(x, (uint8_t *)y, N, C, S);
     MICK();
 }
@@ -150,8 +154,8 @@ __global__ void __launch_bounds__(256) mx_to_f32_pairs_k(const uint8_t *x, float
 }
 template <int B> static void mx_to_f32(const void *x, int N, int C, size_t S, float *y) {
     const size_t n = (size_t)N * mx_nb(C) * S; if (!n) return;
-    if (cvt_pairs(C, S)) mx_to_f32_pairs_k<B><<<rows_grid(N, mx_nb(C), (S + 1) / 2), 256>>>((const uint8_t *)x, y, N, C, S);
-    else if (cvt_stream(y, N, C, S)) mx_to_f32_k<B, true><<<rows_grid(N, mx_nb(C), S), 256>>>((const uint8_t *)x, y, N, C, S);
+    if (cvt_stream(y, N, C, S)) mx_to_f32_k<B, true><<<rows_grid(N, mx_nb(C), S), 256>>>((const uint8_t *)x, y, N, C, S);
+    else if (cvt_pairs(C, S)) mx_to_f32_pairs_k<B><<<rows_grid(N, mx_nb(C), (S + 1) / 2), 256>>>((const uint8_t *)x, y, N, C, S);
     else mx_to_f32_k<B><<<rows_grid(N, mx_nb(C), S), 256>>>((const uint8_t *)x, y, N, C, S);
     MICK();
 }
