@@ -94,6 +94,9 @@ void mi_conv_split(int tiles);
    straight from the stored tensor when the launch has enough output voxels to fill the device, else the general kernel (staged halo);
    0: always the general kernel; 1: the direct kernel whenever its operands allow it. The results are the same conv either way. */
 void mi_conv_s2_direct(int mode);
+/* Extension: up to how many tiles (64 voxels x 32 output channels, of the whole tensor) the calling thread's 3x3x3 convs may run on the kernel that splits
+   the K range over a workgroup's wavefronts. -1 (default): the measured limits; 0: never. The same conv either way, its fp32 sums in another order. */
+void mi_conv_thin(int tiles);
 /* 1x1x1 head with eight outputs on whole 32-channel blocks: where its 8 x 32 products per voxel run. mode 1: the matrix pipe (batched 4 x 4 x 1
    fp32 outer products, one product per accumulator and step, in channel order), 0: fused multiply-adds on the vector ALUs, -1: the default
    (1, or the environment's MI_HEAD_MFMA). The two give the same bits; the setting is the calling thread's. No counterpart in the reference. */

@@ -15,6 +15,14 @@ pytestmark = pytest.mark.gpu
 GRID = np.array([0, .5, 1, 1.5, 2, 3, 4, 6], np.float32)
 
 
+@pytest.fixture(autouse=True)
+def staged_kernels():
+    """This file's convs run on the staged kernels, also those small enough for the kernel that splits K over wavefronts (tests/test_gpu_thin.py has its cases)."""
+    lib.mi_conv_thin(0)
+    yield
+    lib.mi_conv_thin(-1)
+
+
 def rand_case(rng, N, Ci, Co, S):
     x = rng.standard_normal((N, Ci, S)).astype(np.float32)
     w = (rng.standard_normal((Co, Ci, 27)) * np.sqrt(2.0 / (Ci * 27))).astype(np.float32)       # Kaiming normal (src/unet.c:588-607)
@@ -63,8 +71,8 @@ def test_wide_kernel_exact(gpu, slice_split, bits, N, Ci, Co, D, H, W):
 
 @pytest.mark.parametrize("bits,N,Ci,Co,D,H,W", WIDE_SHAPES[:3] + WIDE_SHAPES[5:])
 def test_few_tiles_default_dispatch(gpu, bits, N, Ci, Co, D, H, W):
-    """The default rule for launches of very few tiles (the coarsest levels): one channel tile and two planes per workgroup on the general
-    kernel instead of the wide kernel's slices."""
+    """The staged kernels' rule for launches of very few tiles (past the K-split kernel's range): one channel tile and two planes per workgroup on the
+    general kernel instead of the wide kernel's slices."""
     rng = np.random.default_rng(Ci * 19 + Co + D * 5 + bits)
     S = D * H * W
     x, w, b = exact_case(rng, N, Ci, Co, S)

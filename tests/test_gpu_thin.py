@@ -1,12 +1,11 @@
 """The K-split kernel of conv launches with few output voxels: exact operands equal the oracle byte for byte in every output type at the edges of its
-tiles (64 voxels x 32 channels, eight wavefronts over the K pairs), statistics are the oracle's and identical run to run, and a launch just past its
-range gives the bytes of the staged kernels."""
+tiles (64 voxels x 32 channels, eight wavefronts over the K pairs), statistics are the oracle's and identical run to run, split inputs and z-slabs included."""
 import numpy as np
 import pytest
 
 from ufsm_amd import lib, LP, DevBuf, shape5, gnp_t, split_t
 import orc
-from gpuutil import to_mx, mx_bytes
+from gpuutil import to_mx, mx_bytes, dev_gn
 from test_gpu_conv import exact_case, rand_case, gpu_conv
 
 pytestmark = pytest.mark.gpu
@@ -27,7 +26,11 @@ def test_few_voxels(gpu, bits, N, Ci, Co, D, H, W, stride):
     xq = orc.f32_to_mx(bits, x, N, Ci, S)
     for ydt in (0, 2, xdt):
         want, _ = orc.conv3(xq, xdt, N, Ci, D, H, W, w, b, Co, ydt, cbits=bits, stride=stride, acc64=1)
-        got, _ = gpu_conv(xq, xdt, N, Ci, D, H, W, w, b, Co, ydt, cbits=bits, stride=stride)
+        lib.mi_conv_thin(512)                                     # (the kernel is right for shapes the default rule leaves to others, too)
+        try:
+            got, _ = gpu_conv(xq, xdt, N, Ci, D, H, W, w, b, Co, ydt, cbits=bits, stride=stride)
+        finally:
+            lib.mi_conv_thin(-1)
         assert "conv3_thin_k" in lib.mi_last_kernel().decode(), lib.mi_last_kernel().decode()
         assert np.array_equal(got, want), ydt
     if stride == 2:
@@ -147,3 +150,59 @@ def test_network_in_slabs(gpu, bits, dims, slab):
     assert [n for n, _ in got[0][1]] == [n for n, _ in got[1][1]]
     for (name, a), (_, b) in zip(got[0][1], got[1][1]):
         assert np.array_equal(a, b), name
+
+
+@pytest.mark.parametrize("bits,Cu,Cs,Co", [(8, 64, 96, 64), (4, 96, 32, 128), (8, 256, 128, 128)])
+def test_split_inputs(gpu, bits, Cu, Cs, Co):
+    """[x | x2] read as stored (exact operands: the oracle's bytes), and [2x upsampled coarse | skip] with both GroupNorms (the staged
+    kernels' result but for the order of sums)."""
+    rng = np.random.default_rng(Cu + Cs)
+    N, D, H, W, G, dt = 2, 6, 4, 10, 8, 3 if bits == 8 else 4
+    S = D * H * W
+    x, w, b = exact_case(rng, N, Cu + Cs, Co, S)
+    qu, qs = orc.f32_to_mx(bits, np.ascontiguousarray(x[:, :Cu]), N, Cu, S), orc.f32_to_mx(bits, np.ascontiguousarray(x[:, Cu:]), N, Cs, S)
+    want, _ = orc.conv3(qu, dt, N, Cu + Cs, D, H, W, w, b, Co, dt, cbits=bits, x2=qs, c_split=Cu, acc64=1)
+    got, _ = gpu_conv(qu, dt, N, Cu + Cs, D, H, W, w, b, Co, dt, cbits=bits, x2=qs, c_split=Cu)
+    assert "conv3_thin_k" in lib.mi_last_kernel().decode() and np.array_equal(got, want)
+    xu = rng.standard_normal((N, Cu, S // 8)).astype(np.float32)
+    _, w, b = rand_case(rng, N, Cu + Cs, Co, S)
+    qu = orc.f32_to_mx(bits, xu, N, Cu, S // 8)
+    g = [[rng.uniform(0.5, 1.5, c).astype(np.float32), rng.uniform(-0.3, 0.3, c).astype(np.float32), rng.uniform(-0.2, 0.2, N * G).astype(np.float32), rng.uniform(0.7, 1.4, N * G).astype(np.float32)] for c in (Cu, Cs)]
+    res = []
+    for thin in (-1, 0):
+        lib.mi_conv_thin(thin)
+        try:
+            res.append(gpu_conv(qu, dt, N, Cu + Cs, D, H, W, w, b, Co, 0, cbits=bits, x2=qs, c_split=Cu, up=1, gp=dev_gn(*g[0], G), gp2=dev_gn(*g[1], G))[0])
+        finally:
+            lib.mi_conv_thin(-1)
+        assert ("conv3_thin_k" in lib.mi_last_kernel().decode()) == (thin < 0)
+    assert np.abs(res[0] - res[1]).max() / np.abs(res[1]).max() < 2e-4      # (the same staged operands: fp32 sums in another order)
+
+
+def test_one_memo_id_on_both_kernels(gpu):
+    """Prepared weights are kept per id and layout: one id alternating between a launch of this kernel, a staged one and a thread's other choice gives the
+    bytes of weights prepared per call."""
+    rng = np.random.default_rng(3)
+    Ci, Co = 128, 64
+    w = (rng.standard_normal((Co, Ci, 27)) * 0.03).astype(np.float32)
+    dw, db = DevBuf.from_numpy(w), DevBuf.from_numpy(rng.standard_normal(Co).astype(np.float32))
+    dims = [(8, 8, 8), (24, 24, 24)]
+    xs = [to_mx(8, rng.standard_normal((1, Ci, D * H * W)).astype(np.float32)) for D, H, W in dims]
+
+    def conv(i, wkey, thin):
+        D, H, W = dims[i]
+        sp, y = split_t(), DevBuf(mx_bytes(8, 1, Co, D * H * W))
+        sp.wkey = wkey
+        lib.mi_conv_thin(thin)
+        try:
+            assert lib.lp_conv_fwd_f8(xs[i].ptr, 3, shape5(1, Ci, D, H, W), dw.ptr, db.ptr, Co, y.ptr, 3, gnp_t(), None, 0, sp) == 0
+        finally:
+            lib.mi_conv_thin(-1)
+        LP.check()
+        return y.to_numpy(np.uint8), lib.mi_last_kernel().decode().split("<")[0]
+    ref = {(i, t): conv(i, 0, t) for i in (0, 1) for t in (-1, 0)}
+    assert ref[0, -1][1] == "conv3_thin_k" and all(ref[k][1] != "conv3_thin_k" for k in ((0, 0), (1, -1), (1, 0)))
+    for k in [(0, -1), (1, -1), (0, 0), (0, -1), (1, 0), (1, -1), (0, -1)]:
+        y, name = conv(k[0], 77001, k[1])
+        assert name == ref[k][1] and np.array_equal(y, ref[k][0]), k
+    lib.lp_wmemo_clear()

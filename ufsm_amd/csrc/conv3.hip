@@ -341,6 +341,8 @@ static thread_local int g_x2_dt = 0;
 extern "C" void mi_conv_x2_dt(int dt) { g_x2_dt = dt == 3 || dt == 4 ? dt : 0; }
 static thread_local int g_s2d = -1;         // mi_conv_s2_direct: the calling thread's choice of stride-2 kernel (-1: by launch size)
 extern "C" void mi_conv_s2_direct(int mode) { g_s2d = mode; }
+static thread_local int g_thin = -1;        // mi_conv_thin: the calling thread's tile count up to which the K-split kernel takes a launch (-1: the default rule)
+extern "C" void mi_conv_thin(int tiles) { g_thin = tiles; }
 static int split_s2_env() { static int v = -1; if (v < 0) v = getenv("MI_CONV_SPLIT_S2") ? atoi(getenv("MI_CONV_SPLIT_S2")) : 1; return v; }      // tuning knob: 0 keeps four channel tiles
 static int conv_dispatch(const char *who, int fmt, int stride, const void *x, int xbf, shape5 xs, const float *w, const float *b, int cout, void *y, int ybf,
                          gnp_t gp, double *osum, int Go, split_t sp, const float *ep_a, const float *ep_b, int act) {
@@ -550,8 +552,8 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     // adds in the order of the whole tensor's conv and takes its statistics over the same runs, so that inference in slabs gives its bytes
     static int thin_env = -1;
     if (thin_env < 0) thin_env = getenv("MI_CONV_THIN") ? atoi(getenv("MI_CONV_THIN")) : 256;      // tuning knob: that tile count (0: never)
-    const size_t thin_max = fmt == 8 && a.nbt >= 8 ? 2 * (size_t)thin_env : fmt == 4 && coarse && a.nbt <= 2 ? (size_t)thin_env / 4 : (size_t)thin_env;
-    a.thin = thin_env > 0 && !a.row && !a.areg && !s2d && !act && a.wide && cout > 16 && !(osum && (cout / Go) % 4) && !sp.zlo && !sp.zhi && g_split < 0 && g_s2d < 0 && N <= 65535 &&
+    const size_t thin_max = g_thin >= 0 ? (size_t)g_thin : fmt == 8 && a.nbt >= 8 ? 2 * (size_t)thin_env : fmt == 4 && coarse && a.nbt <= 2 ? (size_t)thin_env / 4 : (size_t)thin_env;
+    a.thin = thin_max > 0 && !a.row && !a.areg && !s2d && !act && a.wide && cout > 16 && !(osum && (cout / Go) % 4) && !sp.zlo && !sp.zhi && g_split < 0 && g_s2d < 0 && N <= 65535 &&
              (size_t)D * H * W * 32 < ((size_t)1 << 31) && mi_thin_tiles(Dr, Ho, Wo) * nmt_all * N <= thin_max;
     if (a.thin) { big = false; MT = 1; NT = 2; a.CB = a.nbt; }
     size_t smem = a.thin ? MI_THIN_LDS : a.row1 ? (size_t)10 * 352 * (RB + 4) : a.row ? (size_t)2 * 2048 * (RB + 4) : a.areg ? (size_t)2 * ((TT + 63) / 64 * 64) * (RB + 4) : big ? (size_t)4 * MT * (WTILE + 256) + (size_t)3 * ((TT + 63) / 64 * 64) * (RB + 4) + (size_t)(((27 * a.nbt + 1) >> 1) + 2) * 32 : lds_bytes(a.CB);
