@@ -1,5 +1,6 @@
 """The K-split kernel of conv launches with few output voxels: exact operands equal the oracle byte for byte in every output type at the edges of its
-tiles (64 voxels x 32 channels, eight wavefronts over the K pairs), statistics are the oracle's and identical run to run, split inputs and z-slabs included."""
+tiles (64 voxels x 32 channels, eight wavefronts over the K pairs), statistics are the oracle's and identical run to run, split inputs and z-slabs included, and
+launches on both sides of its range's edges give the bytes of the staged kernels."""
 import numpy as np
 import pytest
 
@@ -206,3 +207,30 @@ def test_one_memo_id_on_both_kernels(gpu):
         y, name = conv(k[0], 77001, k[1])
         assert name == ref[k][1] and np.array_equal(y, ref[k][0]), k
     lib.lp_wmemo_clear()
+
+# (bits, Ci, Co, stride, [(N, D, H, W, the kernel takes it)]): the last launch of a limit and the one of a plane more
+EDGES = [(8, 64, 64, 1, [(1, 32, 16, 16, True), (1, 33, 16, 16, False)]), (8, 256, 128, 1, [(1, 32, 16, 16, True), (1, 33, 16, 16, False)]),
+         (4, 64, 128, 1, [(1, 16, 16, 16, True), (1, 17, 16, 16, False)]), (4, 256, 128, 1, [(1, 16, 16, 16, True), (1, 17, 16, 16, False)]),
+         (4, 32, 64, 1, [(2, 16, 16, 16, True), (1, 33, 16, 16, False)]), (4, 32, 128, 1, [(1, 4, 4, 4, False), (1, 11, 13, 13, False)]),
+         (4, 32, 32, 2, [(1, 16, 16, 16, False), (2, 8, 12, 16, False)]), (8, 64, 64, 2, [(2, 32, 32, 32, True), (2, 33, 32, 32, False)]),
+         (8, 256, 256, 2, [(1, 16, 32, 32, True), (2, 24, 24, 24, True), (1, 32, 32, 32, False)])]
+
+
+@pytest.mark.parametrize("bits,Ci,Co,stride,launches", EDGES)
+def test_edges_of_the_range(gpu, bits, Ci, Co, stride, launches):
+    """The default choice at its limits, and exact operands: both kernels give the same bytes."""
+    rng = np.random.default_rng(Ci + Co + stride)
+    dt = 3 if bits == 8 else 4
+    for N, D, H, W, thin in launches:
+        x, w, b = exact_case(rng, N, Ci, Co, D * H * W)
+        xq = orc.f32_to_mx(bits, x, N, Ci, D * H * W)
+        got, name = [], []
+        for limit in (-1, 0, 4096):
+            lib.mi_conv_thin(limit)
+            try:
+                got.append(gpu_conv(xq, dt, N, Ci, D, H, W, w, b, Co, dt, cbits=bits, stride=stride)[0])
+            finally:
+                lib.mi_conv_thin(-1)
+            name.append("conv3_thin_k" in lib.mi_last_kernel().decode())
+        assert name == [thin, False, True], (N, D, H, W, name)
+        assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])

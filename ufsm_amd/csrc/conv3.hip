@@ -542,17 +542,22 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     if (a.row && nmt_all >= 2) MT = 1;
     if (a.row) { a.areg = false; a.CB = a.nbt; }
     // few output voxels: the K range split over a workgroup's wavefronts (conv3_thin_k). The staged kernels' time hardly depends on how many workgroups a
-    // launch has until every CU has one, this one's grows with them once it has more than one workgroup per CU. Measured per call with the statistics,
-    // e4m3, 1 x 8^3 / 1 x 16^3 / 2 x 16^3: 64 -> 64 24.6 / 24.7 / 25.1 us on the general kernel, 10.4 / 10.9 / 11.1 here (16 / 128 / 256 tiles of 64
-    // voxels x 32 channels); 192 -> 64 38 / 39 / 39 us on the wide kernel, 13.4 / 14.1 / 14.7; 128 -> 128 20.8 / 21.6 / 22.0 against 12.1 / 13.8 / 21.2 (512
-    // tiles); 256 -> 256 35 / 37 / 38 against 16.7 / 29.0 / 48.5 (1024 tiles); 384 -> 128 47 / 48 / 50 against 18.3 / 20.2 / 33.0 (512 tiles). Hence
-    // 256 tiles, 512 in e4m3 from eight input blocks on; e2m1 of one or two blocks against the coarse form is even (64 -> 128 at 1 x 11 x 13^2: 11.7 and
-    // 12.1 us) and keeps that from 64 tiles on. The row
+    // launch has until every CU has one, this one's grows with its tiles (64 voxels x 32 channels) once each CU has one. Kernel time, us, the other kernel
+    // against this one. e4m3, stride 1, 1 x 8^3 / 1 x 16^3 / 2 x 16^3: 64 -> 64 21.6 / 21.8 / 21.9 against 7.8 / 8.2 / 8.8 (16 / 128 / 256 tiles); 192 -> 64 35 / 35 / 36
+    // against 11.4 / 12.6 / 13.0; 64 -> 128 12.9 / 13.0 / 12.9 against 8.0 / 9.7 / 14.4 (512 tiles); 128 -> 128 18.5 / 18.8 / 19.1 against 9.6 / 11.1 / 17.2 (512);
+    // 256 -> 256 31 / 32 / 34 against 12.8 / 23.5 / 43.1 (1024); 384 -> 128 45 / 45 / 46 against 15.4 / 17.0 / 29.6 (512). e2m1: 64 -> 64 at 2 x 16^3 16.9 against 8.5,
+    // 64 -> 128 at 1 x 16^3 9.4 against 8.5 and at 2 x 16^3 9.6 against 14.0. Hence 256 tiles, and 512 from eight input blocks of e4m3 on. Stride 2, 32 -> 32 at
+    // 16^3 8.6 against 7.0 and 64 -> 64 from 2 x 32^3 (256 tiles) 12.0 against 8.9; with eight blocks it depends on whether the general kernel's workgroups
+    // fit the CUs at once: 256 -> 256 from 1 x 32^3 (512 tiles, 256 of its workgroups) 32.8 against 34.9, 256 -> 128 from 2 x 32^3 32.7 against 38.6, 256 -> 256 from
+    // 2 x 24^3 (432 tiles, 384 of its workgroups) 60.6 against 33.4. One input block of e2m1 has fifteen pairs, too few to split: against the coarse form 32 ->
+    // 128 at 1 x 8^3 7.1 against 7.4 and at 1 x 16^3 7.3 against 7.8, at stride 2 32 -> 32 from 1 x 16^3 6.4 against 6.9; these keep the general kernel. The row
     // kernels' and the one-block, one-tile kernel's launches stay theirs. The tiles counted are the whole tensor's (Dr planes), not a z-range's: a slab
     // adds in the order of the whole tensor's conv and takes its statistics over the same runs, so that inference in slabs gives its bytes
     static int thin_env = -1;
     if (thin_env < 0) thin_env = getenv("MI_CONV_THIN") ? atoi(getenv("MI_CONV_THIN")) : 256;      // tuning knob: that tile count (0: never)
-    const size_t thin_max = g_thin >= 0 ? (size_t)g_thin : fmt == 8 && a.nbt >= 8 ? 2 * (size_t)thin_env : fmt == 4 && coarse && a.nbt <= 2 ? (size_t)thin_env / 4 : (size_t)thin_env;
+    const bool short_k = fmt == 4 && a.nbt == 1 && (coarse || stride == 2);
+    const bool one_round = stride == 2 && (size_t)((Wo + 15) / 16) * ((Ho + 7) / 8) * ((Do + TZ - 1) / TZ) * (nmt_all / MT) * N <= 256;      // (the general kernel's workgroups)
+    const size_t thin_max = g_thin >= 0 ? (size_t)g_thin : short_k ? 0 : fmt == 8 && a.nbt >= 8 && !one_round ? 2 * (size_t)thin_env : (size_t)thin_env;
     a.thin = thin_max > 0 && !a.row && !a.areg && !s2d && !act && a.wide && cout > 16 && !(osum && (cout / Go) % 4) && !sp.zlo && !sp.zhi && g_split < 0 && g_s2d < 0 && N <= 65535 &&
              (size_t)D * H * W * 32 < ((size_t)1 << 31) && mi_thin_tiles(Dr, Ho, Wo) * nmt_all * N <= thin_max;
     if (a.thin) { big = false; MT = 1; NT = 2; a.CB = a.nbt; }
