@@ -210,7 +210,7 @@ def test_one_memo_id_on_both_kernels(gpu):
 
 # (bits, Ci, Co, stride, [(N, D, H, W, the kernel takes it)]): the last launch of a limit and the one of a plane more
 EDGES = [(8, 64, 64, 1, [(1, 32, 16, 16, True), (1, 33, 16, 16, False)]), (8, 256, 128, 1, [(1, 32, 16, 16, True), (1, 33, 16, 16, False)]),
-         (4, 64, 128, 1, [(1, 16, 16, 16, True), (1, 17, 16, 16, False)]), (4, 256, 128, 1, [(1, 16, 16, 16, True), (1, 17, 16, 16, False)]),
+         (4, 64, 128, 1, [(1, 8, 8, 16, True), (1, 9, 8, 16, False)]), (8, 32, 128, 1, [(1, 8, 8, 16, True), (1, 9, 8, 16, False)]), (4, 256, 128, 1, [(1, 16, 16, 16, True), (1, 17, 16, 16, False)]),
          (4, 32, 64, 1, [(2, 16, 16, 16, True), (1, 33, 16, 16, False)]), (4, 32, 128, 1, [(1, 4, 4, 4, False), (1, 11, 13, 13, False)]),
          (4, 32, 32, 2, [(1, 16, 16, 16, False), (2, 8, 12, 16, False)]), (8, 64, 64, 2, [(2, 32, 32, 32, True), (2, 33, 32, 32, False)]),
          (8, 256, 256, 2, [(1, 16, 32, 32, True), (2, 24, 24, 24, True), (1, 32, 32, 32, False)])]

@@ -545,19 +545,22 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     // launch has until every CU has one, this one's grows with its tiles (64 voxels x 32 channels) once each CU has one. Kernel time, us, the other kernel
     // against this one. e4m3, stride 1, 1 x 8^3 / 1 x 16^3 / 2 x 16^3: 64 -> 64 21.6 / 21.8 / 21.9 against 7.8 / 8.2 / 8.8 (16 / 128 / 256 tiles); 192 -> 64 35 / 35 / 36
     // against 11.4 / 12.6 / 13.0; 64 -> 128 12.9 / 13.0 / 12.9 against 8.0 / 9.7 / 14.4 (512 tiles); 128 -> 128 18.5 / 18.8 / 19.1 against 9.6 / 11.1 / 17.2 (512);
-    // 256 -> 256 31 / 32 / 34 against 12.8 / 23.5 / 43.1 (1024); 384 -> 128 45 / 45 / 46 against 15.4 / 17.0 / 29.6 (512). e2m1: 64 -> 64 at 2 x 16^3 16.9 against 8.5,
-    // 64 -> 128 at 1 x 16^3 9.4 against 8.5 and at 2 x 16^3 9.6 against 14.0. Hence 256 tiles, and 512 from eight input blocks of e4m3 on. Stride 2, 32 -> 32 at
+    // 256 -> 256 31 / 32 / 34 against 12.8 / 23.5 / 43.1 (1024); 384 -> 128 45 / 45 / 46 against 15.4 / 17.0 / 29.6 (512). e2m1: 64 -> 64 at 2 x 16^3 16.9 against 8.5.
+    // Hence 256 tiles, and 512 from eight input blocks of e4m3 on. Stride 2, 32 -> 32 at
     // 16^3 8.6 against 7.0 and 64 -> 64 from 2 x 32^3 (256 tiles) 12.0 against 8.9; with eight blocks it depends on whether the general kernel's workgroups
     // fit the CUs at once: 256 -> 256 from 1 x 32^3 (512 tiles, 256 of its workgroups) 32.8 against 34.9, 256 -> 128 from 2 x 32^3 32.7 against 38.6, 256 -> 256 from
-    // 2 x 24^3 (432 tiles, 384 of its workgroups) 60.6 against 33.4. One input block of e2m1 has fifteen pairs, too few to split: against the coarse form 32 ->
-    // 128 at 1 x 8^3 7.1 against 7.4 and at 1 x 16^3 7.3 against 7.8, at stride 2 32 -> 32 from 1 x 16^3 6.4 against 6.9; these keep the general kernel. The row
+    // 2 x 24^3 (432 tiles, 384 of its workgroups) 60.6 against 33.4. Against the coarse form's one channel tile a short K gains little, and the statistics'
+    // reduction reads more records: one block of e4m3 or two of e2m1 are even with it from 64 tiles on (both kernels of a call: e4m3 32 -> 256 at 1 x 4^3
+    // 12.4 against 11.3, 1 x 8^3 (64 tiles) 12.5 and 12.4, 1 x 11 x 13^2 (240) 13.1 and 13.6; e2m1 64 -> 128 at 2 x 8^3 (64) 11.8 and 11.2, 1 x 12^3 (108) 12.1 and 13.1,
+    // 1 x 16^3 (256) 12.2 and 12.1) and stop there. One block of e2m1 has fourteen pairs, too few to split: 32 -> 128 at 1 x 8^3 7.1 against 7.4, at stride 2
+    // 32 -> 32 from 1 x 16^3 6.4 against 6.9; these keep the general kernel. The row
     // kernels' and the one-block, one-tile kernel's launches stay theirs. The tiles counted are the whole tensor's (Dr planes), not a z-range's: a slab
     // adds in the order of the whole tensor's conv and takes its statistics over the same runs, so that inference in slabs gives its bytes
     static int thin_env = -1;
     if (thin_env < 0) thin_env = getenv("MI_CONV_THIN") ? atoi(getenv("MI_CONV_THIN")) : 256;      // tuning knob: that tile count (0: never)
-    const bool short_k = fmt == 4 && a.nbt == 1 && (coarse || stride == 2);
+    const int kb = a.nbt * (fmt == 8 ? 2 : 1);                 // (K in bytes: halves of 16 per tap)
     const bool one_round = stride == 2 && (size_t)((Wo + 15) / 16) * ((Ho + 7) / 8) * ((Do + TZ - 1) / TZ) * (nmt_all / MT) * N <= 256;      // (the general kernel's workgroups)
-    const size_t thin_max = g_thin >= 0 ? (size_t)g_thin : short_k ? 0 : fmt == 8 && a.nbt >= 8 && !one_round ? 2 * (size_t)thin_env : (size_t)thin_env;
+    const size_t thin_max = g_thin >= 0 ? (size_t)g_thin : kb == 1 && (coarse || stride == 2) ? 0 : kb == 2 && coarse ? (size_t)thin_env / 4 : kb >= 16 && fmt == 8 && !one_round ? 2 * (size_t)thin_env : (size_t)thin_env;
     a.thin = thin_max > 0 && !a.row && !a.areg && !s2d && !act && a.wide && cout > 16 && !(osum && (cout / Go) % 4) && !sp.zlo && !sp.zhi && g_split < 0 && g_s2d < 0 && N <= 65535 &&
              (size_t)D * H * W * 32 < ((size_t)1 << 31) && mi_thin_tiles(Dr, Ho, Wo) * nmt_all * N <= thin_max;
     if (a.thin) { big = false; MT = 1; NT = 2; a.CB = a.nbt; }
