@@ -110,11 +110,12 @@ def test_slabs_equal_whole(gpu, bits, N, Ci, Co, D, H, W, slab, up, thin):
     assert np.allclose(s, sz, rtol=1e-12, atol=1e-9)
 
 
-# 128 channels and more: slices of 64 or 128 channels, or the coarse form, by the tiles of the whole tensor; last slabs of one to three planes
+# 128 channels and more: slices of 64 or 128 channels, or the coarse form, by the tiles of the whole tensor (thirteen input blocks: the general kernel's
+# slices); last slabs of one to three planes
 @pytest.mark.parametrize("bits,N,Ci,Co,D,H,W,slab,kern", [(8, 1, 128, 128, 32, 32, 32, 4, "conv3_wide_k"), (8, 1, 256, 256, 32, 32, 32, 8, "conv3_wide_k"), (8, 2, 64, 128, 32, 64, 64, 4, "conv3_wide_k"),
                                                           (8, 1, 64, 128, 18, 32, 32, 8, "conv3_mx_k"), (8, 1, 64, 64, 10, 16, 32, 4, "conv3_row_k"), (8, 2, 32, 32, 9, 16, 48, 4, "conv3_row1_k"),
                                                           (8, 1, 96, 32, 11, 16, 32, 4, "conv3_row_k"), (8, 1, 32, 32, 6, 8, 8, 4, "conv3_small_k"), (8, 1, 64, 128, 21, 32, 64, 4, "conv3_wide_k"),
-                                                          (4, 1, 192, 64, 25, 32, 32, 8, "conv3_wide_k"), (8, 1, 32, 128, 29, 24, 40, 4, "conv3_row1_k")])
+                                                          (8, 1, 416, 128, 16, 64, 128, 4, "conv3_mx_k"), (4, 1, 192, 64, 25, 32, 32, 8, "conv3_wide_k"), (8, 1, 32, 128, 29, 24, 40, 4, "conv3_row1_k")])
 def test_slabs_take_the_whole_tensors_kernel(gpu, bits, N, Ci, Co, D, H, W, slab, kern):
     (y, s, k), (yz, sz, kz) = conv_in_slabs(bits, N, Ci, Co, D, H, W, slab)
     assert kern + "<" in k and kern + "<" in kz, (k, kz)

@@ -432,13 +432,18 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     int MT = nmt_all <= 4 ? nmt_all : nmt_all % 4 == 0 ? 4 : nmt_all % 3 == 0 ? 3 : nmt_all % 2 == 0 ? 2 : 1;
     // channels per group not a multiple of 4 (80 channels in 8 groups): the statistics are per-channel records of one channel tile per workgroup
     if (osum && (cout / Go) % 4) MT = 1;
-    bool halved = false;
+    bool halved = false, halved_whole = false;
     {   // few tiles of 128 channels (the coarse levels): slices of 64 channels double the workgroups of the wide kernel
         static int split_env = -1;
         if (split_env < 0) split_env = getenv("MI_CONV_SPLIT") ? atoi(getenv("MI_CONV_SPLIT")) : 192;    // tuning knob: tile count below which the slices are halved (0: never)
         const int split = g_split >= 0 ? g_split : split_env;
-        if (stride == 1 && MT == 4 && nmt_all % 4 == 0 && Dr >= 3 &&
-            (size_t)((Wo + 15) / 16) * ((Ho + 7) / 8) * ((Do + 3) / 4) * (nmt_all / 4) * N < (size_t)split) { MT = 2; halved = true; }
+        // (a z-range's own tiles count where the wide kernel takes the launch, whose slices of either width add alike; the general kernel's do not)
+        auto few = [&](int d) { return (size_t)((Wo + 15) / 16) * ((Ho + 7) / 8) * ((d + 3) / 4) * (nmt_all / 4) * N < (size_t)split; };
+        if (stride == 1 && MT == 4 && nmt_all % 4 == 0 && Dr >= 3) {
+            halved_whole = few(Dr);
+            halved = few(a.wide && a.nbt <= 12 ? Do : Dr);
+            if (halved) MT = 2;
+        }
     }
     int NT = (stride == 1 && MT <= 2 && Dr >= 4) ? 4 : 2;
     // ... and when even the slices of 64 give fewer than 128 workgroups (256 -> 256 at 2 x 16^3: 64): one channel tile and two planes per workgroup
@@ -448,7 +453,7 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     {
         static int ce = -1;
         if (ce < 0) ce = getenv("MI_CONV_COARSE") ? atoi(getenv("MI_CONV_COARSE")) : 1;      // tuning knob: 0 keeps the wide kernel's slices of 64 there (as does a split forced through mi_conv_split)
-        if (ce && halved && g_split < 0 && (size_t)((Wo + 15) / 16) * ((Ho + 7) / 8) * ((Dr + 3) / 4) * (nmt_all / 2) * N < 128) { coarse = true; NT = 2; MT = 1; halved = false; }
+        if (ce && halved_whole && g_split < 0 && (size_t)((Wo + 15) / 16) * ((Ho + 7) / 8) * ((Dr + 3) / 4) * (nmt_all / 2) * N < 128) { coarse = true; NT = 2; MT = 1; halved = false; }
     }
     // stride 2 with few tiles (the coarse levels): one-plane tiles double the workgroups; with enough tiles the two-plane tile is faster
     // (measured: 128 -> 128 at 32^3 -> 16^3, N 2: 32 tiles 0.072 ms, 64 tiles 0.042 ms; 32 -> 32 at 128^3: 0.090 vs 0.120 ms)
