@@ -569,7 +569,7 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     const bool one_round = stride == 2 && (size_t)((Wo + 15) / 16) * ((Ho + 7) / 8) * ((Do + TZ - 1) / TZ) * (nmt_all / MT) * N <= 256;      // (the general kernel's workgroups)
     const size_t thin_max = g_thin >= 0 ? (size_t)g_thin : kb == 1 && (coarse || stride == 2) ? 0 : kb == 2 && coarse ? (size_t)thin_env / 4 : kb >= 16 && fmt == 8 && !one_round ? 2 * (size_t)thin_env : (size_t)thin_env;
     a.thin = thin_max > 0 && !a.row && !a.areg && !s2d && !act && a.wide && cout > 16 && !(osum && (cout / Go) % 4) && !sp.zlo && !sp.zhi && g_split < 0 && g_s2d < 0 && N <= 65535 &&
-             (size_t)D * H * W * 32 < ((size_t)1 << 31) && mi_thin_tiles(Dr, Ho, Wo) * nmt_all * N <= thin_max;
+             (size_t)D * H * W * 32 < ((size_t)1 << 31) && ((size_t)Dr * Ho * Wo + 63) / 64 * (size_t)nmt_all * N <= thin_max;
     if (a.thin) { big = false; MT = 1; NT = 2; a.CB = a.nbt; }
     size_t smem = a.thin ? MI_THIN_LDS : a.row1 ? (size_t)10 * 352 * (RB + 4) : a.row ? (size_t)2 * 2048 * (RB + 4) : a.areg ? (size_t)2 * ((TT + 63) / 64 * 64) * (RB + 4) : big ? (size_t)4 * MT * (WTILE + 256) + (size_t)3 * ((TT + 63) / 64 * 64) * (RB + 4) + (size_t)(((27 * a.nbt + 1) >> 1) + 2) * 32 : lds_bytes(a.CB);
     if (s2d) smem = 0;
@@ -601,7 +601,7 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     a.nmt_all = nmt_all; a.ncs = nmt_all / MT;
     a.ntx = a.row ? (Wo + 31) / 32 : (Wo + 15) / 16; a.nty = (Ho + 7) / 8; a.ntz = (Do + TZ - 1) / TZ;      // (the row kernel: 4 x 8 x 32 voxels per tile)
     a.ntiles = (unsigned)((size_t)a.ntx * a.nty * a.ntz * a.ncs * N);
-    if (a.thin) { a.ntx = (MI_THIN_ZG * Ho * Wo + 63) / 64; a.ntiles = (unsigned)(mi_thin_tiles(Do, Ho, Wo) * 2 * nmt_all * N); }      // (a statistics record per run of 32 voxels and channel tile)
+    if (a.thin) { a.ntx = (MI_THIN_ZG * Ho * Wo + 31) / 32; a.ntiles = (unsigned)(mi_thin_tiles(Do, Ho, Wo) * 2 * nmt_all * N); }      // (a statistics record per run of 32 voxels and channel tile)
     // ---- weights ----
     int npairs_all = 0;
     for (int b0 = 0; b0 < a.nbt; b0 += a.CB) npairs_all += (27 * (a.nbt - b0 < a.CB ? a.nbt - b0 : a.CB) + 1) >> 1;
