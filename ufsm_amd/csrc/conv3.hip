@@ -601,7 +601,7 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     a.nmt_all = nmt_all; a.ncs = nmt_all / MT;
     a.ntx = a.row ? (Wo + 31) / 32 : (Wo + 15) / 16; a.nty = (Ho + 7) / 8; a.ntz = (Do + TZ - 1) / TZ;      // (the row kernel: 4 x 8 x 32 voxels per tile)
     a.ntiles = (unsigned)((size_t)a.ntx * a.nty * a.ntz * a.ncs * N);
-    if (a.thin) { a.ntx = (MI_THIN_ZG * Ho * Wo + 31) / 32; a.ntiles = (unsigned)(mi_thin_tiles(Do, Ho, Wo) * 2 * nmt_all * N); }      // (a statistics record per run of 32 voxels and channel tile)
+    if (a.thin) a.ntiles = (unsigned)(mi_thin_tiles(Do, Ho, Wo) * 2 * nmt_all * N);      // (a statistics record per run of 32 voxels and channel tile)
     // ---- weights ----
     int npairs_all = 0;
     for (int b0 = 0; b0 < a.nbt; b0 += a.CB) npairs_all += (27 * (a.nbt - b0 < a.CB ? a.nbt - b0 : a.CB) + 1) >> 1;
