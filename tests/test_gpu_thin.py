@@ -96,11 +96,12 @@ def conv_in_slabs(bits, N, Ci, Co, D, H, W, slab, up=0):
     return res
 
 
-# whole tensors past the kernel's range whose slabs are inside it, and whole tensors inside it on planes of an odd voxel count and of one that is no
-# multiple of 32 voxels in four planes
+# whole tensors past the kernel's range whose slabs are inside it, and whole tensors inside it on planes of an odd voxel count, of one that is no
+# multiple of 32 voxels in four planes, and of so few that a run of 32 voxels holds several multiples of four planes
 @pytest.mark.parametrize("bits,N,Ci,Co,D,H,W,slab,up,thin", [(8, 1, 192, 64, 32, 32, 32, 4, 0, False), (8, 1, 192, 64, 32, 32, 32, 8, 1, False), (8, 2, 192, 64, 24, 24, 24, 4, 0, False),
                                                              (4, 1, 96, 96, 24, 24, 24, 4, 0, False), (8, 1, 64, 64, 12, 5, 7, 4, 0, True), (8, 2, 64, 128, 12, 10, 6, 4, 1, True),
-                                                             (8, 1, 256, 64, 10, 9, 5, 4, 0, True), (4, 1, 96, 64, 16, 6, 7, 8, 0, True)])
+                                                             (8, 1, 256, 64, 10, 9, 5, 4, 0, True), (4, 1, 96, 64, 16, 6, 7, 8, 0, True),
+                                                             (8, 1, 64, 64, 13, 1, 3, 4, 0, True), (8, 2, 64, 64, 18, 2, 1, 8, 0, True), (4, 3, 64, 64, 9, 3, 3, 4, 0, True)])
 def test_slabs_equal_whole(gpu, bits, N, Ci, Co, D, H, W, slab, up, thin):
     """A conv run in z-slabs takes the kernel of the whole tensor's conv and its statistics over the same voxels: the same bytes, and sums that differ
     only by the order in which doubles are added."""

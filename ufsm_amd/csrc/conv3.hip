@@ -601,7 +601,7 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     a.nmt_all = nmt_all; a.ncs = nmt_all / MT;
     a.ntx = a.row ? (Wo + 31) / 32 : (Wo + 15) / 16; a.nty = (Ho + 7) / 8; a.ntz = (Do + TZ - 1) / TZ;      // (the row kernel: 4 x 8 x 32 voxels per tile)
     a.ntiles = (unsigned)((size_t)a.ntx * a.nty * a.ntz * a.ncs * N);
-    if (a.thin) a.ntiles = (unsigned)(mi_thin_tiles(Do, Ho, Wo) * 2 * nmt_all * N);      // (a statistics record per run of 32 voxels and channel tile)
+    if (a.thin) { const thin_runs_t t = mi_thin_runs(a.zi0, Do, Ho, Wo); a.zc = t.off; a.ntx = t.step; a.nty = (int)t.recs; a.ntiles = (unsigned)(t.recs * nmt_all * N); }      // (its statistics records)
     // ---- weights ----
     int npairs_all = 0;
     for (int b0 = 0; b0 < a.nbt; b0 += a.CB) npairs_all += (27 * (a.nbt - b0 < a.CB ? a.nbt - b0 : a.CB) + 1) >> 1;
@@ -736,8 +736,8 @@ static size_t conv_scratch_bound(int fmt, const void *x2, int xbf, int ybf, shap
         if (!direct) need += al((size_t)N * ((C + 31) / 32) * S * 33);
         if (upseg) need += al((size_t)N * ((C + 31) / 32) * (S / 8) * 33);
     }
-    if (osum) need += al(tiles * 32 * 2 * sizeof(float));
-    (void)So;
+    const size_t thin_recs = (So + 63) / 64 * nmt_all * N <= (size_t)(g_thin > 1024 ? g_thin : 1024) ? mi_thin_runs(sp.Di ? sp.zi0 : 0, xs.d, xs.h, xs.w).recs * nmt_all * N : 0;      // (the K-split kernel's, 64 bytes each: a few more than its runs)
+    if (osum) need += al((tiles * 256 > thin_recs * 64 ? tiles * 256 : thin_recs * 64));
     return need;
 }
 // set-up, once per device with that device current: the array's address on this device, and the constant page at its head. mi_init calls it
