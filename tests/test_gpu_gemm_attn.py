@@ -160,6 +160,26 @@ def test_attention_four_wavefront_workgroups_and_the_shared_last_tile(gpu, nseq,
         assert d < 1e-5 and np.abs(l4[:, :, first:] - l1[:, :, first:]).max() < 1e-5 and np.isfinite(o4).all() and np.isfinite(l4).all()
 
 
+@pytest.mark.parametrize("nseq,S,H", [(1, 256, 2), (3, 257, 1), (2, 320, 1), (1, 64 * 7 + 32, 2), (1, 64 * 7 + 33, 3)])
+def test_attention_chosen_launch(gpu, nseq, S, H):
+    """The launch chosen by the sequence's length against one wavefront per query tile: odd and even numbers of key tiles, whole and partial last ones, with and
+    without a last query tile alone in its workgroup. The same bits, in a shared tile the same probabilities summed in another order (as above)."""
+    rng = np.random.default_rng(nseq * S + H + 2)
+    qk = normed_qkv(rng, nseq, S, H)
+    o, lse = gpu_attention(qk, nseq, S, H)
+    lib.at_fa8_waves(1)
+    try:
+        o1, l1 = gpu_attention(qk, nseq, S, H)
+    finally:
+        lib.at_fa8_waves(0)
+    first = (S - 1) // 32 * 32 if S > 256 and ((S + 31) // 32) % 4 == 1 else S
+    o, o1 = o.reshape(nseq, S, -1), o1.reshape(nseq, S, -1)
+    assert np.array_equal(o[:, :first], o1[:, :first]) and np.array_equal(lse[:, :, :first], l1[:, :, :first])
+    assert np.abs(o - o1).max() < 1e-5 * np.abs(o1).max() and np.abs(lse - l1).max() < 1e-5
+    wo, _ = orc.fa8_fwd(qk, nseq, S, H)
+    assert np.linalg.norm(o.reshape(wo.shape) - wo) <= 3e-3 * np.linalg.norm(wo)
+
+
 def test_attention_closed_forms(gpu):
     """q = 0: o is the mean of the quantised V over the S valid keys and lse = log2 S, exactly as on the oracle; rows of another
     sequence or of the padding must not leak in."""

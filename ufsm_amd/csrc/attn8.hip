@@ -9,6 +9,7 @@
 // accumulators to the B fragment of the second product in registers with no data exchange at all. The transposed V stores the tokens
 // of a block in the matching order.
 #include <hip/hip_fp16.h>
+#include <type_traits>
 #include "mx_dev.hpp"
 #include "../../include/mi_attn.h"
 
@@ -51,9 +52,9 @@ __global__ void __launch_bounds__(256) a8_rows_k(const __half *__restrict__ src_
     *(uint4 *)(dst + (size_t)hr * 64 + 16 * qt) = make_uint4(d_enc4_e4m3(v[0], v[1], v[2], v[3], e), d_enc4_e4m3(v[4], v[5], v[6], v[7], e), d_enc4_e4m3(v[8], v[9], v[10], v[11], e), d_enc4_e4m3(v[12], v[13], v[14], v[15], e));
     if (!(qt & 1)) sc[(size_t)hr * 2 + (qt >> 1)] = (uint8_t)(e + 127);
 }
-// transposed v: dst [H][48][R] with the 32 tokens of a block in slot order + scales [H][48][R / 32]. One wavefront per (head, 32-token block),
-// lane d < 48 owns dim d: it gathers the block's 32 values of its dim (each gather reads one token's 96 contiguous bytes across the lanes),
-// quantises them as one block and writes 32 contiguous bytes.
+// transposed v: dst [H][R / 64][48][64], the 64 tokens of a key tile in slot order (two blocks of 32) per dim, + scales [H][R / 64][48][2]: what the
+// core reads of a key tile is 3 KB in a row. One wavefront per (head, 32-token block), lane d < 48 owns dim d: it gathers the block's 32 values of its
+// dim (each gather reads one token's 96 contiguous bytes across the lanes), quantises them as one block and writes 32 contiguous bytes.
 __global__ void __launch_bounds__(256) a8_vt_k(const __half *__restrict__ src, uint8_t *__restrict__ dst, uint8_t *__restrict__ sc, int H, int nseq, int S, int Sp, long long Tp) {
     const long long R = (long long)nseq * Sp, nb = R / 32, wb = blockIdx.x * 4ll + (threadIdx.x >> 6);
     const int d = threadIdx.x & 63;
@@ -66,9 +67,10 @@ __global__ void __launch_bounds__(256) a8_vt_k(const __half *__restrict__ src, u
     for (int k = 0; k < 32; k++) { const int ii = i0 + a8_slot_token(k); v[k] = ii < S ? __half2float(base[(size_t)ii * HD]) : 0.f; }
     unsigned codes[8];
     const unsigned sb = d_quant_row<8, false>(v, 32, codes);
-    uint4 *o = (uint4 *)(dst + ((size_t)h * HD + d) * R + r0);
+    const size_t td = ((size_t)h * (R / 64) + (b >> 1)) * HD + d;               // (head, key tile, dim)
+    uint4 *o = (uint4 *)(dst + td * 64 + (b & 1) * 32);
     o[0] = make_uint4(codes[0], codes[1], codes[2], codes[3]); o[1] = make_uint4(codes[4], codes[5], codes[6], codes[7]);
-    sc[((size_t)h * HD + d) * nb + b] = (uint8_t)sb;
+    sc[td * 2 + (b & 1)] = (uint8_t)sb;
 }
 
 __device__ __forceinline__ float a8_xor32f(float x, int h) {
@@ -76,94 +78,79 @@ __device__ __forceinline__ float a8_xor32f(float x, int h) {
     const auto r2 = __builtin_amdgcn_permlane32_swap(u, u, false, false);
     return __uint_as_float(h ? r2[0] : r2[1]);
 }
+// the larger of the lane's and its partner's value
+__device__ __forceinline__ float a8_max32f(float x) {
+    const unsigned u = __float_as_uint(x);
+    const auto r2 = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    return fmaxf(__uint_as_float(r2[0]), __uint_as_float(r2[1]));
+}
+// 2^(s sl2 - m): the scaled logit is rounded before the maximum is taken off, as where the maximum was formed
+__device__ __forceinline__ float a8_prob(float s, float sl2, float m) {
+#pragma clang fp contract(off)
+    return __builtin_amdgcn_exp2f(s * sl2 - m);
+}
 // the lane's fragment of a 64-byte row of two 32-K blocks: bytes 16 h ... of each (p already points at byte 16 h)
 __device__ __forceinline__ v8i a8_frag(const uint8_t *p) {
     const v4i lo = *(const v4i *)p, hi = *(const v4i *)(p + 32);
     return (v8i){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
 }
 
-// grid (ceil(S / (32 nw)), H, nseq), nw = 4 or 1 wavefronts of 32 queries each. Fragments are the quantised tensors' rows as they lie in memory
-// (32 contiguous bytes per lane), loaded from global memory directly: a sequence's K and V of one head are 7 KB per 64 keys and stay in
-// L2 / the vector cache across the workgroup's wavefronts.
-__global__ void __launch_bounds__(256) a8_fwd_k(const uint8_t *__restrict__ Q8, const uint8_t *__restrict__ Q8s, const uint8_t *__restrict__ K8, const uint8_t *__restrict__ K8s,
+// the same through a pointer whose uniform part is in scalar registers (opaque: the address is not folded into the lane's offset) and a 32-bit lane offset
+typedef const __attribute__((address_space(1))) uint8_t *a8_gp;
+__device__ __forceinline__ a8_gp a8_uniform(const uint8_t *p) { a8_gp g = (a8_gp)p; asm("" : "+s"(g)); return g; }
+__device__ __forceinline__ v8i a8_frag(a8_gp p, unsigned o) {
+    typedef const __attribute__((address_space(1))) v4i *g4;
+    const v4i lo = *(g4)(p + o), hi = *(g4)(p + o + 32);
+    return (v8i){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+}
+
+// grid: H nseq (sequence, head) pairs, the pairs fastest, times the query tiles of 32. Consecutive workgroups go to the XCDs in turn, so with 8 pairs (or
+// a divisor or multiple) each XCD's L2 holds one pair's K and V (120 bytes per key, 0.5 MB at 4 100) instead of all of them. Fragments are the quantised
+// tensors' rows as they lie in memory (32 contiguous bytes per lane), loaded from global memory directly.
+// A key tile of 64 keys is four matrix products (256 cycles) and about 210 vector instructions, 34 of them exponentials. Many query tiles (several wavefronts per
+// SIMD): bound by those, 1 300 cycles per tile at 16 x 4 heads of 4 100 tokens (513 -> 340 us; block maxima, masks and rescalings that change nothing left out, 268 + 57
+// instructions before). One wavefront per SIMD (129 x 4 tiles): its own chain, hence the products of the next tile beside the softmax of this one (66 -> 55 us; 202 registers
+// and two wavefronts per SIMD, which costs the many-tile launches 1 %) and loads whose addresses and waits are the hardware's, not the compiler's.
+// A workgroup of four wavefronts whose first alone has queries (the sequence's last query tile: the few tokens past a multiple of 128) shares that
+// tile's keys among its wavefronts, a range of the key tiles each, and merges the four partial softmaxes. Each wavefront starts from the running maximum of the
+// tiles before its range, so the probabilities and their e4m3 codes are those of the one-wavefront pass; only the order in which the partial sums are
+// added differs. The maxima come from a first walk of the wavefronts over their own ranges (the K Q^T products and a maximum per logit), exchanged through LDS.
+__global__ void __launch_bounds__(256, 2) a8_fwd_k(const uint8_t *__restrict__ Q8, const uint8_t *__restrict__ Q8s, const uint8_t *__restrict__ K8, const uint8_t *__restrict__ K8s,
                                                 const uint8_t *__restrict__ Vt, const uint8_t *__restrict__ Vts, float *__restrict__ o, float *__restrict__ lse,
-                                                int S, int Sp, int H, int C, long long R, float sl2) {
-    const int seq = blockIdx.z, hd = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 31, h = lane >> 5;
-    const int nwv = blockDim.x >> 6, tq = blockIdx.x * nwv;
-    // A four-wavefront workgroup whose first wavefront alone has queries (the sequence's last 32-query tile: the few tokens past a multiple
-    // of 128) shares that tile's keys among its wavefronts, a range of the key tiles each, and wavefront 0 merges the four partial
-    // softmaxes: the tile costs a third of a wavefront's full pass instead of one that the rest of the GPU waits for. Each wavefront starts
-    // from the running maximum of the tiles before its range, so the probabilities and their e4m3 codes are those of the one-wavefront
-    // pass; only the order in which the partial sums are added differs
+                                                int S, int Sp, int H, int C, long long R, float sl2, unsigned pairs) {
+    const unsigned bq = blockIdx.x / pairs, bp = blockIdx.x - bq * pairs;
+    const int seq = (int)(bp / (unsigned)H), hd = (int)(bp - (unsigned)seq * (unsigned)H), tid = threadIdx.x, lane = tid & 63, r = lane & 31, h = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nwv = blockDim.x >> 6, tq = (int)bq * nwv;
     const bool split = nwv == 4 && (tq + 1) * 32 >= S;
     const int q0 = (split ? tq : tq + wave) * 32;
     if (q0 >= S) return;                                   // (no barriers outside a split workgroup: a wavefront without queries leaves)
     const long long rb = (long long)hd * R + (long long)seq * Sp;          // the sequence's first row in the row-quantised tensors
-    const long long c0 = (long long)seq * Sp;                              // its first column in the transposed one
+    const long long tb = rb / FT;                                          // ... and its first key tile in the transposed one
     const v8i qf = a8_frag(Q8 + (rb + q0 + r) * 64 + 16 * h);
     const int qs = Q8s[(rb + q0 + r) * 2 + h];
-    const uint8_t *kp = K8 + (rb + r) * 64 + 16 * h, *ksp = K8s + (rb + r) * 2 + h;
-    // V^T rows: dims r and 32 + r (the second tile has 16 real rows; the others multiply zeros)
-    const int d1 = min(32 + r, HD - 1); const bool d1ok = 32 + r < HD;
-    const uint8_t *vp0 = Vt + ((size_t)hd * HD + r) * R + c0 + 16 * h, *vp1 = Vt + ((size_t)hd * HD + d1) * R + c0 + 16 * h;
-    const uint8_t *vs0 = Vts + ((size_t)hd * HD + r) * (R / 32) + c0 / 32 + h, *vs1 = Vts + ((size_t)hd * HD + d1) * (R / 32) + c0 / 32 + h;
-    float m = -INFINITY, l = 0.f;
-    v16f oa[2];
-#pragma unroll
-    for (int t = 0; t < 2; t++)
-#pragma unroll
-        for (int i = 0; i < 16; i++) oa[t][i] = 0.f;
+    // (uniform bases and small lane offsets: one address instruction per load or none)
+    const uint8_t *kp = K8 + rb * 64, *ksp = K8s + rb * 2;
+    const unsigned ko = (unsigned)(r * 64 + 16 * h), kso = (unsigned)(r * 2 + h);
+    // V^T rows: dims r and 32 + r (of the second the first 16 are real; the others repeat the last one into accumulator rows that are never read)
+    const int d1 = min(32 + r, HD - 1);
+    const uint8_t *vp = Vt + tb * (HD * 64), *vsp = Vts + tb * (HD * 2);
+    const unsigned vo0 = (unsigned)(r * 64 + 16 * h), vo1 = (unsigned)(d1 * 64 + 16 * h), vso0 = (unsigned)(r * 2 + h), vso1 = (unsigned)(d1 * 2 + h);
     const int nt = (S + FT - 1) / FT;
-    // (split: later ranges are shorter, since their wavefronts first look through the earlier tiles for the running maximum)
-    const int cut[5] = {0, nt * 34 / 100, nt * 61 / 100, nt * 83 / 100, nt};
-    const int it0 = split ? cut[wave] : 0, it1 = split ? cut[wave + 1] : nt;
-    // The K and V fragments of tile it + 1 are requested before tile it is worked on: with one or a few wavefronts per SIMD nothing else hides
-    // the L2 latency of a tile's loads. (The last iteration re-requests its own tile.)
-    v8i kfn[2], vfn[2]; int ksn[2], evn[2];
-    auto request = [&](int it) {
-        const int kb = it * FT;
+    // the K fragments of a tile are requested behind the products of the one before it, into the registers those products have read, and so are the V
+    // fragments: K then has the softmax and the second products of a tile to arrive, V the next tile's first products and softmax
+    v8i kf[2], vf0, vf1; int ks[2], e0v, e1v;
+    auto request_k = [&](int it) {
+        const a8_gp k = a8_uniform(kp + (size_t)it * (FT * 64)), s = a8_uniform(ksp + (size_t)it * (FT * 2));
 #pragma unroll
-        for (int b = 0; b < 2; b++) { kfn[b] = a8_frag(kp + (size_t)(kb + 32 * b) * 64); ksn[b] = ksp[(size_t)(kb + 32 * b) * 2]; }
-        vfn[0] = a8_frag(vp0 + kb); vfn[1] = a8_frag(vp1 + kb);
-        evn[0] = vs0[kb / 32]; evn[1] = vs1[kb / 32];
+        for (int b = 0; b < 2; b++) { kf[b] = a8_frag(k, ko + 2048u * b); ks[b] = s[kso + 64u * b]; }
     };
-    if (split && it0 > 0) {
-        // the running maximum the single-wavefront pass holds when it reaches tile it0: the logits of the tiles before it (the two products
-        // and the scaling of the main loop, nothing else), so that every probability of this range is the value that pass computes
-        v8i kq[2]; int kqs[2];
-        auto reqk = [&](int it) {
-#pragma unroll
-            for (int b = 0; b < 2; b++) { kq[b] = a8_frag(kp + (size_t)(it * FT + 32 * b) * 64); kqs[b] = ksp[(size_t)(it * FT + 32 * b) * 2]; }
-        };
-        reqk(0);
-        float mx = -INFINITY;
-        for (int it = 0; it < it0; it++) {
-            const v8i kf[2] = {kq[0], kq[1]}; const int ks[2] = {kqs[0], kqs[1]};
-            reqk(min(it + 1, it0 - 1));
-#pragma unroll
-            for (int b = 0; b < 2; b++) {
-                v16f z;
-#pragma unroll
-                for (int i = 0; i < 16; i++) z[i] = 0.f;
-                const v16f sb = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(kf[b], qf, z, 0, 0, 0, ks[b], 0, qs);
-#pragma unroll
-                for (int i = 0; i < 16; i++) {
-                    const int key = it * FT + 32 * b + (i & 3) + 4 * h + 8 * (i >> 2);
-                    mx = fmaxf(mx, key < S ? sb[i] * sl2 : -INFINITY);
-                }
-            }
-        }
-        m = fmaxf(mx, a8_xor32f(mx, h));
-    }
-    request(min(it0, nt - 1));
-    for (int it = it0; it < it1; it++) {
-        const int kb = it * FT;
-        const v8i kf[2] = {kfn[0], kfn[1]}; const int ks[2] = {ksn[0], ksn[1]};
-        v8i vf0 = vfn[0], vf1 = vfn[1];
-        const int e0v = evn[0], e1v = evn[1];
-        request(min(it + 1, nt - 1));
-        // ---- S^T = K Q^T for the tile's two blocks of 32 keys ----
-        v16f s[2];
+    auto request_v = [&](int it) {
+        const a8_gp v = a8_uniform(vp + (size_t)it * (HD * 64)), vs = a8_uniform(vsp + (size_t)it * (HD * 2));
+        vf0 = a8_frag(v, vo0); vf1 = a8_frag(v, vo1); e0v = vs[vso0]; e1v = vs[vso1];
+    };
+    // S^T = K Q^T for the two blocks of 32 keys of tile it, the next tile's K requested behind it (the last tile re-requests itself)
+    auto logits = [&](int it, v16f (&s)[2]) {
 #pragma unroll
         for (int b = 0; b < 2; b++) {
             v16f z;
@@ -171,98 +158,131 @@ __global__ void __launch_bounds__(256) a8_fwd_k(const uint8_t *__restrict__ Q8, 
             for (int i = 0; i < 16; i++) z[i] = 0.f;
             s[b] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(kf[b], qf, z, 0, 0, 0, ks[b], 0, qs);
         }
-        if (!d1ok) vf1 = (v8i){0, 0, 0, 0, 0, 0, 0, 0};
-        // ---- logits in base-2 units, keys past S masked (only the last tile can hold them) ----
-        const bool full = kb + FT <= S;
+        __builtin_amdgcn_sched_barrier(0);
+        request_k(min(it + 1, nt - 1));
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    extern __shared__ float4 cmb4[];                       // split: [range][6][lane] float4 of O^T, then [range][2][lane] floats: m, l; the exchanged maxima before that
+    float m = -INFINITY;
+    int it0 = 0, it1 = nt;
+    if (split) {
+        const int cut[5] = {0, nt * 34 / 100, nt * 61 / 100, nt * 83 / 100, nt};
+        it0 = cut[wave]; it1 = cut[wave + 1];
+        float mx = -INFINITY;
+        if (wave < 3) {                                    // (keys past S count for nothing here: a range that holds the last tile has none behind it)
+            request_k(min(it0, nt - 1));
+            // (the loads of tile it + 1 are requested behind the products of tile it, into the registers these have read)
+            for (int it = it0; it < it1; it++) {
+                v16f s[2];
+                logits(it, s);
 #pragma unroll
-        for (int b = 0; b < 2; b++)
+                for (int b = 0; b < 2; b++)
 #pragma unroll
-            for (int i = 0; i < 16; i++) s[b][i] *= sl2;
-        if (!full) {                                       // (uniform: no per-element key test on the tiles before the last)
+                    for (int i = 0; i < 16; i++) mx = fmaxf(mx, s[b][i]);
+            }
+            mx = a8_max32f(mx) * sl2;        // (sl2 > 0 and rounding is monotone: the largest scaled logit)
+        }
+        float *pm = (float *)cmb4;
+        pm[wave * 64 + lane] = mx;
+        __syncthreads();
+        if (it0 < it1) for (int w = 0; w < wave; w++) m = fmaxf(m, pm[w * 64 + lane]);      // (a range without tiles keeps -inf)
+        __syncthreads();
+    }
+    float l = 0.f;
+    v16f oa0, oa1;                                         // O^T: dims 4 h + 8 g + c in element 4 g + c; of the second tile elements 0 .. 7 are dims below 48
+#pragma unroll
+    for (int i = 0; i < 16; i++) { oa0[i] = 0.f; oa1[i] = 0.f; }
+    auto softmax_pv = [&](int it, v16f (&s)[2], auto last) {
+        if constexpr (decltype(last)::value) {             // keys past S masked (only the last tile can hold them)
 #pragma unroll
             for (int b = 0; b < 2; b++)
 #pragma unroll
-                for (int i = 0; i < 16; i++) { const int key = kb + 32 * b + (i & 3) + 4 * h + 8 * (i >> 2); if (key >= S) s[b][i] = -INFINITY; }
+                for (int i = 0; i < 16; i++) { const int key = it * FT + 32 * b + (i & 3) + 4 * h + 8 * (i >> 2); if (key >= S) s[b][i] = -INFINITY; }
         }
-        float mx = -INFINITY;
+        // ---- the largest logit of each block of 32 keys, in the products' own units (the scaling to base 2 is monotone): it gives the running maximum and, as
+        // the exponential of its scaled value, the largest probability of the block, which fixes the block's scale ----
+        float bm[2] = {s[0][0], s[1][0]};
 #pragma unroll
-        for (int b = 0; b < 2; b++)
+        for (int i = 1; i < 16; i++) { bm[0] = fmaxf(bm[0], s[0][i]); bm[1] = fmaxf(bm[1], s[1][i]); }
+        bm[0] = a8_max32f(bm[0]); bm[1] = a8_max32f(bm[1]);
+        const float mn = fmaxf(m, fmaxf(bm[0], bm[1]) * sl2), corr = __builtin_amdgcn_exp2f(m - mn);
+        m = mn;
+        if (__builtin_amdgcn_ballot_w64(corr != 1.f) != 0ull) {      // (uniform: most tiles late in a row raise no query's maximum)
 #pragma unroll
-            for (int i = 0; i < 16; i++) mx = fmaxf(mx, s[b][i]);
-        mx = fmaxf(mx, a8_xor32f(mx, h));
-        const float mn = fmaxf(m, mx), corr = __builtin_amdgcn_exp2f(m - mn);
-        m = mn; l *= corr;
-        float am[2] = {0.f, 0.f};
+            for (int i = 0; i < 16; i++) oa0[i] *= corr;
 #pragma unroll
-        for (int b = 0; b < 2; b++)
-#pragma unroll
-            for (int i = 0; i < 16; i++) { const float p = __builtin_amdgcn_exp2f(s[b][i] - m); s[b][i] = p; l += p; am[b] = fmaxf(am[b], p); }
-#pragma unroll
-        for (int t = 0; t < 2; t++)
-#pragma unroll
-            for (int i = 0; i < 16; i++) oa[t][i] *= corr;
-        // ---- P -> e4m3 with one scale per query per 32 keys; the lane's codes are its B fragment, its scale operand is block h's ----
+            for (int i = 0; i < 16; i++) oa1[i] *= corr;
+        }
+        // ---- P = 2^(logit - m) -> e4m3 with one scale per query per 32 keys; the lane's codes are its B fragment, its scale operand is block h's ----
         unsigned cw[2][4]; int ep[2];
 #pragma unroll
         for (int b = 0; b < 2; b++) {
-            am[b] = fmaxf(am[b], a8_xor32f(am[b], h));
-            ep[b] = d_mx_exp(am[b], MI_INVQ8);
-            const float p2e = d_exp2i(ep[b]);
+            ep[b] = d_mx_expb_fin(a8_prob(bm[b], sl2, m), MI_INVQ8);
+            const float p2e = __uint_as_float((unsigned)ep[b] << 23);
+#pragma unroll
+            for (int i = 0; i < 16; i++) { s[b][i] = a8_prob(s[b][i], sl2, m); l = b || i ? l + s[b][i] : fmaf(l, corr, s[b][i]); }
 #pragma unroll
             for (int q = 0; q < 4; q++) cw[b][q] = d_enc_e4m3x4_hw(s[b][4 * q], s[b][4 * q + 1], s[b][4 * q + 2], s[b][4 * q + 3], p2e);
         }
         const v8i pf = {(int)cw[0][0], (int)cw[0][1], (int)cw[0][2], (int)cw[0][3], (int)cw[1][0], (int)cw[1][1], (int)cw[1][2], (int)cw[1][3]};
-        const int ps = (h ? ep[1] : ep[0]) + 127;
+        const int ps = h ? ep[1] : ep[0];
         // ---- O^T += V^T P^T ----
-        oa[0] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(vf0, pf, oa[0], 0, 0, 0, e0v, 0, ps);
-        oa[1] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(vf1, pf, oa[1], 0, 0, 0, e1v, 0, ps);
+        oa0 = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(vf0, pf, oa0, 0, 0, 0, e0v, 0, ps);
+        oa1 = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(vf1, pf, oa1, 0, 0, 0, e1v, 0, ps);
+        if constexpr (!decltype(last)::value) { __builtin_amdgcn_sched_barrier(0); request_v(it + 1); __builtin_amdgcn_sched_barrier(0); }
+    };
+    if (it0 < it1) {
+        // the products of tile it + 1 are issued before the softmax of tile it, whose vector instructions run beside them
+        request_k(it0); request_v(it0);
+        v16f sa[2], sb[2];
+        logits(it0, sa);
+        int it = it0;
+        for (; it + 2 < it1; it += 2) {
+            logits(it + 1, sb); softmax_pv(it, sa, std::false_type{});
+            logits(it + 2, sa); softmax_pv(it + 1, sb, std::false_type{});
+        }
+        if (it + 1 < it1) { logits(it + 1, sb); softmax_pv(it, sa, std::false_type{}); softmax_pv(it + 1, sb, std::true_type{}); }
+        else softmax_pv(it, sa, std::true_type{});
     }
     l += a8_xor32f(l, h);
-    if (split) {
-        // partial (m, l, O^T) of the four key ranges -> LDS [wavefront][value][lane]; wavefront 0 adds them in wavefront order at the common
-        // maximum (a wavefront without keys holds m = -inf, l = 0, O = 0: its factor is 0)
-        extern __shared__ float cmb[];
-        float *mine = cmb + (size_t)wave * 34 * 64 + lane;
-        mine[0] = m; mine[64] = l;
+    const int i = q0 + r;
+    float *orow = o + ((size_t)seq * S + (i < S ? i : S - 1)) * C + hd * HD + 4 * h;
+    if (!split) {
+        if (i >= S) return;
+        const float il = 1.f / l;
 #pragma unroll
-        for (int t = 0; t < 2; t++)
+        for (int g = 0; g < 4; g++) *(float4 *)(orow + 8 * g) = make_float4(oa0[4 * g] * il, oa0[4 * g + 1] * il, oa0[4 * g + 2] * il, oa0[4 * g + 3] * il);
 #pragma unroll
-            for (int k = 0; k < 16; k++) mine[(2 + 16 * t + k) * 64] = oa[t][k];
-        __syncthreads();
-        if (wave) return;
-        float mm = m;
+        for (int g = 0; g < 2; g++) *(float4 *)(orow + 32 + 8 * g) = make_float4(oa1[4 * g] * il, oa1[4 * g + 1] * il, oa1[4 * g + 2] * il, oa1[4 * g + 3] * il);
+        if (!h) lse[((size_t)seq * H + hd) * S + i] = m + __log2f(l);
+        return;
+    }
+    // partial (m, l, O^T) of the key ranges -> LDS; every wavefront adds its share of the dims in range order at the common maximum (a wavefront without
+    // keys holds l = 0, O = 0; its factor, of a maximum at most the common one, is finite)
+    float *ml = (float *)(cmb4 + 4 * 6 * 64);
 #pragma unroll
-        for (int w = 1; w < 4; w++) mm = fmaxf(mm, cmb[(size_t)w * 34 * 64 + lane]);
-        float ls = 0.f;
-        v16f os[2];
+    for (int g = 0; g < 4; g++) cmb4[(wave * 6 + g) * 64 + lane] = make_float4(oa0[4 * g], oa0[4 * g + 1], oa0[4 * g + 2], oa0[4 * g + 3]);
 #pragma unroll
-        for (int t = 0; t < 2; t++)
+    for (int g = 0; g < 2; g++) cmb4[(wave * 6 + 4 + g) * 64 + lane] = make_float4(oa1[4 * g], oa1[4 * g + 1], oa1[4 * g + 2], oa1[4 * g + 3]);
+    ml[(wave * 2) * 64 + lane] = m; ml[(wave * 2 + 1) * 64 + lane] = l;
+    __syncthreads();
+    float mw[4], mm = -INFINITY, ls = 0.f;
 #pragma unroll
-            for (int k = 0; k < 16; k++) os[t][k] = 0.f;
+    for (int w = 0; w < 4; w++) { mw[w] = ml[(w * 2) * 64 + lane]; mm = fmaxf(mm, mw[w]); }
+#pragma unroll
+    for (int w = 0; w < 4; w++) { mw[w] = __builtin_amdgcn_exp2f(mw[w] - mm); ls = fmaf(ml[(w * 2 + 1) * 64 + lane], mw[w], ls); }
+    if (i >= S) return;
+    const float il = 1.f / ls;
+    for (int g = wave; g < 6; g += 4) {                    // (float4 group g: dims 8 g + 4 h ...)
+        float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
         for (int w = 0; w < 4; w++) {
-            const float *pw = cmb + (size_t)w * 34 * 64 + lane;
-            const float f = __builtin_amdgcn_exp2f(pw[0] - mm);
-            ls = fmaf(pw[64], f, ls);
-#pragma unroll
-            for (int t = 0; t < 2; t++)
-#pragma unroll
-                for (int k = 0; k < 16; k++) os[t][k] = fmaf(pw[(2 + 16 * t + k) * 64], f, os[t][k]);
+            const float4 p = cmb4[(w * 6 + g) * 64 + lane];
+            a.x = fmaf(p.x, mw[w], a.x); a.y = fmaf(p.y, mw[w], a.y); a.z = fmaf(p.z, mw[w], a.z); a.w = fmaf(p.w, mw[w], a.w);
         }
-        m = mm; l = ls; oa[0] = os[0]; oa[1] = os[1];
+        *(float4 *)(orow + 8 * g) = make_float4(a.x * il, a.y * il, a.z * il, a.w * il);
     }
-    const int i = q0 + r;
-    if (i >= S) return;
-    const float il = 1.f / l;
-    float *orow = o + ((size_t)seq * S + i) * C + hd * HD;
-#pragma unroll
-    for (int t = 0; t < 2; t++)
-#pragma unroll
-        for (int g = 0; g < 4; g++) {
-            const int d0 = 32 * t + 4 * h + 8 * g;         // accumulator elements 4 g ... 4 g + 3: dims d0 ... d0 + 3
-            if (d0 < HD) *(float4 *)(orow + d0) = make_float4(oa[t][4 * g] * il, oa[t][4 * g + 1] * il, oa[t][4 * g + 2] * il, oa[t][4 * g + 3] * il);
-        }
-    if (!h) lse[((size_t)seq * H + hd) * S + i] = m + __log2f(l);
+    if (wave == 3 && !h) lse[((size_t)seq * H + hd) * S + i] = mm + __log2f(ls);
 }
 
 static int g_a8_waves = 0;
@@ -281,10 +301,13 @@ extern "C" int at_fa8_fwd(const void *qkvh, float *o, float *lse, const at_geom 
     // (queries and keys in one launch: their sources, code planes and scale planes each lie one fixed stride apart)
     a8_rows_k<<<dim3(nblk_((size_t)H * R * 4, 256), 2), 256>>>(Qh, q8, qs, H, g->nseq, g->S, Sp, Tp, (size_t)(Kh - Qh), (size_t)(k8 - q8), (size_t)(ks - qs));
     a8_vt_k<<<nblk_((size_t)H * (R / 32), 4), 256>>>(Vh, vt, vts, H, g->nseq, g->S, Sp, Tp);
-    // few query tiles (a 16^3 bottleneck: 129 per head): one wavefront per workgroup, so that every CU gets some
-    const int nw = g_a8_waves ? g_a8_waves : (size_t)((g->S + 127) / 128) * H * g->nseq >= 512 ? 4 : 1;
-    const dim3 grid((unsigned)((g->S + 32 * nw - 1) / (32 * nw)), (unsigned)H, (unsigned)g->nseq);
-    a8_fwd_k<<<grid, 64 * nw, nw == 4 ? 4 * 34 * 64 * sizeof(float) : 0>>>(q8, qs, k8, ks, vt, vts, o, lse, g->S, Sp, H, C, R, 1.4426950408889634f / sqrtf((float)HD));
+    // four wavefronts share a workgroup's reads of K and V, and its last query tile when that is alone (8 stragglers of 1 032 tiles on 1 024 SIMDs otherwise: 90 against 65 us);
+    // sequences of at most 256 tokens have too few key tiles to share (5 tokens: 9.8 against 10.3 us)
+    const size_t pairs = (size_t)H * g->nseq, qt = (size_t)(g->S + 31) / 32;
+    const int nw = g_a8_waves ? g_a8_waves : g->S <= 256 ? 1 : 4;
+    const size_t nblk = pairs * ((qt + nw - 1) / nw);
+    if (nblk * (size_t)(64 * nw) >= (size_t)1 << 32) mi_die("at_fa8_fwd: %zu workgroups exceed the launch grid", nblk);
+    a8_fwd_k<<<(unsigned)nblk, 64 * nw, nw == 4 ? 4 * 26 * 64 * sizeof(float) : 0>>>(q8, qs, k8, ks, vt, vts, o, lse, g->S, Sp, H, C, R, 1.4426950408889634f / sqrtf((float)HD), (unsigned)pairs);
     MICK();
     return 0;
 }
