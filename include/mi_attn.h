@@ -48,7 +48,8 @@ void at_fa8_waves(int nw);
 /* (no counterpart: a knob for tests) 0: at_block_fwd writes the fp32 rows of its LayerNorms and its SwiGLU (at_ws.xn, .xn2, .gg) and the GEMMs
    pack them; 1: with e4m3 linears and C, F multiples of 64 those kernels write the GEMMs' packed operands themselves and the three fp32 buffers
    are left untouched (a forward never reads them again); 2 (default): also, for C <= 256, the up projection forms the SwiGLU in its epilogue and
-   writes the down projection's packed operand, and at_ws.h is left untouched too. The block's output has the same bits in all three */
+   writes the down projection's packed operand, and at_ws.h is left untouched too, and without rays the pack writes the core's quantised operands, with
+   at_ws.qkvh left untouched. The block's output has the same bits in all three */
 void at_fuse_pack(int on);
 
 /* ---- radial attention and scroll coordinates (src/attn.h:83-128, src/nn_attn_ray.cu) ----

@@ -11,6 +11,7 @@
 #include <hip/hip_fp16.h>
 #include <type_traits>
 #include "mx_dev.hpp"
+#include "attn_rope.hpp"
 #include "../../include/mi_attn.h"
 
 typedef int v8i __attribute__((ext_vector_type(8)));
@@ -71,6 +72,86 @@ __global__ void __launch_bounds__(256) a8_vt_k(const __half *__restrict__ src, u
     uint4 *o = (uint4 *)(dst + td * 64 + (b & 1) * 32);
     o[0] = make_uint4(codes[0], codes[1], codes[2], codes[3]); o[1] = make_uint4(codes[4], codes[5], codes[6], codes[7]);
     sc[td * 2 + (b & 1)] = (uint8_t)sb;
+}
+
+// The block forward's way to the same operands: qkv_pack_k's arithmetic (attn_block.hip: QK-norm, gains, rotary embedding, rounding to binary16), a8_rows_k's and
+// a8_vt_k's quantisation in one pass over the projection's rows, without the binary16 tensor between them (three launches of 20 + 5 + 12 us for
+// two 16^3 windows in 4 heads, 11 us as this one: a workgroup forms the rotary angles once for 64 rows). Bound by its vector instructions and the chain of one row, not by
+// the 192 bytes in and 62 out of a row and part. A workgroup takes one part (queries, keys, values) of the 64 tokens of a key tile of one head, thread (row, quarter)
+// 16 dims: the row's sum of squares meets over the quarters in the order of qkv_pack_k's eight lanes; the V tile turns in LDS.
+template <int MODE>
+__global__ void __launch_bounds__(256) a8_pack_k(const float *__restrict__ qkv, const float *__restrict__ qg, const float *__restrict__ kg, uint8_t *__restrict__ q8, uint8_t *__restrict__ q8s,
+                                                 size_t part, size_t part_sc, uint8_t *__restrict__ vt, uint8_t *__restrict__ vts, float *__restrict__ rq, float *__restrict__ rk, float *__restrict__ amx,
+                                                 int H, int S, unsigned tiles, long long R, rope_t rp) {
+    __shared__ float2 rtab[ROPE_TAB * 8];
+    __shared__ float vl[64][HD + 1];
+    __shared__ unsigned bmax;
+    // eight tiles at a time, their 3 H workgroups each on one XCD (workgroups go to the XCDs in turn): the parts' 192-byte pieces of a token's row share cache lines
+    const unsigned u = blockIdx.x >> 3, g = u / (3u * H), hp = u - g * (3u * H), tile = g * 8 + (blockIdx.x & 7);
+    if (tile >= (unsigned)(R >> 6)) return;
+    const int p = (int)(hp / (unsigned)H), h = (int)hp - p * H, C = H * HD, row = threadIdx.x >> 2, qt = threadIdx.x & 3;
+    const unsigned seq = tile / tiles;                                           // (whole tiles of 64 tokens per sequence)
+    const int ii = (int)(tile - seq * tiles) * 64 + row;
+    const long long t = (long long)seq * S + ii;
+    const bool live = ii < S && qt < 3;
+    float v[16];
+    {
+        const float4 *x = (const float4 *)(qkv + t * 3 * C + p * C + h * HD + 16 * qt);
+#pragma unroll
+        for (int k = 0; k < 4; k++) { const float4 a = live ? x[k] : make_float4(0.f, 0.f, 0.f, 0.f); v[4 * k] = a.x; v[4 * k + 1] = a.y; v[4 * k + 2] = a.z; v[4 * k + 3] = a.w; }
+    }
+    if (p < 2) {
+        const float *gs = (p ? kg : qg) + h * HD + 16 * qt;                      // (the gains sit at an arbitrary offset of the flat parameter vector: dword loads)
+        float gn[16];
+#pragma unroll
+        for (int k = 0; k < 16; k++) gn[k] = qt < 3 ? gs[k] : 0.f;
+        const int ts = ii - rp.nreg;
+        const bool turn = rp.on && live && ts >= 0;
+        const float pos = turn ? rope_pos<MODE>(rp, t, ts, qt) : 0.f;
+        if (MODE == ROPE_TABLE && rp.on) { rope_fill(rtab, rope_positions(rp), rp.lbase); __syncthreads(); }
+        float s0 = 0.f, s1 = 0.f;
+#pragma unroll
+        for (int k = 0; k < 8; k++) { s0 = fmaf(v[k], v[k], s0); s1 = fmaf(v[8 + k], v[8 + k], s1); }
+        float ss = s0 + s1;
+        ss += d_quad_xor_f<1>(ss); ss += d_quad_xor_f<2>(ss);
+        const float r = 1.f / sqrtf(ss / HD + 1e-6f);
+        if (!qt && live) (p ? rk : rq)[t * H + h] = r;
+#pragma unroll
+        for (int k = 0; k < 16; k++) v[k] *= r * gn[k];
+        if (turn) {
+#pragma unroll
+            for (int f = 0; f < 8; f++) rope_turn<MODE>(rp, rtab, pos, f, v[2 * f], v[2 * f + 1]);
+        }
+        float am = 0.f;
+#pragma unroll
+        for (int k = 0; k < 16; k++) { v[k] = __half2float(__float2half_rn(v[k])); am = fmaxf(am, fabsf(v[k])); }
+        am = __uint_as_float(max(__float_as_uint(am), d_quad_xor_u<1>(__float_as_uint(am))));      // (quarters (0, 1) and (2, 3) are the two blocks)
+        const int e = d_mx_exp(am, MI_INVQ8);
+        const size_t hr = (size_t)h * R + tile * 64ll + row;
+        *(uint4 *)(q8 + p * part + hr * 64 + 16 * qt) = make_uint4(d_enc4_e4m3(v[0], v[1], v[2], v[3], e), d_enc4_e4m3(v[4], v[5], v[6], v[7], e), d_enc4_e4m3(v[8], v[9], v[10], v[11], e), d_enc4_e4m3(v[12], v[13], v[14], v[15], e));
+        if (!(qt & 1)) q8s[p * part_sc + hr * 2 + (qt >> 1)] = (uint8_t)(e + 127);
+        return;
+    }
+    if (threadIdx.x == 0) bmax = 0u;
+    __syncthreads();
+    float m = 0.f;
+#pragma unroll
+    for (int k = 0; k < 16; k++) { m = fmaxf(m, fabsf(v[k])); if (qt < 3) vl[row][16 * qt + k] = __half2float(__float2half_rn(v[k])); }
+    m = fmaxf(m, d_quad_xor_f<1>(m)); m = fmaxf(m, d_quad_xor_f<2>(m));
+    if (!qt) atomicMax(&bmax, __float_as_uint(m));                               // (non-negative floats order as their bit patterns)
+    __syncthreads();
+    // (the running maximum only grows: a workgroup that does not exceed the value it reads has nothing to add)
+    if (threadIdx.x == 0 && bmax > *(volatile unsigned *)((unsigned *)amx + 1)) atomicMax((unsigned *)amx + 1, bmax);
+    if (threadIdx.x >= HD * 4) return;
+    const int d = threadIdx.x >> 2, b = (threadIdx.x >> 1) & 1, hh = threadIdx.x & 1;      // dim, block of 32 tokens, half of its slots
+    float am = 0.f;
+#pragma unroll
+    for (int k = 0; k < 16; k++) { v[k] = vl[32 * b + a8_slot_token(16 * hh + k)][d]; am = fmaxf(am, fabsf(v[k])); }
+    am = __uint_as_float(max(__float_as_uint(am), d_quad_xor_u<1>(__float_as_uint(am))));
+    const int e = d_mx_exp(am, MI_INVQ8);
+    const size_t td = ((size_t)h * (R / 64) + tile) * HD + d;
+    *(uint4 *)(vt + td * 64 + b * 32 + hh * 16) = make_uint4(d_enc4_e4m3(v[0], v[1], v[2], v[3], e), d_enc4_e4m3(v[4], v[5], v[6], v[7], e), d_enc4_e4m3(v[8], v[9], v[10], v[11], e), d_enc4_e4m3(v[12], v[13], v[14], v[15], e));
+    if (!hh) vts[td * 2 + b] = (uint8_t)(e + 127);
 }
 
 __device__ __forceinline__ float a8_xor32f(float x, int h) {
@@ -287,27 +368,53 @@ __global__ void __launch_bounds__(256, 2) a8_fwd_k(const uint8_t *__restrict__ Q
 
 static int g_a8_waves = 0;
 extern "C" void at_fa8_waves(int nw) { g_a8_waves = nw == 1 || nw == 4 ? nw : 0; }
-extern "C" int at_fa8_fwd(const void *qkvh, float *o, float *lse, const at_geom *g, int H, int C) {
-    if (!g || g->nseq <= 0 || g->S <= 0 || H <= 0) return 0;
-    if (C != H * HD) mi_die("at_fa8_fwd: C %d is not %d heads of %d", C, H, HD);
-    if (g->lens || g->rays) mi_die("at_fa8_fwd: per-sequence lengths and ray geometry are not supported");
-    const long long T = (long long)g->nseq * g->S, Tp = T + FT; const int Sp = (g->S + FT - 1) / FT * FT; const long long R = (long long)g->nseq * Sp;
-    const size_t rq = (size_t)H * R * 64, rqs = (size_t)H * R * 2, tq = (size_t)H * HD * R, tqs = (size_t)H * HD * (R / 32);
+namespace {
+// the quantised operands of one call in the library's scratch, and the core on them
+struct a8_ops { uint8_t *q8, *k8, *qs, *ks, *vt, *vts; int Sp; long long R; };
+bool a8_carve(a8_ops *w, const at_geom *g, int H) {
+    w->Sp = (g->S + FT - 1) / FT * FT; w->R = (long long)g->nseq * w->Sp;
+    const size_t rq = (size_t)H * w->R * 64, rqs = (size_t)H * w->R * 2, tq = (size_t)H * HD * w->R, tqs = (size_t)H * HD * (w->R / 32);
     auto al = [](size_t n) { return (n + 255) & ~(size_t)255; };
     uint8_t *base = (uint8_t *)mi_ws(MI_WS_ATTN, 2 * (al(rq) + al(rqs)) + al(tq) + al(tqs));
-    if (!base) return -1;
-    uint8_t *q8 = base, *k8 = q8 + al(rq), *qs = k8 + al(rq), *ks = qs + al(rqs), *vt = ks + al(rqs), *vts = vt + al(tq);
-    const __half *Qh = (const __half *)qkvh, *Kh = Qh + (size_t)H * Tp * HD, *Vh = Kh + (size_t)H * Tp * HD;
-    // (queries and keys in one launch: their sources, code planes and scale planes each lie one fixed stride apart)
-    a8_rows_k<<<dim3(nblk_((size_t)H * R * 4, 256), 2), 256>>>(Qh, q8, qs, H, g->nseq, g->S, Sp, Tp, (size_t)(Kh - Qh), (size_t)(k8 - q8), (size_t)(ks - qs));
-    a8_vt_k<<<nblk_((size_t)H * (R / 32), 4), 256>>>(Vh, vt, vts, H, g->nseq, g->S, Sp, Tp);
+    if (!base) return false;
+    w->q8 = base; w->k8 = w->q8 + al(rq); w->qs = w->k8 + al(rq); w->ks = w->qs + al(rqs); w->vt = w->ks + al(rqs); w->vts = w->vt + al(tq);
+    return true;
+}
+void a8_core(const a8_ops &w, float *o, float *lse, const at_geom *g, int H, int C) {
     // four wavefronts share a workgroup's reads of K and V, and its last query tile when that is alone (8 stragglers of 1 032 tiles on 1 024 SIMDs otherwise: 90 against 65 us);
     // sequences of at most 256 tokens have too few key tiles to share (5 tokens: 9.8 against 10.3 us)
     const size_t pairs = (size_t)H * g->nseq, qt = (size_t)(g->S + 31) / 32;
     const int nw = g_a8_waves ? g_a8_waves : g->S <= 256 ? 1 : 4;
     const size_t nblk = pairs * ((qt + nw - 1) / nw);
     if (nblk * (size_t)(64 * nw) >= (size_t)1 << 32) mi_die("at_fa8_fwd: %zu workgroups exceed the launch grid", nblk);
-    a8_fwd_k<<<(unsigned)nblk, 64 * nw, nw == 4 ? 4 * 26 * 64 * sizeof(float) : 0>>>(q8, qs, k8, ks, vt, vts, o, lse, g->S, Sp, H, C, R, 1.4426950408889634f / sqrtf((float)HD), (unsigned)pairs);
+    a8_fwd_k<<<(unsigned)nblk, 64 * nw, nw == 4 ? 4 * 26 * 64 * sizeof(float) : 0>>>(w.q8, w.qs, w.k8, w.ks, w.vt, w.vts, o, lse, g->S, w.Sp, H, C, w.R, 1.4426950408889634f / sqrtf((float)HD), (unsigned)pairs);
     MICK();
+}
+}
+extern "C" int at_fa8_fwd(const void *qkvh, float *o, float *lse, const at_geom *g, int H, int C) {
+    if (!g || g->nseq <= 0 || g->S <= 0 || H <= 0) return 0;
+    if (C != H * HD) mi_die("at_fa8_fwd: C %d is not %d heads of %d", C, H, HD);
+    if (g->lens || g->rays) mi_die("at_fa8_fwd: per-sequence lengths and ray geometry are not supported");
+    a8_ops w;
+    if (!a8_carve(&w, g, H)) return -1;
+    const long long Tp = (long long)g->nseq * g->S + FT;
+    const __half *Qh = (const __half *)qkvh, *Kh = Qh + (size_t)H * Tp * HD, *Vh = Kh + (size_t)H * Tp * HD;
+    // (queries and keys in one launch: their sources, code planes and scale planes each lie one fixed stride apart)
+    a8_rows_k<<<dim3(nblk_((size_t)H * w.R * 4, 256), 2), 256>>>(Qh, w.q8, w.qs, H, g->nseq, g->S, w.Sp, Tp, (size_t)(Kh - Qh), (size_t)(w.k8 - w.q8), (size_t)(w.ks - w.qs));
+    a8_vt_k<<<nblk_((size_t)H * (w.R / 32), 4), 256>>>(Vh, w.vt, w.vts, H, g->nseq, g->S, w.Sp, Tp);
+    a8_core(w, o, lse, g, H, C);
+    return 0;
+}
+// (internal) at_fa_pack and at_fa8_fwd from the projection's rows qkv [T][3 C], 16-byte aligned, without the binary16 tensor between them: the same operands, the same
+// outputs, rq / rk / amx included (amx: four floats that are zero when this runs). Tokens x heads below 2^28 (the launch grid)
+int mi_fa8_from_qkv(const float *qkv, const float *qg, const float *kg, float *rq, float *rk, float *amx, float *o, float *lse, const at_geom *g, int nreg, int H, int rope, float base) {
+    a8_ops w;
+    if (!a8_carve(&w, g, H)) return -1;
+    const rope_t rp = {rope, g->S, g->Hh, g->W, nreg, log2f(base), rope ? g->pos : nullptr};
+    const size_t nb = (size_t)(w.R / 64 + 7) / 8 * 8 * 3 * H;
+#define A8P(MODE) a8_pack_k<MODE><<<(unsigned)nb, 256>>>(qkv, qg, kg, w.q8, w.qs, (size_t)(w.k8 - w.q8), (size_t)(w.ks - w.qs), w.vt, w.vts, rq, rk, amx, H, g->S, (unsigned)(w.Sp / 64), w.R, rp)
+    switch (rope_mode(rp)) { case ROPE_TABLE: A8P(ROPE_TABLE); break; case ROPE_REAL: A8P(ROPE_REAL); break; default: A8P(ROPE_EACH); }
+#undef A8P
+    a8_core(w, o, lse, g, H, H * HD);
     return 0;
 }

@@ -5,6 +5,10 @@
 #include "mx_dev.hpp"
 #include "../../include/mi_attn.h"
 #include "attn_ray.hpp"
+#include "attn_rope.hpp"
+
+// (attn8.hip)
+int mi_fa8_from_qkv(const float *qkv, const float *qg, const float *kg, float *rq, float *rk, float *amx, float *o, float *lse, const at_geom *g, int nreg, int H, int rope, float base);
 
 #define HD AT_HD
 #define FT 64
@@ -18,7 +22,8 @@
 // lanes, whose maxima meet through three lane exchanges. C a multiple of 64
 template <int NV, bool PK = false>
 __global__ void __launch_bounds__(256) ln_row_k(const float4 *__restrict__ x, const float *__restrict__ g, const float *__restrict__ b, float4 *__restrict__ y,
-                                                float *__restrict__ mean, float *__restrict__ rstd, long long T, int C4, uint8_t *__restrict__ pq = nullptr, uint8_t *__restrict__ ps = nullptr) {
+                                                float *__restrict__ mean, float *__restrict__ rstd, long long T, int C4, uint8_t *__restrict__ pq = nullptr, uint8_t *__restrict__ ps = nullptr, float *__restrict__ zero4 = nullptr) {
+    if (PK && zero4 && blockIdx.x == 0 && threadIdx.x < 4) zero4[threadIdx.x] = 0.f;      // (four words that a later kernel of the stream accumulates into)
     const long long row = blockIdx.x * 4ll + (threadIdx.x >> 6); const int lane = threadIdx.x & 63;
     if (row >= T) return;
     const float4 *xr = x + row * C4;
@@ -85,10 +90,10 @@ extern "C" void at_ln_fwd(const float *x, const float *g, const float *b, float 
     MICK();
 }
 // at_ln_fwd with the normalised rows written as the packed MX-fp8 A operand of the GEMM that follows (no fp32 rows); C a multiple of 64
-static void ln_pack_fwd(const float *x, const float *g, const float *b, float *mean, float *rstd, long T, int C, uint8_t *pq, uint8_t *ps) {
+static void ln_pack_fwd(const float *x, const float *g, const float *b, float *mean, float *rstd, long T, int C, uint8_t *pq, uint8_t *ps, float *zero4 = nullptr) {
     const int C4 = C / 4, nv = (C4 + 63) / 64;
     const unsigned grid = nblk_((size_t)T, 4);
-#define LN(NV) ln_row_k<NV, true><<<grid, 256>>>((const float4 *)x, g, b, nullptr, mean, rstd, T, C4, pq, ps)
+#define LN(NV) ln_row_k<NV, true><<<grid, 256>>>((const float4 *)x, g, b, nullptr, mean, rstd, T, C4, pq, ps, zero4)
     if (nv <= 1) LN(1); else if (nv <= 2) LN(2); else if (nv <= 4) LN(4); else LN(8);
 #undef LN
     MICK();
@@ -185,17 +190,12 @@ extern "C" void at_tok_to_cs(const float *t, float *x, int n, int C, long Sg, in
 // loads and one 16-byte store of eight halves. The sum of squares meets over the unit's lanes; a rotary pair never leaves its lane
 // (slice j covers pairs 4 (j & 1) .. + 3 of axis j / 2). ----
 struct ray_src { ray_geo G; const float *ray; const int *ad; };      // ray: null = the rows are the tokens' own
+template <int MODE>
 __global__ void __launch_bounds__(256) qkv_pack_k(const float *__restrict__ qkv, const float *__restrict__ qg, const float *__restrict__ kg, __half *__restrict__ out,
-                                                  float *__restrict__ rq, float *__restrict__ rk, float *__restrict__ amx, long long T, int H, int S, int Hh, int W, int nreg, int rope, float lbase,
-                                                  const float *__restrict__ gpos, ray_src rs) {
-    // the rotary angles take few values - position along an axis x frequency - and a sine / cosine pair costs far more than the rest of a unit:
-    // a block forms the table once (the same expression the per-value form evaluates, so the same bits), positions up to RP per axis
-    constexpr int RP = 64;
-    __shared__ float2 rtab[RP * 8];
-    const int pmax = max(max(S / (Hh * W), Hh), W);         // positions along an axis: < pmax (registers included in S: an upper bound)
-    const bool tab = rope && !gpos && pmax <= RP;            // (gpos: per-token coordinates, real numbers: every angle is evaluated)
-    if (tab) {
-        for (int i = threadIdx.x; i < pmax * 8; i += 256) { float sn, cs; sincosf((float)(i >> 3) * exp2f(-lbase * (float)(i & 7) / 8.f), &sn, &cs); rtab[i] = make_float2(sn, cs); }
+                                                  float *__restrict__ rq, float *__restrict__ rk, float *__restrict__ amx, long long T, int H, rope_t rp, ray_src rs) {
+    __shared__ float2 rtab[ROPE_TAB * 8];
+    if (MODE == ROPE_TABLE && rp.on) {
+        rope_fill(rtab, rope_positions(rp), rp.lbase);
         __syncthreads();
     }
     const long long unit = (blockIdx.x * 256ll + threadIdx.x) >> 3; const int j = threadIdx.x & 7;
@@ -245,20 +245,11 @@ __global__ void __launch_bounds__(256) qkv_pack_k(const float *__restrict__ qkv,
                     const float *gs = (p ? kg : qg) + h * HD + 8 * j;      // (the gains sit at an arbitrary offset of the flat parameter vector: dword loads)
 #pragma unroll
                     for (int i = 0; i < 8; i++) v[i] *= r * gs[i];
-                    const int ts = (int)(t % S) - nreg;
-                    if (rope && ts >= 0) {
-                        const int ax = j >> 1;
-                        const float pos = gpos ? gpos[3 * t + ax] : ax == 0 ? (float)(ts / (Hh * W)) : ax == 1 ? (float)((ts / W) % Hh) : (float)(ts % W);
+                    const int ts = (int)(t % rp.S) - rp.nreg;
+                    if (rp.on && ts >= 0) {
+                        const float pos = rope_pos<MODE>(rp, t, ts, j >> 1);
 #pragma unroll
-                        for (int i = 0; i < 4; i++) {
-                            const int fi = 4 * (j & 1) + i;
-                            float sn, cs;
-                            if (tab) { const float2 sc2 = rtab[(int)pos * 8 + fi]; sn = sc2.x; cs = sc2.y; }
-                            else if (gpos) { const float ang = pos * exp2f(-lbase * (float)fi / 8.f); sn = __sinf(ang); cs = __cosf(ang); }      // (real coordinates: the hardware sine / cosine, as the reference's fast-math build)
-                            else sincosf(pos * exp2f(-lbase * (float)fi / 8.f), &sn, &cs);
-                            const float a = v[2 * i], b = v[2 * i + 1];
-                            v[2 * i] = a * cs - b * sn; v[2 * i + 1] = a * sn + b * cs;
-                        }
+                        for (int i = 0; i < 4; i++) rope_turn<MODE>(rp, rtab, pos, 4 * (j & 1) + i, v[2 * i], v[2 * i + 1]);
                     }
                 }
             } else {
@@ -286,7 +277,10 @@ static void fa_pack(const float *qkv, const float *qg, const float *kg, void *qk
     ray_src rs = {};
     if (R) { rs.G = geo_of(R); rs.ray = R->ray; rs.ad = R->ad; }
     at_zero4_k<<<1, 64>>>(amx);
-    qkv_pack_k<<<nblk_((size_t)Tp * H * 3 * 8, 256), 256>>>(qkv, qg, kg, (__half *)qkvh, rq, rk, amx, T, H, g->S, g->Hh, g->W, nreg, rope, log2f(base), rope ? g->pos : nullptr, rs);
+    const rope_t rp = {rope, g->S, g->Hh, g->W, nreg, log2f(base), rope ? g->pos : nullptr};
+#define QP(MODE) qkv_pack_k<MODE><<<nblk_((size_t)Tp * H * 3 * 8, 256), 256>>>(qkv, qg, kg, (__half *)qkvh, rq, rk, amx, T, H, rp, rs)
+    switch (rope_mode(rp)) { case ROPE_TABLE: QP(ROPE_TABLE); break; case ROPE_REAL: QP(ROPE_REAL); break; default: QP(ROPE_EACH); }
+#undef QP
     MICK();
 }
 extern "C" void at_fa_pack(const float *qkv, const float *qg, const float *kg, void *qkvh, float *rq, float *rk, float *amx, const at_geom *g, int nreg, int C, int rope, float base) {
@@ -405,11 +399,14 @@ extern "C" int at_block_fwd(const at_dims *d, const float *P, const at_bp *bp, c
     // read again) are not: per block 1.8 GB less HBM traffic at 250 000 tokens and three launches fewer. The same values quantised the same way
     const bool fuse = g_fuse_pack && g_at_mx == 8 && C % 64 == 0 && F % 64 == 0 && !((uintptr_t)x & 15) && !((uintptr_t)w->x1 & 15) && !((uintptr_t)w->h & 15);
     uint8_t *aq = nullptr, *as = nullptr;
+    // ... and the full attention's pack writes the core's quantised operands from the projection's rows; the binary16 tensor (qkvh) is not stored
+    bool direct = fuse && g_fuse_pack > 1 && !R && !((uintptr_t)w->qkv & 15) && g->S > 0 && (long long)T * d->H < 1ll << 28;
     // attention branch
     if (fuse && mi_mx_gemm_abuf(8, (int)T, 3 * C, C, &aq, &as)) {
-        ln_pack_fwd(x, P + bp->ln1g, P + bp->ln1b, w->m1, w->r1, T, C, aq, as);
+        ln_pack_fwd(x, P + bp->ln1g, P + bp->ln1b, w->m1, w->r1, T, C, aq, as, direct ? w->amx : nullptr);
         if (int e = mi_mx_gemm_apacked(8, 1, (int)T, 3 * C, C, qkv.w, w->qkv, 0.f, qkv.b, nullptr)) return e;
     } else {
+        direct = false;
         at_ln_fwd(x, P + bp->ln1g, P + bp->ln1b, w->xn, w->m1, w->r1, T, C);
         if (int e = linear(qkv, T, w->xn, w->qkv, nullptr)) return e;
     }
@@ -423,6 +420,8 @@ extern "C" int at_block_fwd(const at_dims *d, const float *P, const at_bp *bp, c
         fa_pack(w->qkv, P + bp->qg, P + bp->kg, w->qkvh, w->rq, w->rk, w->amx, &ga, 0, C, d->rope, d->rope_base, R);
         at_fa_fwd(w->qkvh, w->orr, w->lse, &ga, d->H, C);
         at_ray_scatter(R, w->orr, w->o, C, 1);
+    } else if (direct) {
+        if (int e = mi_fa8_from_qkv(w->qkv, P + bp->qg, P + bp->kg, w->rq, w->rk, w->amx, w->o, w->lse, &ga, d->nreg, d->H, d->rope, d->rope_base)) return e;
     } else {
         at_fa_pack(w->qkv, P + bp->qg, P + bp->kg, w->qkvh, w->rq, w->rk, w->amx, &ga, d->nreg, C, d->rope, d->rope_base);
         if (int e = at_fa8_fwd(w->qkvh, w->o, w->lse, &ga, d->H, C)) return e;
