@@ -64,6 +64,23 @@ def test_gemm_epilogue_exact_operands(gpu, bits):
     assert lib.lp_mx_gemm(8, 0, 0, 0, 4, 4, None, None, None, 0.0) == 0          # empty output: nothing to do
 
 
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("M,N,K", [(1, 1, 64), (33, 65, 64), (70, 45, 192), (31, 130, 320), (40, 64, 576), (7105, 576, 64), (8190, 520, 128), (65500, 1030, 64)])
+def test_gemm_tiles_exact(gpu, bits, M, N, K):
+    """The wavefront tiles of 32 and 64 rows (their rule's sides: 1 008 and 1 152 tiles of 64 x 64), the four-wavefront workgroups (17 408 tiles, N above 1 024), partial tiles in
+    both directions, 1 to 9 K steps (groups of two, two in flight): products of small integers are exact, so the output equals them, with a residual that is
+    C itself as well."""
+    rng = np.random.default_rng(M + K)
+    A = rng.integers(-4, 5, (M, K)).astype(np.float32); A[:, ::32] = 4
+    B = rng.integers(-4, 5, (N, K)).astype(np.float32); B[:, ::32] = 4
+    bias = rng.integers(-8, 9, N).astype(np.float32); res = rng.integers(-8, 9, (M, N)).astype(np.float32)
+    exact = A @ B.T + bias + res                                  # (below 2^24: exact in fp32 whatever the order)
+    dA, dB, dC, db = DevBuf.from_numpy(A), DevBuf.from_numpy(B), DevBuf.from_numpy(res), DevBuf.from_numpy(bias)
+    assert lib.lp_mx_gemm_ex(bits, 0, 1, M, N, K, dA.ptr, dB.ptr, dC.ptr, 0.0, db.ptr, dC.ptr) == 0
+    LP.check()
+    assert np.array_equal(dC.to_numpy(np.float32, (M, N)), exact)
+
+
 @pytest.mark.parametrize("bits,beta", [(4, 0.0), (8, 0.0), (8, 1.0)])
 def test_gemm_split_k(gpu, bits, beta):
     """The weight-gradient shape: few output tiles, K = tokens (tests/test_attn.c:447): K is split over workgroups that add atomically."""

@@ -57,20 +57,114 @@ __global__ void gemm_zero_k(float *c, size_t n) {
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) c[i] = 0.f;
 }
 
-// C tile of 64 x 256 per workgroup (four wavefronts side by side along N), 64 x 64 per wavefront = 2 x 2 MFMA tiles of 32 x 32; K in steps of 64 = the two 32-K blocks the
+// A wavefront owns a C tile of 64 or 32 rows x 64 columns, MFMA tiles of 32 x 32; K in steps of 64 = the two 32-K blocks the
 // scale operands of the lane halves of a 32x32x64 MFMA cover. A lane's fragment is 16 bytes of each of the two blocks (e4m3: bytes
-// 16 h ... of both; e2m1: all 16 bytes of block h), so fragments are loaded from the packed rows in global memory directly: the four
-// wavefronts of a workgroup read the same A rows through the vector cache.
+// 16 h ... of both; e2m1: all 16 bytes of block h), so fragments are loaded from the packed rows in global memory directly.
+// Workgroups go to the XCDs in turn: eight row tiles at a time, a row tile's column tiles are those of one XCD, whose L2 then reads its rows of A once.
 // gridDim.z > 1: split K, each split adds its part into C atomically (C zeroed or kept by the host; no bias / residual then).
+struct gemm_tile_t { int m0, n0; };
+__device__ __forceinline__ gemm_tile_t gemm_tile(int nx, int rows, int wn, int wave) {
+    const unsigned u = blockIdx.x >> 3, g = u / (unsigned)nx, x = u - g * (unsigned)nx, y = g * 8 + (blockIdx.x & 7);
+    return gemm_tile_t{(int)y * rows, ((int)x * wn + wave) * 64};
+}
+// 32 x 64 per wavefront, for launches of up to a wavefront per SIMD or so (fewer than 1 024 tiles of 64 x 64): such a launch lasts as long as one tile, so it
+// is one round trip to memory, the products and the stores: the residual (or old) values and the operands of two groups of two steps are requested before the
+// first product. Whole calls with the operand's pack, us, on 192 -> 192 with residual / 512 -> 192 with residual / 192 -> 576, against the 64 x 64 form: 516 rows 7.5 / 9.0 / 7.8 against
+// 10.6 / 13.6 / 10.0; 8 200 rows 9.6 / 16.2 / 15.9 against 12.7 / 19.1 / 14.5; 36 900 rows 24.9 / 51 / 39 against 22.8 / 43 / 37
 template <int BITS>
-__global__ void __launch_bounds__(256) mx_gemm_k(const uint8_t *__restrict__ Aq, const uint8_t *__restrict__ As, const uint8_t *__restrict__ Bq, const uint8_t *__restrict__ Bs,
-                                                 float *C, int M, int N, int nkb, float beta, const float *__restrict__ bias, const float *res, int sper) {
+__global__ void __launch_bounds__(64) mx_gemm_k(const uint8_t *__restrict__ Aq, const uint8_t *__restrict__ As, const uint8_t *__restrict__ Bq, const uint8_t *__restrict__ Bs,
+                                                 float *C, int M, int N, int nkb, float beta, const float *__restrict__ bias, const float *res, int sper, int nx) {
+    constexpr int BPB = BITS == 8 ? 32 : 16, FM = BITS == 8 ? 0 : 4, G = 2;
+    const int lane = threadIdx.x, r = lane & 31, h = lane >> 5;
+    const gemm_tile_t t = gemm_tile(nx, 32, 1, 0);
+    const int m0 = t.m0, n0 = t.n0;
+    if (m0 >= M || n0 >= N) return;
+    const int nst = nkb >> 1, s0 = (int)blockIdx.z * sper, s1 = min(nst, s0 + sper);
+    const size_t ra = (size_t)min(m0 + r, M - 1);           // rows past the edge repeat the last one (never stored)
+    const uint8_t *pa = Aq + ra * nkb * BPB + 16 * h, *sa = As + ra * nkb + h, *pb[2], *sb[2];      // (e2m1: + 16 h is block h of a step; e4m3: the lane's half of both blocks)
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const size_t rb = (size_t)min(n0 + 32 * j + r, N - 1);
+        pb[j] = Bq + rb * nkb * BPB + 16 * h; sb[j] = Bs + rb * nkb + h;
+    }
+    auto frag = [&](const uint8_t *p) {
+        const v4i lo = *(const v4i *)p;
+        if (BITS == 8) { const v4i hi = *(const v4i *)(p + 32); return (v8i){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]}; }
+        return (v8i){lo[0], lo[1], lo[2], lo[3], 0, 0, 0, 0};
+    };
+    struct group_t { v8i fa[G], fb[G][2]; int ea[G], eb[G][2]; };
+    auto load = [&](group_t &g, int s) {                   // (steps past the last re-read it: their products are skipped)
+#pragma unroll
+        for (int k = 0; k < G; k++) {
+            const int sk = min(s + k, s1 - 1);
+            g.fa[k] = frag(pa + (size_t)sk * 2 * BPB); g.ea[k] = sa[2 * sk];
+#pragma unroll
+            for (int j = 0; j < 2; j++) { g.fb[k][j] = frag(pb[j] + (size_t)sk * 2 * BPB); g.eb[k][j] = sb[j][2 * sk]; }
+        }
+    };
+    group_t ga, gb;
+    if (s0 < s1) load(ga, s0);
+    if (s0 + G < s1) load(gb, s0 + G);
+    // accumulator element q of lane (r, h): row (q & 3) + 4 h + 8 (q >> 2), column r of its 32 x 32 tile
+    const bool split = gridDim.z > 1;
+    float add[2][16];
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const int col = min(n0 + 32 * j + r, N - 1);
+        const float bv = bias ? bias[col] : 0.f;
+#pragma unroll
+        for (int q = 0; q < 16; q++) add[j][q] = bv;
+        if (res && !split) {                                // (uniform; res may be C itself: a wavefront reads the very values it stores, before it does)
+#pragma unroll
+            for (int q = 0; q < 16; q++) add[j][q] += res[(size_t)min(m0 + (q & 3) + 4 * h + 8 * (q >> 2), M - 1) * N + col];
+        }
+        if (beta != 0.f && !split) {                        // (uniform)
+#pragma unroll
+            for (int q = 0; q < 16; q++) add[j][q] += beta * C[(size_t)min(m0 + (q & 3) + 4 * h + 8 * (q >> 2), M - 1) * N + col];
+        }
+    }
+    v16f acc[2];
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+        for (int q = 0; q < 16; q++) acc[j][q] = 0.f;
+    auto products = [&](group_t &g, int s) {
+#pragma unroll
+        for (int k = 0; k < G; k++) {
+            if (s + k < s1) {                               // (uniform)
+#pragma unroll
+                for (int j = 0; j < 2; j++) acc[j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(g.fa[k], g.fb[k][j], acc[j], FM, FM, 0, g.ea[k], 0, g.eb[k][j]);
+            }
+        }
+    };
+    for (int s = s0; s < s1; s += 2 * G) {
+        products(ga, s);
+        if (s + 2 * G < s1) load(ga, s + 2 * G);
+        if (s + G < s1) products(gb, s + G);
+        if (s + 3 * G < s1) load(gb, s + 3 * G);
+    }
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const int col = n0 + 32 * j + r;
+        if (col >= N) continue;
+#pragma unroll
+        for (int q = 0; q < 16; q++) {
+            const int row = m0 + (q & 3) + 4 * h + 8 * (q >> 2);
+            if (row >= M) continue;
+            float *p = C + (size_t)row * N + col;
+            if (split) atomicAdd(p, acc[j][q]); else *p = acc[j][q] + add[j][q];
+        }
+    }
+}
+// 64 x 64 per wavefront: a third less of the operands read per product, and three wavefronts per SIMD. One wavefront per workgroup, or four of them side by side along N (wide
+// outputs of many rows: runs of 1 KiB of a C row; 250 000 rows, 192 -> 1 024 389 against 459 us, 192 -> 576 284 against 282)
+template <int BITS>
+__global__ void __launch_bounds__(256) mx_gemm_tall_k(const uint8_t *__restrict__ Aq, const uint8_t *__restrict__ As, const uint8_t *__restrict__ Bq, const uint8_t *__restrict__ Bs,
+                                                 float *C, int M, int N, int nkb, float beta, const float *__restrict__ bias, const float *res, int sper, int nx) {
     constexpr int BPB = BITS == 8 ? 32 : 16, FM = BITS == 8 ? 0 : 4;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 31, h = lane >> 5;
-    // a wavefront owns a 64 x 64 tile; a workgroup is four of them in a row, or a single one (few tiles: more workgroups than CUs that way)
-    // (four wavefronts: side by side along N, so the workgroup writes runs of 1 KiB of a C row and shares its A rows)
-    const int wn = blockDim.x >> 6;
-    const int m0 = blockIdx.y * 64, n0 = (blockIdx.x * wn + wave) * 64;
+    const gemm_tile_t t = gemm_tile(nx, 64, blockDim.x >> 6, wave);
+    const int m0 = t.m0, n0 = t.n0;
     if (m0 >= M || n0 >= N) return;                        // (no barriers in this kernel: a wavefront without work leaves)
     const int nst = nkb >> 1, s0 = (int)blockIdx.z * sper, s1 = min(nst, s0 + sper);
     const uint8_t *pa[2], *pb[2], *sa[2], *sb[2];
@@ -228,11 +322,13 @@ static int gemm_impl(int bits, int ta, int tb, int M, int N, int K, const float 
     const int sper = ns > 1 ? (nst + ns - 1) / ns : (nst > 0 ? nst : 1);
     ns = nst > 0 ? (nst + sper - 1) / sper : 1;
     if (ns > 1 && beta == 0.f) gemm_zero_k<<<nblk_((size_t)M * N, 256 * 4), 256>>>(C, (size_t)M * N);   // (a kernel, not a memset node: safe under graph capture)
-    const int wt = (size_t)tiles * ns >= 512 ? 2 : 1;              // (few tiles: one wavefront per workgroup)
-    const int wn = wt == 2 ? 4 : 1;                                // wavefronts per workgroup, side by side along N
-    const dim3 grid((unsigned)((N + 64 * wn - 1) / (64 * wn)), (unsigned)((M + 63) / 64), (unsigned)ns);
-    if (bits == 8) mx_gemm_k<8><<<grid, 64 * wn>>>(Aq, As, Bq, Bs, C, M, N, nkb, beta, bias, res, sper);
-    else mx_gemm_k<4><<<grid, 64 * wn>>>(Aq, As, Bq, Bs, C, M, N, nkb, beta, bias, res, sper);
+    const size_t t64 = (size_t)((N + 63) / 64) * ((M + 63) / 64) * ns;
+    const bool tall = t64 >= 1024;                                 // (the kernels' comments)
+    const int wn = t64 >= 16384 && N >= 1024 ? 4 : 1, nx = (N + 64 * wn - 1) / (64 * wn), ny = tall ? (M + 63) / 64 : (M + 31) / 32;
+    const dim3 grid((unsigned)((ny + 7) / 8 * 8 * nx), 1, (unsigned)ns);
+#define MG(K) K<<<grid, 64 * wn>>>(Aq, As, Bq, Bs, C, M, N, nkb, beta, bias, res, sper, nx)
+    if (bits == 8) { if (tall) MG(mx_gemm_tall_k<8>); else MG(mx_gemm_k<8>); } else { if (tall) MG(mx_gemm_tall_k<4>); else MG(mx_gemm_k<4>); }
+#undef MG
     MICK();
     return 0;
 }
