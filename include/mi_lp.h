@@ -110,6 +110,9 @@ int mi_conv_prestage(const void *x, int xdt, shape5 s, gnp_t gp, void *y, int yb
    split conv's second segment is stored as MX-fp4 although x is MX-fp8 (3: MX-fp8 beside an MX-fp4 x; the descriptor carries one format) */
 int mi_conv_prestage2(const void *x, shape5 s, gnp_t gp, void *y8, void *y4);
 void mi_conv_x2_dt(int dt);
+/* mi_conv_up_staged(1) before a conv entry: the calling thread's next split conv's upsampled segment is stored as the e4m3 rows that its own pre-pass (GroupNorm + SiLU +
+   re-quantisation) would make, so it is upsampled as it is (MX-fp8, a multiple of 32 channels; its GroupNorm must be none) */
+void mi_conv_up_staged(int on);
 gnp_t gnp_mk(const float *gamma, const float *beta, const float *mean, const float *rstd, int G);   /* src/nn_lp.h:19 */
 int lp_gn_slab_any(void);                                                                         /* src/nn_lp.h:20: any statistics array registered */
 /* the statistics array `mean` holds one row per (sample, z-slab) with this geometry: every gnp_t gnp_mk builds from it (and lp_gn_silu_apply_mx,
@@ -202,6 +205,12 @@ int mi_convt_up2_fwd(int bits, const void *x, int xbf, shape5 xs, const float *w
    mean and 1 / sqrt(var + eps), bit-identical to mi_gn_sums_zero + lp_conv_fwd_f8 / _f4 + mi_gn_finalize. */
 int mi_conv_fwd_gn(int bits, const void *x, int xbf, shape5 xs, const float *w, const float *b, int cout, void *y, int ybf, gnp_t gp,
                    double *osum, int Go, split_t sp, float eps, float *omean, float *orstd);
+/* ... and what mi_conv_prestage then makes of its output under these statistics: silu(gn(y)) with the given affine as MX-fp8 rows st8 and / or MX-fp4 rows st4 (one of them
+   may be null; both: MX-fp8 y). With few records the pre-pass forms the statistics itself, one launch less; the same bytes in y, omean, orstd, st8 and st4 as the separate
+   calls' (the statistics are the same sums added in another order in double: equal but for a last bit now and then). osum is scratch. cout a multiple of 32, an MX y, no z-range;
+   0 on success, -1 for what it does not take (nothing is launched) */
+int mi_conv_fwd_gn_stage(int bits, const void *x, int xbf, shape5 xs, const float *w, const float *b, int cout, void *y, int ybf, gnp_t gp,
+                         double *osum, int Go, split_t sp, float eps, float *omean, float *orstd, const float *gamma, const float *beta, void *st8, void *st4);
 /* timing of the 3x3x3 conv kernel launches alone (benchmarks): on != 0 starts recording an event pair around every launch on the
    stream it runs on and clears the totals; read returns the total milliseconds so far and the number of launches (synchronises) */
 void mi_kernel_timing(int on);

@@ -41,6 +41,9 @@ int nn_conv3d_fwd_split(const float *x, const float *x2, int c_split, shape5 xs,
 /* input-side recompute conv: k 3 stride 1 (split / fused upsample / output statistics), k 3 stride 2, k 1 head (src/nn.h:432) */
 int nn_conv3d_fwd_x(const float *x, const nn_gn_t *gx, const float *x2, const nn_gn_t *gx2, int c_split, int up, shape5 xs,
                     const float *w, const float *b, int cout, int k, int stride, float *y, int G_out, float eps, float *omean, float *orstd);
+/* (no counterpart: the graph's form of the same conv on operand rows; nn_host.c) */
+int mi_nn_conv3d_rows(const void *x, int xrows, const nn_gn_t *gx, const void *x2, const nn_gn_t *gx2, int c_split, int up, int uprows, shape5 xs, const float *w, const float *b, int cout,
+                      void *y, int G_out, float eps, float *omean, float *orstd, const float *gamma, const float *beta, void *st8, void *st4);
 void nn_set_zrange(int zi0, int Di, int first, int last, int Do, int zo);   /* the next stride-1 MX convs compute output planes [zo, zo + xs.d) of a depth-Do tensor, plane z reading
                                                                                input plane z + zi0 of a depth-Di input; sums zeroed by the first, finalised by the last call; Di 0 = off
                                                                                (src/nn_bwd.cu:33-36) */

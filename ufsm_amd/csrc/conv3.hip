@@ -12,31 +12,21 @@ __device__ __forceinline__ void gn_part_finish(double *osum, double s, double ss
     const size_t i = 2 * (size_t)ng;
     if (!fin.mean) { gn_acc_add(osum, i, s); gn_acc_add(osum, i + 1, ss); return; }
     unsigned long long *w = (unsigned long long *)osum + 3 * i;
-    double v[2] = {s, ss}, got[2];
-#pragma unroll
-    for (int k = 0; k < 2; k++) {                       // the slot a single exact add to a cleared slot would leave, and its value read back
-        if (!(fabs(v[k]) < 4.611686018427387904e18)) { w[3 * k] = 0ull; w[3 * k + 1] = 0ull; w[3 * k + 2] = 1ull; got[k] = __longlong_as_double(0x7ff8000000000000ll); continue; }
-        const double f = floor(v[k]);
-        const unsigned long long lo = (unsigned long long)((v[k] - f) * 18446744073709551616.0);
-        w[3 * k] = lo; w[3 * k + 1] = (unsigned long long)(long long)f; w[3 * k + 2] = 0ull;
-        got[k] = (double)(long long)f + (double)lo * 5.42101086242752217e-20;
-    }
-    const double m = got[0] / fin.len, var = got[1] / fin.len - m * m;
-    fin.mean[ng] = (float)m;
-    fin.rstd[ng] = (float)(1.0 / sqrt((var > 0 ? var : 0) + (double)fin.eps));
+    const double gs = gn_slot_value(s, w), gss = gn_slot_value(ss, w + 3);
+    gn_mean_rstd(gs, gss, fin.len, fin.eps, fin.mean + ng, fin.rstd + ng);
 }
 
 // (sum, sum of squares) partials of the tiles -> exact GroupNorm sum slots (src/lp_common.cuh:1575-1597 does the same with one fixed-point atomic
 // per block and channel). A spatial tile's record is Q = Co / 4 (padded to whole channel slices) consecutive float2, one per channel quad; quad
 // Q = co / 4 lives in channel slice Q / (8 MT), slot Q % (8 MT). A block takes one sample's tiles [t0, t1) with ALL their quads: thread (j, q) adds
-// quad q of tiles t0 + j, t0 + j + J, ... in double (consecutive threads read consecutive records: every fetched line is used whole), then thread
-// g adds its group's quads over the J rows in a fixed order. nsplit > 1 (thousands of tiles: the level-0 layers): every block leaves its Go pairs
+// quad q of tiles t0 + j, t0 + j + J, ... in double (consecutive threads read consecutive records: every fetched line is used whole), then the J
+// rows of partial sums are added in halves down to four, and thread g adds its group's quads over these, all in a fixed order. nsplit > 1 (thousands of tiles: the level-0 layers): every block leaves its Go pairs
 // in scr and takes a ticket of its sample; the block that draws the last one adds the nsplit pairs of every group in index order - the result
 // does not depend on which block that is - and puts the ticket counter back to zero for the next launch
 struct gn_split_t { int nsplit; double *scr; unsigned *cnt; };
-__global__ void __launch_bounds__(256) gn_part_reduce_k(const float2 *part, int tiles_per_n, int ncs, int MT, int Co, int Go, double *osum, gn_fin_t fin, gn_split_t sp) {
-    const int n = (int)blockIdx.x / sp.nsplit, pi = (int)blockIdx.x % sp.nsplit, tid = (int)threadIdx.x;
-    const int Q = ncs * MT * 8, nst = tiles_per_n / ncs, qpg = Co / Go / 4, J = 256 / Q;
+__global__ void __launch_bounds__(1024) gn_part_reduce_k(const float2 *part, int tiles_per_n, int ncs, int MT, int Co, int Go, double *osum, gn_fin_t fin, gn_split_t sp) {
+    const int n = (int)blockIdx.x / sp.nsplit, pi = (int)blockIdx.x % sp.nsplit, tid = (int)threadIdx.x, nth = (int)blockDim.x;
+    const int Q = ncs * MT * 8, nst = tiles_per_n / ncs, qpg = Co / Go / 4, J = nth / Q;
     const int per = (nst + sp.nsplit - 1) / sp.nsplit, t0 = pi * per, t1 = min(nst, t0 + per);
     const int q = tid % Q, j = tid / Q;
     const float2 *rec = part + (size_t)n * tiles_per_n * (MT * 8) + q;
@@ -48,14 +38,21 @@ __global__ void __launch_bounds__(256) gn_part_reduce_k(const float2 *part, int 
             s += (double)p.x; ss += (double)p.y;
         }
     }
-    __shared__ double r1[256], r2[256];
+    __shared__ double r1[1024], r2[1024];
     __shared__ unsigned ticket;
     r1[tid] = s; r2[tid] = ss;
     __syncthreads();
+    for (int m = J; m > 4;) {                                                // the J rows of partial sums in halves down to four, in a fixed order
+        const int hlf = (m + 1) >> 1;
+        if (j < m - hlf) { r1[tid] += r1[tid + hlf * Q]; r2[tid] += r2[tid + hlf * Q]; }
+        __syncthreads();
+        m = hlf;
+    }
+    int JJ = J; while (JJ > 4) JJ = (JJ + 1) >> 1;
     s = 0.0; ss = 0.0;
     if (tid < Go)
         for (int k = 0; k < qpg; k++)
-            for (int jj = 0; jj < J; jj++) { s += r1[jj * Q + tid * qpg + k]; ss += r2[jj * Q + tid * qpg + k]; }
+            for (int jj = 0; jj < JJ; jj++) { s += r1[jj * Q + tid * qpg + k]; ss += r2[jj * Q + tid * qpg + k]; }
     if (sp.nsplit == 1) { if (tid < Go) gn_part_finish(osum, s, ss, fin, (unsigned)(n * Go + tid)); return; }
     if (tid < Go) {
         double *mine = sp.scr + 2 * ((size_t)blockIdx.x * Go + tid);
@@ -245,10 +242,28 @@ extern "C" const char *mi_last_kernel(void) { return g_last_kernel; }
 // set by mi_conv_fwd_gn around its conv: finalize the statistics in the reduce kernel
 static thread_local gn_fin_t g_fin = {nullptr, nullptr, 0.0, 0.f};
 // GroupNorm partial sums of a conv's tiles -> the caller's sum slots (and mean / rstd when mi_conv_fwd_gn asked for them)
+// set by mi_conv_fwd_gn_stage around its conv: silu(gn(output)) as the next reader's operand rows
+struct gn_stage_t { const float *gamma, *beta; void *y8, *y4; };
+static thread_local gn_stage_t g_stage = {nullptr, nullptr, nullptr, nullptr};
 static void conv_stats_reduce(const char *who, const conv_args &a, int MT, split_t sp, double *osum) {
     gn_fin_t fin = g_fin;
     fin.len = (double)(a.Co / a.Go) * (double)a.Do * a.Ho * a.Wo;
     if (fin.mean && (sp.zlo || sp.zhi)) mi_die("%s: fused finalize with a z range", who);
+    if (g_stage.gamma) {
+        // few records: the pre-pass that follows adds them itself, one launch less (its rule: mi_restage_records)
+        const gn_stage_t g = g_stage; g_stage.gamma = nullptr;
+        const int xdt = a.ydt; const size_t S = (size_t)a.Do * a.Ho * a.Wo;
+        const gn_records_t rec = {(const float2 *)a.part, (int)(a.ntiles / a.N) * (a.row1 ? 8 : 1) / a.ncs, a.ncs * MT * 8, a.Go, fin.len, fin.eps, fin.mean, fin.rstd};
+        if (!a.stat_ch && mi_restage_records(a.y, xdt, a.N, a.Co, S, g.gamma, g.beta, rec, g.y8, g.y4)) return;
+        conv_stats_reduce(who, a, MT, sp, osum);
+        gnp_t gp; memset(&gp, 0, sizeof gp); gp.gamma = g.gamma; gp.beta = g.beta; gp.mean = fin.mean; gp.rstd = fin.rstd; gp.G = a.Go;
+        if (g.y8 && g.y4 && xdt == 3) mi_restage_sub2(a.y, a.N, a.Co, S, gp, g.y8, g.y4, S, 0);
+        else {
+            if (g.y8) mi_restage_sub(a.y, xdt, a.N, a.Co, S, gp, a.Co, 0, g.y8, 8, S, 0);
+            if (g.y4) mi_restage_sub(a.y, xdt, a.N, a.Co, S, gp, a.Co, 0, g.y4, 4, S, 0);
+        }
+        return;
+    }
     if (a.stat_ch) { gn_part_reduce_ch_k<<<a.N * a.Go, 256>>>((const float2 *)a.part, (int)(a.ntiles / a.N), a.ncs, a.Co, a.Go, osum, fin); MICK(); return; }
     const int tiles_per_n = (int)(a.ntiles / a.N) * (a.row1 ? 8 : 1);      // (row1: eight records per tile)
     const int Q = a.ncs * MT * 8, nst = tiles_per_n / a.ncs;
@@ -271,7 +286,9 @@ static void conv_stats_reduce(const char *who, const conv_args &a, int MT, split
         }
         gs.nsplit = want; gs.scr = scr[dv]; gs.cnt = cnt[dv];
     }
-    gn_part_reduce_k<<<a.N * gs.nsplit, 256>>>((const float2 *)a.part, tiles_per_n, a.ncs, MT, a.Co, a.Go, osum, fin, gs);
+    // (one block per sample over more than a few hundred records: four times the threads, 2 002 records of 8 quads 10.4 -> 8.2 us, 1 232 of 16 7.9 -> 6.6; the split launches' blocks
+    // are few rounds long already and lose by it, 7.3 -> 10.6)
+    gn_part_reduce_k<<<a.N * gs.nsplit, gs.nsplit == 1 && nst * Q > 8192 ? 1024 : 256>>>((const float2 *)a.part, tiles_per_n, a.ncs, MT, a.Co, a.Go, osum, fin, gs);
     MICK();
 }
 
@@ -338,6 +355,9 @@ extern "C" void mi_conv_split(int tiles) { g_split = tiles; }
 // storage format of the calling thread's next split conv's second segment when it differs from the first's (3 MX-fp8, 4 MX-fp4; the descriptor
 // carries one format for both); 0 = the same
 static thread_local int g_x2_dt = 0;
+// the calling thread's next split conv reads its upsampled segment as the e4m3 rows its pre-pass would make of it (MX-fp8, a multiple of 32 channels, no GroupNorm)
+static thread_local bool g_up_staged = false;
+extern "C" void mi_conv_up_staged(int on) { g_up_staged = on != 0; }
 extern "C" void mi_conv_x2_dt(int dt) { g_x2_dt = dt == 3 || dt == 4 ? dt : 0; }
 static thread_local int g_s2d = -1;         // mi_conv_s2_direct: the calling thread's choice of stride-2 kernel (-1: by launch size)
 extern "C" void mi_conv_s2_direct(int mode) { g_s2d = mode; }
@@ -396,6 +416,8 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     const void *segx[2] = {x, sp.x2}; const int segC[2] = {Cx, C2};
     const int segbf[2] = {xbf, sp.x2 && g_x2_dt ? g_x2_dt : xbf};
     g_x2_dt = 0;
+    const bool up_staged = g_up_staged && sp.up && xbf >= 3 && Cx % 32 == 0;
+    g_up_staged = false;
     for (int s = 0; s < (sp.x2 ? 2 : 1); s++) {
         const gnp_t g = s2g ? (s ? sp.gp2 : gp) : gp;
         const int Cg = s2g ? segC[s] : Ci, cg0 = s2g ? 0 : (s ? Cx : 0);
@@ -413,7 +435,8 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
             // the fp4 entry blends the upsample in binary16 unless UFSM_UP_H2=0 (src/lp_f4fwd.cuh:1135-1136); sp.up 2 / 3 force one blend
             static int uph2 = -1;
             if (uph2 < 0) uph2 = getenv("UFSM_UP_H2") ? atoi(getenv("UFSM_UP_H2")) : 1;
-            if (upseg) mi_restage_up_sub(segx[s], xbf, N, segC[s], D, H, W, g, Cg, st, fmt, zlo, zhi, sp.up == 2 || (sp.up == 1 && entry_fmt == 4 && uph2));
+            if (upseg && up_staged) mi_restage_up_rows(segx[s], N, segC[s], D, H, W, st, fmt, zlo, zhi, sp.up == 2 || (sp.up == 1 && entry_fmt == 4 && uph2));
+            else if (upseg) mi_restage_up_sub(segx[s], xbf, N, segC[s], D, H, W, g, Cg, st, fmt, zlo, zhi, sp.up == 2 || (sp.up == 1 && entry_fmt == 4 && uph2));
             else gn_for_slabs(who, g, H * W, zlo, zhi, [&](int z0, int z1, gnp_t gs) { mi_restage_sub(segx[s], xbf, N, segC[s], (size_t)(z1 - z0) * H * W, gs, Cg, cg0, st, fmt, S, (size_t)z0 * H * W); });
             a.xq[s] = st; a.xsc[s] = st + (size_t)N * nbp * S * mx_rb(32, fmt);
             a.nbs[s] = nbp; a.bws[s] = 32;
@@ -695,6 +718,14 @@ extern "C" int mi_conv_fwd_gn(int bits, const void *x, int xbf, shape5 xs, const
     g_fin = gn_fin_t{omean, orstd, 0.0, eps};
     const int rc = conv_dispatch("mi_conv_fwd_gn", bits, 1, x, xbf, xs, w, b, cout, y, ybf, gp, osum, Go, sp, nullptr, nullptr, 0);
     g_fin = gn_fin_t{nullptr, nullptr, 0.0, 0.f};
+    return rc;
+}
+extern "C" int mi_conv_fwd_gn_stage(int bits, const void *x, int xbf, shape5 xs, const float *w, const float *b, int cout, void *y, int ybf, gnp_t gp,
+                                    double *osum, int Go, split_t sp, float eps, float *omean, float *orstd, const float *gamma, const float *beta, void *st8, void *st4) {
+    if (cout % 32 || ybf < 3 || !gamma || !beta || (!st8 && !st4) || sp.Di || sp.yD || sp.zlo || sp.zhi || Go <= 0 || cout % Go || xs.n <= 0 || xs.c <= 0 || xs.d <= 0 || xs.h <= 0 || xs.w <= 0) return -1;
+    g_stage = gn_stage_t{gamma, beta, st8, st4};
+    const int rc = mi_conv_fwd_gn(bits, x, xbf, xs, w, b, cout, y, ybf, gp, osum, Go, sp, eps, omean, orstd);
+    g_stage.gamma = nullptr;
     return rc;
 }
 extern "C" int mi_conv_fwd_fused(int bits, const void *x, int xbf, shape5 xs, const float *w, const float *b, int cout, void *y, int ybf,

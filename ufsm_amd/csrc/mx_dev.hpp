@@ -267,7 +267,27 @@ __device__ __forceinline__ void gn_acc_add(double *b, size_t i, double v) {
     if (hi) atomicAdd(&w[1], (unsigned long long)hi);
 }
 
+// the value a single exact add of v to a cleared slot would leave, read back; w: the slot's three words
+__device__ __forceinline__ double gn_slot_value(double v, unsigned long long *w) {
+    if (!(fabs(v) < 4.611686018427387904e18)) { w[0] = 0ull; w[1] = 0ull; w[2] = 1ull; return __longlong_as_double(0x7ff8000000000000ll); }
+    const double f = floor(v);
+    const unsigned long long lo = (unsigned long long)((v - f) * 18446744073709551616.0);
+    w[0] = lo; w[1] = (unsigned long long)(long long)f; w[2] = 0ull;
+    return (double)(long long)f + (double)lo * 5.42101086242752217e-20;
+}
+// mean and rstd of a group of len elements from its slots' values (src/nn_elem.cu:5-11)
+__device__ __forceinline__ void gn_mean_rstd(double s, double ss, double len, float eps, float *mean, float *rstd) {
+    const double m = s / len, var = ss / len - m * m;
+    *mean = (float)m; *rstd = (float)(1.0 / sqrt((var > 0 ? var : 0) + (double)eps));
+}
+
 // ---- host-side shared declarations of the library's units ----
+// the statistics records of a conv's output (conv3.hip): per sample nst records of Q float2 (sum, sum of squares of a channel quad), quad q = channels 4 q .. 4 q + 3,
+// and what is made of them: mean / rstd [N][Go] of groups of len elements
+struct gn_records_t { const float2 *part; int nst, Q, Go; double len; float eps; float *mean, *rstd; };
+// silu(gn(x)) of the MX tensor x (C a multiple of 32) into y8 (MX-fp8 rows) and / or y4 (MX-fp4), mean and rstd formed from the records by the kernel that applies
+// them; false: not for these records (nothing was launched)
+bool mi_restage_records(const void *x, int xdt, int N, int C, size_t S, const float *gamma, const float *beta, const gn_records_t &rec, void *y8, void *y4);
 void mi_restage(const void *x, int xdt, int N, int C, size_t S, gnp_t gp, int Cg, int cg0, void *y, int ybits);
 void mi_restage_up(const void *x, int xdt, int N, int C, int D, int H, int W, gnp_t gp, int Cg, void *y, int ybits, int h2);    // h2: the binary16 blend
 // the MX GEMM with A's rows quantised by the kernel that produces them (csrc/mx_gemm.hip): where to write them, then the product
@@ -281,6 +301,7 @@ int mi_mx_gemm_glu(int T, int F, int C, const float *W, const float *bias, uint8
 void mi_restage_sub(const void *x, int xdt, int N, int C, size_t S, gnp_t gp, int Cg, int cg0, void *y, int ybits, size_t Ss, size_t v0);     // only voxels [v0, v0 + S) of tensors of Ss voxels
 void mi_restage_sub2(const void *x, int N, int C, size_t S, gnp_t gp, void *y8, void *y4, size_t Ss, size_t v0);      // MX-fp8 source, 32-wide blocks: both formats from one read
 void mi_restage_up_sub(const void *x, int xdt, int N, int C, int D, int H, int W, gnp_t gp, int Cg, void *y, int ybits, int zlo, int zhi, int h2);   // only fine planes [zlo, zhi)
+void mi_restage_up_rows(const void *x, int N, int C, int D, int H, int W, void *y, int ybits, int zlo, int zhi, int h2);   // the coarse tensor already as the e4m3 rows the first pass makes (C a multiple of 32)
 void mi_post_error(hipError_t e, const char *file, int line);
 #define MICK() do { hipError_t e_ = hipGetLastError(); if (e_ != hipSuccess) mi_post_error(e_, __FILE__, __LINE__); } while (0)
 #define MIRT(x) do { hipError_t e_ = (x); if (e_ != hipSuccess) mi_post_error(e_, __FILE__, __LINE__); } while (0)

@@ -830,8 +830,10 @@ __global__ void __launch_bounds__(256) restage_k(const void *xv, uint8_t *y, int
 constexpr int RS32_R = 4;                                          // rows per thread of restage32_k
 // BY2 (4, with BY 8): the same values also leave as a second tensor y2 in MX-fp4 - a skip tensor whose two readers compute in different
 // formats (the stride-2 down conv in e4m3, the decoder's conv in e2m1) is read and transformed once
-template <int BX, int BY, int BY2 = 0>
-__global__ void __launch_bounds__(256) restage32_k(const uint8_t *x, uint8_t *y, int N, int C, size_t S, gnp_t gp, int Cg, int cg0, size_t Ss, size_t v0, uint8_t *y2 = nullptr) {
+// RED: the statistics are not read but formed here, from the records of the conv that wrote x (rec; Cg = C, cg0 = 0): every workgroup adds the records of the groups
+// its 32 channels lie in, in double, while its rows arrive; the first workgroup of a group's first block stores the group's mean and rstd
+template <int BX, int BY, int BY2 = 0, bool RED = false>
+__global__ void __launch_bounds__(256) restage32_k(const uint8_t *x, uint8_t *y, int N, int C, size_t S, gnp_t gp, int Cg, int cg0, size_t Ss, size_t v0, uint8_t *y2 = nullptr, gn_records_t rec = gn_records_t{}) {
     const int nb = C / 32, blk = blockIdx.y, n = blockIdx.z;
     __shared__ float sa[32], sb[32];
     // A workgroup moves RS32_R x 128 consecutive voxels of the block, a thread one 16-channel half of RS32_R rows 128 voxels apart: the rows are
@@ -842,6 +844,20 @@ __global__ void __launch_bounds__(256) restage32_k(const uint8_t *x, uint8_t *y,
     const size_t row0 = ((size_t)n * nb + blk) * Ss + v0;
     const uint8_t *xs = x + (size_t)N * nb * Ss * (IB * 2);
     uint8_t *ys = y + (size_t)N * nb * Ss * (OB * 2);
+    // RED: the groups the block's channels lie in and their quads of channels; thread (q, j) adds quad q of records j, j + 16, ... The first of them and the affine are requested
+    // before the rows (loads return in order: the chain they start is the longer one)
+    constexpr int RK = RED ? 8 : 1;
+    const int cpg = RED ? C / rec.Go : 4, g0 = blk * 32 / cpg, g1 = (blk * 32 + 31) / cpg, qpg = cpg >> 2;      // (cpg a multiple of 4; the groups' quads are at most 16: the host's rule)
+    const int rj = threadIdx.x >> 4;
+    const float2 *rp = nullptr;
+    float2 rv[RK];
+    float ga = 0.f, be = 0.f;
+    if constexpr (RED) {
+        rp = rec.part + (size_t)n * rec.nst * rec.Q + g0 * qpg + min((int)(threadIdx.x & 15), (g1 - g0 + 1) * qpg - 1);
+#pragma unroll
+        for (int k = 0; k < RK; k++) { const int t = rj + 16 * k; rv[k] = rp[(size_t)min(t, rec.nst - 1) * rec.Q]; }
+        if (threadIdx.x < 32) { ga = gp.gamma[blk * 32 + threadIdx.x]; be = gp.beta[blk * 32 + threadIdx.x]; }
+    }
     unsigned w[RS32_R][4]; unsigned sby[RS32_R];
 #pragma unroll
     for (int i = 0; i < RS32_R; i++) {
@@ -852,7 +868,41 @@ __global__ void __launch_bounds__(256) restage32_k(const uint8_t *x, uint8_t *y,
         sby[i] = xs[row];
     }
     // (the rows are requested before the block's coefficients are formed: the two chains of dependent loads overlap)
-    if (threadIdx.x < 32) {
+    if constexpr (RED) {
+        double s = 0.0, ss = 0.0;
+#pragma unroll
+        for (int k = 0; k < RK; k++) if (rj + 16 * k < rec.nst) { s += (double)rv[k].x; ss += (double)rv[k].y; }
+#pragma unroll 8
+        for (int t = rj + 16 * RK; t < rec.nst; t += 16) { const float2 v = rp[(size_t)t * rec.Q]; s += (double)v.x; ss += (double)v.y; }
+        __shared__ double r1[256], r2[256];
+        __shared__ float sm[16], sr[16];
+        r1[threadIdx.x] = s; r2[threadIdx.x] = ss;
+        __syncthreads();
+        if (threadIdx.x < 64) {                               // lane (q, part): a quad's sums over four of the sixteen rows, then over the four lanes of the quad
+            const int qq = threadIdx.x & 15, k0 = threadIdx.x >> 4;
+            s = (r1[(4 * k0) * 16 + qq] + r1[(4 * k0 + 1) * 16 + qq]) + (r1[(4 * k0 + 2) * 16 + qq] + r1[(4 * k0 + 3) * 16 + qq]);
+            ss = (r2[(4 * k0) * 16 + qq] + r2[(4 * k0 + 1) * 16 + qq]) + (r2[(4 * k0 + 2) * 16 + qq] + r2[(4 * k0 + 3) * 16 + qq]);
+            s += __shfl_xor(s, 16); s += __shfl_xor(s, 32); ss += __shfl_xor(ss, 16); ss += __shfl_xor(ss, 32);
+            if (threadIdx.x < 16) { r1[threadIdx.x] = s; r2[threadIdx.x] = ss; }
+        }
+        __syncthreads();
+        if ((int)threadIdx.x <= g1 - g0) {
+            s = 0.0; ss = 0.0;
+            for (int k = 0; k < qpg; k++) { s += r1[threadIdx.x * qpg + k]; ss += r2[threadIdx.x * qpg + k]; }
+            unsigned long long w[3];
+            float m, r;
+            gn_mean_rstd(gn_slot_value(s, w), gn_slot_value(ss, w), rec.len, rec.eps, &m, &r);
+            sm[threadIdx.x] = m; sr[threadIdx.x] = r;
+            const int g = g0 + (int)threadIdx.x;
+            if (blockIdx.x == 0 && g * cpg >= blk * 32) { rec.mean[n * rec.Go + g] = m; rec.rstd[n * rec.Go + g] = r; }
+        }
+        __syncthreads();
+        if (threadIdx.x < 32) {
+            const int k = (blk * 32 + (int)threadIdx.x) / cpg - g0;
+            const float a = sr[k] * ga;
+            sa[threadIdx.x] = a; sb[threadIdx.x] = fmaf(-sm[k], a, be);
+        }
+    } else if (threadIdx.x < 32) {
         float a = 1.f, b = 0.f;
         if (gp.G) { const int c = cg0 + blk * 32 + threadIdx.x, ng = d_gn_row(gp, n) * gp.G + c / (Cg / gp.G); a = gp.rstd[ng] * gp.gamma[c]; b = fmaf(-gp.mean[ng], a, gp.beta[c]); }
         sa[threadIdx.x] = a; sb[threadIdx.x] = b;
@@ -875,7 +925,7 @@ __global__ void __launch_bounds__(256) restage32_k(const uint8_t *x, uint8_t *y,
 #pragma unroll
             for (int k = 0; k < 16; k++) r[k] *= sc;
         }
-        if (gp.G) {                                               // (one uniform branch around sixteen independent chains: a select per value made sixteen blocks of one dependent chain each)
+        if (RED || gp.G) {                                        // (one uniform branch around sixteen independent chains: a select per value made sixteen blocks of one dependent chain each)
 #pragma unroll
             for (int k = 0; k < 16; k++) r[k] = d_act_ab(r[k], ca[k], cb[k]);
         }
@@ -907,6 +957,25 @@ void mi_restage_sub2(const void *x, int N, int C, size_t S, gnp_t gp, void *y8, 
     const dim3 grid(nblk_(S, 128 * RS32_R), (unsigned)(C / 32), (unsigned)N);
     restage32_k<8, 8, 4><<<grid, 256>>>((const uint8_t *)x, (uint8_t *)y8, N, C, S, gp, C, 0, Ss, v0, (uint8_t *)y4);
     MICK();
+}
+bool mi_restage_records(const void *x, int xdt, int N, int C, size_t S, const float *gamma, const float *beta, const gn_records_t &rec, void *y8, void *y4) {
+    const int cpg = C / rec.Go;
+    if (C % 32 || (xdt != 3 && xdt != 4) || cpg % 4 || !N || !S || (y8 && y4 && xdt != 3)) return false;
+    int nq = 0;                                                    // the most quads a block's groups have
+    for (int b = 0; b < C / 32; b++) { const int k = ((b * 32 + 31) / cpg - b * 32 / cpg + 1) * (cpg / 4); if (k > nq) nq = k; }
+    if (nq > 16) return false;
+    const dim3 grid(nblk_(S, 128 * RS32_R), (unsigned)(C / 32), (unsigned)N);
+    // every workgroup reads its groups' records: up to 512 of them per sample (four rounds of its threads' loads) and 16 MB in all the launch they save (4 - 5 us) is longer. 1 x 88 x 104^2,
+    // 154 records and 466 workgroups 8.0 + 4.6 against 10.0 - 11.4 us; 20 - 80 records 5.3 + 4.5 against 6.0; at 2 x 64^3 256 records for 2 048 workgroups (32 MB) are even
+    if (rec.nst > 512 || (size_t)grid.x * grid.y * grid.z * rec.nst * (nq * 8) > (size_t)16 << 20) return false;
+    gnp_t gp = {}; gp.gamma = gamma; gp.beta = beta;
+    const uint8_t *xq = (const uint8_t *)x;
+#define RR(BX, BY, BY2, Y, Y2) restage32_k<BX, BY, BY2, true><<<grid, 256>>>(xq, (uint8_t *)(Y), N, C, S, gp, C, 0, S, 0, (uint8_t *)(Y2), rec)
+    if (xdt == 3) { if (y8 && y4) RR(8, 8, 4, y8, y4); else if (y8) RR(8, 8, 0, y8, nullptr); else RR(8, 4, 0, y4, nullptr); }
+    else if (y8) RR(4, 8, 0, y8, nullptr); else RR(4, 4, 0, y4, nullptr);
+#undef RR
+    MICK();
+    return true;
 }
 // voxels [v0, v0 + S) of tensors holding Ss voxels per (sample, channel / block): the result has the source's geometry, only that range is written
 void mi_restage_sub(const void *x, int xdt, int N, int C, size_t S, gnp_t gp, int Cg, int cg0, void *y, int ybits, size_t Ss, size_t v0) {
@@ -1110,7 +1179,8 @@ __global__ void __launch_bounds__(256) up_blend_k(const uint8_t *xc, uint8_t *y,
     }
 }
 // fine planes [zlo, zhi) of the upsampled depth-D tensor, written at their place in the depth-D MX tensor y
-void mi_restage_up_sub(const void *x, int xdt, int N, int C, int D, int H, int W, gnp_t gp, int Cg, void *y, int ybits, int zlo, int zhi, int h2) {
+// (rows: x is the coarse tensor's e4m3 rows themselves, the first pass done by whoever wrote them)
+static void restage_up(const void *x, int xdt, int N, int C, int D, int H, int W, gnp_t gp, int Cg, void *y, int ybits, int zlo, int zhi, int h2, bool rows) {
     if (!N || zhi <= zlo || !H || !W) return;
     if (xdt != 3 && xdt != 4) mi_die("fused-upsample input must be an MX tensor (dtype %d)", xdt);
     if ((D | H | W) & 1) mi_die("fused-upsample output dims must be even (%d %d %d)", D, H, W);
@@ -1119,8 +1189,8 @@ void mi_restage_up_sub(const void *x, int xdt, int N, int C, int D, int H, int W
     const int mz0 = (zlo - 2) >> 1 < -1 ? -1 : (zlo - 2) >> 1, mz1 = (zhi - 2) >> 1, ncz = mz1 - mz0 + 1;
     const int clo = mz0 < 0 ? 0 : mz0, chi = (mz1 + 1 > Dc - 1 ? Dc - 1 : mz1 + 1) + 1, Dcs = chi - clo;
     const size_t Scp = (size_t)(H / 2) * (W / 2);
-    uint8_t *xc = (uint8_t *)mi_ws(MI_WS_UPCOARSE, (size_t)N * nbo * Dc * Scp * 33);          // the coarse tensor's geometry; planes [clo, clo + Dcs) are filled
-    mi_restage_sub(x, xdt, N, C, (size_t)Dcs * Scp, gp, Cg, 0, xc, 8, (size_t)Dc * Scp, (size_t)clo * Scp);
+    uint8_t *xc = rows ? (uint8_t *)const_cast<void *>(x) : (uint8_t *)mi_ws(MI_WS_UPCOARSE, (size_t)N * nbo * Dc * Scp * 33);          // the coarse tensor's geometry; planes [clo, clo + Dcs) are filled
+    if (!rows) mi_restage_sub(x, xdt, N, C, (size_t)Dcs * Scp, gp, Cg, 0, xc, 8, (size_t)Dc * Scp, (size_t)clo * Scp);
     const size_t cells = (size_t)(H / 2 + 1) * (W / 2 + 1);                                   // per z layer of cells
     if ((size_t)N * nbo > 65535 || ncz > 65535) mi_die("fused upsample: launch grid (%d x %d blocks, %d cell layers)", N, nbo, ncz);
     const dim3 grid(nblk_(cells * (h2 ? 2 : 4), 256), (unsigned)(N * nbo), (unsigned)ncz);      // (threads per cell: two in the binary16 blend, four in the fp32 one)
@@ -1129,6 +1199,8 @@ void mi_restage_up_sub(const void *x, int xdt, int N, int C, int D, int H, int W
 #undef UB
     MICK();
 }
+void mi_restage_up_sub(const void *x, int xdt, int N, int C, int D, int H, int W, gnp_t gp, int Cg, void *y, int ybits, int zlo, int zhi, int h2) { restage_up(x, xdt, N, C, D, H, W, gp, Cg, y, ybits, zlo, zhi, h2, false); }
+void mi_restage_up_rows(const void *x, int N, int C, int D, int H, int W, void *y, int ybits, int zlo, int zhi, int h2) { restage_up(x, 3, N, C, D, H, W, gnp_t{}, C, y, ybits, zlo, zhi, h2, true); }
 void mi_restage_up(const void *x, int xdt, int N, int C, int D, int H, int W, gnp_t gp, int Cg, void *y, int ybits, int h2) { mi_restage_up_sub(x, xdt, N, C, D, H, W, gp, Cg, y, ybits, 0, D, h2); }
 
 // weights w [Co][Ci][T] rounded in place to MX-fp4 values with one E8M0 scale per Bo x Bi (output x input channel) block and tap (src/lp_mx_cvt.cu:369-395):

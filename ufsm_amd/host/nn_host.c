@@ -111,6 +111,29 @@ static int conv_s1(const char *who, const float *x, shape5 xs, const float *w, c
     return 0;
 }
 
+/* a 3^3 stride-1 conv of the graph whose neighbours read and write operand rows: x may be rows already transformed for this conv's compute format (xrows), the upsampled first
+   segment the e4m3 rows its pre-pass would make (uprows), and silu(gn(y)) under the affine (gamma, beta) of the statistics taken here goes to st8 (MX-fp8 rows) and / or st4
+   (MX-fp4), if either is given. The formats are those conv_s1 would choose: the registry gives y's, which is also what x and x2 stand for. -1: not for these operands (nothing was
+   launched) */
+int mi_nn_conv3d_rows(const void *x, int xrows, const nn_gn_t *gx, const void *x2, const nn_gn_t *gx2, int c_split, int up, int uprows, shape5 xs, const float *w, const float *b, int cout,
+                      void *y, int G_out, float eps, float *omean, float *orstd, const float *gamma, const float *beta, void *st8, void *st4) {
+    const int ydt = lp_dt(y);
+    if (g_zr_Di || ydt < 3 || cout % 32 || G_out <= 0 || cout % G_out || (g_gn_stored && !gn_fused_stored(ydt, cout)) || (xrows && x2)) return -1;
+    const int xdt = xrows ? ydt : lp_dt(x), x2dt = x2 ? lp_dt(x2) : 0;
+    if (uprows && (!up || c_split % 32)) return -1;
+    const int fam = conv_family("mi_nn_conv3d_rows", uprows ? ydt : xdt, ydt, x2dt, x2 != nullptr, xs.c, cout, up);
+    const int xbf = xrows ? (fam == 4 ? 4 : 3) : uprows ? 3 : xdt;
+    split_t sp; memset(&sp, 0, sizeof sp);
+    if (x2) { sp.x2 = x2; sp.c_split = c_split; sp.up = (int16_t)up; if (gx2) sp.gp2 = gnp_mk(gx2->gamma, gx2->beta, gx2->mean, gx2->rstd, gx2->G); else sp.gp2.G = -1; }
+    sp.wkey = (unsigned)((uintptr_t)w >> 4) | 1u;
+    sp.stored_stats = gn_fused_stored(ydt, cout);
+    if (x2 && x2dt != xbf) mi_conv_x2_dt(x2dt);
+    mi_conv_up_staged(uprows);
+    const gnp_t gp = gx ? gnp_mk(gx->gamma, gx->beta, gx->mean, gx->rstd, gx->G) : gnp_mk(nullptr, nullptr, nullptr, nullptr, 0);
+    double *sums = gn_dsums((size_t)2 * xs.n * G_out);
+    if (!st8 && !st4) return mi_conv_fwd_gn(fam, x, xbf, xs, w, b, cout, y, ydt, gp, sums, G_out, sp, eps, omean, orstd);
+    return mi_conv_fwd_gn_stage(fam, x, xbf, xs, w, b, cout, y, ydt, gp, sums, G_out, sp, eps, omean, orstd, gamma, beta, st8, st4);
+}
 int nn_conv3d_fwd_x(const float *x, const nn_gn_t *gx, const float *x2, const nn_gn_t *gx2, int c_split, int up, shape5 xs,
                     const float *w, const float *b, int cout, int k, int stride, float *y, int G_out, float eps, float *omean, float *orstd) {
     const int xdt = lp_dt(x), ydt = lp_dt(y);

@@ -44,6 +44,9 @@ struct unet {
     convp down[UNET_MAXLEV], head;
     convp ds[UNET_MAXLEV], eh;         /* cfg.ds_levels / cfg.emb_lev: the deep-supervision heads of decoder levels 1 .. ds_levels and the distillation head: training-time outputs, here only their place in the parameter vector (src/unet.c:467, :511) */
     void *downo[UNET_MAXLEV];
+    /* per level, silu(gn(.)) of the conv output just written, as the operand rows (MX-fp8 or MX-fp4) of its one reader, the next conv of the graph: the level's pre-staged skip's
+       buffer, whose rows are written after conv2 has read conv1's and are dead once the decoder's conv1 has read them, or (levels without one) rows_own, one buffer for all */
+    void *rows[UNET_MAXLEV], *rows_own;
     void *skipst[UNET_MAXLEV];         /* silu(gn(enc[i].a2)) in the compute format, formed once for its two readers (down conv, decoder conv1); null: each reader transforms it */
     void *skipst4[UNET_MAXLEV];        /* precision 3 over MX-fp8 storage: the two readers compute in different formats (the stride-2 conv in e4m3, the decoder's in e2m1);
                                           the same pass writes the MX-fp4 rows here beside the MX-fp8 ones in skipst */
@@ -260,6 +263,8 @@ static void free_acts(unet *u) {
     if (u->tbn) { act_del(u->tb.a2); mi_free(u->tb.m2); mi_free(u->tb.r2); mi_free(u->tb_cs); mi_free(u->tb_tok); mi_free(u->tb_ws); if (u->tb_vr) mi_free(u->tb_vr); u->tb_vr = nullptr; tb_geom_free(u); u->tb.a2 = nullptr; u->tb.m2 = u->tb.r2 = nullptr; u->tb_cs = u->tb_tok = nullptr; u->tb_ws = nullptr; }
     for (int i = 0; i < 2; i++) { act_del(u->slab_tmp[i]); act_del(u->slab_carry[i]); u->slab_tmp[i] = u->slab_carry[i] = nullptr; }
     act_del(u->xin); u->xin = nullptr;
+    if (u->rows_own) mi_free(u->rows_own);
+    u->rows_own = nullptr; memset(u->rows, 0, sizeof u->rows);
     mi_free(u->logits); u->logits = nullptr;
     u->built = 0; u->nouts = 0; u->slab_ip = u->slab_nl = u->slab_s = 0; u->l0s_zs = u->l0s_ns = 0;
 }
@@ -318,6 +323,10 @@ static int build_acts(unet *u, shape5 in) {
         u->slab_tmp[i] = act_new(u, t); t.d = 1; u->slab_carry[i] = act_new(u, t);
     }
     u->xin = act_new(u, in);
+    size_t rows = 0;
+    for (int i = 0; i < L; i++) { const size_t r = nn_mx8_bytes(u->ls[i]); if (!u->skipst[i] && r > rows) rows = r; }      /* (a decoder block is at most as wide as its level) */
+    if (rows) u->rows_own = mi_malloc(rows);
+    for (int i = 0; i < L; i++) u->rows[i] = u->skipst[i] ? u->skipst[i] : u->rows_own;
     u->logits = f32_new((size_t)in.n * cfg->cout * in.d * in.h * in.w);
     if (u->tbn) {
         const shape5 ys = u->ls[L - 1]; const long Sg = (long)ys.d * ys.h * ys.w, S = Sg + u->tbd.nreg, T = (long)ys.n * S; const int C = u->tbd.C;
@@ -554,7 +563,10 @@ static void l0_const_fill(unet *u) {
 }
 /* conv1 -> a1 (+ its statistics), conv2 reads silu(gn(a1)) while staging -> a2 (+ statistics) (src/unet.c:2567-2636); in z-slabs when asked for
    (slab_run, src/unet.c:2499-2545) */
-static int block_fwd(unet *u, block *b, int level, const void *x, const nn_gn_t *gin, const void *xup, const nn_gn_t *gup, int c_split, const char *n1, const char *n2) {
+/* what a block's convs hand on as operand rows: the coarse segment of the block's input (uprows: the level below holds them in its u->rows), and of the block's output silu(gn(a2)) as MX-fp8 rows st8
+   and / or MX-fp4 rows st4 when they are asked for; done: they were written */
+typedef struct { int uprows; void *st8, *st4; int done; } rows_io;
+static int block_fwd(unet *u, block *b, int level, const void *x, const nn_gn_t *gin, const void *xup, const nn_gn_t *gup, int c_split, const char *n1, const char *n2, rows_io *io) {
     const int G = G_of(u, b->c1.cout), D = b->ys.d, ip = u->slab_ip && level < u->slab_nl;
     /* per-slab statistics (level 0 under cfg.l0_norm 4): the convs reduce nothing; a pass over the stored output, seen as n * slabs samples of
        l0_slab planes (one channel block: a slab is a sample of the same layout), fills the [n][slab][G] rows (src/unet.c:996-998) */
@@ -562,6 +574,12 @@ static int block_fwd(unet *u, block *b, int level, const void *x, const nn_gn_t 
     const int s = level >= slab_levels(u) ? 0 : g_infer_slab < D ? g_infer_slab : ip ? D : 0;      /* (in place: a level of fewer planes is one slab) */
     void *tmp = ip ? u->slab_tmp[level] : nullptr, *carry = ip ? u->slab_carry[level] : nullptr;
     int r = 0;
+    /* outside slabs, with statistics of its own, a conv's output leaves its GroupNorm + SiLU to one pass behind the conv (mi_conv_fwd_gn_stage), whose rows the next conv reads as
+       they are; the reader's own pre-pass would make the same rows */
+    const int rows_ok = !s && !ip && Gc > 0, fam4 = u->act_dt == 4 || u->prec == 3;
+    void *const rows = u->rows[level];
+    int have = 0;                                                  /* rows holds silu(gn(a1)) in conv2's compute format */
+    io->done = 0;
     for (int conv = b->single ? 2 : 1; conv <= 2 && !r; conv++) {  /* (one-conv decoder block: its conv, with c1's weights, writes a2 and the statistics m2 / r2, src/unet.c:2581-2582) */
         void *y = conv == 1 ? b->a1 : b->a2;
         const int first = conv == 1 || b->single;                  /* this conv reads the block's input */
@@ -573,6 +591,20 @@ static int block_fwd(unet *u, block *b, int level, const void *x, const nn_gn_t 
             shape5 xs = first ? b->xs : b->ys;
             if (s) { nn_set_zrange(z0, D, z0 == 0, last, D, z0); nn_set_zrange_out(!over); xs.d = sk; }
             void *o = over ? tmp : y;
+            const int more = conv == 1;                            /* (its reader is conv2) */
+            const gnpar *gn = more ? &b->n1 : &b->n2;
+            void *st8 = more ? (fam4 ? nullptr : rows) : io->st8, *st4 = more ? (fam4 ? rows : nullptr) : io->st4;
+            const convp *cp = first ? &b->c1 : &b->c2;
+            const float *cb = P(u, cp->b);
+            if (first && !xup && b == &u->enc[0] && u->cfg.scale_cond) cb = u->stem_b;
+            if (rows_ok && (st8 || st4 || have)) {
+                const int e = !first ? mi_nn_conv3d_rows(have ? rows : b->a1, have, have ? nullptr : &(nn_gn_t){P(u, b->n1.gamma), P(u, b->n1.beta), b->m1, b->r1, G}, nullptr, nullptr, 0, 0, 0, xs,
+                                                         P(u, cp->w), cb, cp->cout, o, Gc, 1e-5f, om, orr, P(u, gn->gamma), P(u, gn->beta), st8, st4)
+                            : xup ? mi_nn_conv3d_rows(io->uprows ? u->rows[level + 1] : xup, 0, io->uprows ? nullptr : gup, x, gin, c_split, 1, io->uprows, xs, P(u, cp->w), cb, cp->cout, o, Gc, 1e-5f, om, orr, P(u, gn->gamma), P(u, gn->beta), st8, st4)
+                                  : mi_nn_conv3d_rows(x, 0, gin, nullptr, nullptr, 0, 0, 0, xs, P(u, cp->w), cb, cp->cout, o, Gc, 1e-5f, om, orr, P(u, gn->gamma), P(u, gn->beta), st8, st4);
+                if (!e) { if (more) have = 1; else io->done = st8 || st4; continue; }
+                if (have) { r = -1; break; }                       /* (conv2 takes what conv1 took) */
+            }
             if (!first) r = nn_conv3d_fwd_gn_stats(b->a1, xs, G, P(u, b->n1.gamma), P(u, b->n1.beta), b->m1, b->r1, P(u, b->c2.w), P(u, b->c2.b), b->c2.cout, o, Gc, 1e-5f, om, orr);
             else if (xup) r = nn_conv3d_fwd_x(xup, gup, x, gin, c_split, 1, xs, P(u, b->c1.w), P(u, b->c1.b), b->c1.cout, 3, 1, o, Gc, 1e-5f, om, orr);   /* [up2(coarse) | skip] */
             else r = nn_conv3d_fwd_x(x, gin, nullptr, nullptr, 0, 0, xs, P(u, b->c1.w), b == &u->enc[0] && u->cfg.scale_cond ? u->stem_b : P(u, b->c1.b), b->c1.cout, 3, 1, o, Gc, 1e-5f, om, orr);
@@ -716,16 +748,20 @@ static int graph_fwd(unet *u, const void *x) {
         nn_axpy(u->stem_b, u->sc_c, P(u, u->sc_w), (size_t)c0);
     }
     const void *cur = x;
+    int uprows = 0;                                                /* the level below holds the coarse segment of the next decoder block as its pre-pass would make it, in its rows */
     for (int i = 0; i < L; i++) {
         nn_gn_t gd; const nn_gn_t *gin = nullptr;                  /* down_norm: conv1 reads silu(gn(down conv output)) (src/unet.c:2593) */
         if (i && u->cfg.down_norm) { gd = (nn_gn_t){P(u, u->dn[i - 1].gamma), P(u, u->dn[i - 1].beta), u->dm[i - 1], u->dr[i - 1], G_of(u, u->cfg.widths[i - 1])}; gin = &gd; }
-        if (block_fwd(u, &u->enc[i], i, cur, gin, nullptr, nullptr, 0, en1[i], en2[i])) return -1;
+        rows_io io = {0};
+        if (!u->cfg.enc_blocks[i]) { if (i < L - 1) { io.st8 = u->skipst[i]; io.st4 = u->skipst4[i]; } else if (L > 1 && !u->tbn) io.st8 = u->rows[i]; }
+        if (block_fwd(u, &u->enc[i], i, cur, gin, nullptr, nullptr, 0, en1[i], en2[i], &io)) return -1;
+        if (i == L - 1) uprows = io.done;
         for (int k = 0; k < u->cfg.enc_blocks[i]; k++) if (rblock_fwd(u, &u->rb[i][k], k ? &u->rb[i][k - 1] : &u->enc[i], u->rbn[i][k])) return -1;      /* (src/unet.c:2963) */
         if (i < L - 1) {                                           /* stride-2 down conv of silu(gn(a2)), width kept (src/unet.c:2970) */
             const block *so = stage_out(u, i);
             const nn_gn_t g = gn_out(u, so);
             const int pre = u->skipst[i] != nullptr;
-            if (pre && (u->skipst4[i] ? mi_conv_prestage2(so->a2, so->ys, gnp_mk(g.gamma, g.beta, g.mean, g.rstd, g.G), u->skipst[i], u->skipst4[i])
+            if (pre && !io.done && (u->skipst4[i] ? mi_conv_prestage2(so->a2, so->ys, gnp_mk(g.gamma, g.beta, g.mean, g.rstd, g.G), u->skipst[i], u->skipst4[i])
                                       : mi_conv_prestage(so->a2, 3, so->ys, gnp_mk(g.gamma, g.beta, g.mean, g.rstd, g.G), u->skipst[i], 8))) return -1;
             if (nn_conv3d_fwd_x(pre ? u->skipst[i] : so->a2, pre ? nullptr : &g, nullptr, nullptr, 0, 0, so->ys, P(u, u->down[i].w), P(u, u->down[i].b), u->cfg.widths[i], 3, 2, u->downo[i], 0, 0.f, nullptr, nullptr)) return -1;
             shape5 ds = u->ls[i + 1]; ds.c = u->cfg.widths[i];
@@ -743,7 +779,9 @@ static int graph_fwd(unet *u, const void *x) {
         if (i == L - 2 && u->tbn) { coarse = &u->tb; gc.mean = u->tb.m2; gc.rstd = u->tb.r2; }      /* the stage's output under the level's n2 affine (src/unet.c:508) */
         static const nn_gn_t none = {nullptr, nullptr, nullptr, nullptr, -1};          /* the pre-staged skip: no GroupNorm left to apply */
         const void *sk = u->skipst4[i] ? u->skipst4[i] : u->skipst[i];      /* (the decoder's conv computes in e2m1 under precision 3: its rows) */
-        if (block_fwd(u, &u->dec[i], i, sk ? sk : skip->a2, sk ? &none : &gs, coarse->a2, &gc, coarse->ys.c, dn1[i], dn2[i])) return -1;
+        rows_io io = {.uprows = uprows, .st8 = i ? u->rows[i] : nullptr};      /* (the coarse rows are e4m3 whatever the decoder's conv computes in) */
+        if (block_fwd(u, &u->dec[i], i, sk ? sk : skip->a2, sk ? &none : &gs, coarse->a2, &gc, coarse->ys.c, dn1[i], dn2[i], &io)) return -1;
+        uprows = io.done;
     }
     const block *last = L > 1 ? &u->dec[0] : &u->enc[0];
     const nn_gn_t g = gn_out(u, last);

@@ -51,6 +51,7 @@ _PROTOS = {
     "mi_conv_prestage": (_I, [_P, _I, shape5, gnp_t, _P, _I]),
     "mi_conv_prestage2": (_I, [_P, shape5, gnp_t, _P, _P]),
     "mi_conv_x2_dt": (None, [_I]),
+    "mi_conv_up_staged": (None, [_I]),
     "gnp_mk": (gnp_t, [_P, _P, _P, _P, _I]),
     "lp_gn_slab_any": (_I, []),
     "lp_gn_slab_reg": (None, [_P, _I, _I, _I, _I]),
@@ -119,6 +120,7 @@ _PROTOS = {
     "mi_conv_down2_fwd": (_I, [_I, _P, _I, shape5, _P, _P, _I, _P, _I, gnp_t]),
     "mi_convt_up2_fwd": (_I, [_I, _P, _I, shape5, _P, _P, _I, _P, _I, gnp_t]),
     "mi_conv_fwd_gn": (_I, [_I, _P, _I, shape5, _P, _P, _I, _P, _I, gnp_t, _P, _I, split_t, C.c_float, _P, _P]),
+    "mi_conv_fwd_gn_stage": (_I, [_I, _P, _I, shape5, _P, _P, _I, _P, _I, gnp_t, _P, _I, split_t, C.c_float, _P, _P, _P, _P, _P, _P]),
     "mi_conv_fwd_static": (_I, [_I, _P, _I, shape5, _P, _P, _I, _P, _I, gnp_t, _P, _I, split_t]),
     "mi_conv_static_scratch_bytes": (_Z, []),
     "mi_alloc_count": (C.c_long, []),
