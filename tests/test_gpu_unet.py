@@ -354,6 +354,13 @@ def test_reference_signature_forwards(gpu):
     want = np.empty_like(got); q = H_.mi_unet_forward_mx(net.h, xin.ptr, xs); lib.mi_sync(); lib.mi_d2h(want.ctypes.data, q, want.nbytes)
     LP.check()
     assert np.array_equal(got, want)
+    # the logits written to the caller's buffer: the same, at any float's address (and through a copy at any other)
+    for off in (0, 4, 1):
+        mine = DevBuf.from_numpy(np.full(got.nbytes + 8, 255, np.uint8))
+        assert H_.mi_unet_forward_ct_to(net.h, dct.ptr, 120.0, 1 / 50.0, ddy.ptr, ddx.ptr, 1, xs, 2, mine.ptr + off) == 0
+        LP.check()
+        b = mine.to_numpy(np.uint8)
+        assert np.array_equal(b[off:off + got.nbytes], got.view(np.uint8)) and (b[:off] == 255).all() and (b[off + got.nbytes:] == 255).all()
     # a configuration field this build does not run is refused by name, not ignored
     bad = make_cfg(4, [32, 64]); bad.fstem = 2
     assert not H_.unet_create(C.byref(bad))

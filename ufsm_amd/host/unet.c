@@ -733,7 +733,7 @@ static int rblock_fwd(unet *u, block *b, block *prev, const char (*nm)[16]) {
     return 0;
 }
 /* the graph on the MX input tensor x (src/unet.c:2939-3105) */
-static int graph_fwd(unet *u, const void *x) {
+static int graph_fwd(unet *u, const void *x, float *logits) {
     static const char *en1[] = {"enc0.c1", "enc1.c1", "enc2.c1", "enc3.c1", "enc4.c1", "enc5.c1", "enc6.c1", "enc7.c1"}, *en2[] = {"enc0.c2", "enc1.c2", "enc2.c2", "enc3.c2", "enc4.c2", "enc5.c2", "enc6.c2", "enc7.c2"};
     static const char *dn1[] = {"dec0.c1", "dec1.c1", "dec2.c1", "dec3.c1", "dec4.c1", "dec5.c1", "dec6.c1"}, *dn2[] = {"dec0.c2", "dec1.c2", "dec2.c2", "dec3.c2", "dec4.c2", "dec5.c2", "dec6.c2"};
     static const char *dwn[] = {"down0", "down1", "down2", "down3", "down4", "down5", "down6"};
@@ -785,19 +785,23 @@ static int graph_fwd(unet *u, const void *x) {
     }
     const block *last = L > 1 ? &u->dec[0] : &u->enc[0];
     const nn_gn_t g = gn_out(u, last);
-    return nn_conv3d_fwd_x(last->a2, &g, nullptr, nullptr, 0, 0, last->ys, P(u, u->head.w), P(u, u->head.b), u->cfg.cout, 1, 1, u->logits, 0, 0.f, nullptr, nullptr);
+    lp_conv1_fwd_mx(last->a2, u->act_dt == 4 ? 4 : 3, last->ys, P(u, u->head.w), P(u, u->head.b), u->cfg.cout, logits, gnp_mk(g.gamma, g.beta, g.mean, g.rstd, g.G));
+    return 0;
 }
 /* every exit of a forward passes here: the caller's tensor leaves the storage registry again (a stale range would make a later allocation
    inside it look like MX storage) */
-const float *mi_unet_forward_mx(unet *u, const void *xmx, shape5 xs) {
-    if (ensure_built(u, xs)) return nullptr;
+int mi_unet_forward_mx_to(unet *u, const void *xmx, shape5 xs, float *logits) {
+    if (ensure_built(u, xs)) return -1;
     fw_refresh(u);
     const int reg_here = xmx != u->xin && nn_storage(xmx) != u->act_dt;     /* the input is looked up by the convs like any activation */
     if (reg_here) nn_set_storage(xmx, act_bytes(u, u->in), u->act_dt);
-    const int rc = graph_fwd(u, xmx);
+    const int own = !logits || ((uintptr_t)logits & 3);            /* (the head stores whole floats: a buffer at another address gets a copy) */
+    const int rc = graph_fwd(u, xmx, own ? u->logits : logits);
     if (reg_here) nn_storage_forget(xmx);
-    return rc ? nullptr : u->logits;
+    if (!rc && own && logits) mi_d2d(logits, u->logits, (size_t)xs.n * u->cfg.cout * xs.d * xs.h * xs.w * sizeof(float));
+    return rc ? -1 : 0;
 }
+const float *mi_unet_forward_mx(unet *u, const void *xmx, shape5 xs) { return mi_unet_forward_mx_to(u, xmx, xs, nullptr) ? nullptr : u->logits; }
 const float *unet_forward_x(unet *u, const void *x, shape5 xs, int train, int x_h16) {
     if (train) { fprintf(stderr, "unet_forward_x: this is an inference build (train must be 0)\n"); abort(); }
     if (ensure_built(u, xs)) return nullptr;
@@ -809,18 +813,24 @@ const float *unet_forward_x(unet *u, const void *x, shape5 xs, int train, int x_
 }
 const float *unet_forward(unet *u, const float *x, shape5 xs, int train) { return unet_forward_x(u, x, xs, train, 0); }
 /* one forward over xs.n windows: window n's input rows go to sample n; logits [n][cout][voxels] */
-const float *mi_unet_forward_ct_n(unet *u, const uint8_t *const *ct, float mean, float isd, const float *const *dyo, const float *const *dxo, int axis, shape5 xs, int h16) {
-    if (xs.c != 4 || u->cfg.cin != 4 || xs.h != xs.w) { fprintf(stderr, "unet_forward_ct: needs square windows of 4 input channels\n"); return nullptr; }
-    if (ensure_built(u, xs)) return nullptr;
+static int forward_ct_n(unet *u, const uint8_t *const *ct, float mean, float isd, const float *const *dyo, const float *const *dxo, int axis, shape5 xs, int h16, float *logits) {
+    if (xs.c != 4 || u->cfg.cin != 4 || xs.h != xs.w) { fprintf(stderr, "unet_forward_ct: needs square windows of 4 input channels\n"); return -1; }
+    if (ensure_built(u, xs)) return -1;
     mi_pred_input_mx_batch(ct, xs.w, mean, isd, dyo, dxo, axis, 0, xs.d, u->xin, h16, u->act_dt == 4 ? 4 : 8, xs.n, 0, xs.n);
-    return mi_unet_forward_mx(u, u->xin, xs);
+    return mi_unet_forward_mx_to(u, u->xin, xs, logits);
 }
-const float *unet_forward_ct(unet *u, const uint8_t *ct, float mean, float isd, const float *dyo, const float *dxo, int axis, shape5 xs, int h16) {
-    if (xs.n < 1 || xs.n > 64) { fprintf(stderr, "unet_forward_ct: %d windows per forward (1 .. 64)\n", xs.n); return nullptr; }
+const float *mi_unet_forward_ct_n(unet *u, const uint8_t *const *ct, float mean, float isd, const float *const *dyo, const float *const *dxo, int axis, shape5 xs, int h16) {
+    return forward_ct_n(u, ct, mean, isd, dyo, dxo, axis, xs, h16, nullptr) ? nullptr : u->logits;
+}
+int mi_unet_forward_ct_to(unet *u, const uint8_t *ct, float mean, float isd, const float *dyo, const float *dxo, int axis, shape5 xs, int h16, float *logits) {
+    if (xs.n < 1 || xs.n > 64) { fprintf(stderr, "unet_forward_ct: %d windows per forward (1 .. 64)\n", xs.n); return -1; }
     const uint8_t *cts[64]; const float *dys[64], *dxs[64];
     const size_t w3 = (size_t)xs.d * xs.h * xs.w;
     for (int n = 0; n < xs.n; n++) { cts[n] = ct + (size_t)n * w3; dys[n] = dyo + (size_t)n * xs.d; dxs[n] = dxo + (size_t)n * xs.d; }
-    return mi_unet_forward_ct_n(u, cts, mean, isd, dys, dxs, axis, xs, h16);
+    return forward_ct_n(u, cts, mean, isd, dys, dxs, axis, xs, h16, logits);
+}
+const float *unet_forward_ct(unet *u, const uint8_t *ct, float mean, float isd, const float *dyo, const float *dxo, int axis, shape5 xs, int h16) {
+    return mi_unet_forward_ct_to(u, ct, mean, isd, dyo, dxo, axis, xs, h16, nullptr) ? nullptr : u->logits;
 }
 int mi_unet_layer_stats(const unet *u, int k, const float **mean, const float **rstd) {
     if (k < 0 || k >= u->nouts) return 0;

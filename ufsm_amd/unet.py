@@ -52,6 +52,8 @@ def load_host():
     L.unet_forward_ct.restype = P; L.unet_forward_ct.argtypes = [P, P, C.c_float, C.c_float, P, P, _I, shape5, _I]
     L.mi_unet_forward_ct_n.restype = P; L.mi_unet_forward_ct_n.argtypes = [P, P, C.c_float, C.c_float, P, P, _I, shape5, _I]
     L.mi_unet_forward_mx.restype = P; L.mi_unet_forward_mx.argtypes = [P, P, shape5]
+    L.mi_unet_forward_mx_to.restype = _I; L.mi_unet_forward_mx_to.argtypes = [P, P, shape5, P]
+    L.mi_unet_forward_ct_to.restype = _I; L.mi_unet_forward_ct_to.argtypes = [P, P, C.c_float, C.c_float, P, P, _I, shape5, _I, P]
     L.mi_unet_get_params.restype = None; L.mi_unet_get_params.argtypes = [P, P]
     L.mi_unet_set_params.restype = None; L.mi_unet_set_params.argtypes = [P, P]
     L.mi_unet_layer_out.restype = P; L.mi_unet_layer_out.argtypes = [P, _I, C.POINTER(shape5), C.POINTER(C.c_char_p)]
@@ -162,13 +164,12 @@ class UNet:
             self._unmode()
 
     def forward_x(self, x_ptr, logits_ptr):
-        """forward_mx, the logits copied into the caller's device buffer; 0 on success."""
-        from .lp import lib
-        p = self.forward_mx(x_ptr)
-        if not p:
-            return -1
-        lib.mi_d2d(logits_ptr, p, self.logits_bytes())
-        return 0
+        """forward_mx, the logits written to the caller's device buffer; 0 on success."""
+        self._mode()
+        try:
+            return -1 if not logits_ptr or self.L.mi_unet_forward_mx_to(self.h, x_ptr, self.shape, logits_ptr) else 0
+        finally:
+            self._unmode()
 
     def forward_planes(self, x_ptr, h16=False):
         """unet_forward_x: fp32 (or fp16) planes in, the net's logits pointer out."""
@@ -179,16 +180,12 @@ class UNet:
             self._unmode()
 
     def forward_ct(self, ct_ptr, mean, isd, dyo_ptr, dxo_ptr, axis, logits_ptr, h16=2):
-        from .lp import lib
+        """The forward from the uint8 CT window(s), the logits written to the caller's device buffer; 0 on success."""
         self._mode()
         try:
-            p = self.L.unet_forward_ct(self.h, ct_ptr, mean, isd, dyo_ptr, dxo_ptr, axis, self.shape, h16)
+            return -1 if not logits_ptr or self.L.mi_unet_forward_ct_to(self.h, ct_ptr, mean, isd, dyo_ptr, dxo_ptr, axis, self.shape, h16, logits_ptr) else 0
         finally:
             self._unmode()
-        if not p:
-            return -1
-        lib.mi_d2d(logits_ptr, p, self.logits_bytes())
-        return 0
 
     def predict_volume(self, vol_ptr, dims, halo, feather, mean, isd, axis, cy, cx, out_ptr):
         """Sliding-window prediction of a device uint8 volume; returns (rc, windows, windows computed)."""
