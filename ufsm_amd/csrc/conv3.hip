@@ -257,7 +257,7 @@ static void conv_stats_reduce(const char *who, const conv_args &a, int MT, split
         if (!a.stat_ch && mi_restage_records(a.y, xdt, a.N, a.Co, S, g.gamma, g.beta, rec, g.y8, g.y4)) return;
         conv_stats_reduce(who, a, MT, sp, osum);
         gnp_t gp; memset(&gp, 0, sizeof gp); gp.gamma = g.gamma; gp.beta = g.beta; gp.mean = fin.mean; gp.rstd = fin.rstd; gp.G = a.Go;
-        if (g.y8 && g.y4 && xdt == 3) mi_restage_sub2(a.y, a.N, a.Co, S, gp, g.y8, g.y4, S, 0);
+        if (g.y8 && g.y4) mi_restage_sub2(a.y, xdt, a.N, a.Co, S, gp, g.y8, g.y4, S, 0);
         else {
             if (g.y8) mi_restage_sub(a.y, xdt, a.N, a.Co, S, gp, a.Co, 0, g.y8, 8, S, 0);
             if (g.y4) mi_restage_sub(a.y, xdt, a.N, a.Co, S, gp, a.Co, 0, g.y4, 4, S, 0);
@@ -687,7 +687,7 @@ extern "C" int mi_conv_prestage(const void *x, int xdt, shape5 s, gnp_t gp, void
 extern "C" int mi_conv_prestage2(const void *x, shape5 s, gnp_t gp, void *y8, void *y4) {
     if (s.c % 32 || (gp.G > 0 && s.c % gp.G) || !y8 || !y4) return -1;
     const size_t hw = (size_t)s.h * s.w;
-    gn_for_slabs("mi_conv_prestage2", gp, s.h * s.w, 0, s.d, [&](int z0, int z1, gnp_t gs) { mi_restage_sub2(x, s.n, s.c, (size_t)(z1 - z0) * hw, gs, y8, y4, (size_t)s.d * hw, (size_t)z0 * hw); });
+    gn_for_slabs("mi_conv_prestage2", gp, s.h * s.w, 0, s.d, [&](int z0, int z1, gnp_t gs) { mi_restage_sub2(x, 3, s.n, s.c, (size_t)(z1 - z0) * hw, gs, y8, y4, (size_t)s.d * hw, (size_t)z0 * hw); });
     return 0;
 }
 extern "C" int lp_conv_fwd_f8(const void *x, int xbf, shape5 xs, const float *w, const float *b, int cout, void *y, int ybf, gnp_t gp, double *osum, int Go, split_t sp) {

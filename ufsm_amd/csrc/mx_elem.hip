@@ -951,16 +951,17 @@ __global__ void __launch_bounds__(256) restage32_k(const uint8_t *x, uint8_t *y,
         }
     }
 }
-// MX-fp8 source with 32-wide blocks -> the transformed rows in both formats from one read (y8 MX-fp8, y4 MX-fp4), the bytes of the two single calls
-void mi_restage_sub2(const void *x, int N, int C, size_t S, gnp_t gp, void *y8, void *y4, size_t Ss, size_t v0) {
+// source with 32-wide blocks (xdt 3 / 4) -> the transformed rows in both formats from one read (y8 MX-fp8, y4 MX-fp4), the bytes of the two single calls
+void mi_restage_sub2(const void *x, int xdt, int N, int C, size_t S, gnp_t gp, void *y8, void *y4, size_t Ss, size_t v0) {
     if (!N || !S) return;
     const dim3 grid(nblk_(S, 128 * RS32_R), (unsigned)(C / 32), (unsigned)N);
-    restage32_k<8, 8, 4><<<grid, 256>>>((const uint8_t *)x, (uint8_t *)y8, N, C, S, gp, C, 0, Ss, v0, (uint8_t *)y4);
+    if (xdt == 3) restage32_k<8, 8, 4><<<grid, 256>>>((const uint8_t *)x, (uint8_t *)y8, N, C, S, gp, C, 0, Ss, v0, (uint8_t *)y4);
+    else restage32_k<4, 8, 4><<<grid, 256>>>((const uint8_t *)x, (uint8_t *)y8, N, C, S, gp, C, 0, Ss, v0, (uint8_t *)y4);
     MICK();
 }
 bool mi_restage_records(const void *x, int xdt, int N, int C, size_t S, const float *gamma, const float *beta, const gn_records_t &rec, void *y8, void *y4) {
     const int cpg = C / rec.Go;
-    if (C % 32 || (xdt != 3 && xdt != 4) || cpg % 4 || !N || !S || (y8 && y4 && xdt != 3)) return false;
+    if (C % 32 || (xdt != 3 && xdt != 4) || cpg % 4 || !N || !S) return false;
     int nq = 0;                                                    // the most quads a block's groups have
     for (int b = 0; b < C / 32; b++) { const int k = ((b * 32 + 31) / cpg - b * 32 / cpg + 1) * (cpg / 4); if (k > nq) nq = k; }
     if (nq > 16) return false;
@@ -972,7 +973,7 @@ bool mi_restage_records(const void *x, int xdt, int N, int C, size_t S, const fl
     const uint8_t *xq = (const uint8_t *)x;
 #define RR(BX, BY, BY2, Y, Y2) restage32_k<BX, BY, BY2, true><<<grid, 256>>>(xq, (uint8_t *)(Y), N, C, S, gp, C, 0, S, 0, (uint8_t *)(Y2), rec)
     if (xdt == 3) { if (y8 && y4) RR(8, 8, 4, y8, y4); else if (y8) RR(8, 8, 0, y8, nullptr); else RR(8, 4, 0, y4, nullptr); }
-    else if (y8) RR(4, 8, 0, y8, nullptr); else RR(4, 4, 0, y4, nullptr);
+    else if (y8 && y4) RR(4, 8, 4, y8, y4); else if (y8) RR(4, 8, 0, y8, nullptr); else RR(4, 4, 0, y4, nullptr);
 #undef RR
     MICK();
     return true;

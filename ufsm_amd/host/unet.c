@@ -45,11 +45,12 @@ struct unet {
     convp ds[UNET_MAXLEV], eh;         /* cfg.ds_levels / cfg.emb_lev: the deep-supervision heads of decoder levels 1 .. ds_levels and the distillation head: training-time outputs, here only their place in the parameter vector (src/unet.c:467, :511) */
     void *downo[UNET_MAXLEV];
     /* per level, silu(gn(.)) of the conv output just written, as the operand rows (MX-fp8 or MX-fp4) of its one reader, the next conv of the graph: the level's pre-staged skip's
-       buffer, whose rows are written after conv2 has read conv1's and are dead once the decoder's conv1 has read them, or (levels without one) rows_own, one buffer for all */
-    void *rows[UNET_MAXLEV], *rows_own;
+       buffer of that format, whose rows are written after conv2 has read conv1's and are dead once the decoder's conv1 has read them, or (levels without one) rows_own, one buffer for all */
+    void *rows8[UNET_MAXLEV], *rows4[UNET_MAXLEV], *rows_own;
     void *skipst[UNET_MAXLEV];         /* silu(gn(enc[i].a2)) in the compute format, formed once for its two readers (down conv, decoder conv1); null: each reader transforms it */
-    void *skipst4[UNET_MAXLEV];        /* precision 3 over MX-fp8 storage: the two readers compute in different formats (the stride-2 conv in e4m3, the decoder's in e2m1);
-                                          the same pass writes the MX-fp4 rows here beside the MX-fp8 ones in skipst */
+    void *skipst4[UNET_MAXLEV];        /* precision 3 over MX-fp8 storage, and MX-fp4 storage: the two readers compute in different formats (the stride-2 conv in e4m3, the decoder's
+                                          in e2m1); the same pass writes the MX-fp4 rows here beside the MX-fp8 ones in skipst. MX-fp4 storage where the stride-2 conv computes
+                                          in e2m1 as well (32 channels): only these */
     gnpar dn[UNET_MAXLEV]; float *dm[UNET_MAXLEV], *dr[UNET_MAXLEV];   /* down_norm: GroupNorm after down[i], its statistics */
     size_t np; float *p, *ema, *params;                            /* device: live weights, EMA copy, the one the forward reads */
     float *src, *wm; int wm_ok;                                    /* cfg.w4_2d: the selected weights (p or ema), their forward copy with the fp4 convs' weights rounded per 32 x 32 block, whether it is current */
@@ -264,7 +265,7 @@ static void free_acts(unet *u) {
     for (int i = 0; i < 2; i++) { act_del(u->slab_tmp[i]); act_del(u->slab_carry[i]); u->slab_tmp[i] = u->slab_carry[i] = nullptr; }
     act_del(u->xin); u->xin = nullptr;
     if (u->rows_own) mi_free(u->rows_own);
-    u->rows_own = nullptr; memset(u->rows, 0, sizeof u->rows);
+    u->rows_own = nullptr; memset(u->rows8, 0, sizeof u->rows8); memset(u->rows4, 0, sizeof u->rows4);
     mi_free(u->logits); u->logits = nullptr;
     u->built = 0; u->nouts = 0; u->slab_ip = u->slab_nl = u->slab_s = 0; u->l0s_zs = u->l0s_ns = 0;
 }
@@ -311,9 +312,10 @@ static int build_acts(unet *u, shape5 in) {
             /* both readers of the skip compute in e4m3 from MX-fp8 storage: one shared pre-stage (any other combination: the readers' formats differ) */
             static int skip2 = -1;                                 /* tuning knob MI_UNET_SKIP2=0: under precision 3 each reader transforms the skip itself */
             if (skip2 < 0) skip2 = getenv("MI_UNET_SKIP2") ? atoi(getenv("MI_UNET_SKIP2")) : 1;
-            if (u->act_dt == 8 && (u->prec != 3 || skip2) && w[i] % 32 == 0 && i >= u->slab_nl) {
-                u->skipst[i] = act_new(u, u->enc[i].ys);
-                if (u->prec == 3) { const size_t b4 = nn_mx4_bytes(u->enc[i].ys); u->skipst4[i] = mi_malloc(b4); mi_zero(u->skipst4[i], b4); nn_set_storage(u->skipst4[i], b4, 4); }
+            if ((u->act_dt == 4 || u->prec != 3 || skip2) && w[i] % 32 == 0 && i >= u->slab_nl) {
+                if (u->act_dt == 8) u->skipst[i] = act_new(u, u->enc[i].ys);
+                else if (w[i] > 32) { const size_t b8 = nn_mx8_bytes(u->enc[i].ys); u->skipst[i] = mi_malloc(b8); mi_zero(u->skipst[i], b8); nn_set_storage(u->skipst[i], b8, 8); }
+                if (u->act_dt == 4 || u->prec == 3) { const size_t b4 = nn_mx4_bytes(u->enc[i].ys); u->skipst4[i] = mi_malloc(b4); mi_zero(u->skipst4[i], b4); nn_set_storage(u->skipst4[i], b4, 4); }
             }
             if (cfg->down_norm) { const size_t ng = (size_t)in.n * G_of(u, w[i]); u->dm[i] = f32_new(ng); u->dr[i] = f32_new(ng); }
         }
@@ -324,9 +326,12 @@ static int build_acts(unet *u, shape5 in) {
     }
     u->xin = act_new(u, in);
     size_t rows = 0;
-    for (int i = 0; i < L; i++) { const size_t r = nn_mx8_bytes(u->ls[i]); if (!u->skipst[i] && r > rows) rows = r; }      /* (a decoder block is at most as wide as its level) */
+    for (int i = 0; i < L; i++) {                                  /* (a decoder block is at most as wide as its level) */
+        const size_t r = !u->skipst[i] && (i || u->act_dt == 8) ? nn_mx8_bytes(u->ls[i]) : !u->skipst4[i] && (u->act_dt == 4 || u->prec == 3) ? nn_mx4_bytes(u->ls[i]) : 0;      /* (level 0 hands no coarse rows on) */
+        if (r > rows) rows = r;
+    }
     if (rows) u->rows_own = mi_malloc(rows);
-    for (int i = 0; i < L; i++) u->rows[i] = u->skipst[i] ? u->skipst[i] : u->rows_own;
+    for (int i = 0; i < L; i++) { u->rows8[i] = u->skipst[i] ? u->skipst[i] : u->rows_own; u->rows4[i] = u->skipst4[i] ? u->skipst4[i] : u->rows_own; }
     u->logits = f32_new((size_t)in.n * cfg->cout * in.d * in.h * in.w);
     if (u->tbn) {
         const shape5 ys = u->ls[L - 1]; const long Sg = (long)ys.d * ys.h * ys.w, S = Sg + u->tbd.nreg, T = (long)ys.n * S; const int C = u->tbd.C;
@@ -563,7 +568,7 @@ static void l0_const_fill(unet *u) {
 }
 /* conv1 -> a1 (+ its statistics), conv2 reads silu(gn(a1)) while staging -> a2 (+ statistics) (src/unet.c:2567-2636); in z-slabs when asked for
    (slab_run, src/unet.c:2499-2545) */
-/* what a block's convs hand on as operand rows: the coarse segment of the block's input (uprows: the level below holds them in its u->rows), and of the block's output silu(gn(a2)) as MX-fp8 rows st8
+/* what a block's convs hand on as operand rows: the coarse segment of the block's input (uprows: the level below holds them in its rows8), and of the block's output silu(gn(a2)) as MX-fp8 rows st8
    and / or MX-fp4 rows st4 when they are asked for; done: they were written */
 typedef struct { int uprows; void *st8, *st4; int done; } rows_io;
 static int block_fwd(unet *u, block *b, int level, const void *x, const nn_gn_t *gin, const void *xup, const nn_gn_t *gup, int c_split, const char *n1, const char *n2, rows_io *io) {
@@ -577,7 +582,7 @@ static int block_fwd(unet *u, block *b, int level, const void *x, const nn_gn_t 
     /* outside slabs, with statistics of its own, a conv's output leaves its GroupNorm + SiLU to one pass behind the conv (mi_conv_fwd_gn_stage), whose rows the next conv reads as
        they are; the reader's own pre-pass would make the same rows */
     const int rows_ok = !s && !ip && Gc > 0, fam4 = u->act_dt == 4 || u->prec == 3;
-    void *const rows = u->rows[level];
+    void *const rows = fam4 ? u->rows4[level] : u->rows8[level];
     int have = 0;                                                  /* rows holds silu(gn(a1)) in conv2's compute format */
     io->done = 0;
     for (int conv = b->single ? 2 : 1; conv <= 2 && !r; conv++) {  /* (one-conv decoder block: its conv, with c1's weights, writes a2 and the statistics m2 / r2, src/unet.c:2581-2582) */
@@ -600,7 +605,7 @@ static int block_fwd(unet *u, block *b, int level, const void *x, const nn_gn_t 
             if (rows_ok && (st8 || st4 || have)) {
                 const int e = !first ? mi_nn_conv3d_rows(have ? rows : b->a1, have, have ? nullptr : &(nn_gn_t){P(u, b->n1.gamma), P(u, b->n1.beta), b->m1, b->r1, G}, nullptr, nullptr, 0, 0, 0, xs,
                                                          P(u, cp->w), cb, cp->cout, o, Gc, 1e-5f, om, orr, P(u, gn->gamma), P(u, gn->beta), st8, st4)
-                            : xup ? mi_nn_conv3d_rows(io->uprows ? u->rows[level + 1] : xup, 0, io->uprows ? nullptr : gup, x, gin, c_split, 1, io->uprows, xs, P(u, cp->w), cb, cp->cout, o, Gc, 1e-5f, om, orr, P(u, gn->gamma), P(u, gn->beta), st8, st4)
+                            : xup ? mi_nn_conv3d_rows(io->uprows ? u->rows8[level + 1] : xup, 0, io->uprows ? nullptr : gup, x, gin, c_split, 1, io->uprows, xs, P(u, cp->w), cb, cp->cout, o, Gc, 1e-5f, om, orr, P(u, gn->gamma), P(u, gn->beta), st8, st4)
                                   : mi_nn_conv3d_rows(x, 0, gin, nullptr, nullptr, 0, 0, 0, xs, P(u, cp->w), cb, cp->cout, o, Gc, 1e-5f, om, orr, P(u, gn->gamma), P(u, gn->beta), st8, st4);
                 if (!e) { if (more) have = 1; else io->done = st8 || st4; continue; }
                 if (have) { r = -1; break; }                       /* (conv2 takes what conv1 took) */
@@ -753,17 +758,25 @@ static int graph_fwd(unet *u, const void *x, float *logits) {
         nn_gn_t gd; const nn_gn_t *gin = nullptr;                  /* down_norm: conv1 reads silu(gn(down conv output)) (src/unet.c:2593) */
         if (i && u->cfg.down_norm) { gd = (nn_gn_t){P(u, u->dn[i - 1].gamma), P(u, u->dn[i - 1].beta), u->dm[i - 1], u->dr[i - 1], G_of(u, u->cfg.widths[i - 1])}; gin = &gd; }
         rows_io io = {0};
-        if (!u->cfg.enc_blocks[i]) { if (i < L - 1) { io.st8 = u->skipst[i]; io.st4 = u->skipst4[i]; } else if (L > 1 && !u->tbn) io.st8 = u->rows[i]; }
+        if (!u->cfg.enc_blocks[i]) { if (i < L - 1) { io.st8 = u->skipst[i]; io.st4 = u->skipst4[i]; } else if (L > 1 && !u->tbn) io.st8 = u->rows8[i]; }
         if (block_fwd(u, &u->enc[i], i, cur, gin, nullptr, nullptr, 0, en1[i], en2[i], &io)) return -1;
         if (i == L - 1) uprows = io.done;
         for (int k = 0; k < u->cfg.enc_blocks[i]; k++) if (rblock_fwd(u, &u->rb[i][k], k ? &u->rb[i][k - 1] : &u->enc[i], u->rbn[i][k])) return -1;      /* (src/unet.c:2963) */
         if (i < L - 1) {                                           /* stride-2 down conv of silu(gn(a2)), width kept (src/unet.c:2970) */
             const block *so = stage_out(u, i);
             const nn_gn_t g = gn_out(u, so);
-            const int pre = u->skipst[i] != nullptr;
-            if (pre && !io.done && (u->skipst4[i] ? mi_conv_prestage2(so->a2, so->ys, gnp_mk(g.gamma, g.beta, g.mean, g.rstd, g.G), u->skipst[i], u->skipst4[i])
-                                      : mi_conv_prestage(so->a2, 3, so->ys, gnp_mk(g.gamma, g.beta, g.mean, g.rstd, g.G), u->skipst[i], 8))) return -1;
-            if (nn_conv3d_fwd_x(pre ? u->skipst[i] : so->a2, pre ? nullptr : &g, nullptr, nullptr, 0, 0, so->ys, P(u, u->down[i].w), P(u, u->down[i].b), u->cfg.widths[i], 3, 2, u->downo[i], 0, 0.f, nullptr, nullptr)) return -1;
+            const int pre = u->skipst[i] || u->skipst4[i];
+            if (pre && !io.done) {
+                const gnp_t gp = gnp_mk(g.gamma, g.beta, g.mean, g.rstd, g.G);
+                const int dt = u->act_dt == 4 ? 4 : 3;
+                if (dt == 3 && u->skipst4[i]) { if (mi_conv_prestage2(so->a2, so->ys, gp, u->skipst[i], u->skipst4[i])) return -1; }
+                else if ((u->skipst[i] && mi_conv_prestage(so->a2, dt, so->ys, gp, u->skipst[i], 8)) || (u->skipst4[i] && mi_conv_prestage(so->a2, dt, so->ys, gp, u->skipst4[i], 4))) return -1;
+            }
+            if (pre && u->act_dt == 4) {                           /* the rows in the format the stride-2 entry computes in for MX-fp4 storage (lp_conv_fwd_s2_f8: e2m1 for 32 channels, else e4m3) */
+                shape5 ds = u->ls[i + 1]; ds.c = u->cfg.widths[i];
+                mi_conv_s2_wkey((unsigned)((uintptr_t)P(u, u->down[i].w) >> 4) | 1u);
+                lp_conv_fwd_s2_f8(u->skipst[i] ? u->skipst[i] : u->skipst4[i], u->skipst[i] ? 3 : 4, so->ys, P(u, u->down[i].w), P(u, u->down[i].b), ds.c, u->downo[i], 4, ds, gnp_mk(nullptr, nullptr, nullptr, nullptr, 0));
+            } else if (nn_conv3d_fwd_x(pre ? u->skipst[i] : so->a2, pre ? nullptr : &g, nullptr, nullptr, 0, 0, so->ys, P(u, u->down[i].w), P(u, u->down[i].b), u->cfg.widths[i], 3, 2, u->downo[i], 0, 0.f, nullptr, nullptr)) return -1;
             shape5 ds = u->ls[i + 1]; ds.c = u->cfg.widths[i];
             if (u->cfg.down_norm) {                                /* statistics of the stored down-conv output now, the transform in the next conv1's staging (src/unet.c:2974-2979) */
                 if (!ge_const(u) && nn_gn_stats(u->downo[i], ds, G_of(u, ds.c), 1e-5f, u->dm[i], u->dr[i])) { fprintf(stderr, "unet: down_norm GroupNorm statistics unsupported for this storage\n"); return -1; }
@@ -779,7 +792,7 @@ static int graph_fwd(unet *u, const void *x, float *logits) {
         if (i == L - 2 && u->tbn) { coarse = &u->tb; gc.mean = u->tb.m2; gc.rstd = u->tb.r2; }      /* the stage's output under the level's n2 affine (src/unet.c:508) */
         static const nn_gn_t none = {nullptr, nullptr, nullptr, nullptr, -1};          /* the pre-staged skip: no GroupNorm left to apply */
         const void *sk = u->skipst4[i] ? u->skipst4[i] : u->skipst[i];      /* (the decoder's conv computes in e2m1 under precision 3: its rows) */
-        rows_io io = {.uprows = uprows, .st8 = i ? u->rows[i] : nullptr};      /* (the coarse rows are e4m3 whatever the decoder's conv computes in) */
+        rows_io io = {.uprows = uprows, .st8 = i ? u->rows8[i] : nullptr};      /* (the coarse rows are e4m3 whatever the decoder's conv computes in) */
         if (block_fwd(u, &u->dec[i], i, sk ? sk : skip->a2, sk ? &none : &gs, coarse->a2, &gc, coarse->ys.c, dn1[i], dn2[i], &io)) return -1;
         uprows = io.done;
     }
