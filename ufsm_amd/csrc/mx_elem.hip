@@ -54,9 +54,15 @@ static dim3 rows_grid(int N, int nb, size_t S) {
 //   146 -> 119 (pairs: 160 and 142). Blocks of 8 channels stay pairs (305 MB, to MX and back: 161 and 158, streamed 172 and 165). Lines shared by two
 //   wavefronts lose their meeting in the cache (64 channels, 999999: 53 / 68 -> 61 / 100 and 48 / 59 -> 55 / 98), and planes that fit the cache are found there (64
 //   channels, 96^3 to MX: 43 -> 46 and 39 -> 44).
+//   These kernels ask for LDS that they do not use, which leaves 4 blocks of them on a CU (6 with blocks of 16 channels): the fewer wavefronts run, the
+//   nearer together are the addresses that a plane's stream is at, and the fewer DRAM pages are open at once. Blocks a CU, all (8) / 6 / 5 / 4 / 3, us to MX and back:
+//   32 channels, 2 x 128^3, e4m3 242 / 231 / 223 / 219 / 216 and e2m1 228 / 215 / 207 / 203 / 200; 160^3 204 / 202 / 201 / 202 / 204 and 197 / 196 / 195 / 194 / 195; 8 x 294912
+//   116 / 115 / 115 / 114 / 117; 96 channels, 96^3 131 / 130 / 130 / 129 / 130; 64 channels, 4 x 393216 156 / 156 / 155 / 155 / 157 (planes of a power of two gain
+//   most: their streams meet in one channel). 16 channels, 2 x 128^3 124 / 120 / 122 / 132 / 136, 192^3 172 / 169 / 169 / 173 / 189.
 constexpr int CVT_BW = 16;         // widest block of the pairs
 static bool cvt_pairs(int C, size_t S) { return mx_bw(C) <= CVT_BW && S >= (size_t)1 << 17; }
 static bool cvt_stream(const void *planes, int N, int C, size_t S) { return mx_bw(C) > 8 && S % 32 == 0 && !((uintptr_t)planes & 127) && (size_t)N * C * S * 4 >= (size_t)256 << 20; }
+static unsigned cvt_lds(int C) { return mx_bw(C) > 16 ? (160u << 10) / 4 : 21 * 1280; }      // of a CU's 160 KB (in 1280 bytes), for 4 and for 6 blocks
 typedef float plane2_t __attribute__((ext_vector_type(2), aligned(4)));      // two neighbouring voxels of a plane (any element's address)
 template <int B, typename TI, bool STREAM = false>
 __global__ void __launch_bounds__(256) f32_to_mx_k(const TI *x, uint8_t *y, int N, int C, size_t S) {
@@ -98,7 +104,7 @@ __global__ void __launch_bounds__(256) f32_to_mx_pairs_k(const float *x, uint8_t
 template <int B> static void f32_to_mx(const float *x, int N, int C, size_t S, void *y) {
     const size_t n = (size_t)N * mx_nb(C) * S;
     if (!n) return;
-    if (cvt_stream(x, N, C, S)) f32_to_mx_k<B, float, true><<<rows_grid(N, mx_nb(C), S), 256>>>(x, (uint8_t *)y, N, C, S);
+    if (cvt_stream(x, N, C, S)) f32_to_mx_k<B, float, true><<<rows_grid(N, mx_nb(C), S), 256, cvt_lds(C)>>>(x, (uint8_t *)y, N, C, S);
     else if (cvt_pairs(C, S)) f32_to_mx_pairs_k<B><<<rows_grid(N, mx_nb(C), (S + 1) / 2), 256>>>(x, (uint8_t *)y, N, C, S);
     else f32_to_mx_k<B, float><<<rows_grid(N, mx_nb(C), S), 256>>>(x, (uint8_t *)y, N, C, S);
     MICK();
@@ -154,7 +160,7 @@ __global__ void __launch_bounds__(256) mx_to_f32_pairs_k(const uint8_t *x, float
 }
 template <int B> static void mx_to_f32(const void *x, int N, int C, size_t S, float *y) {
     const size_t n = (size_t)N * mx_nb(C) * S; if (!n) return;
-    if (cvt_stream(y, N, C, S)) mx_to_f32_k<B, true><<<rows_grid(N, mx_nb(C), S), 256>>>((const uint8_t *)x, y, N, C, S);
+    if (cvt_stream(y, N, C, S)) mx_to_f32_k<B, true><<<rows_grid(N, mx_nb(C), S), 256, cvt_lds(C)>>>((const uint8_t *)x, y, N, C, S);
     else if (cvt_pairs(C, S)) mx_to_f32_pairs_k<B><<<rows_grid(N, mx_nb(C), (S + 1) / 2), 256>>>((const uint8_t *)x, y, N, C, S);
     else mx_to_f32_k<B><<<rows_grid(N, mx_nb(C), S), 256>>>((const uint8_t *)x, y, N, C, S);
     MICK();
