@@ -19,14 +19,15 @@ __device__ __forceinline__ void gn_part_finish(double *osum, double s, double ss
 // (sum, sum of squares) partials of the tiles -> exact GroupNorm sum slots (src/lp_common.cuh:1575-1597 does the same with one fixed-point atomic
 // per block and channel). A spatial tile's record is Q = Co / 4 (padded to whole channel slices) consecutive float2, one per channel quad; quad
 // Q = co / 4 lives in channel slice Q / (8 MT), slot Q % (8 MT). A block takes one sample's tiles [t0, t1) with ALL their quads: thread (j, q) adds
-// quad q of tiles t0 + j, t0 + j + J, ... in double (consecutive threads read consecutive records: every fetched line is used whole), then the J
-// rows of partial sums are added in halves down to four, and thread g adds its group's quads over these, all in a fixed order. nsplit > 1 (thousands of tiles: the level-0 layers): every block leaves its Go pairs
+// quad q of tiles t0 + j, t0 + j + J, ... in double (consecutive threads read consecutive records: every fetched line is used whole), then thread g
+// adds its group's quads over the J rows (of 1024 threads: added in halves down to four first), all in a fixed order. nsplit > 1 (thousands of tiles: the level-0 layers): every block leaves its Go pairs
 // in scr and takes a ticket of its sample; the block that draws the last one adds the nsplit pairs of every group in index order - the result
 // does not depend on which block that is - and puts the ticket counter back to zero for the next launch
 struct gn_split_t { int nsplit; double *scr; unsigned *cnt; };
-__global__ void __launch_bounds__(1024) gn_part_reduce_k(const float2 *part, int tiles_per_n, int ncs, int MT, int Co, int Go, double *osum, gn_fin_t fin, gn_split_t sp) {
-    const int n = (int)blockIdx.x / sp.nsplit, pi = (int)blockIdx.x % sp.nsplit, tid = (int)threadIdx.x, nth = (int)blockDim.x;
-    const int Q = ncs * MT * 8, nst = tiles_per_n / ncs, qpg = Co / Go / 4, J = nth / Q;
+template <int NTH>
+__global__ void __launch_bounds__(NTH) gn_part_reduce_k(const float2 *part, int tiles_per_n, int ncs, int MT, int Co, int Go, double *osum, gn_fin_t fin, gn_split_t sp) {
+    const int n = (int)blockIdx.x / sp.nsplit, pi = (int)blockIdx.x % sp.nsplit, tid = (int)threadIdx.x;
+    const int Q = ncs * MT * 8, nst = tiles_per_n / ncs, qpg = Co / Go / 4, J = NTH / Q;
     const int per = (nst + sp.nsplit - 1) / sp.nsplit, t0 = pi * per, t1 = min(nst, t0 + per);
     const int q = tid % Q, j = tid / Q;
     const float2 *rec = part + (size_t)n * tiles_per_n * (MT * 8) + q;
@@ -38,17 +39,19 @@ __global__ void __launch_bounds__(1024) gn_part_reduce_k(const float2 *part, int
             s += (double)p.x; ss += (double)p.y;
         }
     }
-    __shared__ double r1[1024], r2[1024];
+    __shared__ double r1[NTH], r2[NTH];
     __shared__ unsigned ticket;
     r1[tid] = s; r2[tid] = ss;
     __syncthreads();
-    for (int m = J; m > 4;) {                                                // the J rows of partial sums in halves down to four, in a fixed order
-        const int hlf = (m + 1) >> 1;
-        if (j < m - hlf) { r1[tid] += r1[tid + hlf * Q]; r2[tid] += r2[tid + hlf * Q]; }
-        __syncthreads();
-        m = hlf;
+    int JJ = J;
+    if constexpr (NTH > 256) {                                               // the J rows of partial sums in halves down to four, in a fixed order
+        while (JJ > 4) {
+            const int hlf = (JJ + 1) >> 1;
+            if (j < JJ - hlf) { r1[tid] += r1[tid + hlf * Q]; r2[tid] += r2[tid + hlf * Q]; }
+            __syncthreads();
+            JJ = hlf;
+        }
     }
-    int JJ = J; while (JJ > 4) JJ = (JJ + 1) >> 1;
     s = 0.0; ss = 0.0;
     if (tid < Go)
         for (int k = 0; k < qpg; k++)
@@ -288,7 +291,9 @@ static void conv_stats_reduce(const char *who, const conv_args &a, int MT, split
     }
     // (one block per sample over more than a few hundred records: four times the threads, 2 002 records of 8 quads 10.4 -> 8.2 us, 1 232 of 16 7.9 -> 6.6; the split launches' blocks
     // are few rounds long already and lose by it, 7.3 -> 10.6)
-    gn_part_reduce_k<<<a.N * gs.nsplit, gs.nsplit == 1 && nst * Q > 8192 ? 1024 : 256>>>((const float2 *)a.part, tiles_per_n, a.ncs, MT, a.Co, a.Go, osum, fin, gs);
+    const float2 *part = (const float2 *)a.part;
+    if (gs.nsplit == 1 && nst * Q > 8192) gn_part_reduce_k<1024><<<a.N, 1024>>>(part, tiles_per_n, a.ncs, MT, a.Co, a.Go, osum, fin, gs);
+    else gn_part_reduce_k<256><<<a.N * gs.nsplit, 256>>>(part, tiles_per_n, a.ncs, MT, a.Co, a.Go, osum, fin, gs);
     MICK();
 }
 
