@@ -344,10 +344,11 @@ __device__ __forceinline__ void conv_epilogue(const conv_args &a, v16f (&acc)[MT
                     const float p2e = d_exp2i(e);
 #pragma unroll
                     for (int q4 = 0; q4 < 4; q4++) d[q4] = d_enc_e4m3x4_hw(v[4 * q4], v[4 * q4 + 1], v[4 * q4 + 2], v[4 * q4 + 3], p2e);
-                    if (__builtin_amdgcn_ballot_w64(e == 128) != 0ull) {      // a block with an infinity or NaN: closed-form codes (never taken by finite data)
+                    if (d_any_nf(e)) {                   // a block with an infinity or NaN: closed-form codes (never taken by finite data)
+                        const unsigned z = d_opaque_zero();
                         if (e == 128) {
 #pragma unroll
-                            for (int q4 = 0; q4 < 4; q4++) d[q4] = d_enc4_e4m3_nf(v[4 * q4], v[4 * q4 + 1], v[4 * q4 + 2], v[4 * q4 + 3]);
+                            for (int q4 = 0; q4 < 4; q4++) d[q4] = d_enc4_e4m3_nf(v[4 * q4], v[4 * q4 + 1], v[4 * q4 + 2], v[4 * q4 + 3], z);
                         }
                     }
                     if (a.stored_stats) {                // the statistics are those of the stored values: decode the codes at the block's scale
@@ -367,8 +368,9 @@ __device__ __forceinline__ void conv_epilogue(const conv_args &a, v16f (&acc)[MT
                 } else {
                     const float p2e = d_exp2i(e);
                     unsigned w01 = d_enc_e2m1x8_hw(v, p2e), w23 = d_enc_e2m1x8_hw(v + 8, p2e);
-                    if (__builtin_amdgcn_ballot_w64(e == 128) != 0ull) {
-                        if (e == 128) { w01 = d_enc8_e2m1_nf(v); w23 = d_enc8_e2m1_nf(v + 8); }
+                    if (d_any_nf(e)) {
+                        const unsigned z = d_opaque_zero();
+                        if (e == 128) { w01 = d_enc8_e2m1_nf(v, z); w23 = d_enc8_e2m1_nf(v + 8, z); }
                     }
                     if (a.stored_stats) {
                         const float sc = d_exp2i(e);

@@ -119,35 +119,42 @@ __device__ __forceinline__ unsigned d_enc_e2m1x8_hw(const float *v, float pow2e)
 }
 // encode with the block exponent e. 128 marks a block holding an infinity or NaN: the reference then multiplies by exp2i(-128), the
 // bits of -inf (src/lp_common.cuh:501), so a finite non-zero value or an infinity saturates with the opposite sign and a zero or a
-// NaN becomes NaN. Those codes have a closed form; they are formed under a wave-uniform branch that finite data never takes.
-__device__ __forceinline__ unsigned d_enc_e4m3_nf(float x) {
-    const unsigned u = __float_as_uint(x), a = u & 0x7fffffffu;
+// NaN becomes NaN. Those codes have a closed form; they are formed under a wave-uniform branch that finite data never takes. z is a zero the
+// compiler does not know, made inside that branch (d_opaque_zero): the closed forms need it, so they stay there. Without it the compiler moved their 38 instructions per
+// word in front of the branch, where every wavefront ran them (a row of restage32_k: 250 vector instructions instead of 125 beside its transcendentals).
+__device__ __forceinline__ unsigned d_opaque_zero() { unsigned z; asm volatile("v_mov_b32 %0, 0" : "=v"(z)); return z; }
+__device__ __forceinline__ unsigned d_enc_e4m3_nf(float x, unsigned z) {
+    const unsigned u = __float_as_uint(x) | z, a = u & 0x7fffffffu;
     return (a == 0u || a > 0x7f800000u) ? 0x7fu : (0x7eu | ((~u >> 24) & 0x80u));
 }
-__device__ __forceinline__ unsigned d_enc_e2m1_nf(float x) {
-    const unsigned u = __float_as_uint(x), a = u & 0x7fffffffu;
+__device__ __forceinline__ unsigned d_enc_e2m1_nf(float x, unsigned z) {
+    const unsigned u = __float_as_uint(x) | z, a = u & 0x7fffffffu;
     return (a == 0u || a > 0x7f800000u) ? 7u : (7u | ((~u >> 28) & 8u));
 }
-__device__ __forceinline__ unsigned d_enc4_e4m3_nf(float a, float b, float c, float d) {
-    return d_enc_e4m3_nf(a) | (d_enc_e4m3_nf(b) << 8) | (d_enc_e4m3_nf(c) << 16) | (d_enc_e4m3_nf(d) << 24);
+__device__ __forceinline__ unsigned d_enc4_e4m3_nf(float a, float b, float c, float d, unsigned z) {
+    return d_enc_e4m3_nf(a, z) | (d_enc_e4m3_nf(b, z) << 8) | (d_enc_e4m3_nf(c, z) << 16) | (d_enc_e4m3_nf(d, z) << 24);
 }
-__device__ __forceinline__ unsigned d_enc8_e2m1_nf(const float *v) {
+__device__ __forceinline__ unsigned d_enc8_e2m1_nf(const float *v, unsigned z) {
     unsigned w = 0u;
 #pragma unroll
-    for (int k = 0; k < 8; k++) w |= d_enc_e2m1_nf(v[k]) << (4 * k);
+    for (int k = 0; k < 8; k++) w |= d_enc_e2m1_nf(v[k], z) << (4 * k);
     return w;
 }
+// (uniform) some lane's block holds an infinity or NaN
+__device__ __forceinline__ bool d_any_nf(int e) { return __builtin_expect(__builtin_amdgcn_ballot_w64(e == 128) != 0ull, 0); }
 __device__ __forceinline__ unsigned d_enc4_e4m3(float a, float b, float c, float d, int e) {
     unsigned w = d_enc_e4m3x4_hw(a, b, c, d, d_exp2i(e));
-    if (__builtin_amdgcn_ballot_w64(e == 128) != 0ull) {
-        if (e == 128) w = d_enc4_e4m3_nf(a, b, c, d);
+    if (d_any_nf(e)) {
+        const unsigned z = d_opaque_zero();
+        if (e == 128) w = d_enc4_e4m3_nf(a, b, c, d, z);
     }
     return w;
 }
 __device__ __forceinline__ unsigned d_enc8_e2m1(const float *v, int e) {
     unsigned w = d_enc_e2m1x8_hw(v, d_exp2i(e));
-    if (__builtin_amdgcn_ballot_w64(e == 128) != 0ull) {
-        if (e == 128) w = d_enc8_e2m1_nf(v);
+    if (d_any_nf(e)) {
+        const unsigned z = d_opaque_zero();
+        if (e == 128) w = d_enc8_e2m1_nf(v, z);
     }
     return w;
 }
@@ -178,12 +185,25 @@ __device__ __forceinline__ unsigned d_quant_row(const float *v, int bw, unsigned
         for (int k = 0; k < 32; k++) if (k < bw) amax = fmaxf(amax, fabsf(v[k]));
     }
     const int e = d_mx_exp(amax, BITS == 8 ? MI_INVQ8 : MI_INVQ4);
+    const float p2e = d_exp2i(e);
     if (BITS == 8) {
 #pragma unroll
-        for (int j = 0; j < 8; j++) codes[j] = 4 * j < bw ? d_enc4_e4m3(v[4 * j], v[4 * j + 1], v[4 * j + 2], v[4 * j + 3], e) : 0u;
+        for (int j = 0; j < 8; j++) codes[j] = 4 * j < bw ? d_enc_e4m3x4_hw(v[4 * j], v[4 * j + 1], v[4 * j + 2], v[4 * j + 3], p2e) : 0u;
     } else {
 #pragma unroll
-        for (int j = 0; j < 4; j++) codes[j] = 8 * j < bw ? d_enc8_e2m1(v + 8 * j, e) : 0u;
+        for (int j = 0; j < 4; j++) codes[j] = 8 * j < bw ? d_enc_e2m1x8_hw(v + 8 * j, p2e) : 0u;
+    }
+    if (d_any_nf(e)) {                                                    // (one branch for the row)
+        const unsigned z = d_opaque_zero();
+        if (e == 128) {
+            if (BITS == 8) {
+#pragma unroll
+                for (int j = 0; j < 8; j++) codes[j] = 4 * j < bw ? d_enc4_e4m3_nf(v[4 * j], v[4 * j + 1], v[4 * j + 2], v[4 * j + 3], z) : 0u;
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; j++) codes[j] = 8 * j < bw ? d_enc8_e2m1_nf(v + 8 * j, z) : 0u;
+            }
+        }
     }
     return (unsigned)(e + 127);
 }
