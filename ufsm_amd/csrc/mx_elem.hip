@@ -49,8 +49,8 @@ static dim3 rows_grid(int N, int nb, size_t S) {
 //   (4 channels: 4.1 / 3.9 and 4.1 / 4.0), hence from 2^17 voxels. Blocks of 32 channels have 32 streams already and lose (2 x 128^3, e4m3: 132 / 142 -> 149 / 140),
 //   and four voxels are no faster than two.
 // * STREAM, blocks of 16 and 32 channels: planes past the 256 MB of the last-level cache are read and written past it where a wavefront's accesses are
-//   whole 128-byte lines (S a multiple of 32, aligned planes). 32 channels, 2 x 128^3: 135 / 146 -> 123 / 116 and 123 / 126 -> 112 / 111 (a large copy reaches
-//   5.3 TB/s, these 5.5 / 5.9); to MX and back 294 -> 240 and 270 -> 222; 1 x 128^3, the smallest: 151 -> 122 and 142 -> 111; 16 channels, 2 x 128^3: 153 -> 124 and
+//   whole 128-byte lines (S a multiple of 32, aligned planes). 32 channels, 2 x 128^3: 135 / 146 -> 123 / 116 and 123 / 126 -> 112 / 111 (before the block
+//   cap below); to MX and back 294 -> 240 and 270 -> 222; 1 x 128^3, the smallest: 151 -> 122 and 142 -> 111; 16 channels, 2 x 128^3: 153 -> 124 and
 //   146 -> 119 (pairs: 160 and 142). Blocks of 8 channels stay pairs (305 MB, to MX and back: 161 and 158, streamed 172 and 165). Lines shared by two
 //   wavefronts lose their meeting in the cache (64 channels, 999999: 53 / 68 -> 61 / 100 and 48 / 59 -> 55 / 98), and planes that fit the cache are found there (64
 //   channels, 96^3 to MX: 43 -> 46 and 39 -> 44).
