@@ -106,12 +106,14 @@ void mi_conv1_matrix(int mode);
    input, gp2.G = -1 says "x2 carries no GroupNorm, gp is x's own" (gp2.G = 0 keeps the reference's meaning: gp spans both segments). */
 int mi_conv_prestage(const void *x, int xdt, shape5 s, gnp_t gp, void *y, int ybits);
 /* the same from an MX-fp8 tensor into both formats at once (y8 MX-fp8, y4 MX-fp4: the bytes of the two single calls from one read and one
-   evaluation): a tensor whose readers compute in different formats. mi_conv_x2_dt(4) before a conv entry says that the calling thread's next
-   split conv's second segment is stored as MX-fp4 although x is MX-fp8 (3: MX-fp8 beside an MX-fp4 x; the descriptor carries one format) */
+   evaluation): a tensor whose readers compute in different formats. mi_conv_x2_dt(4) before a conv entry says that the second segment of the
+   calling thread's next conv is stored as MX-fp4 although x is MX-fp8 (3: MX-fp8 beside an MX-fp4 x; the descriptor carries one format); that call takes
+   the word, whatever becomes of it */
 int mi_conv_prestage2(const void *x, shape5 s, gnp_t gp, void *y8, void *y4);
 void mi_conv_x2_dt(int dt);
-/* mi_conv_up_staged(1) before a conv entry: the calling thread's next split conv's upsampled segment is stored as the e4m3 rows that its own pre-pass (GroupNorm + SiLU +
-   re-quantisation) would make, so it is upsampled as it is (MX-fp8, a multiple of 32 channels; its GroupNorm must be none) */
+/* mi_conv_up_staged(1) before a conv entry: the upsampled segment of the calling thread's next conv is stored as the e4m3 rows that its own pre-pass (GroupNorm + SiLU +
+   re-quantisation) would make, so it is upsampled as it is. It must be MX-fp8, a multiple of 32 channels, with no GroupNorm given (the call ends the process with a
+   message otherwise); that call takes the word, whatever becomes of it, and a conv without an upsampled segment ignores it */
 void mi_conv_up_staged(int on);
 gnp_t gnp_mk(const float *gamma, const float *beta, const float *mean, const float *rstd, int G);   /* src/nn_lp.h:19 */
 int lp_gn_slab_any(void);                                                                         /* src/nn_lp.h:20: any statistics array registered */

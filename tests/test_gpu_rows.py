@@ -86,3 +86,31 @@ def test_upsampled_segment_as_rows(gpu, bits, n, cc, cs, dims):
     conv(rows.ptr, 3, shape5(n, cc + cs, *dims), w.ptr, b.ptr, co, y1.ptr, dt, gnp_t(), None, 0, sp)
     LP.check()
     assert np.array_equal(y0.to_numpy(np.uint8), y1.to_numpy(np.uint8)) and y0.to_numpy(np.uint8).any()
+
+
+@pytest.mark.parametrize("how", ["empty", "refused", "static"])
+def test_words_for_one_call_end_with_it(gpu, how):
+    """mi_conv_up_staged and mi_conv_x2_dt belong to the next call: one that has nothing to do or is refused takes them, and the conv after it reads its operands as they are."""
+    rng = np.random.default_rng(5)
+    n, cc, cs, dims, co, G = 1, 32, 32, (4, 8, 8), 32, 8
+    s = int(np.prod(dims))
+    coarse, skip = to_mx(8, rng.standard_normal((n, cc, s // 8)).astype(np.float32)), to_mx(8, rng.standard_normal((n, cs, s)).astype(np.float32))
+    w = DevBuf.from_numpy((rng.standard_normal((co, cc + cs, 27)) * 0.05).astype(np.float32)); b = DevBuf.from_numpy((0.1 * rng.standard_normal(co)).astype(np.float32))
+    v = [DevBuf.from_numpy(a.astype(np.float32)) for a in (rng.uniform(0.7, 1.3, cc), 0.2 * rng.standard_normal(cc), 0.1 * rng.standard_normal(n * G), rng.uniform(0.8, 1.2, n * G))]
+    g = gnp_t(v[0].ptr, v[1].ptr, v[2].ptr, v[3].ptr, G)
+    sp = split_t(); sp.x2, sp.c_split, sp.up = skip.ptr, cc, 1
+    sp.gp2.G = -1
+    ys = [DevBuf(_bytes(8, n, co, s)) for _ in range(2)]
+    for y, words in zip(ys, (False, True)):
+        if words:
+            lib.mi_conv_up_staged(1); lib.mi_conv_x2_dt(4)
+            p = w.ptr
+            if how == "empty":
+                assert lib.lp_conv_fwd_f8(p, 3, shape5(0, 32, 4, 4, 4), p, p, 32, y.ptr, 3, gnp_t(), None, 0, split_t()) == 0
+            elif how == "refused":
+                assert lib.mi_conv_fwd_gn_stage(8, p, 3, shape5(1, 32, 4, 4, 4), p, p, 48, y.ptr, 3, gnp_t(), p, 8, split_t(), 1e-5, p, p, p, p, y.ptr, None) == -1
+            else:
+                assert lib.mi_conv_fwd_static(8, p, 3, shape5(1, 512, 64, 64, 64), p, p, 512, y.ptr, 3, g, None, 0, split_t()) == -1      # (more than the fixed scratch)
+        lib.lp_conv_fwd_f8(coarse.ptr, 3, shape5(n, cc + cs, *dims), w.ptr, b.ptr, co, y.ptr, 3, g, None, 0, sp)
+    LP.check()
+    assert np.array_equal(ys[0].to_numpy(np.uint8), ys[1].to_numpy(np.uint8)) and ys[0].to_numpy(np.uint8).any()

@@ -364,6 +364,9 @@ static thread_local int g_x2_dt = 0;
 static thread_local bool g_up_staged = false;
 extern "C" void mi_conv_up_staged(int on) { g_up_staged = on != 0; }
 extern "C" void mi_conv_x2_dt(int dt) { g_x2_dt = dt == 3 || dt == 4 ? dt : 0; }
+// both belong to one call of a conv entry and are taken at its start, also where it refuses or has nothing to do: none is left for a later call
+struct conv_once_t { int x2_dt; bool up_staged; };
+static conv_once_t take_once(void) { const conv_once_t o = {g_x2_dt, g_up_staged}; g_x2_dt = 0; g_up_staged = false; return o; }
 static thread_local int g_s2d = -1;         // mi_conv_s2_direct: the calling thread's choice of stride-2 kernel (-1: by launch size)
 extern "C" void mi_conv_s2_direct(int mode) { g_s2d = mode; }
 static thread_local int g_thin = -1;        // mi_conv_thin: the calling thread's tile count up to which the K-split kernel takes a launch (-1: the default rule)
@@ -371,6 +374,7 @@ extern "C" void mi_conv_thin(int tiles) { g_thin = tiles; }
 static int split_s2_env() { static int v = -1; if (v < 0) v = getenv("MI_CONV_SPLIT_S2") ? atoi(getenv("MI_CONV_SPLIT_S2")) : 1; return v; }      // tuning knob: 0 keeps four channel tiles
 static int conv_dispatch(const char *who, int fmt, int stride, const void *x, int xbf, shape5 xs, const float *w, const float *b, int cout, void *y, int ybf,
                          gnp_t gp, double *osum, int Go, split_t sp, const float *ep_a, const float *ep_b, int act) {
+    const conv_once_t once = take_once();
     if (sp.y2 || sp.o_split || sp.accum || sp.sr || sp.osr || sp.o_pad || sp.zw0 || sp.zw1)
         mi_die("%s: split outputs, accumulate, stochastic rounding and the z-window fields of split_t are not built here (inference forward only)", who);
     // z-range (src/nn_lp.h:36-40, src/nn_bwd.cu:33-36): the xs.d output planes read input plane z + zi0 of depth-Di inputs; direct slab output:
@@ -391,6 +395,8 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     if (sp.x2 && (Cx <= 0 || C2 <= 0)) mi_die("%s: channel split %d of %d", who, sp.c_split, Ci);
     if (sp.x2 && xbf < 3) mi_die("%s: split inputs need MX storage", who);
     if (sp.up && (!sp.x2 || xbf < 3 || ((sp.Di ? sp.Di : xs.d) & 1) || (xs.h & 1) || (xs.w & 1) || stride != 1)) mi_die("%s: the fused upsample needs an MX split input and even dims", who);
+    // (rows that are not what mi_restage_up_rows reads, 33 bytes each, would be read past their end; a GroupNorm on them would be one too many)
+    if (once.up_staged && sp.up && (xbf != 3 || Cx % 32 || gp.G)) mi_die("%s: mi_conv_up_staged needs an MX-fp8 first segment of a multiple of 32 channels with no GroupNorm (storage %d, %d channels, %d groups)", who, xbf, Cx, gp.G);
     if (osum && (Go <= 0 || cout % Go)) mi_die("%s: %d output channels in %d groups", who, cout, Go);
     if (gp.G > 0 && ((sp.x2 && sp.gp2.G ? Cx : Ci) % gp.G)) mi_die("%s: GroupNorm groups %d do not divide the channels", who, gp.G);
     if (sp.gp2.G > 0 && (!sp.x2 || C2 % sp.gp2.G)) mi_die("%s: second GroupNorm without a matching x2 segment", who);
@@ -419,10 +425,7 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     const bool s2g = sp.x2 && sp.gp2.G;
     if (sp.gp2.G < 0) sp.gp2 = gnp_mk(nullptr, nullptr, nullptr, nullptr, 0);
     const void *segx[2] = {x, sp.x2}; const int segC[2] = {Cx, C2};
-    const int segbf[2] = {xbf, sp.x2 && g_x2_dt ? g_x2_dt : xbf};
-    g_x2_dt = 0;
-    const bool up_staged = g_up_staged && sp.up && xbf >= 3 && Cx % 32 == 0;
-    g_up_staged = false;
+    const int segbf[2] = {xbf, sp.x2 && once.x2_dt ? once.x2_dt : xbf};
     for (int s = 0; s < (sp.x2 ? 2 : 1); s++) {
         const gnp_t g = s2g ? (s ? sp.gp2 : gp) : gp;
         const int Cg = s2g ? segC[s] : Ci, cg0 = s2g ? 0 : (s ? Cx : 0);
@@ -440,7 +443,7 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
             // the fp4 entry blends the upsample in binary16 unless UFSM_UP_H2=0 (src/lp_f4fwd.cuh:1135-1136); sp.up 2 / 3 force one blend
             static int uph2 = -1;
             if (uph2 < 0) uph2 = getenv("UFSM_UP_H2") ? atoi(getenv("UFSM_UP_H2")) : 1;
-            if (upseg && up_staged) mi_restage_up_rows(segx[s], N, segC[s], D, H, W, st, fmt, zlo, zhi, sp.up == 2 || (sp.up == 1 && entry_fmt == 4 && uph2));
+            if (upseg && once.up_staged) mi_restage_up_rows(segx[s], N, segC[s], D, H, W, st, fmt, zlo, zhi, sp.up == 2 || (sp.up == 1 && entry_fmt == 4 && uph2));
             else if (upseg) mi_restage_up_sub(segx[s], xbf, N, segC[s], D, H, W, g, Cg, st, fmt, zlo, zhi, sp.up == 2 || (sp.up == 1 && entry_fmt == 4 && uph2));
             else gn_for_slabs(who, g, H * W, zlo, zhi, [&](int z0, int z1, gnp_t gs) { mi_restage_sub(segx[s], xbf, N, segC[s], (size_t)(z1 - z0) * H * W, gs, Cg, cg0, st, fmt, S, (size_t)z0 * H * W); });
             a.xq[s] = st; a.xsc[s] = st + (size_t)N * nbp * S * mx_rb(32, fmt);
@@ -727,7 +730,7 @@ extern "C" int mi_conv_fwd_gn(int bits, const void *x, int xbf, shape5 xs, const
 }
 extern "C" int mi_conv_fwd_gn_stage(int bits, const void *x, int xbf, shape5 xs, const float *w, const float *b, int cout, void *y, int ybf, gnp_t gp,
                                     double *osum, int Go, split_t sp, float eps, float *omean, float *orstd, const float *gamma, const float *beta, void *st8, void *st4) {
-    if (cout % 32 || ybf < 3 || !gamma || !beta || (!st8 && !st4) || sp.Di || sp.yD || sp.zlo || sp.zhi || Go <= 0 || cout % Go || xs.n <= 0 || xs.c <= 0 || xs.d <= 0 || xs.h <= 0 || xs.w <= 0) return -1;
+    if (cout % 32 || ybf < 3 || !gamma || !beta || (!st8 && !st4) || sp.Di || sp.yD || sp.zlo || sp.zhi || Go <= 0 || cout % Go || xs.n <= 0 || xs.c <= 0 || xs.d <= 0 || xs.h <= 0 || xs.w <= 0) { take_once(); return -1; }
     g_stage = gn_stage_t{gamma, beta, st8, st4};
     const int rc = mi_conv_fwd_gn(bits, x, xbf, xs, w, b, cout, y, ybf, gp, osum, Go, sp, eps, omean, orstd);
     g_stage.gamma = nullptr;
@@ -793,11 +796,12 @@ int mi_conv_static_setup(const char *who) {
 }
 static int conv_fwd_static(const char *who, int fmt, const void *x, int xbf, shape5 xs, const float *w, const float *b, int cout, void *y, int ybf, gnp_t gp, double *osum, int Go, split_t sp) {
     int dv = 0; MIRT(hipGetDevice(&dv)); dv &= 7;
-    if (!g_scratch_ptr[dv] && mi_conv_static_setup(who)) return -2;
+    if (!g_scratch_ptr[dv] && mi_conv_static_setup(who)) { take_once(); return -2; }
     const size_t need = conv_scratch_bound(fmt, sp.x2, xbf, ybf, xs, cout, gp, osum, sp);
     if (need > MI_STATIC_SCRATCH_BYTES) {
         fprintf(stderr, "%s: this call needs up to %zu bytes of scratch (prepared weights, re-staged operands, statistics partials); the fixed scratch holds %zu. "
                         "Use lp_conv_fwd_f8 / lp_conv_fwd_f4, which allocate, or pass an input that is already in the compute format without GroupNorm\n", who, need, (size_t)MI_STATIC_SCRATCH_BYTES);
+        take_once();
         return -1;
     }
     unsigned char *ptr = g_scratch_ptr[dv];
@@ -809,6 +813,6 @@ static int conv_fwd_static(const char *who, int fmt, const void *x, int xbf, sha
     return rc;
 }
 extern "C" int mi_conv_fwd_static(int bits, const void *x, int xbf, shape5 xs, const float *w, const float *b, int cout, void *y, int ybf, gnp_t gp, double *osum, int Go, split_t sp) {
-    if (bits != 8 && bits != 4) { fprintf(stderr, "mi_conv_fwd_static: compute format %d (8 or 4)\n", bits); return -1; }
+    if (bits != 8 && bits != 4) { fprintf(stderr, "mi_conv_fwd_static: compute format %d (8 or 4)\n", bits); take_once(); return -1; }
     return conv_fwd_static("mi_conv_fwd_static", bits, x, xbf, xs, w, b, cout, y, ybf, gp, osum, Go, sp);
 }
