@@ -51,6 +51,9 @@ void at_fa8_waves(int nw);
    writes the down projection's packed operand, and at_ws.h is left untouched too, and without rays the pack writes the core's quantised operands, with
    at_ws.qkvh left untouched. The block's output has the same bits in all three */
 void at_fuse_pack(int on);
+/* (no counterpart) whether the launch of that last form fits: nseq sequences of S tokens in H heads, every sequence padded to whole tiles of 64. Where it does not, at_block_fwd runs
+   at_fa_pack and at_fa8_fwd */
+int at_fa8_one_pass(int nseq, int S, int H);
 
 /* ---- radial attention and scroll coordinates (src/attn.h:83-128, src/nn_attn_ray.cu) ----
    Each sample's grid (D x Hh x W tokens, no registers) has a scroll axis along grid dim ad (0 D, 1 Hh, 2 W) with a centre (cu, cv) per plane k

@@ -145,3 +145,18 @@ def test_oracle_is_not_reachable_from_the_product():
                 text = open(os.path.join(dirpath, f), errors="ignore").read()
                 assert "liboracle" not in text or f == "build.py", f
                 assert "mx_oracle" not in text and "orc_" not in text, f
+
+
+@pytest.mark.parametrize("S", [1, 5, 63, 64, 65, 129, 4097])
+@pytest.mark.parametrize("H", [1, 4, 7])
+def test_one_pass_pack_takes_what_its_launch_holds(S, H):
+    """The attention block's one-pass pack launches 256 threads per part, head and 64-token tile (sequences padded to whole tiles, tiles to eight); a launch has fewer than 2^32."""
+    from ufsm_amd import lp
+    L = lp.load()
+    tiles = -(-S // 64)
+    def threads(nseq):
+        return -(-nseq * tiles // 8) * 8 * 3 * H * 256
+    edge = 2 ** 32 // (tiles * 3 * H * 256)                       # the limit lies within eight tiles of this many sequences
+    for nseq in [1, 2, max(1, edge // 2)] + list(range(max(1, edge - 9), edge + 10)) + [2 * edge, 2 ** 28 // (S * H) - 1]:
+        assert L.at_fa8_one_pass(nseq, S, H) == (1 if 0 < nseq and threads(nseq) < 2 ** 32 else 0), nseq
+    assert not L.at_fa8_one_pass(0, S, H) and not L.at_fa8_one_pass(5, 0, H)

@@ -405,14 +405,18 @@ extern "C" int at_fa8_fwd(const void *qkvh, float *o, float *lse, const at_geom 
     a8_core(w, o, lse, g, H, C);
     return 0;
 }
+// workgroups of a8_pack_k: the three parts of every 64-token tile (sequences padded to whole tiles) and head, tiles rounded up to eight
+static unsigned long long a8_pack_blocks(int nseq, int S, int H) { return ((unsigned long long)nseq * (((unsigned)S + FT - 1) / FT) + 7) / 8 * 8 * 3 * (unsigned)H; }
+// a launch has fewer than 2^32 threads. Short sequences reach that first, every one of them being a tile (5.6 million sequence x head pairs of up to 64 tokens); the separate passes'
+// launches have a third of the threads at most
+extern "C" int at_fa8_one_pass(int nseq, int S, int H) { return nseq > 0 && S > 0 && H > 0 && a8_pack_blocks(nseq, S, H) < (1ull << 32) / 256; }
 // (internal) at_fa_pack and at_fa8_fwd from the projection's rows qkv [T][3 C], 16-byte aligned, without the binary16 tensor between them: the same operands, the same
-// outputs, rq / rk / amx included (amx: four floats that are zero when this runs). Tokens x heads below 2^28 (the launch grid)
+// outputs, rq / rk / amx included (amx: four floats that are zero when this runs). at_fa8_one_pass(g->nseq, g->S, H) must hold
 int mi_fa8_from_qkv(const float *qkv, const float *qg, const float *kg, float *rq, float *rk, float *amx, float *o, float *lse, const at_geom *g, int nreg, int H, int rope, float base) {
     a8_ops w;
     if (!a8_carve(&w, g, H)) return -1;
     const rope_t rp = {rope, g->S, g->Hh, g->W, nreg, log2f(base), rope ? g->pos : nullptr};
-    const size_t nb = (size_t)(w.R / 64 + 7) / 8 * 8 * 3 * H;
-#define A8P(MODE) a8_pack_k<MODE><<<(unsigned)nb, 256>>>(qkv, qg, kg, w.q8, w.qs, (size_t)(w.k8 - w.q8), (size_t)(w.ks - w.qs), w.vt, w.vts, rq, rk, amx, H, g->S, (unsigned)(w.Sp / 64), w.R, rp)
+#define A8P(MODE) a8_pack_k<MODE><<<(unsigned)a8_pack_blocks(g->nseq, g->S, H), 256>>>(qkv, qg, kg, w.q8, w.qs, (size_t)(w.k8 - w.q8), (size_t)(w.ks - w.qs), w.vt, w.vts, rq, rk, amx, H, g->S, (unsigned)(w.Sp / 64), w.R, rp)
     switch (rope_mode(rp)) { case ROPE_TABLE: A8P(ROPE_TABLE); break; case ROPE_REAL: A8P(ROPE_REAL); break; default: A8P(ROPE_EACH); }
 #undef A8P
     a8_core(w, o, lse, g, H, H * HD);

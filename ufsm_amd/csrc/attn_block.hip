@@ -400,7 +400,7 @@ extern "C" int at_block_fwd(const at_dims *d, const float *P, const at_bp *bp, c
     const bool fuse = g_fuse_pack && g_at_mx == 8 && C % 64 == 0 && F % 64 == 0 && !((uintptr_t)x & 15) && !((uintptr_t)w->x1 & 15) && !((uintptr_t)w->h & 15);
     uint8_t *aq = nullptr, *as = nullptr;
     // ... and the full attention's pack writes the core's quantised operands from the projection's rows; the binary16 tensor (qkvh) is not stored
-    bool direct = fuse && g_fuse_pack > 1 && !R && !((uintptr_t)w->qkv & 15) && g->S > 0 && (long long)T * d->H < 1ll << 28;
+    bool direct = fuse && g_fuse_pack > 1 && !R && !((uintptr_t)w->qkv & 15) && at_fa8_one_pass(g->nseq, g->S, d->H);
     // attention branch
     if (fuse && mi_mx_gemm_abuf(8, (int)T, 3 * C, C, &aq, &as)) {
         ln_pack_fwd(x, P + bp->ln1g, P + bp->ln1b, w->m1, w->r1, T, C, aq, as, direct ? w->amx : nullptr);

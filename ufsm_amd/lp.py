@@ -181,6 +181,7 @@ _ATTN_PROTOS = {
     "at_fa8_fwd": (_I, [_P, _P, _P, C.POINTER(at_geom), _I, _I]),
     "at_fa8_waves": (None, [_I]),
     "at_fuse_pack": (None, [_I]),
+    "at_fa8_one_pass": (_I, [_I, _I, _I]),
     "at_ws_bytes_r": (_Z, [C.POINTER(at_dims), C.c_long, C.c_long]),
     "at_ws_carve_r": (None, [C.POINTER(at_ws), C.POINTER(at_dims), C.c_long, C.c_long, _P]),
     "at_rays_dims": (None, [_I, _I, _I, _F, C.POINTER(C.c_int), C.POINTER(C.c_int), C.POINTER(C.c_int)]),
