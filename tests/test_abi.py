@@ -160,3 +160,14 @@ def test_one_pass_pack_takes_what_its_launch_holds(S, H):
     for nseq in [1, 2, max(1, edge // 2)] + list(range(max(1, edge - 9), edge + 10)) + [2 * edge, 2 ** 28 // (S * H) - 1]:
         assert L.at_fa8_one_pass(nseq, S, H) == (1 if 0 < nseq and threads(nseq) < 2 ** 32 else 0), nseq
     assert not L.at_fa8_one_pass(0, S, H) and not L.at_fa8_one_pass(5, 0, H)
+
+
+@pytest.mark.parametrize("rope", [0, 1])
+def test_pack_of_an_empty_geometry_ends_normally(rope):
+    """at_fa_pack on a geometry of no tokens and no grid: the choice of how angles are formed divides by nothing on the host (no GPU: the launches are errors that lp_check reports)."""
+    import subprocess
+    import sys
+    code = ("from ufsm_amd import lp\nL = lp.load()\n"
+            "L.at_fa_pack(4096, 4096, 4096, 4096, 4096, 4096, 4096, lp.C.byref(lp.at_geom()), 0, 48, %d, 100.0)\nprint('done')" % rope)
+    r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, env=dict(os.environ, HIP_VISIBLE_DEVICES="-1"), capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0 and "done" in r.stdout, (r.returncode, r.stderr)

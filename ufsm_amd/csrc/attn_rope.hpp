@@ -23,6 +23,7 @@ template <int MODE> __device__ __forceinline__ float rope_pos(const rope_t &R, l
 inline int rope_mode(const rope_t &R) {
     if (!R.on) return ROPE_TABLE;                              // (nothing turns: no table is formed either)
     if (R.gpos) return ROPE_REAL;
+    if (R.Hh <= 0 || R.W <= 0) return ROPE_EACH;               // (no grid: an empty call's geometry; nothing here may divide by it)
     const int a = R.S / (R.Hh * R.W), b = R.Hh > R.W ? R.Hh : R.W;
     return (a > b ? a : b) <= ROPE_TAB ? ROPE_TABLE : ROPE_EACH;
 }
