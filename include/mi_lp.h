@@ -209,7 +209,7 @@ int mi_conv_fwd_gn(int bits, const void *x, int xbf, shape5 xs, const float *w, 
                    double *osum, int Go, split_t sp, float eps, float *omean, float *orstd);
 /* ... and what mi_conv_prestage then makes of its output under these statistics: silu(gn(y)) with the given affine as MX-fp8 rows st8 and / or MX-fp4 rows st4 (one of them
    may be null). With few records the pre-pass forms the statistics itself, one launch less; the same bytes in y, omean, orstd, st8 and st4 as the separate
-   calls' (the statistics are the same sums added in another order in double: equal but for a last bit now and then). osum is scratch. cout a multiple of 32, an MX y, no z-range;
+   calls' (the records are added in one order whoever adds them). osum is scratch. cout a multiple of 32, an MX y, no z-range;
    0 on success, -1 for what it does not take (nothing is launched) */
 int mi_conv_fwd_gn_stage(int bits, const void *x, int xbf, shape5 xs, const float *w, const float *b, int cout, void *y, int ybf, gnp_t gp,
                          double *osum, int Go, split_t sp, float eps, float *omean, float *orstd, const float *gamma, const float *beta, void *st8, void *st4);

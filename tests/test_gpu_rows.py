@@ -43,15 +43,50 @@ def test_conv_with_rows_equals_the_separate_calls(gpu, bits, n, ci, co, dims, G)
                                         st8.ptr if f8 else None, st4.ptr if f4 else None) == 0
         LP.check()
         assert np.array_equal(y.to_numpy(np.uint8), y0.to_numpy(np.uint8))
-        # the same sums added in another order in double (relative 2^-52 per addition, far inside half a step of fp32): equal, or the neighbouring float
-        a, c = m.to_numpy(np.float32), m0.to_numpy(np.float32)
-        assert np.allclose(a, c, rtol=2.0 ** -23, atol=1e-12) and np.allclose(r.to_numpy(np.float32), r0.to_numpy(np.float32), rtol=2.0 ** -23, atol=0)
+        assert np.array_equal(m.to_numpy(np.float32), m0.to_numpy(np.float32)) and np.array_equal(r.to_numpy(np.float32), r0.to_numpy(np.float32))      # (added in one order)
         g = gnp_t(gamma.ptr, beta.ptr, m.ptr, r.ptr, G)
         for st, sb, on in ((st8, 8, f8), (st4, 4, f4)):      # the rows are those of the pre-pass under the statistics returned
             if on:
                 want = DevBuf(_bytes(sb, n, co, s))
                 assert lib.mi_conv_prestage(y.ptr, dt, ys, g, want.ptr, sb) == 0
                 assert np.array_equal(st.to_numpy(np.uint8), want.to_numpy(np.uint8))
+
+
+@pytest.mark.parametrize("bits,ci,co,dims", [(8, 64, 64, (64, 64, 64)), (4, 64, 64, (64, 64, 64))])
+def test_statistics_do_not_depend_on_the_batch(gpu, bits, ci, co, dims):
+    """A sample's mean, rstd and rows alone and as the first of two, on both sides of the size where the pre-pass stops adding the records itself (16 MB of records read over the
+    launch: 1 x 64 channels at 64^3 is the last, 2 the first past it). The input's second half in y is the first one's negative except near the halves' edges, large further in, and
+    there is no bias: the large tiles' records cancel exactly, and what is left of the small ones, some ten bits, shows in which order they were added."""
+    rng = np.random.default_rng(co)
+    H, h, s, G = dims[1], dims[1] // 2, int(np.prod(dims)), 8
+    a = 2.0 ** -22 * rng.standard_normal((ci, dims[0], h, dims[2])).astype(np.float32)
+    a[:, :, 10:h - 10] *= 2.0 ** 40                               # (output rows 8 .. h - 9, whole tiles, are the other half's negative, and every large one among them)
+    x1 = np.concatenate([a, -a], 2)
+    small = np.r_[0:6, h - 6:h + 6, H - 6:H]
+    x1[:, :, small] = 2.0 ** -22 * rng.standard_normal((ci, dims[0], len(small), dims[2]))
+    x2 = np.stack([x1, rng.standard_normal(x1.shape).astype(np.float32)]).reshape(2, ci, s)
+    w = DevBuf.from_numpy((rng.standard_normal((co, ci, 27)) * np.sqrt(2.0 / (ci * 27))).astype(np.float32)); b = DevBuf(co * 4)
+    gamma, beta = DevBuf.from_numpy(rng.uniform(0.7, 1.3, co).astype(np.float32)), DevBuf.from_numpy((0.2 * rng.standard_normal(co)).astype(np.float32))
+    dt, got = (3 if bits == 8 else 4), []
+    for n in (1, 2):
+        x = to_mx(bits, x2[:n])
+        for staged in (True, False):
+            y, st, sums, m, r = DevBuf(_bytes(bits, n, co, s)), DevBuf(_bytes(bits, n, co, s)), DevBuf(n * G * 48), DevBuf(n * G * 4), DevBuf(n * G * 4)
+            args = (bits, x.ptr, dt, shape5(n, ci, *dims), w.ptr, b.ptr, co, y.ptr, dt, gnp_t(), sums.ptr, G, split_t(), 1e-5, m.ptr, r.ptr)
+            if staged:
+                assert lib.mi_conv_fwd_gn_stage(*args, gamma.ptr, beta.ptr, st.ptr if bits == 8 else None, st.ptr if bits == 4 else None) == 0
+            else:
+                assert lib.mi_conv_fwd_gn(*args) == 0
+                assert lib.mi_conv_prestage(y.ptr, dt, shape5(n, co, *dims), gnp_t(gamma.ptr, beta.ptr, m.ptr, r.ptr, G), st.ptr, bits) == 0
+            LP.check()
+            nb, rb = co // 32, 32 if bits == 8 else 16
+            rows = st.to_numpy(np.uint8)
+            codes, scales = rows[:n * nb * s * rb].reshape(n, -1), rows[n * nb * s * rb:n * nb * s * (rb + 1)].reshape(n, -1)
+            got.append((m.to_numpy(np.float32)[:G], r.to_numpy(np.float32)[:G], codes[0], scales[0]))
+    assert np.abs(got[0][0]).max() > 0
+    for other in got[1:]:
+        for p, q in zip(got[0], other):
+            assert np.array_equal(p, q)
 
 
 def test_conv_with_rows_refuses(gpu):

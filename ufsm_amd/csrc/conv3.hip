@@ -78,6 +78,21 @@ __global__ void __launch_bounds__(NTH) gn_part_reduce_k(const float2 *part, int 
     for (int k = 0; k < sp.nsplit; k++) { s += r1[k * Go + tid]; ss += r2[k * Go + tid]; }
     gn_part_finish(osum, s, ss, fin, (unsigned)(n * Go + tid));
 }
+// the same for few records (mi_records_few): a block per 32 channels and sample, whose threads add in the order of the pre-pass that forms statistics itself
+// (restage32_k<..., RED>); a group is finished by the block it starts in. Bound by the launch and one chain of loads: 3.9 - 5.2 us where the kernel above takes 3.9 - 5.8 (8 to 512
+// records of 8 to 128 quads, 1 and 2 samples; even at 32 and 64 channels, 4.7 -> 3.1 at 512 from 16^3)
+__global__ void __launch_bounds__(256) gn_part_reduce_few_k(gn_records_t rec, int C, double *osum, gn_fin_t fin) {
+    __shared__ double r1[256], r2[256];
+    const int nb = C / 32, n = (int)blockIdx.x / nb, blk = (int)blockIdx.x - n * nb;
+    const gn_rec_lane_t l = gn_rec_lane(rec, C, n, blk);
+    float2 rv[8];
+    double s, ss;
+    gn_rec_request(rec, l, rv);
+    gn_rec_sums(rec, l, rv, r1, r2, s, ss);
+    const int g = l.g0 + (int)threadIdx.x;
+    if (g <= l.g1 && g * l.cpg >= blk * 32) gn_part_finish(osum, s, ss, fin, (unsigned)(n * rec.Go + g));
+}
+
 // the same with one block per (sample, group), for records wider than a block (more than 1024 channels) or more than 256 groups
 __global__ void __launch_bounds__(256) gn_part_reduce_g_k(const float2 *part, int tiles_per_n, int ncs, int MT, int Co, int Go, double *osum, gn_fin_t fin) {
     const int n = blockIdx.x / Go, gidx = blockIdx.x % Go, qpg = Co / Go / 4, nq = MT * 8, nst = tiles_per_n / ncs;
@@ -270,6 +285,10 @@ static void conv_stats_reduce(const char *who, const conv_args &a, int MT, split
     if (a.stat_ch) { gn_part_reduce_ch_k<<<a.N * a.Go, 256>>>((const float2 *)a.part, (int)(a.ntiles / a.N), a.ncs, a.Co, a.Go, osum, fin); MICK(); return; }
     const int tiles_per_n = (int)(a.ntiles / a.N) * (a.row1 ? 8 : 1);      // (row1: eight records per tile)
     const int Q = a.ncs * MT * 8, nst = tiles_per_n / a.ncs;
+    if (mi_records_few(a.Co, a.Go, nst)) {
+        const gn_records_t rec = {(const float2 *)a.part, nst, Q, a.Go, fin.len, fin.eps, nullptr, nullptr};
+        gn_part_reduce_few_k<<<a.N * (a.Co / 32), 256>>>(rec, a.Co, osum, fin); MICK(); return;
+    }
     if (Q > 256 || a.Go > 256) { gn_part_reduce_g_k<<<a.N * a.Go, 256>>>((const float2 *)a.part, tiles_per_n, a.ncs, MT, a.Co, a.Go, osum, fin); MICK(); return; }
     // thousands of tiles per sample: several blocks each (512 tiles or more per block), folded by the last one done. The pairs and ticket
     // counters live in a small buffer per device, allocated on first use and left zeroed by every launch (the entry point that must not

@@ -850,18 +850,14 @@ __global__ void __launch_bounds__(256) restage32_k(const uint8_t *x, uint8_t *y,
     const size_t row0 = ((size_t)n * nb + blk) * Ss + v0;
     const uint8_t *xs = x + (size_t)N * nb * Ss * (IB * 2);
     uint8_t *ys = y + (size_t)N * nb * Ss * (OB * 2);
-    // RED: the groups the block's channels lie in and their quads of channels; thread (q, j) adds quad q of records j, j + 16, ... The first of them and the affine are requested
-    // before the rows (loads return in order: the chain they start is the longer one)
+    // RED: the first of the thread's records and the affine are requested before the rows (loads return in order: the chain they start is the longer one)
     constexpr int RK = RED ? 8 : 1;
-    const int cpg = RED ? C / rec.Go : 4, g0 = blk * 32 / cpg, g1 = (blk * 32 + 31) / cpg, qpg = cpg >> 2;      // (cpg a multiple of 4; the groups' quads are at most 16: the host's rule)
-    const int rj = threadIdx.x >> 4;
-    const float2 *rp = nullptr;
+    gn_rec_lane_t rl;
     float2 rv[RK];
     float ga = 0.f, be = 0.f;
     if constexpr (RED) {
-        rp = rec.part + (size_t)n * rec.nst * rec.Q + g0 * qpg + min((int)(threadIdx.x & 15), (g1 - g0 + 1) * qpg - 1);
-#pragma unroll
-        for (int k = 0; k < RK; k++) { const int t = rj + 16 * k; rv[k] = rp[(size_t)min(t, rec.nst - 1) * rec.Q]; }
+        rl = gn_rec_lane(rec, C, n, blk);
+        gn_rec_request(rec, rl, rv);
         if (threadIdx.x < 32) { ga = gp.gamma[blk * 32 + threadIdx.x]; be = gp.beta[blk * 32 + threadIdx.x]; }
     }
     unsigned w[RS32_R][4]; unsigned sby[RS32_R];
@@ -875,36 +871,21 @@ __global__ void __launch_bounds__(256) restage32_k(const uint8_t *x, uint8_t *y,
     }
     // (the rows are requested before the block's coefficients are formed: the two chains of dependent loads overlap)
     if constexpr (RED) {
-        double s = 0.0, ss = 0.0;
-#pragma unroll
-        for (int k = 0; k < RK; k++) if (rj + 16 * k < rec.nst) { s += (double)rv[k].x; ss += (double)rv[k].y; }
-#pragma unroll 8
-        for (int t = rj + 16 * RK; t < rec.nst; t += 16) { const float2 v = rp[(size_t)t * rec.Q]; s += (double)v.x; ss += (double)v.y; }
         __shared__ double r1[256], r2[256];
         __shared__ float sm[16], sr[16];
-        r1[threadIdx.x] = s; r2[threadIdx.x] = ss;
-        __syncthreads();
-        if (threadIdx.x < 64) {                               // lane (q, part): a quad's sums over four of the sixteen rows, then over the four lanes of the quad
-            const int qq = threadIdx.x & 15, k0 = threadIdx.x >> 4;
-            s = (r1[(4 * k0) * 16 + qq] + r1[(4 * k0 + 1) * 16 + qq]) + (r1[(4 * k0 + 2) * 16 + qq] + r1[(4 * k0 + 3) * 16 + qq]);
-            ss = (r2[(4 * k0) * 16 + qq] + r2[(4 * k0 + 1) * 16 + qq]) + (r2[(4 * k0 + 2) * 16 + qq] + r2[(4 * k0 + 3) * 16 + qq]);
-            s += __shfl_xor(s, 16); s += __shfl_xor(s, 32); ss += __shfl_xor(ss, 16); ss += __shfl_xor(ss, 32);
-            if (threadIdx.x < 16) { r1[threadIdx.x] = s; r2[threadIdx.x] = ss; }
-        }
-        __syncthreads();
-        if ((int)threadIdx.x <= g1 - g0) {
-            s = 0.0; ss = 0.0;
-            for (int k = 0; k < qpg; k++) { s += r1[threadIdx.x * qpg + k]; ss += r2[threadIdx.x * qpg + k]; }
+        double s, ss;
+        gn_rec_sums(rec, rl, rv, r1, r2, s, ss);
+        if ((int)threadIdx.x <= rl.g1 - rl.g0) {
             unsigned long long w[3];
             float m, r;
             gn_mean_rstd(gn_slot_value(s, w), gn_slot_value(ss, w), rec.len, rec.eps, &m, &r);
             sm[threadIdx.x] = m; sr[threadIdx.x] = r;
-            const int g = g0 + (int)threadIdx.x;
-            if (blockIdx.x == 0 && g * cpg >= blk * 32) { rec.mean[n * rec.Go + g] = m; rec.rstd[n * rec.Go + g] = r; }
+            const int g = rl.g0 + (int)threadIdx.x;
+            if (blockIdx.x == 0 && g * rl.cpg >= blk * 32) { rec.mean[n * rec.Go + g] = m; rec.rstd[n * rec.Go + g] = r; }
         }
         __syncthreads();
         if (threadIdx.x < 32) {
-            const int k = (blk * 32 + (int)threadIdx.x) / cpg - g0;
+            const int k = (blk * 32 + (int)threadIdx.x) / rl.cpg - rl.g0;
             const float a = sr[k] * ga;
             sa[threadIdx.x] = a; sb[threadIdx.x] = fmaf(-sm[k], a, be);
         }
@@ -966,15 +947,11 @@ void mi_restage_sub2(const void *x, int xdt, int N, int C, size_t S, gnp_t gp, v
     MICK();
 }
 bool mi_restage_records(const void *x, int xdt, int N, int C, size_t S, const float *gamma, const float *beta, const gn_records_t &rec, void *y8, void *y4) {
-    const int cpg = C / rec.Go;
-    if (C % 32 || (xdt != 3 && xdt != 4) || cpg % 4 || !N || !S) return false;
-    int nq = 0;                                                    // the most quads a block's groups have
-    for (int b = 0; b < C / 32; b++) { const int k = ((b * 32 + 31) / cpg - b * 32 / cpg + 1) * (cpg / 4); if (k > nq) nq = k; }
-    if (nq > 16) return false;
+    if (!mi_records_few(C, rec.Go, rec.nst) || (xdt != 3 && xdt != 4) || !N || !S) return false;
     const dim3 grid(nblk_(S, 128 * RS32_R), (unsigned)(C / 32), (unsigned)N);
-    // every workgroup reads its groups' records: up to 512 of them per sample (four rounds of its threads' loads) and 16 MB in all the launch they save (4 - 5 us) is longer. 1 x 88 x 104^2,
+    // every workgroup reads its groups' records: up to 512 of them per sample (four rounds of its threads' loads; mi_records_few) and 16 MB in all the launch they save (4 - 5 us) is longer. 1 x 88 x 104^2,
     // 154 records and 466 workgroups 8.0 + 4.6 against 10.0 - 11.4 us; 20 - 80 records 5.3 + 4.5 against 6.0; at 2 x 64^3 256 records for 2 048 workgroups (32 MB) are even
-    if (rec.nst > 512 || (size_t)grid.x * grid.y * grid.z * rec.nst * (nq * 8) > (size_t)16 << 20) return false;
+    if ((size_t)grid.x * grid.y * grid.z * rec.nst * (mi_records_quads(C, rec.Go) * 8) > (size_t)16 << 20) return false;
     gnp_t gp = {}; gp.gamma = gamma; gp.beta = beta;
     const uint8_t *xq = (const uint8_t *)x;
 #define RR(BX, BY, BY2, Y, Y2) restage32_k<BX, BY, BY2, true><<<grid, 256>>>(xq, (uint8_t *)(Y), N, C, S, gp, C, 0, S, 0, (uint8_t *)(Y2), rec)
