@@ -566,6 +566,21 @@ static void l0_const_fill(unet *u) {
         nn_gn_const_fill(k == 1 ? b->m1 : b->m2, k == 1 ? b->r1 : b->r2, run, N, G, 1e-5f);
     }
 }
+/* planes per z-slab of a level's convs in this forward (0: whole) */
+static int level_slab(const unet *u, int level) {
+    const int D = u->ls[level].d;
+    return level >= slab_levels(u) ? 0 : g_infer_slab < D ? g_infer_slab : u->slab_ip && level < u->slab_nl ? D : 0;      /* (in place: a level of fewer planes is one slab) */
+}
+/* the level's convs reduce GroupNorm statistics of their outputs (constant statistics: nothing to reduce; per-slab statistics of level 0: a pass over the stored output) */
+static int level_stats(const unet *u, int level) { return !(level == 0 && (u->l0s_ns || l0_const(u))) && !ge_const(u); }
+/* a block's convs hand silu(gn(.)) of their outputs on as operand rows (mi_nn_conv3d_rows): outside slabs, with statistics of their own, on whole blocks of 32 channels */
+static int rows_block(const unet *u, const block *b, int level) { return !(u->slab_ip && level < u->slab_nl) && !level_slab(u, level) && level_stats(u, level) && b->c1.cout % 32 == 0; }
+/* ... of its output as the coarse rows of the decoder block above, if that block takes them: a decoder block, or the bottom level's where neither residual blocks nor the attention
+   stage lie between */
+static int rows_up(const unet *u, const block *b, int level) {
+    if (level == 0 || !rows_block(u, b, level) || !rows_block(u, &u->dec[level - 1], level - 1)) return 0;
+    return b == &u->dec[level] || (level == u->cfg.nlev - 1 && !u->tbn && !u->cfg.enc_blocks[level]);
+}
 /* conv1 -> a1 (+ its statistics), conv2 reads silu(gn(a1)) while staging -> a2 (+ statistics) (src/unet.c:2567-2636); in z-slabs when asked for
    (slab_run, src/unet.c:2499-2545) */
 /* what a block's convs hand on as operand rows: the coarse segment of the block's input (uprows: the level below holds them in its rows8), and of the block's output silu(gn(a2)) as MX-fp8 rows st8
@@ -575,13 +590,13 @@ static int block_fwd(unet *u, block *b, int level, const void *x, const nn_gn_t 
     const int G = G_of(u, b->c1.cout), D = b->ys.d, ip = u->slab_ip && level < u->slab_nl;
     /* per-slab statistics (level 0 under cfg.l0_norm 4): the convs reduce nothing; a pass over the stored output, seen as n * slabs samples of
        l0_slab planes (one channel block: a slab is a sample of the same layout), fills the [n][slab][G] rows (src/unet.c:996-998) */
-    const int l0s = level == 0 && u->l0s_ns, Gc = l0s || (level == 0 && l0_const(u)) || ge_const(u) ? 0 : G;       /* (constant statistics: nothing to reduce either) */
-    const int s = level >= slab_levels(u) ? 0 : g_infer_slab < D ? g_infer_slab : ip ? D : 0;      /* (in place: a level of fewer planes is one slab) */
+    const int l0s = level == 0 && u->l0s_ns, Gc = level_stats(u, level) ? G : 0;
+    const int s = level_slab(u, level);
     void *tmp = ip ? u->slab_tmp[level] : nullptr, *carry = ip ? u->slab_carry[level] : nullptr;
     int r = 0;
-    /* outside slabs, with statistics of its own, a conv's output leaves its GroupNorm + SiLU to one pass behind the conv (mi_conv_fwd_gn_stage), whose rows the next conv reads as
-       they are; the reader's own pre-pass would make the same rows */
-    const int rows_ok = !s && !ip && Gc > 0, fam4 = u->act_dt == 4 || u->prec == 3;
+    /* a conv's output leaves its GroupNorm + SiLU to one pass behind the conv (mi_conv_fwd_gn_stage), whose rows the next conv reads as they are; the reader's own pre-pass would
+       make the same rows */
+    const int rows_ok = rows_block(u, b, level), fam4 = u->act_dt == 4 || u->prec == 3;
     void *const rows = fam4 ? u->rows4[level] : u->rows8[level];
     int have = 0;                                                  /* rows holds silu(gn(a1)) in conv2's compute format */
     io->done = 0;
@@ -602,7 +617,7 @@ static int block_fwd(unet *u, block *b, int level, const void *x, const nn_gn_t 
             const convp *cp = first ? &b->c1 : &b->c2;
             const float *cb = P(u, cp->b);
             if (first && !xup && b == &u->enc[0] && u->cfg.scale_cond) cb = u->stem_b;
-            if (rows_ok && (st8 || st4 || have)) {
+            if (rows_ok && (st8 || st4 || have || (first && io->uprows))) {
                 const int e = !first ? mi_nn_conv3d_rows(have ? rows : b->a1, have, have ? nullptr : &(nn_gn_t){P(u, b->n1.gamma), P(u, b->n1.beta), b->m1, b->r1, G}, nullptr, nullptr, 0, 0, 0, xs,
                                                          P(u, cp->w), cb, cp->cout, o, Gc, 1e-5f, om, orr, P(u, gn->gamma), P(u, gn->beta), st8, st4)
                             : xup ? mi_nn_conv3d_rows(io->uprows ? u->rows8[level + 1] : xup, 0, io->uprows ? nullptr : gup, x, gin, c_split, 1, io->uprows, xs, P(u, cp->w), cb, cp->cout, o, Gc, 1e-5f, om, orr, P(u, gn->gamma), P(u, gn->beta), st8, st4)
@@ -758,7 +773,7 @@ static int graph_fwd(unet *u, const void *x, float *logits) {
         nn_gn_t gd; const nn_gn_t *gin = nullptr;                  /* down_norm: conv1 reads silu(gn(down conv output)) (src/unet.c:2593) */
         if (i && u->cfg.down_norm) { gd = (nn_gn_t){P(u, u->dn[i - 1].gamma), P(u, u->dn[i - 1].beta), u->dm[i - 1], u->dr[i - 1], G_of(u, u->cfg.widths[i - 1])}; gin = &gd; }
         rows_io io = {0};
-        if (!u->cfg.enc_blocks[i]) { if (i < L - 1) { io.st8 = u->skipst[i]; io.st4 = u->skipst4[i]; } else if (L > 1 && !u->tbn) io.st8 = u->rows8[i]; }
+        if (!u->cfg.enc_blocks[i]) { if (i < L - 1) { io.st8 = u->skipst[i]; io.st4 = u->skipst4[i]; } else if (rows_up(u, &u->enc[i], i)) io.st8 = u->rows8[i]; }
         if (block_fwd(u, &u->enc[i], i, cur, gin, nullptr, nullptr, 0, en1[i], en2[i], &io)) return -1;
         if (i == L - 1) uprows = io.done;
         for (int k = 0; k < u->cfg.enc_blocks[i]; k++) if (rblock_fwd(u, &u->rb[i][k], k ? &u->rb[i][k - 1] : &u->enc[i], u->rbn[i][k])) return -1;      /* (src/unet.c:2963) */
@@ -792,7 +807,7 @@ static int graph_fwd(unet *u, const void *x, float *logits) {
         if (i == L - 2 && u->tbn) { coarse = &u->tb; gc.mean = u->tb.m2; gc.rstd = u->tb.r2; }      /* the stage's output under the level's n2 affine (src/unet.c:508) */
         static const nn_gn_t none = {nullptr, nullptr, nullptr, nullptr, -1};          /* the pre-staged skip: no GroupNorm left to apply */
         const void *sk = u->skipst4[i] ? u->skipst4[i] : u->skipst[i];      /* (the decoder's conv computes in e2m1 under precision 3: its rows) */
-        rows_io io = {.uprows = uprows, .st8 = i ? u->rows8[i] : nullptr};      /* (the coarse rows are e4m3 whatever the decoder's conv computes in) */
+        rows_io io = {.uprows = uprows, .st8 = rows_up(u, &u->dec[i], i) ? u->rows8[i] : nullptr};      /* (the coarse rows are e4m3 whatever the decoder's conv computes in) */
         if (block_fwd(u, &u->dec[i], i, sk ? sk : skip->a2, sk ? &none : &gs, coarse->a2, &gc, coarse->ys.c, dn1[i], dn2[i], &io)) return -1;
         uprows = io.done;
     }
