@@ -150,3 +150,64 @@ def test_rows_are_handed_on_where_they_can_be(graph, name):
     skips = (2 if "mx4" in name or "precision" in name else 1) * (blocks - 1) - ("mx4" in name)      # (MX-fp4: level 0 of 32 channels has one form for both readers)
     assert len(rows) == (2 * blocks - 1 - singles) + skips + (blocks - 1)
     assert not [e for e in log if e[0] == "pass"]
+
+
+@pytest.mark.parametrize("name", CONFIGS)
+def test_every_buffer_of_a_forward_is_used(graph, name):
+    """The graph holds no tensor that its forwards neither read nor write, and no buffer of operand rows larger than the rows it is given. (Of the buffers that are allocated:
+    the statistics and the sum slots are reached through pointers that the stand-ins do not follow, so only those of tensor size count.)"""
+    log, _ = run(graph, forwards=2, **CONFIGS[name])
+    dims, n = CONFIGS[name].get("dims", (32, 32, 32)), CONFIGS[name].get("n", 1)
+    small = 1 << 13                                                # (statistics of the widest level and two samples: 8 KB; the smallest tensor, 128 channels at 8^3 in e2m1: 34 KB)
+    held = {e[1]: e[2] for e in log if e[0] == "alloc" and e[2] > small}
+    freed = {e[1] for e in log if e[0] == "free"}
+    used = {e[1] for e in log if e[0] in ("read", "write", "rows")}
+    unused = {p: b for p, b in held.items() if p not in used and p not in freed}
+    # the net's own input tensor (MX, one block of 8 channels) takes another forward entry's rows
+    s = dims[0] * dims[1] * dims[2]
+    own_input = {n * s * 9, n * s * 5}
+    assert all(b in own_input for b in unused.values()) and len(unused) <= 1, unused
+    written = {}
+    for e in log:
+        if e[0] == "rows":
+            written[e[1]] = max(written.get(e[1], 0), e[2])
+    assert all(b <= held[p] for p, b in written.items())          # they fit
+    assert not [(held[p], b) for p, b in written.items() if held[p] > b]      # (a skip's buffer is filled by the skip itself, the blocks' own one by their widest rows)
+    assert len(freed) == 0                                         # (two forwards of one kind: nothing is given back or grown)
+
+
+@pytest.mark.parametrize("mx4,prec", [(0, 0), (0, 3), (1, 0)])
+def test_slabs_switched_between_forwards(graph, mx4, prec):
+    """A net built in the direct slab form and then run whole makes its rows in buffers that hold them, and goes back to slabs: no rebuild, no rows that nothing reads."""
+    c = unet_cfg()
+    c.nlev, c.cin, c.cout, c.G = 3, 4, 8, 8
+    c.widths[0], c.widths[1], c.widths[2] = 16, 48, 64
+    c.dec_widths[1] = 32
+    graph.unet_set_act_mx4(mx4); graph.nn_set_prec(prec)
+    graph.stub_clear()
+    u = graph.unet_create(C.byref(c))
+    xin = C.create_string_buffer(64)
+    counts = []
+    try:
+        for slab in (8, 0, 8, 0):
+            graph.unet_set_infer_slab(slab)
+            before = len(graph.stub_log())
+            assert graph.mi_unet_forward_mx(u, C.addressof(xin), shape5(1, 4, 32, 32, 32))
+            counts.append(graph.stub_log()[before:].count(b"rows"))
+        log = [(l.split()[0],) + tuple(int(v) for v in l.split()[1:]) for l in graph.stub_log().decode().splitlines()]
+    finally:
+        graph.unet_free(u)
+        graph.unet_set_act_mx4(0); graph.nn_set_prec(0); graph.unet_set_infer_slab(0)
+    assert counts[1] == counts[3] > counts[0] == counts[2]
+    held, open_rows = {}, set()
+    for e in log:
+        if e[0] == "alloc":
+            held[e[1]] = e[2]
+        elif e[0] == "free":
+            del held[e[1]]
+        elif e[0] == "rows":
+            assert e[1] not in open_rows and e[2] <= held[e[1]]
+            open_rows.add(e[1])
+        elif e[0] == "read":
+            open_rows.discard(e[1])
+    assert not open_rows

@@ -45,8 +45,9 @@ struct unet {
     convp ds[UNET_MAXLEV], eh;         /* cfg.ds_levels / cfg.emb_lev: the deep-supervision heads of decoder levels 1 .. ds_levels and the distillation head: training-time outputs, here only their place in the parameter vector (src/unet.c:467, :511) */
     void *downo[UNET_MAXLEV];
     /* per level, silu(gn(.)) of the conv output just written, as the operand rows (MX-fp8 or MX-fp4) of its one reader, the next conv of the graph: the level's pre-staged skip's
-       buffer of that format, whose rows are written after conv2 has read conv1's and are dead once the decoder's conv1 has read them, or (levels without one) rows_own, one buffer for all */
-    void *rows8[UNET_MAXLEV], *rows4[UNET_MAXLEV], *rows_own;
+       buffer of that format, whose rows are written after conv2 has read conv1's and are dead once the decoder's conv1 has read them, or (levels without one) rows_own, one buffer for
+       all, held only where a block of such a level makes rows (rows_buffers) */
+    void *rows8[UNET_MAXLEV], *rows4[UNET_MAXLEV], *rows_own; size_t rows_cap;
     void *skipst[UNET_MAXLEV];         /* silu(gn(enc[i].a2)) in the compute format, formed once for its two readers (down conv, decoder conv1); null: each reader transforms it */
     void *skipst4[UNET_MAXLEV];        /* precision 3 over MX-fp8 storage, and MX-fp4 storage: the two readers compute in different formats (the stride-2 conv in e4m3, the decoder's
                                           in e2m1); the same pass writes the MX-fp4 rows here beside the MX-fp8 ones in skipst. MX-fp4 storage where the stride-2 conv computes
@@ -265,7 +266,7 @@ static void free_acts(unet *u) {
     for (int i = 0; i < 2; i++) { act_del(u->slab_tmp[i]); act_del(u->slab_carry[i]); u->slab_tmp[i] = u->slab_carry[i] = nullptr; }
     act_del(u->xin); u->xin = nullptr;
     if (u->rows_own) mi_free(u->rows_own);
-    u->rows_own = nullptr; memset(u->rows8, 0, sizeof u->rows8); memset(u->rows4, 0, sizeof u->rows4);
+    u->rows_own = nullptr; u->rows_cap = 0; memset(u->rows8, 0, sizeof u->rows8); memset(u->rows4, 0, sizeof u->rows4);
     mi_free(u->logits); u->logits = nullptr;
     u->built = 0; u->nouts = 0; u->slab_ip = u->slab_nl = u->slab_s = 0; u->l0s_zs = u->l0s_ns = 0;
 }
@@ -325,13 +326,6 @@ static int build_acts(unet *u, shape5 in) {
         u->slab_tmp[i] = act_new(u, t); t.d = 1; u->slab_carry[i] = act_new(u, t);
     }
     u->xin = act_new(u, in);
-    size_t rows = 0;
-    for (int i = 0; i < L; i++) {                                  /* (a decoder block is at most as wide as its level) */
-        const size_t r = !u->skipst[i] && (i || u->act_dt == 8) ? nn_mx8_bytes(u->ls[i]) : !u->skipst4[i] && (u->act_dt == 4 || u->prec == 3) ? nn_mx4_bytes(u->ls[i]) : 0;      /* (level 0 hands no coarse rows on) */
-        if (r > rows) rows = r;
-    }
-    if (rows) u->rows_own = mi_malloc(rows);
-    for (int i = 0; i < L; i++) { u->rows8[i] = u->skipst[i] ? u->skipst[i] : u->rows_own; u->rows4[i] = u->skipst4[i] ? u->skipst4[i] : u->rows_own; }
     u->logits = f32_new((size_t)in.n * cfg->cout * in.d * in.h * in.w);
     if (u->tbn) {
         const shape5 ys = u->ls[L - 1]; const long Sg = (long)ys.d * ys.h * ys.w, S = Sg + u->tbd.nreg, T = (long)ys.n * S; const int C = u->tbd.C;
@@ -581,6 +575,25 @@ static int rows_up(const unet *u, const block *b, int level) {
     if (level == 0 || !rows_block(u, b, level) || !rows_block(u, &u->dec[level - 1], level - 1)) return 0;
     return b == &u->dec[level] || (level == u->cfg.nlev - 1 && !u->tbn && !u->cfg.enc_blocks[level]);
 }
+/* the buffers of a forward's rows: rows_own grown to the largest tensor of the blocks that make rows now (slabs and constant statistics can be switched between forwards) and have no
+   skip buffer of the format to put them in */
+static void rows_buffers(unet *u) {
+    const int L = u->cfg.nlev, fam4 = u->act_dt == 4 || u->prec == 3;
+    size_t need = 0;
+    for (int i = 0; i < L; i++) for (int s = 0; s < (i < L - 1 ? 2 : 1); s++) {
+        const block *b = s ? &u->dec[i] : &u->enc[i];              /* (a decoder block is at most as wide as its level, whose skip buffers hold its rows) */
+        if (!rows_block(u, b, i)) continue;
+        const size_t inner = b->single || (fam4 ? u->skipst4[i] : u->skipst[i]) ? 0 : fam4 ? nn_mx4_bytes(b->ys) : nn_mx8_bytes(b->ys);      /* conv1's, in conv2's compute format */
+        const size_t up = rows_up(u, b, i) && !u->skipst[i] ? nn_mx8_bytes(b->ys) : 0;                                                       /* (coarse rows are e4m3 whatever the convs compute in) */
+        if (inner > need) need = inner;
+        if (up > need) need = up;
+    }
+    if (need > u->rows_cap) {
+        if (u->rows_own) { mi_sync(); mi_free(u->rows_own); }
+        u->rows_own = mi_malloc(need); u->rows_cap = need;
+    }
+    for (int i = 0; i < L; i++) { u->rows8[i] = u->skipst[i] ? u->skipst[i] : u->rows_own; u->rows4[i] = u->skipst4[i] ? u->skipst4[i] : u->rows_own; }
+}
 /* conv1 -> a1 (+ its statistics), conv2 reads silu(gn(a1)) while staging -> a2 (+ statistics) (src/unet.c:2567-2636); in z-slabs when asked for
    (slab_run, src/unet.c:2499-2545) */
 /* what a block's convs hand on as operand rows: the coarse segment of the block's input (uprows: the level below holds them in its rows8), and of the block's output silu(gn(a2)) as MX-fp8 rows st8
@@ -759,6 +772,7 @@ static int graph_fwd(unet *u, const void *x, float *logits) {
     static const char *dwn[] = {"down0", "down1", "down2", "down3", "down4", "down5", "down6"};
     const int L = u->cfg.nlev;
     u->nouts = 0;
+    rows_buffers(u);
     if (l0_const(u)) l0_const_fill(u);
     if (ge_const(u)) ge_const_fill(u);
     if (u->cfg.scale_cond) {                                       /* the stem bias of this forward: b + c v (src/unet.c:2880-2885) */
