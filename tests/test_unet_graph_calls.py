@@ -70,7 +70,10 @@ int lp_gn_sums_mx(const void *x, int xdt, int n, int c, int G, size_t S, double 
 
 @pytest.fixture(scope="module")
 def graph(tmp_path_factory):
-    d = tmp_path_factory.mktemp("graph")
+    return link(tmp_path_factory.mktemp("graph"))
+
+
+def link(d):
     host = [os.path.join(ROOT, "ufsm_amd", "host", f) for f in ("nn_host.c", "unet.c", "predict.c")]
     (d / "stub.c").write_text("#include <stdarg.h>\n" + STUB)
     def cc(out, src, *more):
@@ -139,6 +142,23 @@ def test_no_rows_are_made_that_nothing_reads(graph, name):
         elif e[0] == "read":
             open_rows.pop(e[1], None)
     assert not open_rows
+
+
+@pytest.mark.parametrize("name", CONFIGS)
+def test_a_skip_has_one_pass_of_its_own_at_most(graph, name):
+    """A skip that no conv's pass has transformed gets one pass for both readers or, under MX-fp4 storage, none and no buffers: each reader transforms it."""
+    log, _ = run(graph, **CONFIGS[name])
+    passes = [e[1] for e in log if e[0] == "pass"]
+    assert len(passes) == len(set(passes)) and not (passes and "mx4" in name)
+
+
+@pytest.mark.parametrize("name,skips", [("mx4", 0), ("precision 3", 0), ("plain", 2)])
+def test_skip_knob(tmp_path, monkeypatch, name, skips):
+    """MI_UNET_SKIP2=0: where a skip's readers compute in different formats each transforms it itself; nothing is held or made for both (MX-fp8 alone shares its skips as ever)."""
+    monkeypatch.setenv("MI_UNET_SKIP2", "0")
+    L = link(tmp_path)
+    log, _ = run(L, **CONFIGS[name])
+    assert len([e for e in log if e[0] == "rows"]) == (2 * 3 - 1) + 2 + skips and not [e for e in log if e[0] == "pass"]      # (five blocks' conv1, two coarse segments, the skips)
 
 
 @pytest.mark.parametrize("name", ["plain", "mx4", "precision 3", "dec_convs 1 at level 0", "dec_convs 1", "two levels"])

@@ -51,7 +51,7 @@ struct unet {
     void *skipst[UNET_MAXLEV];         /* silu(gn(enc[i].a2)) in the compute format, formed once for its two readers (down conv, decoder conv1); null: each reader transforms it */
     void *skipst4[UNET_MAXLEV];        /* precision 3 over MX-fp8 storage, and MX-fp4 storage: the two readers compute in different formats (the stride-2 conv in e4m3, the decoder's
                                           in e2m1); the same pass writes the MX-fp4 rows here beside the MX-fp8 ones in skipst. MX-fp4 storage where the stride-2 conv computes
-                                          in e2m1 as well (32 channels): only these */
+                                          in e2m1 as well (32 channels): only these. Under MX-fp4 storage both are held and read only where the pass behind conv2 writes them */
     gnpar dn[UNET_MAXLEV]; float *dm[UNET_MAXLEV], *dr[UNET_MAXLEV];   /* down_norm: GroupNorm after down[i], its statistics */
     size_t np; float *p, *ema, *params;                            /* device: live weights, EMA copy, the one the forward reads */
     float *src, *wm; int wm_ok;                                    /* cfg.w4_2d: the selected weights (p or ema), their forward copy with the fp4 convs' weights rounded per 32 x 32 block, whether it is current */
@@ -84,7 +84,8 @@ static size_t add_conv(convp *c, int cin, int cout, int k, size_t off) { c->cin 
 static int dw_of(const unet_cfg *c, int i) { return i >= c->nlev - 1 || !c->dec_widths[i] ? c->widths[i] : c->dec_widths[i]; }
 static size_t add_gn(gnpar *g, int c, size_t off) { g->c = c; g->gamma = off; g->beta = off + c; return off + 2 * (size_t)c; }
 static size_t act_bytes(const unet *u, shape5 s) { return u->act_dt == 4 ? nn_mx4_bytes(s) : nn_mx8_bytes(s); }
-static void *act_new(const unet *u, shape5 s) { const size_t b = act_bytes(u, s); void *p = mi_malloc(b); mi_zero(p, b); nn_set_storage(p, b, u->act_dt); return p; }
+static void *mx_new(shape5 s, int dt) { const size_t b = dt == 4 ? nn_mx4_bytes(s) : nn_mx8_bytes(s); void *p = mi_malloc(b); mi_zero(p, b); nn_set_storage(p, b, dt); return p; }
+static void *act_new(const unet *u, shape5 s) { return mx_new(s, u->act_dt); }
 static void act_del(void *p) { if (p) { nn_storage_forget(p); mi_free(p); } }
 static float *f32_new(size_t n) { float *p = mi_malloc(n * 4); mi_zero(p, n * 4); return p; }
 
@@ -242,6 +243,9 @@ static int slab_levels(const unet *u) {      /* how many of the finest levels ru
 }
 static int slab_inplace_now(const unet *u) { return g_infer_slab && !g_slab_direct && u->cfg.nlev > 1; }
 
+/* tuning knob MI_UNET_SKIP2=0: where a skip's two readers compute in different formats (precision 3, MX-fp4 storage) each transforms it itself */
+static int skip2(void) { static int v = -1; if (v < 0) v = getenv("MI_UNET_SKIP2") ? atoi(getenv("MI_UNET_SKIP2")) : 1; return v; }
+
 /* the activation buffers of the current build */
 static void free_acts(unet *u) {
     if (!u->built) return;
@@ -310,13 +314,11 @@ static int build_acts(unet *u, shape5 in) {
         }
         if (i < L - 1) {
             shape5 ds = u->ls[i + 1]; ds.c = w[i]; u->downo[i] = act_new(u, ds);
-            /* both readers of the skip compute in e4m3 from MX-fp8 storage: one shared pre-stage (any other combination: the readers' formats differ) */
-            static int skip2 = -1;                                 /* tuning knob MI_UNET_SKIP2=0: under precision 3 each reader transforms the skip itself */
-            if (skip2 < 0) skip2 = getenv("MI_UNET_SKIP2") ? atoi(getenv("MI_UNET_SKIP2")) : 1;
-            if ((u->act_dt == 4 || u->prec != 3 || skip2) && w[i] % 32 == 0 && i >= u->slab_nl) {
-                if (u->act_dt == 8) u->skipst[i] = act_new(u, u->enc[i].ys);
-                else if (w[i] > 32) { const size_t b8 = nn_mx8_bytes(u->enc[i].ys); u->skipst[i] = mi_malloc(b8); mi_zero(u->skipst[i], b8); nn_set_storage(u->skipst[i], b8, 8); }
-                if (u->act_dt == 4 || u->prec == 3) { const size_t b4 = nn_mx4_bytes(u->enc[i].ys); u->skipst4[i] = mi_malloc(b4); mi_zero(u->skipst4[i], b4); nn_set_storage(u->skipst4[i], b4, 4); }
+            /* MX-fp8 storage: the skip is transformed once for its two readers, into e4m3 rows and under precision 3, where the decoder's conv computes in e2m1, both forms (MX-fp4
+               storage: rows_buffers) */
+            if (u->act_dt == 8 && (u->prec != 3 || skip2()) && w[i] % 32 == 0 && i >= u->slab_nl) {
+                u->skipst[i] = act_new(u, u->enc[i].ys);
+                if (u->prec == 3) u->skipst4[i] = mx_new(u->enc[i].ys, 4);
             }
             if (cfg->down_norm) { const size_t ng = (size_t)in.n * G_of(u, w[i]); u->dm[i] = f32_new(ng); u->dr[i] = f32_new(ng); }
         }
@@ -575,10 +577,16 @@ static int rows_up(const unet *u, const block *b, int level) {
     if (level == 0 || !rows_block(u, b, level) || !rows_block(u, &u->dec[level - 1], level - 1)) return 0;
     return b == &u->dec[level] || (level == u->cfg.nlev - 1 && !u->tbn && !u->cfg.enc_blocks[level]);
 }
-/* the buffers of a forward's rows: rows_own grown to the largest tensor of the blocks that make rows now (slabs and constant statistics can be switched between forwards) and have no
+/* the buffers of a forward's rows: MX-fp4 storage's skips, and rows_own grown to the largest tensor of the blocks that make rows now (slabs and constant statistics can be switched between forwards) and have no
    skip buffer of the format to put them in */
 static void rows_buffers(unet *u) {
     const int L = u->cfg.nlev, fam4 = u->act_dt == 4 || u->prec == 3;
+    /* MX-fp4 storage: the skips that the pass behind conv2 writes; where there is none (slabs, constant statistics, residual blocks) each reader transforms the skip itself
+       and no buffers are held */
+    for (int i = 0; u->act_dt == 4 && skip2() && i < L - 1; i++) if (!u->skipst4[i] && !u->cfg.enc_blocks[i] && rows_block(u, &u->enc[i], i)) {
+        u->skipst4[i] = mx_new(u->enc[i].ys, 4);
+        if (u->cfg.widths[i] > 32) u->skipst[i] = mx_new(u->enc[i].ys, 8);
+    }
     size_t need = 0;
     for (int i = 0; i < L; i++) for (int s = 0; s < (i < L - 1 ? 2 : 1); s++) {
         const block *b = s ? &u->dec[i] : &u->enc[i];              /* (a decoder block is at most as wide as its level, whose skip buffers hold its rows) */
@@ -781,7 +789,7 @@ static int graph_fwd(unet *u, const void *x, float *logits) {
         mi_d2d(u->stem_b, P(u, u->enc[0].c1.b), (size_t)c0 * 4);
         nn_axpy(u->stem_b, u->sc_c, P(u, u->sc_w), (size_t)c0);
     }
-    const void *cur = x;
+    const void *cur = x, *sk[UNET_MAXLEV] = {0};                    /* sk: the level's skip as its decoder block's conv reads it, transformed */
     int uprows = 0;                                                /* the level below holds the coarse segment of the next decoder block as its pre-pass would make it, in its rows */
     for (int i = 0; i < L; i++) {
         nn_gn_t gd; const nn_gn_t *gin = nullptr;                  /* down_norm: conv1 reads silu(gn(down conv output)) (src/unet.c:2593) */
@@ -794,13 +802,12 @@ static int graph_fwd(unet *u, const void *x, float *logits) {
         if (i < L - 1) {                                           /* stride-2 down conv of silu(gn(a2)), width kept (src/unet.c:2970) */
             const block *so = stage_out(u, i);
             const nn_gn_t g = gn_out(u, so);
-            const int pre = u->skipst[i] || u->skipst4[i];
+            const int pre = u->act_dt == 4 ? io.done : u->skipst[i] != nullptr;
             if (pre && !io.done) {
                 const gnp_t gp = gnp_mk(g.gamma, g.beta, g.mean, g.rstd, g.G);
-                const int dt = u->act_dt == 4 ? 4 : 3;
-                if (dt == 3 && u->skipst4[i]) { if (mi_conv_prestage2(so->a2, so->ys, gp, u->skipst[i], u->skipst4[i])) return -1; }
-                else if ((u->skipst[i] && mi_conv_prestage(so->a2, dt, so->ys, gp, u->skipst[i], 8)) || (u->skipst4[i] && mi_conv_prestage(so->a2, dt, so->ys, gp, u->skipst4[i], 4))) return -1;
+                if (u->skipst4[i] ? mi_conv_prestage2(so->a2, so->ys, gp, u->skipst[i], u->skipst4[i]) : mi_conv_prestage(so->a2, 3, so->ys, gp, u->skipst[i], 8)) return -1;
             }
+            if (pre) sk[i] = u->skipst4[i] ? u->skipst4[i] : u->skipst[i];      /* (the decoder's conv computes in e2m1 where there are MX-fp4 rows) */
             if (pre && u->act_dt == 4) {                           /* the rows in the format the stride-2 entry computes in for MX-fp4 storage (lp_conv_fwd_s2_f8: e2m1 for 32 channels, else e4m3) */
                 shape5 ds = u->ls[i + 1]; ds.c = u->cfg.widths[i];
                 mi_conv_s2_wkey((unsigned)((uintptr_t)P(u, u->down[i].w) >> 4) | 1u);
@@ -820,9 +827,8 @@ static int graph_fwd(unet *u, const void *x, float *logits) {
         nn_gn_t gc = gn_out(u, coarse); const nn_gn_t gs = gn_out(u, skip);
         if (i == L - 2 && u->tbn) { coarse = &u->tb; gc.mean = u->tb.m2; gc.rstd = u->tb.r2; }      /* the stage's output under the level's n2 affine (src/unet.c:508) */
         static const nn_gn_t none = {nullptr, nullptr, nullptr, nullptr, -1};          /* the pre-staged skip: no GroupNorm left to apply */
-        const void *sk = u->skipst4[i] ? u->skipst4[i] : u->skipst[i];      /* (the decoder's conv computes in e2m1 under precision 3: its rows) */
         rows_io io = {.uprows = uprows, .st8 = rows_up(u, &u->dec[i], i) ? u->rows8[i] : nullptr};      /* (the coarse rows are e4m3 whatever the decoder's conv computes in) */
-        if (block_fwd(u, &u->dec[i], i, sk ? sk : skip->a2, sk ? &none : &gs, coarse->a2, &gc, coarse->ys.c, dn1[i], dn2[i], &io)) return -1;
+        if (block_fwd(u, &u->dec[i], i, sk[i] ? sk[i] : skip->a2, sk[i] ? &none : &gs, coarse->a2, &gc, coarse->ys.c, dn1[i], dn2[i], &io)) return -1;
         uprows = io.done;
     }
     const block *last = L > 1 ? &u->dec[0] : &u->enc[0];
