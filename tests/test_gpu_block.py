@@ -111,6 +111,48 @@ def test_block_with_packed_operands_from_the_producers_has_the_same_bits(gpu):
     assert np.array_equal(ys[0], ys[1]) and np.array_equal(ys[0], ys[2])
 
 
+# rope off; the grid's indices from the table (an axis of 64 is the last) and one by one (70, 65; 64 with registers, which count as an upper bound); real coordinates; sequences of
+# 64 k, 64 k + 1 and fewer than 64 tokens; the one- and four-wavefront cores
+@pytest.mark.parametrize("rope,nseq,nreg,dims", [(0, 2, 0, (4, 4, 4)), (0, 3, 1, (4, 4, 4)), (1, 1, 0, (4, 4, 8)), (1, 9, 2, (1, 1, 3)), (1, 1, 0, (1, 1, 64)), (1, 2, 3, (1, 2, 70)),
+                                                 (1, 1, 0, (65, 1, 1)), (1, 1, 4, (64, 1, 1)), (2, 2, 3, (3, 5, 7)), (2, 1, 0, (4, 4, 4)), (1, 2, 4, (8, 8, 8))])
+def test_one_pass_pack_equals_the_separate_passes(gpu, rope, nseq, nreg, dims):
+    """at_fuse_pack 2 forms the core's operands from the projection's rows in one pass; 0 and 1 go through the binary16 tensor. The output, the rows' scales rq / rk, the maximum of
+    V in amx and the core's lse are the same bits, whatever the scratch held."""
+    rng = np.random.default_rng(7 * nseq + dims[0])
+    Cc, H, F = 192, 4, 512
+    S = nreg + int(np.prod(dims)); T = nseq * S
+    P, lay = make_block(rng, Cc, F)
+    for k in ("qg", "kg"):
+        P[lay[k]:lay[k] + Cc] = 1 + 0.2 * rng.standard_normal(Cc)
+    x = (rng.standard_normal((T, Cc)) * np.exp(rng.uniform(-2, 2, (T, 1)))).astype(np.float32)
+    pos = DevBuf.from_numpy(rng.uniform(-40, 40, (T, 3)).astype(np.float32))
+    d = at_dims(); d.C, d.H, d.F, d.rope, d.nreg, d.rope_base = Cc, H, F, rope, nreg, 100.0
+    bp = at_bp(); lib.at_block_layout(C.byref(d), C.byref(bp), 0)
+    g = at_geom(); g.nseq, g.S, g.D, g.Hh, g.W = (nseq, S) + dims
+    if rope == 2:
+        g.pos = pos.ptr
+    dP, dx = DevBuf.from_numpy(P), DevBuf.from_numpy(x)
+    nb = lib.at_ws_bytes(C.byref(d), T)
+    out = []
+    try:
+        for mode in (0, 1, 2):
+            lib.at_fuse_pack(mode)
+            wsb = DevBuf.from_numpy(np.full(nb // 4, 9.0, np.float32))
+            ws = at_ws(); lib.at_ws_carve(C.byref(ws), C.byref(d), T, wsb.ptr)
+            dy = DevBuf(x.nbytes)
+            assert lib.at_block_fwd(C.byref(d), dP.ptr, C.byref(bp), dx.ptr, dy.ptr, C.byref(g), C.byref(ws)) == 0
+            LP.check()
+            whole = wsb.to_numpy(np.float32)
+            part = lambda p, n: whole[(p - wsb.ptr) // 4:(p - wsb.ptr) // 4 + n].copy()
+            out.append([dy.to_numpy(np.float32), part(ws.rq, T * H), part(ws.rk, T * H), part(ws.amx, 4), part(ws.lse, T * H)])
+    finally:
+        lib.at_fuse_pack(2)
+    assert np.isfinite(out[0][0]).all() and out[0][3][1] > 0 and (out[0][1] != 9.0).all()
+    for mode in (1, 2):
+        for a, b, what in zip(out[0], out[mode], ("y", "rq", "rk", "amx", "lse")):
+            assert np.array_equal(a, b), (mode, what)
+
+
 @pytest.mark.parametrize("nseq,dims,nreg,Cc", [(2, (3, 4, 5), 2, 96), (1, (8, 8, 8), 0, 192), (3, (1, 1, 7), 4, 48), (1, (2, 2, 2), 1, 4)])
 def test_peg_matches_oracle_bit_for_bit(gpu, nseq, dims, nreg, Cc):
     """at_peg_fwd (src/attn.h:141-144): x + b + depthwise 3^3 conv on the grid tokens, the taps in (dz, dy, dx) order as fused multiply-adds:

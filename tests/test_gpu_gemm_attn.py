@@ -81,6 +81,23 @@ def test_gemm_tiles_exact(gpu, bits, M, N, K):
     assert np.array_equal(dC.to_numpy(np.float32, (M, N)), exact)
 
 
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("N,K,many", [(192, 192, 22000), (576, 320, 7300), (1030, 64, 65500)])
+def test_gemm_tiles_round_alike(gpu, bits, N, K, many):
+    """A row of the output does not depend on how many rows the product has: the same A rows alone (tiles of 32 rows) and at the head of a product that takes the tiles of 64 rows,
+    one or four wavefronts to a workgroup, give the same bits, with a bias, a residual and the old C."""
+    rng = np.random.default_rng(K)
+    A = (rng.standard_normal((many, K)) * np.exp(rng.uniform(-3, 3, (many, 1)))).astype(np.float32); B = rng.standard_normal((N, K)).astype(np.float32)
+    bias = rng.standard_normal(N).astype(np.float32); res = rng.standard_normal((many, N)).astype(np.float32); C0 = rng.standard_normal((many, N)).astype(np.float32)
+    few, out = 77, []
+    for M in (few, many):
+        dA, dB, dC, db, dr = (DevBuf.from_numpy(v) for v in (A[:M], B, C0[:M], bias, res[:M]))
+        assert lib.lp_mx_gemm_ex(bits, 0, 1, M, N, K, dA.ptr, dB.ptr, dC.ptr, 0.3, db.ptr, dr.ptr) == 0
+        LP.check()
+        out.append(dC.to_numpy(np.float32, (M, N)))
+    assert np.array_equal(out[0], out[1][:few]) and np.isfinite(out[1]).all()
+
+
 @pytest.mark.parametrize("bits,beta", [(4, 0.0), (8, 0.0), (8, 1.0)])
 def test_gemm_split_k(gpu, bits, beta):
     """The weight-gradient shape: few output tiles, K = tokens (tests/test_attn.c:447): K is split over workgroups that add atomically."""
