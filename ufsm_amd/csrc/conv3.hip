@@ -79,18 +79,31 @@ __global__ void __launch_bounds__(NTH) gn_part_reduce_k(const float2 *part, int 
     gn_part_finish(osum, s, ss, fin, (unsigned)(n * Go + tid));
 }
 // the same for few records (mi_records_few): a block per 32 channels and sample, whose threads add in the order of the pre-pass that forms statistics itself
-// (restage32_k<..., RED>); a group is finished by the block it starts in. Bound by the launch and one chain of loads: 3.9 - 5.2 us where the kernel above takes 3.9 - 5.8 (8 to 512
-// records of 8 to 128 quads, 1 and 2 samples; even at 32 and 64 channels, 4.7 -> 3.1 at 512 from 16^3)
+// (restage32_k<..., RED>, mx_elem.hip: a change here is one there); a group is finished by the block it starts in. Bound by the launch and one chain of loads: 3.9 - 5.2 us where
+// the kernel above takes 3.9 - 5.8 (8 to 512 records of 8 to 128 quads, 1 and 2 samples; even at 32 and 64 channels, 4.7 -> 3.1 at 512 from 16^3)
 __global__ void __launch_bounds__(256) gn_part_reduce_few_k(gn_records_t rec, int C, double *osum, gn_fin_t fin) {
     __shared__ double r1[256], r2[256];
     const int nb = C / 32, n = (int)blockIdx.x / nb, blk = (int)blockIdx.x - n * nb;
-    const gn_rec_lane_t l = gn_rec_lane(rec, C, n, blk);
-    float2 rv[8];
-    double s, ss;
-    gn_rec_request(rec, l, rv);
-    gn_rec_sums(rec, l, rv, r1, r2, s, ss);
-    const int g = l.g0 + (int)threadIdx.x;
-    if (g <= l.g1 && g * l.cpg >= blk * 32) gn_part_finish(osum, s, ss, fin, (unsigned)(n * rec.Go + g));
+    const int cpg = C / rec.Go, g0 = blk * 32 / cpg, g1 = (blk * 32 + 31) / cpg, qpg = cpg >> 2;      // (the groups the block's channels lie in and their quads: at most 16)
+    const float2 *rp = rec.part + (size_t)n * rec.nst * rec.Q + g0 * qpg + min((int)(threadIdx.x & 15), (g1 - g0 + 1) * qpg - 1);
+    double s = 0.0, ss = 0.0;
+#pragma unroll 8
+    for (int t = threadIdx.x >> 4; t < rec.nst; t += 16) { const float2 v = rp[(size_t)t * rec.Q]; s += (double)v.x; ss += (double)v.y; }      // thread (quad q, j): records j, j + 16, ...
+    r1[threadIdx.x] = s; r2[threadIdx.x] = ss;
+    __syncthreads();
+    if (threadIdx.x < 64) {                                   // lane (q, part): a quad's sums over four of the sixteen rows, then over the four lanes of the quad
+        const int qq = threadIdx.x & 15, k0 = threadIdx.x >> 4;
+        s = (r1[(4 * k0) * 16 + qq] + r1[(4 * k0 + 1) * 16 + qq]) + (r1[(4 * k0 + 2) * 16 + qq] + r1[(4 * k0 + 3) * 16 + qq]);
+        ss = (r2[(4 * k0) * 16 + qq] + r2[(4 * k0 + 1) * 16 + qq]) + (r2[(4 * k0 + 2) * 16 + qq] + r2[(4 * k0 + 3) * 16 + qq]);
+        s += __shfl_xor(s, 16); s += __shfl_xor(s, 32); ss += __shfl_xor(ss, 16); ss += __shfl_xor(ss, 32);
+        if (threadIdx.x < 16) { r1[threadIdx.x] = s; r2[threadIdx.x] = ss; }
+    }
+    __syncthreads();
+    const int g = g0 + (int)threadIdx.x;
+    if (g > g1 || g * cpg < blk * 32) return;
+    s = 0.0; ss = 0.0;
+    for (int k = 0; k < qpg; k++) { s += r1[threadIdx.x * qpg + k]; ss += r2[threadIdx.x * qpg + k]; }
+    gn_part_finish(osum, s, ss, fin, (unsigned)(n * rec.Go + g));
 }
 
 // the same with one block per (sample, group), for records wider than a block (more than 1024 channels) or more than 256 groups

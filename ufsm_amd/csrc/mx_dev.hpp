@@ -305,7 +305,7 @@ __device__ __forceinline__ void gn_mean_rstd(double s, double ss, double len, fl
 // the statistics records of a conv's output (conv3.hip): per sample nst records of Q float2 (sum, sum of squares of a channel quad), quad q = channels 4 q .. 4 q + 3,
 // and what is made of them: mean / rstd [N][Go] of groups of len elements
 struct gn_records_t { const float2 *part; int nst, Q, Go; double len; float eps; float *mean, *rstd; };
-// whether a conv's statistics are formed from its records 32 channels at a time, a workgroup each (the sums below): whole blocks, groups of whole quads, at most 16 quads in the
+// whether a conv's statistics are formed from its records 32 channels at a time, a workgroup each: whole blocks, groups of whole quads, at most 16 quads in the
 // groups that a block meets and at most 512 records. A matter of one sample, never of how many there are: whoever adds such records - the pre-pass behind the conv, or the
 // reduction where that pass would read too much - adds them in this order, so that a sample's mean and rstd are the same bits alone and in a batch
 inline int mi_records_quads(int C, int Go) {                        // the most quads a block's groups have
@@ -315,39 +315,6 @@ inline int mi_records_quads(int C, int Go) {                        // the most 
     return nq;
 }
 inline bool mi_records_few(int C, int Go, int nst) { return C % 32 == 0 && C / Go % 4 == 0 && nst <= 512 && mi_records_quads(C, Go) <= 16; }
-// thread (quad q, j) of 256: its quad of the groups block blk's channels lie in, records j, j + 16, ...
-struct gn_rec_lane_t { const float2 *rp; int rj, cpg, g0, g1, qpg; };
-__device__ __forceinline__ gn_rec_lane_t gn_rec_lane(const gn_records_t &rec, int C, int n, int blk) {
-    gn_rec_lane_t l;
-    l.cpg = C / rec.Go; l.g0 = blk * 32 / l.cpg; l.g1 = (blk * 32 + 31) / l.cpg; l.qpg = l.cpg >> 2; l.rj = threadIdx.x >> 4;
-    l.rp = rec.part + (size_t)n * rec.nst * rec.Q + l.g0 * l.qpg + min((int)(threadIdx.x & 15), (l.g1 - l.g0 + 1) * l.qpg - 1);
-    return l;
-}
-template <int RK> __device__ __forceinline__ void gn_rec_request(const gn_records_t &rec, const gn_rec_lane_t &l, float2 (&rv)[RK]) {
-#pragma unroll
-    for (int k = 0; k < RK; k++) rv[k] = l.rp[(size_t)min(l.rj + 16 * k, rec.nst - 1) * rec.Q];
-}
-// the sums of group g0 + threadIdx.x for threads up to g1 - g0; r1, r2: 256 doubles of LDS. Ends with the scratch still being read
-template <int RK> __device__ __forceinline__ void gn_rec_sums(const gn_records_t &rec, const gn_rec_lane_t &l, const float2 (&rv)[RK], double *r1, double *r2, double &s, double &ss) {
-    s = 0.0; ss = 0.0;
-#pragma unroll
-    for (int k = 0; k < RK; k++) if (l.rj + 16 * k < rec.nst) { s += (double)rv[k].x; ss += (double)rv[k].y; }
-#pragma unroll 8
-    for (int t = l.rj + 16 * RK; t < rec.nst; t += 16) { const float2 v = l.rp[(size_t)t * rec.Q]; s += (double)v.x; ss += (double)v.y; }
-    r1[threadIdx.x] = s; r2[threadIdx.x] = ss;
-    __syncthreads();
-    if (threadIdx.x < 64) {                                   // lane (q, part): a quad's sums over four of the sixteen rows, then over the four lanes of the quad
-        const int qq = threadIdx.x & 15, k0 = threadIdx.x >> 4;
-        s = (r1[(4 * k0) * 16 + qq] + r1[(4 * k0 + 1) * 16 + qq]) + (r1[(4 * k0 + 2) * 16 + qq] + r1[(4 * k0 + 3) * 16 + qq]);
-        ss = (r2[(4 * k0) * 16 + qq] + r2[(4 * k0 + 1) * 16 + qq]) + (r2[(4 * k0 + 2) * 16 + qq] + r2[(4 * k0 + 3) * 16 + qq]);
-        s += __shfl_xor(s, 16); s += __shfl_xor(s, 32); ss += __shfl_xor(ss, 16); ss += __shfl_xor(ss, 32);
-        if (threadIdx.x < 16) { r1[threadIdx.x] = s; r2[threadIdx.x] = ss; }
-    }
-    __syncthreads();
-    s = 0.0; ss = 0.0;
-    if ((int)threadIdx.x <= l.g1 - l.g0)
-        for (int k = 0; k < l.qpg; k++) { s += r1[threadIdx.x * l.qpg + k]; ss += r2[threadIdx.x * l.qpg + k]; }
-}
 // silu(gn(x)) of the MX tensor x (C a multiple of 32) into y8 (MX-fp8 rows) and / or y4 (MX-fp4), mean and rstd formed from the records by the kernel that applies
 // them; false: not for these records (nothing was launched)
 bool mi_restage_records(const void *x, int xdt, int N, int C, size_t S, const float *gamma, const float *beta, const gn_records_t &rec, void *y8, void *y4);

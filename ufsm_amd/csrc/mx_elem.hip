@@ -837,7 +837,8 @@ constexpr int RS32_R = 4;                                          // rows per t
 // BY2 (4, with BY 8): the same values also leave as a second tensor y2 in MX-fp4 - a skip tensor whose two readers compute in different
 // formats (the stride-2 down conv in e4m3, the decoder's conv in e2m1) is read and transformed once
 // RED: the statistics are not read but formed here, from the records of the conv that wrote x (rec; Cg = C, cg0 = 0): every workgroup adds the records of the groups
-// its 32 channels lie in, in double, while its rows arrive; the first workgroup of a group's first block stores the group's mean and rstd
+// its 32 channels lie in, in double, while its rows arrive; the first workgroup of a group's first block stores the group's mean and rstd. The order of the additions is
+// gn_part_reduce_few_k's (conv3.hip), which runs where this pass would read too many records: a change here is one there
 template <int BX, int BY, int BY2 = 0, bool RED = false>
 __global__ void __launch_bounds__(256) restage32_k(const uint8_t *x, uint8_t *y, int N, int C, size_t S, gnp_t gp, int Cg, int cg0, size_t Ss, size_t v0, uint8_t *y2 = nullptr, gn_records_t rec = gn_records_t{}) {
     const int nb = C / 32, blk = blockIdx.y, n = blockIdx.z;
@@ -850,14 +851,18 @@ __global__ void __launch_bounds__(256) restage32_k(const uint8_t *x, uint8_t *y,
     const size_t row0 = ((size_t)n * nb + blk) * Ss + v0;
     const uint8_t *xs = x + (size_t)N * nb * Ss * (IB * 2);
     uint8_t *ys = y + (size_t)N * nb * Ss * (OB * 2);
-    // RED: the first of the thread's records and the affine are requested before the rows (loads return in order: the chain they start is the longer one)
+    // RED: the groups the block's channels lie in and their quads of channels; thread (q, j) adds quad q of records j, j + 16, ... The first of them and the affine are requested
+    // before the rows (loads return in order: the chain they start is the longer one)
     constexpr int RK = RED ? 8 : 1;
-    gn_rec_lane_t rl;
+    const int cpg = RED ? C / rec.Go : 4, g0 = blk * 32 / cpg, g1 = (blk * 32 + 31) / cpg, qpg = cpg >> 2;      // (cpg a multiple of 4; the groups' quads are at most 16: mi_records_few)
+    const int rj = threadIdx.x >> 4;
+    const float2 *rp = nullptr;
     float2 rv[RK];
     float ga = 0.f, be = 0.f;
     if constexpr (RED) {
-        rl = gn_rec_lane(rec, C, n, blk);
-        gn_rec_request(rec, rl, rv);
+        rp = rec.part + (size_t)n * rec.nst * rec.Q + g0 * qpg + min((int)(threadIdx.x & 15), (g1 - g0 + 1) * qpg - 1);
+#pragma unroll
+        for (int k = 0; k < RK; k++) { const int t = rj + 16 * k; rv[k] = rp[(size_t)min(t, rec.nst - 1) * rec.Q]; }
         if (threadIdx.x < 32) { ga = gp.gamma[blk * 32 + threadIdx.x]; be = gp.beta[blk * 32 + threadIdx.x]; }
     }
     unsigned w[RS32_R][4]; unsigned sby[RS32_R];
@@ -871,21 +876,36 @@ __global__ void __launch_bounds__(256) restage32_k(const uint8_t *x, uint8_t *y,
     }
     // (the rows are requested before the block's coefficients are formed: the two chains of dependent loads overlap)
     if constexpr (RED) {
+        double s = 0.0, ss = 0.0;
+#pragma unroll
+        for (int k = 0; k < RK; k++) if (rj + 16 * k < rec.nst) { s += (double)rv[k].x; ss += (double)rv[k].y; }
+#pragma unroll 8
+        for (int t = rj + 16 * RK; t < rec.nst; t += 16) { const float2 v = rp[(size_t)t * rec.Q]; s += (double)v.x; ss += (double)v.y; }
         __shared__ double r1[256], r2[256];
         __shared__ float sm[16], sr[16];
-        double s, ss;
-        gn_rec_sums(rec, rl, rv, r1, r2, s, ss);
-        if ((int)threadIdx.x <= rl.g1 - rl.g0) {
+        r1[threadIdx.x] = s; r2[threadIdx.x] = ss;
+        __syncthreads();
+        if (threadIdx.x < 64) {                               // lane (q, part): a quad's sums over four of the sixteen rows, then over the four lanes of the quad
+            const int qq = threadIdx.x & 15, k0 = threadIdx.x >> 4;
+            s = (r1[(4 * k0) * 16 + qq] + r1[(4 * k0 + 1) * 16 + qq]) + (r1[(4 * k0 + 2) * 16 + qq] + r1[(4 * k0 + 3) * 16 + qq]);
+            ss = (r2[(4 * k0) * 16 + qq] + r2[(4 * k0 + 1) * 16 + qq]) + (r2[(4 * k0 + 2) * 16 + qq] + r2[(4 * k0 + 3) * 16 + qq]);
+            s += __shfl_xor(s, 16); s += __shfl_xor(s, 32); ss += __shfl_xor(ss, 16); ss += __shfl_xor(ss, 32);
+            if (threadIdx.x < 16) { r1[threadIdx.x] = s; r2[threadIdx.x] = ss; }
+        }
+        __syncthreads();
+        if ((int)threadIdx.x <= g1 - g0) {
+            s = 0.0; ss = 0.0;
+            for (int k = 0; k < qpg; k++) { s += r1[threadIdx.x * qpg + k]; ss += r2[threadIdx.x * qpg + k]; }
             unsigned long long w[3];
             float m, r;
             gn_mean_rstd(gn_slot_value(s, w), gn_slot_value(ss, w), rec.len, rec.eps, &m, &r);
             sm[threadIdx.x] = m; sr[threadIdx.x] = r;
-            const int g = rl.g0 + (int)threadIdx.x;
-            if (blockIdx.x == 0 && g * rl.cpg >= blk * 32) { rec.mean[n * rec.Go + g] = m; rec.rstd[n * rec.Go + g] = r; }
+            const int g = g0 + (int)threadIdx.x;
+            if (blockIdx.x == 0 && g * cpg >= blk * 32) { rec.mean[n * rec.Go + g] = m; rec.rstd[n * rec.Go + g] = r; }
         }
         __syncthreads();
         if (threadIdx.x < 32) {
-            const int k = (blk * 32 + (int)threadIdx.x) / rl.cpg - rl.g0;
+            const int k = (blk * 32 + (int)threadIdx.x) / cpg - g0;
             const float a = sr[k] * ga;
             sa[threadIdx.x] = a; sb[threadIdx.x] = fmaf(-sm[k], a, be);
         }
