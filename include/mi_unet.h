@@ -169,8 +169,8 @@ void mi_unet_get_params(const unet *u, float *host);           /* the live weigh
 void mi_unet_set_params(unet *u, const float *host);           /* ... and the EMA copy with them; drops the prepared-weight memos */
 /* the forward on an input that already is the net's MX tensor (lp_f32_to_mx* output or lp_pred_input_mx rows), device pointer */
 const float *mi_unet_forward_mx(unet *u, const void *xmx, shape5 xs);
-/* the same and unet_forward_ct with the logits written to the caller's device buffer (fp32 [n][cout][d][h][w]) by the head itself; the net's own buffer need not
-   hold them. 0 on success. logits null: the net's own */
+/* the same and unet_forward_ct with the logits written to the caller's device buffer (fp32 [n][cout][d][h][w]) by the head itself; the net's own buffer is left as
+   it is, so that a pointer an earlier forward returned does not see them. 0 on success. logits null: the net's own */
 int mi_unet_forward_mx_to(unet *u, const void *xmx, shape5 xs, float *logits);
 int mi_unet_forward_ct_to(unet *u, const uint8_t *ct, float mean, float isd, const float *dyo, const float *dxo, int axis, shape5 xs, int h16, float *logits);
 /* unet_forward_ct with the windows and their offset rows given one pointer each (window n -> sample n; windows of a batch need not be contiguous) */

@@ -54,11 +54,11 @@ static dim3 rows_grid(int N, int nb, size_t S) {
 //   146 -> 119 (pairs: 160 and 142). Blocks of 8 channels stay pairs (305 MB, to MX and back: 161 and 158, streamed 172 and 165). Lines shared by two
 //   wavefronts lose their meeting in the cache (64 channels, 999999: 53 / 68 -> 61 / 100 and 48 / 59 -> 55 / 98), and planes that fit the cache are found there (64
 //   channels, 96^3 to MX: 43 -> 46 and 39 -> 44).
-//   These kernels ask for LDS that they do not use, which leaves 4 blocks of them on a CU (6 with blocks of 16 channels): the fewer wavefronts run, the
-//   nearer together are the addresses that a plane's stream is at, and the fewer DRAM pages are open at once. Blocks a CU, all (8) / 6 / 5 / 4 / 3, us to MX and back:
+//   These kernels ask for LDS that they do not use, which leaves 4 blocks of them on a CU (6 with blocks of 16 channels). These times are the rule's only ground (the fewer wavefronts
+//   run, the nearer together are the addresses that a plane's stream is at; that this opens fewer DRAM pages was not counted). Blocks a CU, all (8) / 6 / 5 / 4 / 3, us to MX and back:
 //   32 channels, 2 x 128^3, e4m3 242 / 231 / 223 / 219 / 216 and e2m1 228 / 215 / 207 / 203 / 200; 160^3 204 / 202 / 201 / 202 / 204 and 197 / 196 / 195 / 194 / 195; 8 x 294912
 //   116 / 115 / 115 / 114 / 117; 96 channels, 96^3 131 / 130 / 130 / 129 / 130; 64 channels, 4 x 393216 156 / 156 / 155 / 155 / 157 (planes of a power of two gain
-//   most: their streams meet in one channel). 16 channels, 2 x 128^3 124 / 120 / 122 / 132 / 136, 192^3 172 / 169 / 169 / 173 / 189.
+//   most). 16 channels, 2 x 128^3 124 / 120 / 122 / 132 / 136, 192^3 172 / 169 / 169 / 173 / 189.
 constexpr int CVT_BW = 16;         // widest block of the pairs
 static bool cvt_pairs(int C, size_t S) { return mx_bw(C) <= CVT_BW && S >= (size_t)1 << 17; }
 static bool cvt_stream(const void *planes, int N, int C, size_t S) { return mx_bw(C) > 8 && S % 32 == 0 && !((uintptr_t)planes & 127) && (size_t)N * C * S * 4 >= (size_t)256 << 20; }

@@ -164,7 +164,8 @@ class UNet:
             self._unmode()
 
     def forward_x(self, x_ptr, logits_ptr):
-        """forward_mx, the logits written to the caller's device buffer; 0 on success."""
+        """forward_mx, the logits written to the caller's device buffer by the head itself; 0 on success. The net's own buffer is left as it is: a pointer that
+        an earlier forward_mx or forward_planes returned keeps that forward's logits."""
         self._mode()
         try:
             return -1 if not logits_ptr or self.L.mi_unet_forward_mx_to(self.h, x_ptr, self.shape, logits_ptr) else 0
@@ -180,7 +181,7 @@ class UNet:
             self._unmode()
 
     def forward_ct(self, ct_ptr, mean, isd, dyo_ptr, dxo_ptr, axis, logits_ptr, h16=2):
-        """The forward from the uint8 CT window(s), the logits written to the caller's device buffer; 0 on success."""
+        """The forward from the uint8 CT window(s), the logits written to the caller's device buffer (the net's own is left as it is: forward_x); 0 on success."""
         self._mode()
         try:
             return -1 if not logits_ptr or self.L.mi_unet_forward_ct_to(self.h, ct_ptr, mean, isd, dyo_ptr, dxo_ptr, axis, self.shape, h16, logits_ptr) else 0
