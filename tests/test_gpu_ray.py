@@ -67,6 +67,12 @@ def test_ray_maps(gpu, D, Hh, W, mult):
     assert (G[slot >= lens] == 0).all()
 
 
+@pytest.mark.parametrize("D,Hh,W,mult", [(5, 6, 4, 11.0), (1, 9, 3, 3.6), (4, 4, 4, 0.25)])
+def test_ray_maps_at_the_edges_of_a_tokens_lanes(gpu, D, Hh, W, mult):
+    """a plane's rays fill a token's 32 lanes twice over and two more (66), once and one more (33), or are a single one"""
+    test_ray_maps(gpu, D, Hh, W, mult)
+
+
 def test_scroll_pos_on_the_device(gpu):
     D, Hh, W, n, nreg = 5, 6, 4, 3, 2
     axr = make_axr(n, D, Hh, W, (1, 0, 2), (0, 1, 2))

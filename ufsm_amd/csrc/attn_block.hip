@@ -206,7 +206,8 @@ __global__ void __launch_bounds__(256) qkv_pack_k(const float *__restrict__ qkv,
     if (threadIdx.x == 0) bmax = 0u;
     __syncthreads();
     if (unit < nunits) {
-        const int h = (int)(unit % H); const long long tp = unit / H; const int p = (int)(tp % 3); const long long t = tp / 3;      // units of a token are neighbours: its 3 H x 192 bytes are read together
+        // units of a token are neighbours: its 3 H x 192 bytes are read together. (Fewer than 2^32 units: their rows are 96 bytes each)
+        const unsigned tp = (unsigned)unit / (unsigned)H; const int h = (int)((unsigned)unit - tp * (unsigned)H), p = (int)(tp % 3u); const long long t = tp / 3u;
         const int C = H * HD;
         __half *dst = out + (((size_t)p * H + h) * Tp + t) * HD + 8 * j;
         if (t >= T) { if (j < 6) *(uint4 *)dst = make_uint4(0u, 0u, 0u, 0u); }
@@ -245,7 +246,7 @@ __global__ void __launch_bounds__(256) qkv_pack_k(const float *__restrict__ qkv,
                     const float *gs = (p ? kg : qg) + h * HD + 8 * j;      // (the gains sit at an arbitrary offset of the flat parameter vector: dword loads)
 #pragma unroll
                     for (int i = 0; i < 8; i++) v[i] *= r * gs[i];
-                    const int ts = (int)(t % rp.S) - rp.nreg;
+                    const int ts = (int)((unsigned)t % (unsigned)rp.S) - rp.nreg;
                     if (rp.on && ts >= 0) {
                         const float pos = rope_pos<MODE>(rp, t, ts, j >> 1);
 #pragma unroll
