@@ -144,6 +144,24 @@ def test_core_on_other_sequence_lengths(gpu, nseq, S, lens):
     assert rel(do.to_numpy(np.float32, (T, Cc)), ro.attend(qh, kh, vh, nseq, S, lens)) < 2e-3
 
 
+@pytest.mark.parametrize("S", [1, 8, 13, 24, 31, 32])
+def test_short_sequences_give_the_long_ones_bits(gpu, S):
+    """sequences of up to 32 slots run on their own kernel, in the order of the general one: the same rows under a geometry of 40 slots give the same bits"""
+    rng = np.random.default_rng(60 + S)
+    nseq, H, L = 9, 2, 40; Cc = 48 * H
+    lens = rng.integers(0, S + 1, nseq).astype(np.int32); lens[:3] = (S, 0, 1)
+    rows = rng.standard_normal((3, H, nseq, S, 48)).astype(np.float16) * 2
+    out = []
+    for n in (S, L):
+        buf = np.zeros((3, H, nseq * n + 64, 48), np.float16)
+        buf[:, :, :nseq * n].reshape(3, H, nseq, n, 48)[:, :, :, :S] = rows
+        dq, dl, do, dlse = DevBuf.from_numpy(buf.view(np.uint16)), DevBuf.from_numpy(lens), DevBuf(nseq * n * Cc * 4), DevBuf(nseq * H * n * 4)
+        g = at_geom(); g.nseq, g.S, g.D, g.Hh, g.W = nseq, n, 1, 1, n; g.lens = dl.ptr
+        lib.at_fa_fwd(dq.ptr, do.ptr, dlse.ptr, C.byref(g), H, Cc); LP.check()
+        out.append((do.to_numpy(np.float32, (nseq, n, Cc))[:, :S], dlse.to_numpy(np.float32, (nseq, H, n))[:, :, :S]))
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+
+
 def run_block(P, lay, x, d, g, Tr=0):
     bp = at_bp(); assert lib.at_block_layout(C.byref(d), C.byref(bp), 0) == P.size
     T = x.shape[0]

@@ -242,21 +242,15 @@ __global__ void __launch_bounds__(256) scroll_pos_k(long long n, long long S, in
 // multiply-adds as scalar operands (no LDS, no lane exchange). Probabilities are rounded to fp16 before they meet v, the denominator adds the
 // unrounded ones: the rounding points of the fp16 tensor-core kernel this replaces. Ray sequences are 20 - 50 slots long: the arithmetic is
 // a few percent of a block's and the kernel is latency-bound.
-// QL: queries per (sequence, head) unit, 64 or - for sequences of at most 32 tokens - 32, two units per wavefront: a ray of 24 slots fills 75 % of
-// the lanes instead of 37 % (the keys' rows are per-lane addresses either way; the walk runs to the longer of the two units' lengths)
-template <int QL>
 __global__ void __launch_bounds__(256) fa16_rows_k(const __half *__restrict__ Qh, const __half *__restrict__ Kh, const __half *__restrict__ Vh, float *__restrict__ o, float *__restrict__ lse,
                                                    int S, int H, int C, long long Tp, int nseq, float sl2, const int *__restrict__ lens) {
-    const int nqt = (S + QL - 1) / QL, lane = threadIdx.x & 63;
-    const long long nun = (long long)nseq * H * nqt;
-    long long un = ((long long)blockIdx.x * 4 + (threadIdx.x >> 6)) * (64 / QL) + lane / QL;
-    const bool live = un < nun;
-    if (!live) un = nun - 1;                                       // (an idle half: the last unit's rows, nothing stored)
+    const int nqt = (S + 63) / 64, lane = threadIdx.x & 63;
+    const long long nun = (long long)nseq * H * nqt, un = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (un >= nun) return;
     const int qt = (int)(un % nqt), h = (int)(un / nqt % H), seq = (int)(un / nqt / H);
     const size_t base = ((size_t)h * Tp + (size_t)seq * S) * HD;
-    const int SK = !live ? 0 : lens ? min(lens[seq], S) : S;
-    const int SKw = QL == 64 ? SK : max(SK, __shfl_xor(SK, 32));   // how far this wavefront walks
-    const int i = qt * QL + lane % QL;
+    const int SK = lens ? min(lens[seq], S) : S;
+    const int i = qt * 64 + lane;
     float q[HD], acc[HD];
     {
         const uint4 *qr = (const uint4 *)(Qh + base + (size_t)i * HD);      // (rows past the sequence's end are other rows of the padded array: read, never stored)
@@ -271,8 +265,7 @@ __global__ void __launch_bounds__(256) fa16_rows_k(const __half *__restrict__ Qh
     for (int d = 0; d < HD; d++) acc[d] = 0.f;
     float m = -INFINITY, l = 0.f;
     const __half *K = Kh + base, *V = Vh + base;
-    for (int j0 = 0; j0 < SKw; j0 += 8) {
-        if (j0 >= SK) continue;                                    // (the other unit of the wavefront is longer)
+    for (int j0 = 0; j0 < SK; j0 += 8) {
         float s[8];
 #pragma unroll
         for (int jj = 0; jj < 8; jj++) {
@@ -298,12 +291,89 @@ __global__ void __launch_bounds__(256) fa16_rows_k(const __half *__restrict__ Qh
             for (int d = 0; d < HD; d++) acc[d] = fmaf(ph, __half2float(vr[d]), acc[d]);
         }
     }
-    if (i >= S || !live) return;
+    if (i >= S) return;
     const float il = l > 0.f ? 1.f / l : 0.f;
     float4 *orow = (float4 *)(o + ((size_t)seq * S + i) * C + h * HD);
 #pragma unroll
     for (int c = 0; c < HD / 4; c++) orow[c] = make_float4(acc[4 * c] * il, acc[4 * c + 1] * il, acc[4 * c + 2] * il, acc[4 * c + 3] * il);
     lse[((size_t)seq * H + h) * S + i] = l > 0.f ? m + log2f(l) : 0.f;    // (a length-0 sequence: zero output)
+}
+// The same for sequences of at most 32 tokens - every ray of a bottleneck grid of up to 21^3 -, where one query per lane leaves two wavefronts on a SIMD, waiting
+// for rows: a workgroup of two wavefronts takes one (sequence, head), four lanes per query. The rows of K and V lie in LDS; each of a query's lanes forms the logits
+// of every fourth key, and - after these have met in LDS - its quarter of the output dims over all keys. Every logit, maximum, probability and sum is formed
+// in the order of the kernel above (in groups of eight keys), so the results are its bits. Bound by its multiply-adds and the LDS reads that feed them:
+// 2 x 512 rays of 24 slots, four heads, 45 -> 21 us (the multiply-adds and conversions alone take about 9)
+__global__ void __launch_bounds__(128) fa16_short_k(const __half *__restrict__ Qh, const __half *__restrict__ Kh, const __half *__restrict__ Vh, float *__restrict__ o, float *__restrict__ lse,
+                                                    int S, int H, int C, long long Tp, float sl2, const int *__restrict__ lens) {
+    __shared__ __align__(16) __half ks[32 * HD], vs[32 * HD];
+    __shared__ float lg[32 * 33];                                  // [key][query]
+    const int tid = threadIdx.x, i = tid & 31, part = tid >> 5;
+    const int seq = (int)(blockIdx.x / (unsigned)H), h = (int)(blockIdx.x - (unsigned)seq * (unsigned)H);
+    const size_t base = ((size_t)h * Tp + (size_t)seq * S) * HD;
+    const int SK = lens ? min(lens[seq], S) : S;
+    float q[HD];
+    {
+        const uint4 *qr = (const uint4 *)(Qh + base + (size_t)min(i, S - 1) * HD);
+#pragma unroll
+        for (int c = 0; c < HD / 8; c++) {
+            const uint4 u = qr[c]; const __half2 *hp = (const __half2 *)&u;
+#pragma unroll
+            for (int e = 0; e < 4; e++) { const float2 f = __half22float2(hp[e]); q[8 * c + 2 * e] = f.x; q[8 * c + 2 * e + 1] = f.y; }
+        }
+    }
+    for (int c = tid; c < 32 * (HD / 8); c += 128) {               // (rows past the length: zeros; a group's probabilities there are 0)
+        const bool in = c / (HD / 8) < SK;
+        ((uint4 *)ks)[c] = in ? ((const uint4 *)(Kh + base))[c] : make_uint4(0u, 0u, 0u, 0u);
+        ((uint4 *)vs)[c] = in ? ((const uint4 *)(Vh + base))[c] : make_uint4(0u, 0u, 0u, 0u);
+    }
+    __syncthreads();
+    for (int j = part; j < SK; j += 4) {
+        float a = 0.f;
+#pragma unroll
+        for (int c = 0; c < HD / 8; c++) {
+            const uint4 u = ((const uint4 *)ks)[j * (HD / 8) + c]; const __half *kr = (const __half *)&u;
+#pragma unroll
+            for (int e = 0; e < 8; e++) a = fmaf(q[8 * c + e], __half2float(kr[e]), a);
+        }
+        lg[j * 33 + i] = j & 7 ? a * sl2 : a;                      // (a group's first key is scaled inside its difference to the maximum, one rounding, as the compiler has it above)
+    }
+    __syncthreads();
+    constexpr int PD = HD / 4;                                     // the lane's output dims
+    float acc[PD];
+#pragma unroll
+    for (int d = 0; d < PD; d++) acc[d] = 0.f;
+    float m = -INFINITY, l = 0.f;
+    for (int j0 = 0; j0 < SK; j0 += 8) {
+        float s[8];
+        s[0] = lg[j0 * 33 + i];
+#pragma unroll
+        for (int jj = 1; jj < 8; jj++) s[jj] = j0 + jj < SK ? lg[(j0 + jj) * 33 + i] : -INFINITY;
+        float mt = s[0] * sl2;
+#pragma unroll
+        for (int jj = 1; jj < 8; jj++) mt = fmaxf(mt, s[jj]);
+        const float mn = fmaxf(m, mt), corr = exp2f(m - mn);
+        m = mn; l *= corr;
+#pragma unroll
+        for (int d = 0; d < PD; d++) acc[d] *= corr;
+#pragma unroll
+        for (int jj = 0; jj < 8; jj++) {
+            const float p = exp2f(jj ? s[jj] - m : fmaf(s[0], sl2, -m)), ph = __half2float(__float2half_rn(p));
+            l += p;
+            const uint2 *vr = (const uint2 *)(vs + (j0 + jj) * HD + part * PD);
+#pragma unroll
+            for (int c = 0; c < PD / 4; c++) {
+                const uint2 u = vr[c]; const __half *vv = (const __half *)&u;
+#pragma unroll
+                for (int e = 0; e < 4; e++) acc[4 * c + e] = fmaf(ph, __half2float(vv[e]), acc[4 * c + e]);
+            }
+        }
+    }
+    if (i >= S) return;
+    const float il = l > 0.f ? 1.f / l : 0.f;
+    float4 *orow = (float4 *)(o + ((size_t)seq * S + i) * C + h * HD + part * PD);
+#pragma unroll
+    for (int c = 0; c < PD / 4; c++) orow[c] = make_float4(acc[4 * c] * il, acc[4 * c + 1] * il, acc[4 * c + 2] * il, acc[4 * c + 3] * il);
+    if (!part) lse[((size_t)seq * H + h) * S + i] = l > 0.f ? m + log2f(l) : 0.f;
 }
 }
 
@@ -374,11 +444,11 @@ extern "C" void at_fa_fwd(const void *qkvh, float *o, float *lse, const at_geom 
     const long long T = (long long)g->nseq * g->S, Tp = T + FT;
     if (!T) return;
     const __half *Qh = (const __half *)qkvh, *Kh = Qh + (size_t)H * Tp * HD, *Vh = Kh + (size_t)H * Tp * HD;
-    const int QL = g->S <= 32 ? 32 : 64;
-    const long long nw = ((long long)g->nseq * H * ((g->S + QL - 1) / QL) + 64 / QL - 1) / (64 / QL);      // wavefronts
+    const bool shrt = g->S <= 32;
+    const long long nw = (long long)g->nseq * H * (shrt ? 1 : (g->S + 63) / 64);      // (sequence, head) units, or wavefronts
     if (nw > 0x7fffffffll) mi_die("at_fa_fwd: %lld wavefronts", nw);
     const float sl2 = 1.4426950408889634f / sqrtf((float)HD);
-    if (QL == 32) fa16_rows_k<32><<<nblk_((size_t)nw, 4), 256>>>(Qh, Kh, Vh, o, lse, g->S, H, C, Tp, g->nseq, sl2, g->lens);
-    else fa16_rows_k<64><<<nblk_((size_t)nw, 4), 256>>>(Qh, Kh, Vh, o, lse, g->S, H, C, Tp, g->nseq, sl2, g->lens);
+    if (shrt) fa16_short_k<<<(unsigned)nw, 128>>>(Qh, Kh, Vh, o, lse, g->S, H, C, Tp, sl2, g->lens);
+    else fa16_rows_k<<<nblk_((size_t)nw, 4), 256>>>(Qh, Kh, Vh, o, lse, g->S, H, C, Tp, g->nseq, sl2, g->lens);
     MICK();
 }
