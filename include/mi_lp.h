@@ -97,6 +97,10 @@ void mi_conv_s2_direct(int mode);
 /* Extension: up to how many tiles (64 voxels x 32 output channels, of the whole tensor) the calling thread's 3x3x3 convs may run on the kernel that splits
    the K range over a workgroup's wavefronts. -1 (default): the measured limits; 0: never. The same conv either way, its fp32 sums in another order. */
 void mi_conv_thin(int tiles);
+/* Extension: whether the calling thread's 3x3x3 convs run on the kernel of flat 128-voxel tiles whose taps are split over a workgroup's wavefronts: 1 wherever
+   that kernel can (stride 1, an even number of input blocks, more than 32 output channels, rows of at most 41 voxels), 0 nowhere, -1 (default) by size. The same
+   conv either way, its fp32 sums in another order. */
+void mi_conv_flat(int mode);
 /* 1x1x1 head with eight outputs on whole 32-channel blocks: where its 8 x 32 products per voxel run. mode 1: the matrix pipe (batched 4 x 4 x 1
    fp32 outer products, one product per accumulator and step, in channel order), 0: fused multiply-adds on the vector ALUs, -1: the default
    (1, or the environment's MI_HEAD_MFMA). The two give the same bits; the setting is the calling thread's. No counterpart in the reference. */

@@ -350,7 +350,7 @@ static int conv_stem(const char *who, const void *x, int xbf, shape5 xs, const f
     const int nmt_all = (cout + 31) / 32, MT = nmt_all % 2 == 0 && CP && CP < 16 && !(osum && (cout / Go) % 4) ? 2 : 1;
     size_t smem = rows ? (size_t)720 * 16 + 16 + 40 * 4 + 16 * 8 : ((size_t)720 * CP + 16 + CP * 8 + 15) & ~(size_t)15;     // staged tile, (zero row, row words | amax word), channel affine
     if (a.sns > 1) smem += (size_t)(a.sns - 1) * (rows ? 16 : CP) * 8;      // (one affine table per slab)
-    a.epi_o = (unsigned)smem; smem += (size_t)3 * MT * 32 * sizeof(float);
+    a.epi_o = (unsigned)smem; smem += (size_t)3 * (a.flat ? 2 : MT) * 32 * sizeof(float);
     a.red_o = (unsigned)smem; smem += 1024;
     a.nmt_all = nmt_all; a.ncs = nmt_all / MT;
     a.ntx = (W + 15) / 16; a.nty = (H + 7) / 8; a.ntz = (Do + 1) / 2;
@@ -403,6 +403,8 @@ static thread_local int g_s2d = -1;         // mi_conv_s2_direct: the calling th
 extern "C" void mi_conv_s2_direct(int mode) { g_s2d = mode; }
 static thread_local int g_thin = -1;        // mi_conv_thin: the calling thread's tile count up to which the K-split kernel takes a launch (-1: the default rule)
 extern "C" void mi_conv_thin(int tiles) { g_thin = tiles; }
+static thread_local int g_flat = -1;        // mi_conv_flat: whether the calling thread's convs run on the flat kernel wherever it can (1), nowhere (0), or by size (-1)
+extern "C" void mi_conv_flat(int mode) { g_flat = mode; }
 static int split_s2_env() { static int v = -1; if (v < 0) v = getenv("MI_CONV_SPLIT_S2") ? atoi(getenv("MI_CONV_SPLIT_S2")) : 1; return v; }      // tuning knob: 0 keeps four channel tiles
 static int conv_dispatch(const char *who, int fmt, int stride, const void *x, int xbf, shape5 xs, const float *w, const float *b, int cout, void *y, int ybf,
                          gnp_t gp, double *osum, int Go, split_t sp, const float *ep_a, const float *ep_b, int act) {
@@ -633,11 +635,29 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     const size_t thin_max = g_thin >= 0 ? (size_t)g_thin : kb == 1 && (coarse || stride == 2) ? 0 : kb == 2 && coarse ? (size_t)thin_env / 4 : kb >= 16 && fmt == 8 && !one_round ? 2 * (size_t)thin_env : (size_t)thin_env;
     a.thin = thin_max > 0 && !a.row && !a.areg && !s2d && !act && a.wide && cout > 16 && !(osum && (cout / Go) % 4) && !sp.zlo && !sp.zhi && g_split < 0 && g_s2d < 0 && N <= 65535 &&
              (size_t)D * H * W * 32 < ((size_t)1 << 31) && ((size_t)Dr * Ho * Wo + 63) / 64 * (size_t)nmt_all * N <= thin_max;
-    if (a.thin) { big = false; MT = 1; NT = 2; a.CB = a.nbt; }
-    size_t smem = a.thin ? MI_THIN_LDS : a.row1 ? (size_t)10 * 352 * (RB + 4) : a.row ? (size_t)2 * 2048 * (RB + 4) : a.areg ? (size_t)2 * ((TT + 63) / 64 * 64) * (RB + 4) : big ? (size_t)4 * MT * (WTILE + 256) + (size_t)3 * ((TT + 63) / 64 * 64) * (RB + 4) + (size_t)(((27 * a.nbt + 1) >> 1) + 2) * 32 : lds_bytes(a.CB);
+    // about one tile of 128 flat voxels x 64 channels per CU, past the K-split kernel's launches: the flat kernel, whose time goes by its rounds of 256 workgroups -
+    // some 8 us and 2.2 (e2m1 1) per pair of input blocks each - where the staged kernels' goes by one tile's chain of loads and barriers. Kernel time, us, the other
+    // kernel against this one, and workgroups here. e4m3: 256 -> 256 at 2 x 16^3 37.2 against 22.2 (256); at 1 x 22 x 26^2 (234) 64 -> 128 18.4 against 14.4, 128 -> 128 26.8 and
+    // 16.5, 384 -> 128 62.9 and 26.5; 192 -> 64 at 24^3 38.4 and 18.2 (108), at 32^3 38.8 and 21.0 (256); 192 -> 192 at 16^3 47.1 and 18.2 (96); 64 -> 64 at 24^3 20.3 and 13.6 (108);
+    // against the K-split kernel 256 -> 256 at 16^3 26.9 and 20.0 (128), with fewer than 257 of its tiles 192 -> 64 at 16 x 20^2 15.1 and 17.2 (its launches of 257 .. 512 tiles
+    // into 128 channels gain as much, 256 -> 128 at 32 x 16^2 28.2 and 20.9, but its limit of 512 tiles is a tested one and stays). e2m1: 128 -> 192 and 192 -> 192
+    // at 2 x 16^3 26.6 and 36.7 against 14.0 and 15.4 (192), 384 -> 128 at 2 x 16^3 31.9 and 20.2; with two blocks 64 -> 128 at 16^3 11.5 and 12.1. In two rounds a long K pays: e4m3
+    // 256 -> 256 at 4 x 16^3 50.1 and 38.1 (512), 384 -> 128 at 28^3 63.6 and 44.8 (344), 128 -> 128 at 28^3 28.0 and 27.3; e2m1 384 -> 128 at 2 x 24^3 48.5 and 34.5 (432), 128 -> 128 25.1
+    // and 23.4; in four it does not: 384 -> 128 at 2 x 32^3 75.4 and 90.9 (1024). A record per run of 32 voxels is four to eight times the staged kernels': past 512 a sample their
+    // sums take a launch more (3 - 5 us), which e2m1's shorter products do not always win back: 256 -> 128 at 28^3 (686 runs) 33.1 against 37.7 with it. As above, the whole
+    // tensor's voxels count, not a z-range's
+    static int flat_env = -1;
+    if (flat_env < 0) flat_env = getenv("MI_CONV_FLAT") ? atoi(getenv("MI_CONV_FLAT")) : 1;      // tuning knob: 0 never
+    const bool flat_ok = stride == 1 && a.wide && !act && nmt_all >= 2 && a.nbt % 2 == 0 && W <= flat_t<8>::WMAX && !(osum && (cout / Go) % 4) && !sp.zlo && !sp.zhi && N <= 65535 && (size_t)D * H * W < ((size_t)1 << 24);
+    const size_t frun = ((size_t)Dr * Ho * Wo + 31) / 32, fwg = (frun + 3) / 4 * (size_t)((nmt_all + 1) / 2) * N;
+    a.flat = flat_ok && (g_flat > 0 || (g_flat < 0 && flat_env && g_thin < 0 && g_split < 0 && g_s2d < 0 && ((size_t)Dr * Ho * Wo + 63) / 64 * (size_t)nmt_all * N > (a.thin && nmt_all <= 4 ? 512u : 256u) &&
+                         (fmt == 8 ? a.nbt >= 2 : a.nbt >= 4 && frun <= 512) && fwg <= (a.nbt >= 8 ? 512u : 256u)));
+    if (a.flat) a.thin = a.row = a.row1 = a.areg = false;
+    if (a.thin || a.flat) { big = false; MT = 1; NT = 2; a.CB = a.flat ? 2 : a.nbt; }
+    size_t smem = a.flat ? (size_t)(fmt == 8 ? flat_t<8>::LDS : flat_t<4>::LDS) : a.thin ? MI_THIN_LDS : a.row1 ? (size_t)10 * 352 * (RB + 4) : a.row ? (size_t)2 * 2048 * (RB + 4) : a.areg ? (size_t)2 * ((TT + 63) / 64 * 64) * (RB + 4) : big ? (size_t)4 * MT * (WTILE + 256) + (size_t)3 * ((TT + 63) / 64 * 64) * (RB + 4) + (size_t)(((27 * a.nbt + 1) >> 1) + 2) * 32 : lds_bytes(a.CB);
     if (s2d) smem = 0;
     smem = (smem + 15) & ~(size_t)15;
-    a.epi_o = (unsigned)smem; smem += (size_t)3 * MT * 32 * sizeof(float);      // bias, affine a, b of the workgroup's channels
+    a.epi_o = (unsigned)smem; smem += (size_t)3 * (a.flat ? 2 : MT) * 32 * sizeof(float);      // bias, affine a, b of the workgroup's channels
     a.red_o = (unsigned)smem; smem += a.row1 ? 3 * 2048 + 3 * 1024 : 1024;      // statistics scratch (the one-block row kernel: the weight fragments of two tap classes instead)
     if (s2d) smem += (size_t)(27 * a.nbt + 1 + 8) * sizeof(int);                // the direct stride-2 kernel's K-order table
     // the row kernel in e2m1: the prepared weights of up to four input blocks stay in LDS (MI_CONV_ROW_WL=0: loaded from global memory per tap class)
@@ -664,7 +684,11 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     a.nmt_all = nmt_all; a.ncs = nmt_all / MT;
     a.ntx = a.row ? (Wo + 31) / 32 : (Wo + 15) / 16; a.nty = (Ho + 7) / 8; a.ntz = (Do + TZ - 1) / TZ;      // (the row kernel: 4 x 8 x 32 voxels per tile)
     a.ntiles = (unsigned)((size_t)a.ntx * a.nty * a.ntz * a.ncs * N);
-    if (a.thin) { const thin_runs_t t = mi_thin_runs(a.zi0, Do, Ho, Wo); a.zc = t.off; a.ntx = t.step; a.nty = (int)t.recs; a.ntiles = (unsigned)(t.recs * nmt_all * N); }      // (its statistics records)
+    if (a.thin || a.flat) {                                       // (their statistics records)
+        const thin_runs_t t = mi_thin_runs(a.zi0, Do, Ho, Wo);
+        a.zc = t.off; a.ntx = t.step; a.nty = (int)t.recs; a.ntz = (int)t.runs; a.ntiles = (unsigned)(t.recs * nmt_all * N);
+        a.ngrp = (unsigned)((t.runs + 3) / 4);
+    }
     // ---- weights ----
     int npairs_all = 0;
     for (int b0 = 0; b0 < a.nbt; b0 += a.CB) npairs_all += (27 * (a.nbt - b0 < a.CB ? a.nbt - b0 : a.CB) + 1) >> 1;
@@ -807,7 +831,7 @@ static size_t conv_scratch_bound(int fmt, const void *x2, int xbf, int ybf, shap
         if (!direct) need += al((size_t)N * ((C + 31) / 32) * S * 33);
         if (upseg) need += al((size_t)N * ((C + 31) / 32) * (S / 8) * 33);
     }
-    const size_t thin_recs = (So + 63) / 64 * nmt_all * N <= (size_t)(g_thin > 1024 ? g_thin : 1024) ? mi_thin_runs(sp.Di ? sp.zi0 : 0, xs.d, xs.h, xs.w).recs * nmt_all * N : 0;      // (the K-split kernel's, 64 bytes each: a few more than its runs)
+    const size_t thin_recs = xs.w <= flat_t<8>::WMAX || (So + 63) / 64 * nmt_all * N <= (size_t)(g_thin > 1024 ? g_thin : 1024) ? mi_thin_runs(sp.Di ? sp.zi0 : 0, xs.d, xs.h, xs.w).recs * nmt_all * N : 0;      // (the K-split kernel's, 64 bytes each: a few more than its runs)
     if (osum) need += al((tiles * 256 > thin_recs * 64 ? tiles * 256 : thin_recs * 64));
     return need;
 }

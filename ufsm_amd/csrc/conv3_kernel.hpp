@@ -122,6 +122,7 @@ struct conv_args {
     bool row;                          // the row kernel (one channel tile, any number of input blocks, 4 x 8 x 32 voxel tiles) takes the launch
     bool row1;                         // ... its one-input-block form (weights in registers, the two halves of the workgroup half a tile apart)
     bool thin;                         // the K-split kernel of the launches of few output voxels takes the launch
+    bool flat;                         // ... the one of about a tile of 128 voxels x 64 channels per CU (flat runs, the taps split over the wavefronts)
 };
 
 template <int FMT> struct fmt_t;
@@ -664,9 +665,11 @@ static void launch_conv(const conv_args &a, size_t smem) {
 #include "conv3_row.hpp"
 #include "conv3_row1.hpp"
 #include "conv3_thin.hpp"
+#include "conv3_flat.hpp"
 template <int FMT, int STRIDE, int OUT, bool EPI>
 static void launch_mt(int MT, int NT, const conv_args &a, size_t smem) {
     if constexpr (!EPI) { if (a.thin) { launch_thin<FMT, STRIDE, OUT>(a, smem); return; } }
+    if constexpr (!EPI && STRIDE == 1) { if (a.flat) { launch_flat<FMT, OUT>(a, smem); return; } }
     switch (MT * 10 + NT) {
     case 44: if constexpr (STRIDE == 1) launch_wide<FMT, OUT, EPI>(a, smem); else mi_die("conv3: the wide kernel is stride 1 only"); break;
     // (one-plane tiles, stride 2 only: its halo is 8 input positions per output, and a 3 x 17 x 33 halo lets two workgroups share a CU)
