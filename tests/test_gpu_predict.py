@@ -60,6 +60,13 @@ def test_feather_blend_is_bit_exact(gpu, S, B, nss, bn, absent):
     assert lib.mi_feather_blend(dE.ptr, dp.ptr, S, S + 1, nss_a, bn_a, do.ptr) == -1     # B > S: refused
 
 
+# steps and widths of whole runs of 8: a core of one run, none, rows that end inside a run or start at any byte, cells without a left, upper or present neighbour
+@pytest.mark.parametrize("S,B,nss,bn,absent", [(16, 8, (2, 2, 3), (31, 32, 43), [4]), (24, 16, (2, 3, 2), (40, 70, 47), [0, 7]), (8, 8, (3, 3, 3), (24, 19, 17), [13]),
+                                                (40, 0, (1, 1, 2), (7, 40, 41), []), (64, 16, (1, 2, 2), (20, 100, 127), [3])])
+def test_feather_blend_by_runs_is_bit_exact(gpu, S, B, nss, bn, absent):
+    test_feather_blend_is_bit_exact(gpu, S, B, nss, bn, absent)
+
+
 @pytest.mark.parametrize("W", [24, 32])          # rows of 24 voxels are stored byte by byte, rows of a multiple of 16 as 16-byte vectors
 def test_ct_window_gather(gpu, W):
     rng = np.random.default_rng(9)
