@@ -62,7 +62,7 @@ def test_feather_blend_is_bit_exact(gpu, S, B, nss, bn, absent):
 
 # steps and widths of whole runs of 8: a core of one run, none, rows that end inside a run or start at any byte, cells without a left, upper or present neighbour
 @pytest.mark.parametrize("S,B,nss,bn,absent", [(16, 8, (2, 2, 3), (31, 32, 43), [4]), (24, 16, (2, 3, 2), (40, 70, 47), [0, 7]), (8, 8, (3, 3, 3), (24, 19, 17), [13]),
-                                                (40, 0, (1, 1, 2), (7, 40, 41), []), (64, 16, (1, 2, 2), (20, 100, 127), [3])])
+                                                (40, 0, (1, 1, 2), (7, 40, 41), []), (64, 16, (1, 2, 2), (20, 100, 127), [3]), (128, 128, (1, 1, 2), (5, 9, 200), []), (136, 136, (1, 1, 2), (5, 9, 200), [])])
 def test_feather_blend_by_runs_is_bit_exact(gpu, S, B, nss, bn, absent):
     test_feather_blend_is_bit_exact(gpu, S, B, nss, bn, absent)
 

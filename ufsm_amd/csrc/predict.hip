@@ -1,6 +1,7 @@
 // Sliding-window prediction: logits -> uint8 placement (src/nn_elem.cu:1103-1130 of the reference), window gather from a resident volume,
 // and the feather blend of window borders (src/predict.c:282-333) as a device kernel over the whole output box. All HBM-bound byte work.
 #include <math.h>
+#include <string.h>
 #include "mx_dev.hpp"
 #include "../../include/mi_predict.h"
 
@@ -156,9 +157,13 @@ extern "C" void mi_ct_flags(const uint8_t *vol, int64_t Z, int64_t Y, int64_t X,
 }
 
 struct blend_geo { int S, B, En; long long n0, n1, n2, b0, b1, b2; };
+// the blend's weights u(j), 1 - u(j): in the launch's arguments up to a width of BLEND_ARG (no copy to wait for), else [2][1024] in device memory
+constexpr int BLEND_ARG = 128;
+struct blend_u { const float *p; float v[2][BLEND_ARG]; };
+__device__ __forceinline__ float blend_w(const blend_u &u, int q, int j) { return u.p ? u.p[q * 1024 + j] : u.v[q][j]; }
 // one thread per output voxel. Core voxels (the bulk) copy a byte; shell voxels gather up to eight windows in the reference's order
 // (delta = 0 first, then bit 0 x, bit 1 y, bit 2 z) with separately rounded fp32 products and sums, as the host routine computes them.
-__global__ void __launch_bounds__(256) feather_blend_k(const uint8_t *__restrict__ E, const uint8_t *__restrict__ present, blend_geo G, const float *__restrict__ u,
+__global__ void __launch_bounds__(256) feather_blend_k(const uint8_t *__restrict__ E, const uint8_t *__restrict__ present, blend_geo G, const blend_u u,
                                                        uint8_t *__restrict__ out) {
 #pragma clang fp contract(off)       // products and sums round separately, as the host routine's do (no fused multiply-add)
     const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
@@ -179,7 +184,7 @@ __global__ void __launch_bounds__(256) feather_blend_k(const uint8_t *__restrict
         const long long qid = (qa * G.n1 + qb) * G.n2 + qc;
         if (d && !present[qid]) continue;
         if ((dz && z >= B) || (dy && y >= B) || (dx && x >= B)) continue;
-        const float wz = z < B ? u[dz * 1024 + z] : 1.f, wy = y < B ? u[dy * 1024 + y] : 1.f, wx = x < B ? u[dx * 1024 + x] : 1.f;
+        const float wz = z < B ? blend_w(u, dz, z) : 1.f, wy = y < B ? blend_w(u, dy, y) : 1.f, wx = x < B ? blend_w(u, dx, x) : 1.f;
         const float wi = (wz * wy) * wx;
         const float v = (float)E[(size_t)qid * e3 + ((size_t)(z + dz * G.S) * En + (y + dy * G.S)) * En + (x + dx * G.S)];
         s += wi * v; w += wi;
@@ -189,7 +194,7 @@ __global__ void __launch_bounds__(256) feather_blend_k(const uint8_t *__restrict
 // the same for window steps and blend widths of whole runs of 8 (windows of 64 / 96 / 128 with halo 16, blend 16): a thread owns 8 consecutive x of a row, which
 // share cell, presence and - inside the shell or outside it - the windows they gather; 8 bytes per window at a time. Bound by the bytes' arithmetic in the
 // shell (42 % of the voxels at step 96, blend 16: up to eight windows, a quotient each); 190 x 280 x 260: 111 us one voxel per thread, 27 so
-__global__ void __launch_bounds__(256) feather_runs_k(const uint8_t *__restrict__ E, const uint8_t *__restrict__ present, blend_geo G, unsigned nrun, unsigned nthreads, const float *__restrict__ u,
+__global__ void __launch_bounds__(256) feather_runs_k(const uint8_t *__restrict__ E, const uint8_t *__restrict__ present, blend_geo G, unsigned nrun, unsigned nthreads, const blend_u u,
                                                       uint8_t *__restrict__ out) {
 #pragma clang fp contract(off)
     const unsigned i = blockIdx.x * 256u + threadIdx.x;
@@ -212,11 +217,11 @@ __global__ void __launch_bounds__(256) feather_runs_k(const uint8_t *__restrict_
                 if ((dz && (z >= B || !a)) || (dy && (y >= B || !b)) || (dx && (x >= B || !c))) continue;
                 const long long qid = (((long long)a - dz) * G.n1 + ((long long)b - dy)) * G.n2 + ((long long)c - dx);
                 if (d && !present[qid]) continue;
-                const float wz = z < B ? u[dz * 1024 + z] : 1.f, wy = y < B ? u[dy * 1024 + y] : 1.f, wzy = wz * wy;
+                const float wz = z < B ? blend_w(u, dz, z) : 1.f, wy = y < B ? blend_w(u, dy, y) : 1.f, wzy = wz * wy;
                 const uint2 q = ld_any<uint2>(E + (size_t)qid * e3 + ((size_t)(z + dz * G.S) * En + (y + dy * G.S)) * En + (x + dx * G.S));
 #pragma unroll
                 for (int k = 0; k < 8; k++) {
-                    const float wx = x < B ? u[dx * 1024 + x + k] : 1.f, wi = wzy * wx, v = (float)(((k < 4 ? q.x : q.y) >> (8 * (k & 3))) & 255u);
+                    const float wx = x < B ? blend_w(u, dx, x + k) : 1.f, wi = wzy * wx, v = (float)(((k < 4 ? q.x : q.y) >> (8 * (k & 3))) & 255u);
                     s[k] += wi * v; w[k] += wi;
                 }
             }
@@ -234,18 +239,25 @@ __global__ void __launch_bounds__(256) feather_runs_k(const uint8_t *__restrict_
 extern "C" int mi_feather_blend(const uint8_t *E, const uint8_t *present, int S, int B, const int64_t nss[3], const int64_t bn[3], uint8_t *out) {
     if (S <= 0 || B < 0 || B > S || B > 1024) return -1;            // (B 0: no blend, every voxel is its window's own)
     for (int d = 0; d < 3; d++) if (nss[d] <= 0 || bn[d] <= 0 || bn[d] > nss[d] * S) return -1;
-    // u(j) = sin^2(pi/2 (j + .5) / B) and 1 - u(j) in double, rounded to fp32 (src/predict.c:337); the table lives in per-device scratch
+    // u(j) = sin^2(pi/2 (j + .5) / B) and 1 - u(j) in double, rounded to fp32 (src/predict.c:337)
+    blend_u bu; memset(&bu, 0, sizeof bu);
     static thread_local float hu[2048];
-    for (int j = 0; j < B; j++) { const double s = sin(M_PI / 2 * (j + 0.5) / B); hu[j] = (float)(s * s); hu[1024 + j] = (float)(1 - s * s); }
-    float *du = (float *)mi_ws(MI_WS_MISC, sizeof hu);
-    MIRT(hipMemcpyAsync(du, hu, sizeof hu, hipMemcpyHostToDevice, 0));
-    MIRT(hipStreamSynchronize(0));                           // (hu is reused by the next call)
+    for (int j = 0; j < B; j++) {
+        const double s = sin(M_PI / 2 * (j + 0.5) / B); const float u0 = (float)(s * s), u1 = (float)(1 - s * s);
+        if (B <= BLEND_ARG) { bu.v[0][j] = u0; bu.v[1][j] = u1; } else { hu[j] = u0; hu[1024 + j] = u1; }
+    }
+    if (B > BLEND_ARG) {
+        float *du = (float *)mi_ws(MI_WS_MISC, sizeof hu);
+        MIRT(hipMemcpyAsync(du, hu, sizeof hu, hipMemcpyHostToDevice, 0));
+        MIRT(hipStreamSynchronize(0));                           // (hu is reused by the next call)
+        bu.p = du;
+    }
     blend_geo g = {S, B, S + B, nss[0], nss[1], nss[2], bn[0], bn[1], bn[2]};
     const size_t n = (size_t)bn[0] * bn[1] * bn[2];
     // (runs and coordinates of 32 bits; a run never crosses from a cell's shell to its core or into the next cell)
     const unsigned long long nrun = ((unsigned long long)bn[2] + 7) / 8, nth = nrun * (unsigned long long)bn[0] * bn[1];
-    if (S % 8 == 0 && B % 8 == 0 && nth < (1ull << 32) - 256 && bn[2] < (1ll << 31)) feather_runs_k<<<nblk_(nth, 256), 256>>>(E, present, g, (unsigned)nrun, (unsigned)nth, du, out);
-    else feather_blend_k<<<nblk_(n, 256), 256>>>(E, present, g, du, out);
+    if (S % 8 == 0 && B % 8 == 0 && nth < (1ull << 32) - 256 && bn[2] < (1ll << 31)) feather_runs_k<<<nblk_(nth, 256), 256>>>(E, present, g, (unsigned)nrun, (unsigned)nth, bu, out);
+    else feather_blend_k<<<nblk_(n, 256), 256>>>(E, present, g, bu, out);
     MICK();
     return 0;
 }

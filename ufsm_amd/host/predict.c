@@ -5,6 +5,9 @@
 #include "../../include/mi_unet.h"
 #include "../../include/mi_predict.h"
 
+/* (unet.c) the handle's device memory for a prediction, grown on demand; 0 bytes: the prediction is over */
+void *unet_pred_ws(unet *u, size_t bytes);
+
 int mi_unet_predict_volume(unet *u, int window, int nbatch, const uint8_t *vol, const int64_t dims[3], int halo, int feather, float mean, float isd,
                            int axis, float cy, float cx, uint8_t *out, int64_t nwin[2]) {
     shape5 in = {nbatch, 4, window, window, window};
@@ -17,14 +20,17 @@ int mi_unet_predict_volume(unet *u, int window, int nbatch, const uint8_t *vol, 
     int64_t nss[3], total = 1;
     for (int d = 0; d < 3; d++) { if (dims[d] <= 0) return -1; nss[d] = (dims[d] + S - 1) / S; total *= nss[d]; }
     const size_t w3 = (size_t)W * W * W, e3 = (size_t)En * En * En;
-    uint8_t *E = mi_malloc((size_t)total * e3), *ctw = mi_malloc((size_t)in.n * w3), *dpres = mi_malloc((size_t)total);
+    /* device memory of a prediction, one piece: the windows' axis offsets and presence bytes (one copy from the host fills both), their flags, the gathered windows, E */
+    const size_t offb = (size_t)total * 2 * W * sizeof(float), o_any = (offb + (size_t)total + 255) & ~(size_t)255, o_ctw = (o_any + (size_t)total * sizeof(unsigned) + 255) & ~(size_t)255,
+                 o_E = (o_ctw + (size_t)in.n * w3 + 255) & ~(size_t)255;
+    uint8_t *const dw = unet_pred_ws(u, o_E + (size_t)total * e3), *E = dw + o_E, *ctw = dw + o_ctw, *dpres = dw + offb;
     const size_t lgn = (size_t)unet_cfg_of(u)->cout * w3;      /* logits of one window */
-    float *doff = mi_malloc((size_t)total * 2 * W * sizeof(float));
-    unsigned *dany = mi_malloc((size_t)total * sizeof(unsigned));
-    uint8_t *present = calloc((size_t)total, 1);
+    float *doff = (float *)dw;
+    unsigned *dany = (unsigned *)(dw + o_any);
     unsigned *hany = malloc((size_t)total * sizeof(unsigned));
-    float *hoff = malloc((size_t)total * 2 * W * sizeof(float));
-    int rc = present && hoff && hany ? 0 : -1;
+    float *hoff = malloc(offb + (size_t)total);
+    uint8_t *present = hoff ? (uint8_t *)hoff + offb : NULL;
+    int rc = hoff && hany ? 0 : -1;
     int64_t done = 0;
     const int iso = nn_get_pred_iso();
     /* Pass 1, no host round trip per window: every window's "holds a voxel >= iso in its interior" flag (air windows are not computed; their
@@ -39,7 +45,8 @@ int mi_unet_predict_volume(unet *u, int window, int nbatch, const uint8_t *vol, 
             for (int z = 0; z < W; z++) { ho[z] = (float)oy - cy; ho[W + z] = (float)ox - cx; }
         }
         mi_d2h(hany, dany, (size_t)total * sizeof(unsigned));
-        mi_h2d(doff, hoff, (size_t)total * 2 * W * sizeof(float));
+        for (int64_t id = 0; id < total; id++) present[id] = hany[id] != 0;
+        mi_h2d(doff, hoff, offb + (size_t)total);
     }
     /* Pass 2: the windows that hold material, in z-y-x order, in.n per forward (window j of a batch -> sample j; samples are independent, so a
      * window's prediction does not depend on its batch; a last, incomplete batch repeats its last window and places it once) */
@@ -76,18 +83,17 @@ int mi_unet_predict_volume(unet *u, int window, int nbatch, const uint8_t *vol, 
         if (!lg) { rc = -1; break; }
         /* E: the interior and B voxels of the upper halo, window coordinates [halo, halo + S + B) -> [0, S + B) (src/predict.c:3426-3427) */
         mi_pred_place_n(lg, lgn, ctw, w3, nreal, eoff, W, W, halo - B, halo - B, -halo, -halo, -halo, En, En, En, En, E);
-        for (int j = 0; j < nreal; j++) { present[list[k + j]] = 1; done++; }
+        done += nreal;
     }
     free(list); free(axrec);
     if (!rc) {
-        mi_h2d(dpres, present, (size_t)total);
         rc = mi_feather_blend(E, dpres, S, B, nss, dims, out);
         mi_sync();
         if (lp_check()) rc = -1;
     }
     if (nwin) { nwin[0] = total; nwin[1] = done; }
     mi_sync();
-    mi_free(E); mi_free(ctw); mi_free(dpres); mi_free(doff); mi_free(dany);
-    free(present); free(hoff); free(hany);
+    unet_pred_ws(u, 0);
+    free(hoff); free(hany);
     return rc;
 }

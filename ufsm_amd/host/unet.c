@@ -37,6 +37,7 @@ struct unet {
        ge_run = [live weights: ge_ns values][EMA weights: the same], per site pair [mean G | var G] in the order of gn_sites (src/unet.c:5125-5135) */
     float *ge_run; size_t ge_ns; long ge_n; int ge_warm, ge_live; float ge_mom;
     int l0s_zs, l0s_ns;                /* cfg.l0_norm 4: planes per statistics slab and slabs of the current build (0: per-sample statistics) */
+    void *pred_ws; size_t pred_cap;    /* a prediction's device memory (unet_pred_ws) */
     int slab_ip, slab_nl, slab_s;      /* the build's in-place slab plan: on, and over how many levels (a level's tensors all live in enc[i].a2's buffer) */
     void *slab_tmp[2], *slab_carry[2]; /* per such level: one slab of output planes, and the plane that waits for the next slab */
     block enc[UNET_MAXLEV], dec[UNET_MAXLEV];
@@ -368,6 +369,18 @@ static int ensure_built(unet *u, shape5 xs) {
     if (u->built && !memcmp(&u->in, &xs, sizeof xs) && u->act_dt == act_dt_now() && u->prec == nn_get_prec() && u->slab_ip == ip && (!ip || u->slab_s == g_infer_slab)) return 0;
     return build_acts(u, xs);
 }
+/* Device memory of a sliding-window prediction, grown on demand and kept in the handle between predictions: allocating and freeing it took 0.2 ms of each. At most
+   PRED_WS_KEEP stays (a volume of 18 windows of 128^3 with borders takes 44 MB): a larger piece is given back when its prediction is over (bytes 0), any with the
+   handle. A handle runs one prediction at a time, as it runs one forward */
+#define PRED_WS_KEEP ((size_t)256 << 20)
+void *unet_pred_ws(unet *u, size_t bytes) {
+    if (bytes ? bytes > u->pred_cap : u->pred_cap > PRED_WS_KEEP) {
+        if (u->pred_ws) mi_free(u->pred_ws);
+        u->pred_ws = NULL; u->pred_cap = 0;
+        if (bytes) { u->pred_ws = mi_malloc(bytes); u->pred_cap = bytes; }
+    }
+    return u->pred_ws;
+}
 void unet_free(unet *u) {
     if (!u) return;
     mi_sync();
@@ -375,6 +388,7 @@ void unet_free(unet *u) {
     mi_free(u->p); mi_free(u->ema); if (u->wm) mi_free(u->wm); if (u->l0run) mi_free(u->l0run); if (u->ge_run) mi_free(u->ge_run);
     for (int i = 0; i < UNET_MAXLEV; i++) { free(u->rb[i]); free(u->rbn[i]); }
     if (u->stem_b) mi_free(u->stem_b);
+    if (u->pred_ws) mi_free(u->pred_ws);
     free(u->tb_axh);
     if (u->gf_g) { mi_free(u->gf_g); mi_free(u->gf_g1); }
     lp_wmemo_clear();
