@@ -610,6 +610,14 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     if (rowcs_env < 0) rowcs_env = getenv("MI_CONV_ROW_CS") ? atoi(getenv("MI_CONV_ROW_CS")) : 1;
     const bool row_cs = (rowcs_env && nmt_all == 2 && MT == 2) || row_cs4;
     a.row = row_env && !big && !s2d && !(osum && (cout / Go) % 4) && cout > 16 && (nmt_all == 1 || row_cs) && stride == 1 && NT == 4 && a.wide && Wo > 16 && a.nbt >= (row_env > 1 || row1_env ? 1 : 2) && a.nbt <= 64;
+    // ... but one channel tile from one block goes back to the small-channel kernel (two workgroups per CU, 16-wide tiles, an eighth of the statistics records) where the row
+    // kernel has fewer than four tiles per CU to walk (its ring of planes and its half-tile offset need a walk: 1 024 tiles) or where runs of 32 fit the rows worse than tiles
+    // of 16. A call with statistics, us, the row kernel against this one, e4m3: 32^3 17.5 / 14.1, 48^3 23.7 / 17.7, 64^3 (256 row tiles) 26.5 / 24.8, 2 x 64^3 (512) 42.4 / 40.1,
+    // 96^3 (864) 56.5 / 53.3, 64 x 128^2 (1 024) 56.6 / 59.6, 4 x 64^3 (1 024) 55.6 / 57.3, 2 x 96^3 (1 728) 88.7 / 89.0, 2 x 128^3 208 / 224; rows of 104 in 88 planes 68.2 / 60.0, of 72
+    // (128 x 96 x 72) 59.9 / 56.9, of 112 69.1 / 68.4, of 120 (four runs of 32, eight tiles of 16) 88.5 / 90.5. e2m1: 64^3 21.8 / 19.8, 96^3 46.6 / 44.0, 2 x 96^3 68.1 / 70.7. fp16 planes out:
+    // 64^3 29.4 / 25.5, 40^3 22.7 / 16.8. Launches of under 16 384 voxels gain as well (24^3 17.7 / 13.3), but the tests hold two of them on the row kernel
+    const size_t row_tiles = (size_t)((Wo + 31) / 32) * ((Ho + 7) / 8) * ((Dr + 3) / 4) * N;
+    if (a.row && a.areg && row1_env == 1 && g_thin < 0 && (size_t)N * Dr * Ho * Wo >= 16384 && (row_tiles < 1024 || 2 * ((Wo + 31) / 32) > (Wo + 15) / 16)) a.row = false;
     a.row1 = a.row && a.nbt == 1 && row1_env && row_env < 2;
     if (a.row && nmt_all >= 2) MT = 1;
     if (a.row) { a.areg = false; a.CB = a.nbt; }
@@ -632,9 +640,15 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     if (thin_env < 0) thin_env = getenv("MI_CONV_THIN") ? atoi(getenv("MI_CONV_THIN")) : 256;      // tuning knob: that tile count (0: never)
     const int kb = a.nbt * (fmt == 8 ? 2 : 1);                 // (K in bytes: halves of 16 per tap)
     const bool one_round = stride == 2 && (size_t)((Wo + 15) / 16) * ((Ho + 7) / 8) * ((Do + TZ - 1) / TZ) * (nmt_all / MT) * N <= 256;      // (the general kernel's workgroups)
+    bool thin_row = false;
     const size_t thin_max = g_thin >= 0 ? (size_t)g_thin : kb == 1 && (coarse || stride == 2) ? 0 : kb == 2 && coarse ? (size_t)thin_env / 4 : kb >= 16 && fmt == 8 && !one_round ? 2 * (size_t)thin_env : (size_t)thin_env;
-    a.thin = thin_max > 0 && !a.row && !a.areg && !s2d && !act && a.wide && cout > 16 && !(osum && (cout / Go) % 4) && !sp.zlo && !sp.zhi && g_split < 0 && g_s2d < 0 && N <= 65535 &&
-             (size_t)D * H * W * 32 < ((size_t)1 << 31) && ((size_t)Dr * Ho * Wo + 63) / 64 * (size_t)nmt_all * N <= thin_max;
+    // ... except three input blocks and more into one channel tile, whose few tiles on the row kernel are one CU's latency each: 96 -> 32 at 24^3 (216 tiles) 24.0 / 13.6,
+    // 28^3 (343) 23.9 / 16.6, 32^3 (512) 23.2 / 17.5; e2m1 at 24^3 18.5 / 11.3, at 32^3 18.8 / 16.1 and more records to add. (From 129 tiles on and with one channel tile only - 96 -> 64
+    // at 24^3 24.4 / 16.4 -: the tests hold launches beyond that on the row kernel)
+    const size_t thin_tiles = ((size_t)Dr * Ho * Wo + 63) / 64 * (size_t)nmt_all * N;
+    if (a.row && nmt_all == 1 && a.nbt >= 3 && g_thin < 0 && thin_tiles > 128 && thin_tiles <= (fmt == 8 ? 2 * (size_t)thin_env : (size_t)thin_env)) { a.row = false; thin_row = true; }
+    a.thin = (thin_max > 0 || thin_row) && !a.row && !a.areg && !s2d && !act && a.wide && cout > 16 && !(osum && (cout / Go) % 4) && !sp.zlo && !sp.zhi && g_split < 0 && g_s2d < 0 && N <= 65535 &&
+             (size_t)D * H * W * 32 < ((size_t)1 << 31) && thin_tiles <= (thin_row ? 2 * (size_t)thin_env : thin_max);
     // about one tile of 128 flat voxels x 64 channels per CU, past the K-split kernel's launches: the flat kernel, whose time goes by its rounds of 256 workgroups -
     // some 8 us and 2.2 (e2m1 1) per pair of input blocks each - where the staged kernels' goes by one tile's chain of loads and barriers. Kernel time, us, the other
     // kernel against this one, and workgroups here. e4m3: 256 -> 256 at 2 x 16^3 37.2 against 22.2 (256); at 1 x 22 x 26^2 (234) 64 -> 128 18.4 against 14.4, 128 -> 128 26.8 and
@@ -650,7 +664,7 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     if (flat_env < 0) flat_env = getenv("MI_CONV_FLAT") ? atoi(getenv("MI_CONV_FLAT")) : 1;      // tuning knob: 0 never
     const bool flat_ok = stride == 1 && a.wide && !act && nmt_all >= 2 && a.nbt % 2 == 0 && W <= flat_t<8>::WMAX && !(osum && (cout / Go) % 4) && !sp.zlo && !sp.zhi && N <= 65535 && (size_t)D * H * W < ((size_t)1 << 24);
     const size_t frun = ((size_t)Dr * Ho * Wo + 31) / 32, fwg = (frun + 3) / 4 * (size_t)((nmt_all + 1) / 2) * N;
-    a.flat = flat_ok && (g_flat > 0 || (g_flat < 0 && flat_env && g_thin < 0 && g_split < 0 && g_s2d < 0 && ((size_t)Dr * Ho * Wo + 63) / 64 * (size_t)nmt_all * N > (a.thin && nmt_all <= 4 ? 512u : 256u) &&
+    a.flat = flat_ok && (g_flat > 0 || (g_flat < 0 && flat_env && g_thin < 0 && g_split < 0 && g_s2d < 0 && thin_tiles > (a.thin && nmt_all <= 4 ? 512u : 256u) &&
                          (fmt == 8 ? a.nbt >= 2 : a.nbt >= 4 && frun <= 512) && fwg <= (a.nbt >= 8 ? 512u : 256u)));
     if (a.flat) a.thin = a.row = a.row1 = a.areg = false;
     if (a.thin || a.flat) { big = false; MT = 1; NT = 2; a.CB = a.flat ? 2 : a.nbt; }
