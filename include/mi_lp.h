@@ -91,8 +91,9 @@ void mi_conv_stem_zc(int zc);
    slices of 64 channels, twice the workgroups; 0: never, -1: the default (192, or MI_CONV_SPLIT). The results do not depend on it. */
 void mi_conv_split(int tiles);
 /* Extension: which kernel takes the calling thread's 3x3x3 stride-2 convs on 32-channel rows. -1 (default): the kernel that reads the taps' rows
-   straight from the stored tensor when the launch has enough output voxels to fill the device, else the general kernel (staged halo);
-   0: always the general kernel; 1: the direct kernel whenever its operands allow it. The results are the same conv either way. */
+   straight from the stored tensor when the launch has enough output voxels to fill the device, else the general kernel (staged halo); one input block
+   into 17 .. 32 channels runs on a row kernel (rows staged as stored, weights in registers) on rows of more than 16 output voxels;
+   0: always the general kernel; 1: the direct kernel, 2: the row kernel whenever its operands allow it. The results are the same conv either way. */
 void mi_conv_s2_direct(int mode);
 /* Extension: up to how many tiles (64 voxels x 32 output channels, of the whole tensor) the calling thread's 3x3x3 convs may run on the kernel that splits
    the K range over a workgroup's wavefronts. -1 (default): the measured limits; 0: never. The same conv either way, its fp32 sums in another order. */

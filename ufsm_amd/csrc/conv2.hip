@@ -5,6 +5,8 @@
 bool mi_wmemo_other(unsigned key, const float *w, int fmt, int Co, int Ci, int nmt_all, int lay, size_t wq_bytes, size_t wsc_bytes, uint8_t **wq, uint8_t **wsc);     // conv3.hip
 unsigned mi_take_s2_wkey(void);
 
+size_t conv3s2_row_lds(int fmt) { return fmt == 8 ? s2row_t<8>::LDS : s2row_t<4>::LDS; }
+
 // weights -> the MFMA's lane order, one tile per (K pair, channel tile) as the 3x3x3 kernels read them. down: w [Co][Ci][8], pair gp = units 2 gp,
 // 2 gp + 1 of the tap-major (tap, block) order; up: w [Ci][Co][8], pair gp = (tap gp / npt, blocks 2 (gp % npt), + 1), a missing second block = zeros
 template <int FMT>

@@ -265,8 +265,10 @@ static void launch_conv3s2_mt(const conv_args &a, dim3 grid, size_t smem) {
     MICK();
     snprintf(g_last_kernel, sizeof g_last_kernel, "conv3s2_mx_k<fmt %d, out %d, MT %d> blocks %d grid %u x %u x %u", FMT, OUT, MT, a.nbt, grid.x, grid.y, grid.z);
 }
+#include "conv3s2_row.hpp"
 template <int FMT>
 static void launch_conv3s2(int out, int MT, const conv_args &a, dim3 grid, size_t smem) {
+    if (a.s2row) { if (out == 8) launch_s2row<FMT, 8>(a, smem); else if (out == 4) launch_s2row<FMT, 4>(a, smem); else launch_s2row<FMT, 0>(a, smem); return; }
 #define C3S2_MT(OUT) do { if (MT == 4) launch_conv3s2_mt<FMT, OUT, 4>(a, grid, smem); else if (MT == 2) launch_conv3s2_mt<FMT, OUT, 2>(a, grid, smem); else launch_conv3s2_mt<FMT, OUT, 1>(a, grid, smem); } while (0)
     if (out == 8) C3S2_MT(8); else if (out == 4) C3S2_MT(4); else C3S2_MT(0);
 #undef C3S2_MT

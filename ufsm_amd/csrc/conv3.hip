@@ -538,8 +538,15 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     const size_t s2runs = ((size_t)Do * Ho * Wo + 63) / 64;
     // (by default only one input block and one channel tile, the shape it is measured faster on: 64 -> 64 takes 0.034 against 0.030 ms from 2 x 64^3
     // and 0.36 against 0.09 ms from 8 x 64^3)
-    const bool s2d = s2d_env && g_s2d != 0 && stride == 2 && a.wide && !act && N <= 65535 &&
-                     (g_s2d > 0 || (a.nbt == 1 && nmt_all == 1 && (s2runs + 3) / 4 * N >= (size_t)s2d_env * 128));
+    // ... on rows of more than 16 output voxels the row kernel does: the tile's rows staged in LDS as they lie in memory, the weights in registers. us, general / direct / row kernel,
+    // e4m3: 2 x 128^3 85.8 / 59.0 / 43.6, 9 x 128^3 364 / 278 / 170, 88 x 104^2 30.8 / 19.1 / 13.8, 64^3 8.3 / 12.6 / 7.5; e2m1: 128^3 19.7 / 28.1 / 15.9, 2 x 96^3 17.0 / 28.0 / 16.4, 48^3 6.6 / 12.5 / 6.3. On rows of
+    // 16 and fewer half its lanes idle (4 x 64^2 x 32: 10.8 general, 13.7); up to 256 tiles of the K-split kernel e4m3 stays there (48^3 7.2 / 7.8 here, 32 x 64^2 7.4 / 7.7)
+    static int s2row_env = -1;
+    if (s2row_env < 0) s2row_env = getenv("MI_CONV_S2ROW") ? atoi(getenv("MI_CONV_S2ROW")) : 1;      // tuning knob: 0 never
+    a.s2row = stride == 2 && a.nbt == 1 && nmt_all == 1 && cout > 16 && a.wide && !act && S < ((size_t)1 << 31) && (size_t)((Wo + 31) / 32) * ((Ho + 3) / 4) * Do * N < ((size_t)1 << 31) &&
+              (g_s2d == 2 || (g_s2d < 0 && s2row_env && Wo > 16 && (fmt == 4 || s2runs * N > 256)));
+    const bool s2d = a.s2row || (s2d_env && g_s2d != 0 && stride == 2 && a.wide && !act && N <= 65535 &&
+                     (g_s2d > 0 || (a.nbt == 1 && nmt_all == 1 && (s2runs + 3) / 4 * N >= (size_t)s2d_env * 128)));
     if (s2d) {
         MT = nmt_all % 4 == 0 ? 4 : nmt_all % 2 == 0 ? 2 : 1;
         while (MT > 1 && (s2runs + 3) / 4 * (size_t)(nmt_all / MT) * N < 512) MT >>= 1;
@@ -669,17 +676,17 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     if (a.flat) a.thin = a.row = a.row1 = a.areg = false;
     if (a.thin || a.flat) { big = false; MT = 1; NT = 2; a.CB = a.flat ? 2 : a.nbt; }
     size_t smem = a.flat ? (size_t)(fmt == 8 ? flat_t<8>::LDS : flat_t<4>::LDS) : a.thin ? MI_THIN_LDS : a.row1 ? (size_t)10 * 352 * (RB + 4) : a.row ? (size_t)2 * 2048 * (RB + 4) : a.areg ? (size_t)2 * ((TT + 63) / 64 * 64) * (RB + 4) : big ? (size_t)4 * MT * (WTILE + 256) + (size_t)3 * ((TT + 63) / 64 * 64) * (RB + 4) + (size_t)(((27 * a.nbt + 1) >> 1) + 2) * 32 : lds_bytes(a.CB);
-    if (s2d) smem = 0;
+    if (s2d) smem = a.s2row ? conv3s2_row_lds(fmt) : 0;
     smem = (smem + 15) & ~(size_t)15;
     a.epi_o = (unsigned)smem; smem += (size_t)3 * (a.flat ? 2 : MT) * 32 * sizeof(float);      // bias, affine a, b of the workgroup's channels
     a.red_o = (unsigned)smem; smem += a.row1 ? 3 * 2048 + 3 * 1024 : 1024;      // statistics scratch (the one-block row kernel: the weight fragments of two tap classes instead)
-    if (s2d) smem += (size_t)(27 * a.nbt + 1 + 8) * sizeof(int);                // the direct stride-2 kernel's K-order table
+    if (s2d && !a.s2row) smem += (size_t)(27 * a.nbt + 1 + 8) * sizeof(int);                // the direct stride-2 kernel's K-order table
     // the row kernel in e2m1: the prepared weights of up to four input blocks stay in LDS (MI_CONV_ROW_WL=0: loaded from global memory per tap class)
     static int wl_env = -1;
     if (wl_env < 0) wl_env = getenv("MI_CONV_ROW_WL") ? atoi(getenv("MI_CONV_ROW_WL")) : 1;
     a.wl_o = 0;
     if (a.row && !a.row1 && fmt == 4 && wl_env && smem + (size_t)a.nbt * 15 * 1280 <= 160 * 1024) { a.wl_o = (unsigned)smem; smem += (size_t)a.nbt * 15 * 1280; }
-    if (big || a.areg || a.row) {
+    if (big || a.areg || a.row || a.s2row) {
         // rows and scale bytes of positions outside the volume: 64 zero bytes, then 64 bytes of value 1; one page per device, kept for the process
         // (the entry point that must not allocate keeps its own at the head of its fixed scratch)
         static uint8_t *zpage[8];
@@ -703,6 +710,7 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
         a.zc = t.off; a.ntx = t.step; a.nty = (int)t.recs; a.ntz = (int)t.runs; a.ntiles = (unsigned)(t.recs * nmt_all * N);
         a.ngrp = (unsigned)((t.runs + 3) / 4);
     }
+    if (a.s2row) { a.ntx = (Wo + 31) / 32; a.nty = (Ho + 3) / 4; a.ntz = Do; a.ntiles = (unsigned)((size_t)a.ntx * a.nty * Do * N); }
     // ---- weights ----
     int npairs_all = 0;
     for (int b0 = 0; b0 < a.nbt; b0 += a.CB) npairs_all += (27 * (a.nbt - b0 < a.CB ? a.nbt - b0 : a.CB) + 1) >> 1;

@@ -122,6 +122,7 @@ struct conv_args {
     bool row;                          // the row kernel (one channel tile, any number of input blocks, 4 x 8 x 32 voxel tiles) takes the launch
     bool row1;                         // ... its one-input-block form (weights in registers, the two halves of the workgroup half a tile apart)
     bool thin;                         // the K-split kernel of the launches of few output voxels takes the launch
+    bool s2row;                        // the stride-2 row kernel takes the launch (one block, one channel tile)
     bool flat;                         // ... the one of about a tile of 128 voxels x 64 channels per CU (flat runs, the taps split over the wavefronts)
 };
 
@@ -708,6 +709,7 @@ __host__ __device__ __forceinline__ bool mi_s2_unit(int gp, int side, int nb, in
     *tap = row * 3 + kx; *blk = b;
     return ok;
 }
+size_t conv3s2_row_lds(int fmt);
 void conv3s2_launch_f8(int out, int MT, const conv_args &a, dim3 grid, size_t smem);      // (the direct stride-2 kernel: conv2_kernel.hpp)
 void conv3s2_launch_f4(int out, int MT, const conv_args &a, dim3 grid, size_t smem);
 #define CONV3_LAUNCH_DECL(FMT, OUT) void conv3_launch_f##FMT##_o##OUT(int stride, bool epi, int MT, int NT, const conv_args &a, size_t smem)
