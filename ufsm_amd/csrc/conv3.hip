@@ -350,7 +350,7 @@ static int conv_stem(const char *who, const void *x, int xbf, shape5 xs, const f
     const int nmt_all = (cout + 31) / 32, MT = nmt_all % 2 == 0 && CP && CP < 16 && !(osum && (cout / Go) % 4) ? 2 : 1;
     size_t smem = rows ? (size_t)720 * 16 + 16 + 40 * 4 + 16 * 8 : ((size_t)720 * CP + 16 + CP * 8 + 15) & ~(size_t)15;     // staged tile, (zero row, row words | amax word), channel affine
     if (a.sns > 1) smem += (size_t)(a.sns - 1) * (rows ? 16 : CP) * 8;      // (one affine table per slab)
-    a.epi_o = (unsigned)smem; smem += (size_t)3 * (a.flat ? 2 : MT) * 32 * sizeof(float);
+    a.epi_o = (unsigned)smem; smem += (size_t)3 * MT * 32 * sizeof(float);
     a.red_o = (unsigned)smem; smem += 1024;
     a.nmt_all = nmt_all; a.ncs = nmt_all / MT;
     a.ntx = (W + 15) / 16; a.nty = (H + 7) / 8; a.ntz = (Do + 1) / 2;
@@ -405,6 +405,8 @@ static thread_local int g_thin = -1;        // mi_conv_thin: the calling thread'
 extern "C" void mi_conv_thin(int tiles) { g_thin = tiles; }
 static thread_local int g_flat = -1;        // mi_conv_flat: whether the calling thread's convs run on the flat kernel wherever it can (1), nowhere (0), or by size (-1)
 extern "C" void mi_conv_flat(int mode) { g_flat = mode; }
+static thread_local bool g_records = false;  // mi_conv_keep_records: the calling thread's convs with statistics keep to the kernels whose records a network's logits were made with
+extern "C" int mi_conv_keep_records(int on) { const int was = g_records; g_records = on != 0; return was; }
 static int split_s2_env() { static int v = -1; if (v < 0) v = getenv("MI_CONV_SPLIT_S2") ? atoi(getenv("MI_CONV_SPLIT_S2")) : 1; return v; }      // tuning knob: 0 keeps four channel tiles
 static int conv_dispatch(const char *who, int fmt, int stride, const void *x, int xbf, shape5 xs, const float *w, const float *b, int cout, void *y, int ybf,
                          gnp_t gp, double *osum, int Go, split_t sp, const float *ep_a, const float *ep_b, int act) {
@@ -623,8 +625,12 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     // 96^3 (864) 56.5 / 53.3, 64 x 128^2 (1 024) 56.6 / 59.6, 4 x 64^3 (1 024) 55.6 / 57.3, 2 x 96^3 (1 728) 88.7 / 89.0, 2 x 128^3 208 / 224; rows of 104 in 88 planes 68.2 / 60.0, of 72
     // (128 x 96 x 72) 59.9 / 56.9, of 112 69.1 / 68.4, of 120 (four runs of 32, eight tiles of 16) 88.5 / 90.5. e2m1: 64^3 21.8 / 19.8, 96^3 46.6 / 44.0, 2 x 96^3 68.1 / 70.7. fp16 planes out:
     // 64^3 29.4 / 25.5, 40^3 22.7 / 16.8. Launches of under 16 384 voxels gain as well (24^3 17.7 / 13.3), but the tests hold two of them on the row kernel
+    // A conv's fp32 statistics records add up in another order on another kernel, which moves a mean or 1 / std by its last bit now and then; a code of the next conv's rows at a rounding
+    // boundary then moves, and with it the rest of a network (e4m3: up to 2 % of the logits, one window size in ten; e2m1 more). Inside a network the three rules that came with the
+    // flat kernel (this one, the short 96 -> 32 walks and the flat tiles) therefore leave convs with statistics where they were
+    const bool rec = g_records && osum;
     const size_t row_tiles = (size_t)((Wo + 31) / 32) * ((Ho + 7) / 8) * ((Dr + 3) / 4) * N;
-    if (a.row && a.areg && row1_env == 1 && g_thin < 0 && (size_t)N * Dr * Ho * Wo >= 16384 && (row_tiles < 1024 || 2 * ((Wo + 31) / 32) > (Wo + 15) / 16)) a.row = false;
+    if (a.row && a.areg && row1_env == 1 && !rec && g_thin < 0 && (size_t)N * Dr * Ho * Wo >= 16384 && (row_tiles < 1024 || 2 * ((Wo + 31) / 32) > (Wo + 15) / 16)) a.row = false;
     a.row1 = a.row && a.nbt == 1 && row1_env && row_env < 2;
     if (a.row && nmt_all >= 2) MT = 1;
     if (a.row) { a.areg = false; a.CB = a.nbt; }
@@ -653,7 +659,7 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     // 28^3 (343) 23.9 / 16.6, 32^3 (512) 23.2 / 17.5; e2m1 at 24^3 18.5 / 11.3, at 32^3 18.8 / 16.1 and more records to add. (From 129 tiles on and with one channel tile only - 96 -> 64
     // at 24^3 24.4 / 16.4 -: the tests hold launches beyond that on the row kernel)
     const size_t thin_tiles = ((size_t)Dr * Ho * Wo + 63) / 64 * (size_t)nmt_all * N;
-    if (a.row && nmt_all == 1 && a.nbt >= 3 && g_thin < 0 && thin_tiles > 128 && thin_tiles <= (fmt == 8 ? 2 * (size_t)thin_env : (size_t)thin_env)) { a.row = false; thin_row = true; }
+    if (a.row && nmt_all == 1 && a.nbt >= 3 && !rec && g_thin < 0 && thin_tiles > 128 && thin_tiles <= (fmt == 8 ? 2 * (size_t)thin_env : (size_t)thin_env)) { a.row = false; thin_row = true; }
     a.thin = (thin_max > 0 || thin_row) && !a.row && !a.areg && !s2d && !act && a.wide && cout > 16 && !(osum && (cout / Go) % 4) && !sp.zlo && !sp.zhi && g_split < 0 && g_s2d < 0 && N <= 65535 &&
              (size_t)D * H * W * 32 < ((size_t)1 << 31) && thin_tiles <= (thin_row ? 2 * (size_t)thin_env : thin_max);
     // about one tile of 128 flat voxels x 64 channels per CU, past the K-split kernel's launches: the flat kernel, whose time goes by its rounds of 256 workgroups -
@@ -671,7 +677,7 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     if (flat_env < 0) flat_env = getenv("MI_CONV_FLAT") ? atoi(getenv("MI_CONV_FLAT")) : 1;      // tuning knob: 0 never
     const bool flat_ok = stride == 1 && a.wide && !act && nmt_all >= 2 && a.nbt % 2 == 0 && W <= flat_t<8>::WMAX && !(osum && (cout / Go) % 4) && !sp.zlo && !sp.zhi && N <= 65535 && (size_t)D * H * W < ((size_t)1 << 24);
     const size_t frun = ((size_t)Dr * Ho * Wo + 31) / 32, fwg = (frun + 3) / 4 * (size_t)((nmt_all + 1) / 2) * N;
-    a.flat = flat_ok && (g_flat > 0 || (g_flat < 0 && flat_env && g_thin < 0 && g_split < 0 && g_s2d < 0 && thin_tiles > (a.thin && nmt_all <= 4 ? 512u : 256u) &&
+    a.flat = flat_ok && (g_flat > 0 || (g_flat < 0 && flat_env && !rec && g_thin < 0 && g_split < 0 && g_s2d < 0 && thin_tiles > (a.thin && nmt_all <= 4 ? 512u : 256u) &&
                          (fmt == 8 ? a.nbt >= 2 : a.nbt >= 4 && frun <= 512) && fwg <= (a.nbt >= 8 ? 512u : 256u)));
     if (a.flat) a.thin = a.row = a.row1 = a.areg = false;
     if (a.thin || a.flat) { big = false; MT = 1; NT = 2; a.CB = a.flat ? 2 : a.nbt; }

@@ -788,7 +788,7 @@ static int rblock_fwd(unet *u, block *b, block *prev, const char (*nm)[16]) {
     return 0;
 }
 /* the graph on the MX input tensor x (src/unet.c:2939-3105) */
-static int graph_fwd(unet *u, const void *x, float *logits) {
+static int graph_convs(unet *u, const void *x, float *logits) {
     static const char *en1[] = {"enc0.c1", "enc1.c1", "enc2.c1", "enc3.c1", "enc4.c1", "enc5.c1", "enc6.c1", "enc7.c1"}, *en2[] = {"enc0.c2", "enc1.c2", "enc2.c2", "enc3.c2", "enc4.c2", "enc5.c2", "enc6.c2", "enc7.c2"};
     static const char *dn1[] = {"dec0.c1", "dec1.c1", "dec2.c1", "dec3.c1", "dec4.c1", "dec5.c1", "dec6.c1"}, *dn2[] = {"dec0.c2", "dec1.c2", "dec2.c2", "dec3.c2", "dec4.c2", "dec5.c2", "dec6.c2"};
     static const char *dwn[] = {"down0", "down1", "down2", "down3", "down4", "down5", "down6"};
@@ -849,6 +849,12 @@ static int graph_fwd(unet *u, const void *x, float *logits) {
     const nn_gn_t g = gn_out(u, last);
     lp_conv1_fwd_mx(last->a2, u->act_dt == 4 ? 4 : 3, last->ys, P(u, u->head.w), P(u, u->head.b), u->cfg.cout, logits, gnp_mk(g.gamma, g.beta, g.mean, g.rstd, g.G));
     return 0;
+}
+/* the logits of a window are the same bits whatever kernels later convs of their sizes are given: its statistics keep their records (mi_conv_keep_records) */
+static int graph_fwd(unet *u, const void *x, float *logits) {
+    const int was = mi_conv_keep_records(1), rc = graph_convs(u, x, logits);
+    mi_conv_keep_records(was);
+    return rc;
 }
 /* every exit of a forward passes here: the caller's tensor leaves the storage registry again (a stale range would make a later allocation
    inside it look like MX storage) */

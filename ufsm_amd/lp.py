@@ -48,6 +48,7 @@ _PROTOS = {
     "mi_conv_s2_direct": (None, [C.c_int]),
     "mi_conv_thin": (None, [C.c_int]),
     "mi_conv_flat": (None, [C.c_int]),
+    "mi_conv_keep_records": (C.c_int, [C.c_int]),
     "mi_conv1_matrix": (None, [C.c_int]),
     "mi_conv_prestage": (_I, [_P, _I, shape5, gnp_t, _P, _I]),
     "mi_conv_prestage2": (_I, [_P, shape5, gnp_t, _P, _P]),
