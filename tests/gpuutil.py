@@ -31,8 +31,8 @@ def out_dims(D, H, W, stride):
 
 
 def gpu_conv(xq, xdt, N, Ci, D, H, W, w, b, Co, ydt, cbits=8, stride=1, x2=None, c_split=0, up=0, gp=None, gp2=None, Go=0, stats=False,
-             stored_stats=0, wkey=0, fused=None):
-    """xq / x2: host arrays holding the input as stored (MX bytes, fp32 or fp16 planes). Returns (y host array, sums [N][Go][2] or None)."""
+             stored_stats=0, wkey=0, fused=None, zrange=(0, 0)):
+    """xq / x2: host arrays holding the input as stored (MX bytes, fp32 or fp16 planes). zrange: planes at either end that the statistics leave out. Returns (y host array, sums [N][Go][2] or None)."""
     dxq = DevBuf.from_numpy(xq)
     dx2 = DevBuf.from_numpy(x2) if x2 is not None else None
     dw = DevBuf.from_numpy(w.astype(np.float32))
@@ -51,6 +51,7 @@ def gpu_conv(xq, xdt, N, Ci, D, H, W, w, b, Co, ydt, cbits=8, stride=1, x2=None,
     if gp2 is not None:
         sp.gp2 = gp2
     sp.stored_stats, sp.wkey = stored_stats, wkey
+    sp.zlo, sp.zhi = zrange
     g = gp if gp is not None else gnp_t()
     xs = shape5(N, Ci, D, H, W)
     bp = db.ptr if db is not None else None

@@ -4,7 +4,8 @@ import pytest
 
 from ufsm_amd import lib
 import orc
-from test_gpu_conv import exact_case, gpu_conv
+from gpuutil import code_mismatch_fraction
+from test_gpu_conv import exact_case, rand_case, gpu_conv
 
 pytestmark = pytest.mark.gpu
 
@@ -30,3 +31,39 @@ def test_default_rule_at_its_edges(gpu, bits, N, Ci, Co, D, H, W, kern):
     assert kern in lib.mi_last_kernel().decode(), lib.mi_last_kernel().decode()
     want, _ = orc.conv3(xq, xdt, N, Ci, D, H, W, w, b, Co, xdt, cbits=bits, acc64=1)
     assert np.array_equal(got, want)
+
+
+# (bits, input channels): three blocks; four of e4m3 and seven of e2m1, whose halo chunk would not fit LDS in one piece on the general kernel
+@pytest.mark.parametrize("bits,Ci", [(8, 96), (8, 128), (4, 96), (4, 224)])
+@pytest.mark.parametrize("call", ["act", "split", "range"])
+def test_few_tiles_that_the_k_split_kernel_does_not_take(gpu, bits, Ci, call):
+    """three blocks and more into one channel tile of 129 tiles and more go to the K-split kernel by default; a call it cannot run stays on the row kernel"""
+    rng = np.random.default_rng(Ci + bits)
+    N, Co, D, H, W, G, xdt = 1, 32, 9, 30, 31, 8, 3 if bits == 8 else 4
+    x, w, b = (rand_case if call == "act" else exact_case)(rng, N, Ci, Co, D * H * W)
+    xq = orc.f32_to_mx(bits, x, N, Ci, D * H * W)
+    if call == "act":
+        got = []
+        for thin in (-1, 0):
+            lib.mi_conv_thin(thin)
+            try:
+                got.append(gpu_conv(xq, xdt, N, Ci, D, H, W, w, b, Co, xdt, cbits=bits, fused=(1, None, None))[0])
+            finally:
+                lib.mi_conv_thin(-1)
+            assert "conv3_row_k" in lib.mi_last_kernel().decode(), lib.mi_last_kernel().decode()
+        assert np.array_equal(got[0], got[1])
+        want, _ = orc.conv3(xq, xdt, N, Ci, D, H, W, w, b, Co, xdt, cbits=bits, fused_act=1)
+        assert code_mismatch_fraction(bits, got[0], want, N, Co, D * H * W)[1]
+        return
+    zr = (2, 3) if call == "range" else (0, 0)
+    if call == "split":
+        lib.mi_conv_split(0)
+    try:
+        got, gs = gpu_conv(xq, xdt, N, Ci, D, H, W, w, b, Co, xdt, cbits=bits, Go=G, stats=True, zrange=zr)
+    finally:
+        lib.mi_conv_split(-1)
+    assert "conv3_row_k" in lib.mi_last_kernel().decode(), lib.mi_last_kernel().decode()
+    want, _ = orc.conv3(xq, xdt, N, Ci, D, H, W, w, b, Co, xdt, cbits=bits, acc64=1)
+    f, _ = orc.conv3(xq, xdt, N, Ci, D, H, W, w, b, Co, 0, cbits=bits, acc64=1)
+    v = f.reshape(N, G, Co // G, D, H * W)[:, :, :, zr[0]:D - zr[1]].astype(np.float64)
+    assert np.array_equal(got, want) and np.allclose(gs, np.stack([v.sum((2, 3, 4)), (v * v).sum((2, 3, 4))], -1), rtol=1e-6)

@@ -653,15 +653,16 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     if (thin_env < 0) thin_env = getenv("MI_CONV_THIN") ? atoi(getenv("MI_CONV_THIN")) : 256;      // tuning knob: that tile count (0: never)
     const int kb = a.nbt * (fmt == 8 ? 2 : 1);                 // (K in bytes: halves of 16 per tap)
     const bool one_round = stride == 2 && (size_t)((Wo + 15) / 16) * ((Ho + 7) / 8) * ((Do + TZ - 1) / TZ) * (nmt_all / MT) * N <= 256;      // (the general kernel's workgroups)
-    bool thin_row = false;
     const size_t thin_max = g_thin >= 0 ? (size_t)g_thin : kb == 1 && (coarse || stride == 2) ? 0 : kb == 2 && coarse ? (size_t)thin_env / 4 : kb >= 16 && fmt == 8 && !one_round ? 2 * (size_t)thin_env : (size_t)thin_env;
     // ... except three input blocks and more into one channel tile, whose few tiles on the row kernel are one CU's latency each: 96 -> 32 at 24^3 (216 tiles) 24.0 / 13.6,
     // 28^3 (343) 23.9 / 16.6, 32^3 (512) 23.2 / 17.5; e2m1 at 24^3 18.5 / 11.3, at 32^3 18.8 / 16.1 and more records to add. (From 129 tiles on and with one channel tile only - 96 -> 64
     // at 24^3 24.4 / 16.4 -: the tests hold launches beyond that on the row kernel)
+    // thin_ok: what the K-split kernel can take; a call it cannot - an activation, statistics of a range of planes, the thread's own choice of slices - stays on the row kernel
+    const bool thin_ok = !s2d && !act && a.wide && cout > 16 && !(osum && (cout / Go) % 4) && !sp.zlo && !sp.zhi && g_split < 0 && g_s2d < 0 && N <= 65535 && (size_t)D * H * W * 32 < ((size_t)1 << 31);
     const size_t thin_tiles = ((size_t)Dr * Ho * Wo + 63) / 64 * (size_t)nmt_all * N;
-    if (a.row && nmt_all == 1 && a.nbt >= 3 && !rec && g_thin < 0 && thin_tiles > 128 && thin_tiles <= (fmt == 8 ? 2 * (size_t)thin_env : (size_t)thin_env)) { a.row = false; thin_row = true; }
-    a.thin = (thin_max > 0 || thin_row) && !a.row && !a.areg && !s2d && !act && a.wide && cout > 16 && !(osum && (cout / Go) % 4) && !sp.zlo && !sp.zhi && g_split < 0 && g_s2d < 0 && N <= 65535 &&
-             (size_t)D * H * W * 32 < ((size_t)1 << 31) && thin_tiles <= (thin_row ? 2 * (size_t)thin_env : thin_max);
+    const bool thin_row = thin_ok && a.row && nmt_all == 1 && a.nbt >= 3 && !rec && g_thin < 0 && thin_tiles > 128 && thin_tiles <= (fmt == 8 ? 2 * (size_t)thin_env : (size_t)thin_env);
+    if (thin_row) a.row = false;
+    a.thin = thin_row || (thin_ok && !a.row && !a.areg && thin_tiles <= thin_max);
     // about one tile of 128 flat voxels x 64 channels per CU, past the K-split kernel's launches: the flat kernel, whose time goes by its rounds of 256 workgroups -
     // some 8 us and 2.2 (e2m1 1) per pair of input blocks each - where the staged kernels' goes by one tile's chain of loads and barriers. Kernel time, us, the other
     // kernel against this one, and workgroups here. e4m3: 256 -> 256 at 2 x 16^3 37.2 against 22.2 (256); at 1 x 22 x 26^2 (234) 64 -> 128 18.4 against 14.4, 128 -> 128 26.8 and
@@ -692,6 +693,7 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     if (wl_env < 0) wl_env = getenv("MI_CONV_ROW_WL") ? atoi(getenv("MI_CONV_ROW_WL")) : 1;
     a.wl_o = 0;
     if (a.row && !a.row1 && fmt == 4 && wl_env && smem + (size_t)a.nbt * 15 * 1280 <= 160 * 1024) { a.wl_o = (unsigned)smem; smem += (size_t)a.nbt * 15 * 1280; }
+    if (smem > 160 * 1024) mi_die("%s: %zu bytes of LDS for %d input blocks in chunks of %d", who, smem, a.nbt, a.CB);      // (every form above sizes its chunks to fit)
     if (big || a.areg || a.row || a.s2row) {
         // rows and scale bytes of positions outside the volume: 64 zero bytes, then 64 bytes of value 1; one page per device, kept for the process
         // (the entry point that must not allocate keeps its own at the head of its fixed scratch)
