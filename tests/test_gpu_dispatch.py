@@ -35,7 +35,7 @@ def test_default_rule_at_its_edges(gpu, bits, N, Ci, Co, D, H, W, kern):
 
 # (bits, input channels): three blocks; four of e4m3 and seven of e2m1, whose halo chunk would not fit LDS in one piece on the general kernel
 @pytest.mark.parametrize("bits,Ci", [(8, 96), (8, 128), (4, 96), (4, 224)])
-@pytest.mark.parametrize("call", ["act", "split", "range"])
+@pytest.mark.parametrize("call", ["act", "split"])
 def test_few_tiles_that_the_k_split_kernel_does_not_take(gpu, bits, Ci, call):
     """three blocks and more into one channel tile of 129 tiles and more go to the K-split kernel by default; a call it cannot run stays on the row kernel"""
     rng = np.random.default_rng(Ci + bits)
@@ -55,15 +55,36 @@ def test_few_tiles_that_the_k_split_kernel_does_not_take(gpu, bits, Ci, call):
         want, _ = orc.conv3(xq, xdt, N, Ci, D, H, W, w, b, Co, xdt, cbits=bits, fused_act=1)
         assert code_mismatch_fraction(bits, got[0], want, N, Co, D * H * W)[1]
         return
-    zr = (2, 3) if call == "range" else (0, 0)
-    if call == "split":
-        lib.mi_conv_split(0)
+    lib.mi_conv_split(0)
     try:
-        got, gs = gpu_conv(xq, xdt, N, Ci, D, H, W, w, b, Co, xdt, cbits=bits, Go=G, stats=True, zrange=zr)
+        got, gs = gpu_conv(xq, xdt, N, Ci, D, H, W, w, b, Co, xdt, cbits=bits, Go=G, stats=True)
     finally:
         lib.mi_conv_split(-1)
     assert "conv3_row_k" in lib.mi_last_kernel().decode(), lib.mi_last_kernel().decode()
-    want, _ = orc.conv3(xq, xdt, N, Ci, D, H, W, w, b, Co, xdt, cbits=bits, acc64=1)
-    f, _ = orc.conv3(xq, xdt, N, Ci, D, H, W, w, b, Co, 0, cbits=bits, acc64=1)
-    v = f.reshape(N, G, Co // G, D, H * W)[:, :, :, zr[0]:D - zr[1]].astype(np.float64)
-    assert np.array_equal(got, want) and np.allclose(gs, np.stack([v.sum((2, 3, 4)), (v * v).sum((2, 3, 4))], -1), rtol=1e-6)
+    want, ws = orc.conv3(xq, xdt, N, Ci, D, H, W, w, b, Co, xdt, cbits=bits, acc64=1, Go=G, want_stats=True)
+    assert np.array_equal(got, want) and np.allclose(gs, ws, rtol=1e-6)
+
+
+# few output voxels (runs of 32 that meet several planes, or part of one), three blocks into one channel tile, flat tiles of whole and of ragged rows, and the staged kernels beside them
+@pytest.mark.parametrize("bits,N,Ci,Co,D,H,W,kern", [(8, 2, 64, 64, 7, 3, 5, "conv3_thin_k"), (4, 1, 96, 64, 6, 6, 7, "conv3_thin_k"), (8, 1, 96, 32, 9, 30, 31, "conv3_thin_k"),
+                                                     (8, 1, 64, 64, 10, 23, 41, "conv3_flat_k"), (4, 1, 128, 64, 16, 32, 32, "conv3_flat_k"), (8, 1, 96, 32, 8, 32, 32, "conv3_row_k"),
+                                                     (8, 1, 32, 32, 16, 32, 32, "conv3_small_k"), (8, 1, 96, 96, 16, 16, 24, "conv3_mx_k")])
+def test_statistics_of_a_range_of_planes(gpu, bits, N, Ci, Co, D, H, W, kern):
+    """A conv whose statistics leave planes at its ends out (zlo, zhi) runs on the kernel of the whole call: the same fp32 outputs on operands of several
+    magnitudes, whose sums depend on their order, and the sums over the planes that are left (none, too)."""
+    rng = np.random.default_rng(Ci + Co + D + W)
+    S, G, xdt = D * H * W, 8, 3 if bits == 8 else 4
+    x, w, b = rand_case(rng, N, Ci, Co, S)
+    x *= np.exp(2 * rng.standard_normal(x.shape)).astype(np.float32)
+    xq = orc.f32_to_mx(bits, x, N, Ci, S)
+    y, _ = gpu_conv(xq, xdt, N, Ci, D, H, W, w, b, Co, 0, cbits=bits, Go=G, stats=True)
+    assert kern in lib.mi_last_kernel().decode(), lib.mi_last_kernel().decode()
+    v = y.reshape(N, G, Co // G, D, H * W).astype(np.float64)
+    for lo, hi in ((1, 2), (0, D - 1), (4, 0), (D, 0)):
+        got, gs = gpu_conv(xq, xdt, N, Ci, D, H, W, w, b, Co, 0, cbits=bits, Go=G, stats=True, zrange=(lo, hi))
+        assert kern in lib.mi_last_kernel().decode(), lib.mi_last_kernel().decode()
+        assert np.array_equal(got, y), (lo, hi)
+        u = v[:, :, :, lo:max(lo, D - hi)]
+        want = np.stack([u.sum((2, 3, 4)), (u * u).sum((2, 3, 4))], -1)
+        # (sums in fp32 within a record of at most 512 voxels x 4 channels, in double between them: 2^-24 per addition, a random walk of them, against the sum of magnitudes)
+        assert np.abs(gs - want).max() <= 1e-5 * max(np.abs(u).sum((2, 3, 4)).max(), (u * u).sum((2, 3, 4)).max(), 1e-30), (lo, hi)

@@ -271,10 +271,11 @@ __device__ __forceinline__ void conv_epi_consts(const conv_args &a, unsigned cha
 // holds voxel (oz0 + lz, oy0 + ly0 + j, ox0 + r) of a 32-voxel run along x
 // WPART: every wavefront writes its own statistics record (record tile NW + wave: the reduce kernel then sees NW records per tile) and the
 // epilogue has no workgroup barrier and touches no LDS scratch, so the wavefronts of a workgroup need not run it at the same time (one channel tile)
-// SEG: the wavefront's record ends before lane seg of the run and another begins (every seg_step lanes from there on; seg past 32: one record)
+// SEG: the wavefront's record ends before lane seg of the run and another begins (every seg_step lanes from there on; seg past 32: one record); seg_in: the
+// statistics cover the lane's voxel (its plane lies in [zs0, zs1): the caller's voxel mapping knows no planes here)
 template <int MT, int NT, int OUT, bool EPI, bool PIN = false, bool W32 = false, bool FULL = false, bool NOCH = false, int NW = 4, bool ROW = false, bool WPART = false, bool SEG = false>
 __device__ __forceinline__ void conv_epilogue(const conv_args &a, v16f (&acc)[MT][NT], unsigned char *lds, unsigned tile, int n, int cs,
-                                              int oz0, int oy0, int ox0, int lz, int ly0, int tid, const long long *ovx = nullptr, int seg = 33, int seg_step = 0) {
+                                              int oz0, int oy0, int ox0, int lz, int ly0, int tid, const long long *ovx = nullptr, int seg = 33, int seg_step = 0, bool seg_in = true) {
     const int lane = tid & 63, wave = tid >> 6, r = lane & 31, h = lane >> 5;
     // accumulator layout of the 32x32 MFMA: lane (r = voxel within the tile, h), register i -> row (i & 3) + 4 h + 8 (i >> 2) = channel 16 h + i
     const size_t So = (size_t)(a.yD ? a.yD : a.Do) * a.Ho * a.Wo;      // voxels per channel plane of the output tensor
@@ -417,7 +418,7 @@ __device__ __forceinline__ void conv_epilogue(const conv_args &a, v16f (&acc)[MT
         static_assert(!WPART || (MT == 1 && NOCH), "per-wavefront statistics records: one channel tile, no per-channel records");
         if (stats) {
             for (int lo = 0, rec = 0;; rec++) {
-                const bool in = !SEG || (r >= lo && r < seg);
+                const bool in = !SEG || (seg_in && r >= lo && r < seg);
                 float v[8];
 #pragma unroll
                 for (int q4 = 0; q4 < 4; q4++) { v[q4 * 2] = in ? qs[0][q4] : 0.f; v[q4 * 2 + 1] = in ? qss[0][q4] : 0.f; }
