@@ -88,6 +88,26 @@ def test_ct_window_gather(gpu, W):
     assert da.to_numpy(np.uint32)[0] == 0
 
 
+# cells of one workgroup, of several and of a last partial one; rows that start at any byte
+@pytest.mark.parametrize("S,dims", [(16, (33, 50, 61)), (40, (90, 81, 123)), (64, (130, 128, 200))])
+def test_ct_flags_of_dense_cells(gpu, S, dims):
+    """Every workgroup of a cell finds material and looks at the flag while others set it; cells of air beside them, and flags that are set already, stay as they are."""
+    rng = np.random.default_rng(S)
+    vol = rng.integers(3, 256, dims, dtype=np.uint8)
+    nss = np.array([(d + S - 1) // S for d in dims], np.int64); tot = int(nss.prod())
+    air = rng.permutation(tot)[:tot // 3]
+    for k in air:
+        a, b, c = np.unravel_index(k, nss); vol[a * S:a * S + S, b * S:b * S + S, c * S:c * S + S] = 2
+    dv = DevBuf.from_numpy(vol)
+    want = np.ones(tot, np.uint32); want[air] = 0
+    before = np.zeros(tot, np.uint32); before[air[:2]] = 1; want[air[:2]] = 1
+    for _ in range(3):
+        df = DevBuf.from_numpy(before)
+        lib.mi_ct_flags(dv.ptr, *dims, S, nss.ctypes.data_as(C.POINTER(C.c_int64)), 3, df.ptr)
+        LP.check()
+        assert np.array_equal(df.to_numpy(np.uint32), want)
+
+
 @pytest.mark.parametrize("W,n", [(24, 3), (32, 18)])     # 18: more windows than one launch carries
 def test_ct_windows_and_flags_equal_the_single_window_calls(gpu, W, n):
     rng = np.random.default_rng(19)

@@ -122,11 +122,17 @@ extern "C" void mi_ct_window(const uint8_t *vol, int64_t Z, int64_t Y, int64_t X
 // "holds a voxel >= iso" of every cell of a grid over the volume: cell (a, b, c) of nss[3] is [a S, a S + S) x [b S, ..) x [c S, ..) clipped to the
 // volume, i.e. the interior of the sliding window with that index. The cells tile the volume, so this is one read of it. A thread tests 16
 // consecutive x of a cell row (one 16-byte load of a whole piece, else bytes); a workgroup's rows belong to one cell, and a cell whose flag is set already
-// needs no more of them. (190 x 280 x 260 in cells of 96, rows that start at any byte: 94 us with byte loads of every row, 45 now)
+// needs no more of them. (a call over 190 x 280 x 260 in cells of 96, dense: 30 us with a look per wavefront and the compiler's workgroup reduction, 16 now;
+// 512 x 1024^2 64 and 46)
 __global__ void __launch_bounds__(256) ct_flags_k(const uint8_t *__restrict__ vol, long long Z, long long Y, long long X, int S, int n1, int n2, int iso, unsigned *any) {
     const int S16 = (S + 15) >> 4;
     const unsigned cell = blockIdx.x, c = cell % (unsigned)n2, b = (cell / (unsigned)n2) % (unsigned)n1, a = cell / ((unsigned)n2 * (unsigned)n1);
-    if (*(volatile unsigned *)(any + cell) != 0u) return;          // (as this XCD's L2 has it: a stale 0 only costs the read)
+    // one thread looks (as this XCD's L2 has it: a stale 0 only costs the read) and the workgroup goes by what it saw: by themselves its wavefronts could see different values, and
+    // those that stayed would meet at a barrier without the others
+    __shared__ unsigned seen, hit;
+    if (threadIdx.x == 0) { seen = *(volatile unsigned *)(any + cell); hit = 0u; }
+    __syncthreads();
+    if (seen != 0u) return;
     const unsigned i = blockIdx.y * 256u + threadIdx.x;            // (fewer than 2^24 of them: 65535 workgroups)
     unsigned found = 0u;
     if (i < (unsigned)S * S * S16) {
@@ -145,7 +151,9 @@ __global__ void __launch_bounds__(256) ct_flags_k(const uint8_t *__restrict__ vo
     }
     // one store per workgroup that finds material and does not see the flag: all write the same 1. (Accesses that must meet outside the L2s - an atomic per wavefront, or a
     // device-scope look at the flag per workgroup - queue on the flags' two cache lines, 5 ns each: 94 and 86 us)
-    if (__syncthreads_or(found != 0u) && threadIdx.x == 0 && *(volatile unsigned *)(any + cell) == 0u) *(volatile unsigned *)(any + cell) = 1u;
+    if (found) hit = 1u;
+    __syncthreads();
+    if (threadIdx.x == 0 && hit != 0u && *(volatile unsigned *)(any + cell) == 0u) *(volatile unsigned *)(any + cell) = 1u;
 }
 extern "C" void mi_ct_flags(const uint8_t *vol, int64_t Z, int64_t Y, int64_t X, int S, const int64_t nss[3], int iso, unsigned *any) {
     const int64_t total = nss[0] * nss[1] * nss[2];
