@@ -162,6 +162,49 @@ def test_short_sequences_give_the_long_ones_bits(gpu, S):
     assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
 
 
+def test_more_short_sequences_than_one_launch_holds(gpu):
+    """2^25 + 10 (sequence, head) units of 128 threads: past the 2^32 threads of a launch. One slot each, so a unit's output is its v row."""
+    nseq, S, H = (1 << 24) + 5, 1, 2; Cc, Tp = 48 * H, nseq + 64
+    dq, do, dlse = DevBuf(3 * H * Tp * 96, zero=False), DevBuf(nseq * Cc * 4, zero=False), DevBuf(nseq * H * 4, zero=False)
+    rng = np.random.default_rng(3); k = 64
+    rows, nan = {}, np.full((k, Cc), np.nan, np.float32)
+    for a in (0, (1 << 23) - k // 2, nseq - k):                                    # the ends, and the sequences where the launch is cut
+        lib.mi_h2d(do.ptr + a * Cc * 4, nan.ctypes.data, nan.nbytes)
+        rows[a] = rng.standard_normal((3, H, k, 48)).astype(np.float16)
+        for p, h in np.ndindex(3, H):
+            lib.mi_h2d(dq.ptr + ((p * H + h) * Tp + a) * 96, np.ascontiguousarray(rows[a][p, h]).ctypes.data, k * 96)
+    g = at_geom(); g.nseq, g.S, g.D, g.Hh, g.W = nseq, S, 1, 1, S
+    lib.at_fa_fwd(dq.ptr, do.ptr, dlse.ptr, C.byref(g), H, Cc); LP.check()
+    lib.mi_sync()
+    for a, r in rows.items():
+        got = np.empty((k, Cc), np.float32); lib.mi_d2h(got.ctypes.data, do.ptr + a * Cc * 4, got.nbytes)
+        want = r[2].transpose(1, 0, 2).reshape(k, Cc).astype(np.float32)           # (the one probability is 1 up to the rounding of its logit)
+        assert np.abs(got - want).max() < 1e-5, (a, np.abs(got - want).max())
+
+
+def test_more_grid_tokens_than_one_launch_holds(gpu):
+    """the sample lists of 512 x 512 x 513 tokens at 32 threads each: past the 2^32 threads of a launch; one ray per plane keeps the lists small"""
+    D, Hh, W, mult = 512, 512, 513, 0.001
+    axr = make_axr(1, D, Hh, W, (0,), (0,))
+    q, nt, nr = C.c_int(), C.c_int(), C.c_int()
+    lib.at_rays_dims(D, Hh, W, C.c_float(mult), C.byref(q), C.byref(nt), C.byref(nr))
+    Q, Nt, Nr, P, Tg = q.value, nt.value, nr.value, max(D, Hh, W), D * Hh * W
+    assert Nt == 1 and Tg * 32 > 1 << 32
+    ray = np.zeros((1, Q, 8), np.float32); lens = np.zeros((1, Q), np.int32); ad = np.zeros(1, np.int32); cen = np.zeros((1, P, 4), np.float32)
+    lib.at_rays_plan(1, D, Hh, W, C.c_float(mult), axr.ctypes.data, ray.ctypes.data, lens.ctypes.data, ad.ctypes.data, cen.ctypes.data)
+    b = [DevBuf.from_numpy(a) for a in (ad, ray, lens)] + [DevBuf(Q * Nr * 12), DevBuf(Tg * 4, zero=False)]
+    lib.mi_sync()
+    R = at_rays(); R.n, R.Q, R.Nt, R.Nr, R.D, R.Hh, R.W = 1, Q, Nt, Nr, D, Hh, W
+    R.ad, R.ray, R.lens, R.pos, R.wsum = (x.ptr for x in b)
+    lib.at_rays_setup(C.byref(R)); LP.check()
+    got = b[4].to_numpy(np.float32, (Tg,))
+    rows, w = ro.stencil(ray, ad, Nr, D, Hh, W)
+    want = ro.wsum_inv(rows, w, Tg)
+    on = want > 0
+    assert on.sum() > 512 * 100 and on[-Hh * W:].any() and np.array_equal(got > 0, on)
+    assert np.abs(got[on] - want[on]).max() < 1e-5 * np.sqrt((want[on] ** 2).mean())
+
+
 def run_block(P, lay, x, d, g, Tr=0):
     bp = at_bp(); assert lib.at_block_layout(C.byref(d), C.byref(bp), 0) == P.size
     T = x.shape[0]

@@ -130,9 +130,9 @@ __global__ void __launch_bounds__(256) ray_pos_k(const float *__restrict__ ray, 
 // walked 32 rays each, with 64-bit divisions per sample: 131 us; 7.6 now.)
 struct ray_ent { int slot; float w; };
 __global__ void __launch_bounds__(256) ray_inverse_k(ray_geo G, const float *__restrict__ ray, const int *__restrict__ ad, long long Tg, int Nt, int cap,
-                                                     ray_ent *__restrict__ tab, int *__restrict__ cnt, float *__restrict__ winv) {
+                                                     ray_ent *__restrict__ tab, int *__restrict__ cnt, float *__restrict__ winv, long long t0) {
     const int l = threadIdx.x & 31;
-    const long long t = blockIdx.x * 8ll + (threadIdx.x >> 5);
+    const long long t = t0 + blockIdx.x * 8ll + (threadIdx.x >> 5);
     const bool live = t < Tg;                                      // (all lanes stay for the exchanges)
     const long long tc = live ? t : Tg - 1;
     const int b = (int)(Tg >> 32 ? tc / G.Sg : (unsigned)tc / (unsigned)G.Sg), ts = (int)(tc - (long long)b * G.Sg);      // (a sample's tokens: below 2^31 by far)
@@ -304,11 +304,12 @@ __global__ void __launch_bounds__(256) fa16_rows_k(const __half *__restrict__ Qh
 // in the order of the kernel above (in groups of eight keys), so the results are its bits. Bound by its multiply-adds and the LDS reads that feed them:
 // 2 x 512 rays of 24 slots, four heads, 45 -> 21 us (the multiply-adds and conversions alone take about 9)
 __global__ void __launch_bounds__(128) fa16_short_k(const __half *__restrict__ Qh, const __half *__restrict__ Kh, const __half *__restrict__ Vh, float *__restrict__ o, float *__restrict__ lse,
-                                                    int S, int H, int C, long long Tp, float sl2, const int *__restrict__ lens) {
+                                                    int S, int H, int C, long long Tp, float sl2, const int *__restrict__ lens, unsigned u0) {
     __shared__ __align__(16) __half ks[32 * HD], vs[32 * HD];
     __shared__ float lg[32 * 33];                                  // [key][query]
     const int tid = threadIdx.x, i = tid & 31, part = tid >> 5;
-    const int seq = (int)(blockIdx.x / (unsigned)H), h = (int)(blockIdx.x - (unsigned)seq * (unsigned)H);
+    const unsigned un = u0 + blockIdx.x;
+    const int seq = (int)(un / (unsigned)H), h = (int)(un - (unsigned)seq * (unsigned)H);
     const size_t base = ((size_t)h * Tp + (size_t)seq * S) * HD;
     const int SK = lens ? min(lens[seq], S) : S;
     float q[HD];
@@ -393,7 +394,9 @@ inv_tab inverse_table(const at_rays *R, float *winv) {
     const inv_tab t = {cnt, (ray_ent *)(cnt + ((Tg + 63) & ~(size_t)63)), cap};
     const inv_key k = {R->ray, R->ad, cnt, R->n, R->Q, R->Nt, R->Nr, R->D, R->Hh, R->W};
     if (!winv && k == g_inv) return t;
-    ray_inverse_k<<<nblk_(Tg, 8), 256>>>(G, R->ray, R->ad, (long long)Tg, R->Nt, cap, t.tab, t.cnt, winv);
+    // (a launch has fewer than 2^32 threads: 32 of them per token, 2^31 per piece)
+    constexpr size_t PIECE = (size_t)1 << 26;
+    for (size_t t0 = 0; t0 < Tg; t0 += PIECE) ray_inverse_k<<<nblk_(Tg - t0 < PIECE ? Tg - t0 : PIECE, 8), 256>>>(G, R->ray, R->ad, (long long)Tg, R->Nt, cap, t.tab, t.cnt, winv, (long long)t0);
     g_inv = k;
     return t;
 }
@@ -448,7 +451,9 @@ extern "C" void at_fa_fwd(const void *qkvh, float *o, float *lse, const at_geom 
     const long long nw = (long long)g->nseq * H * (shrt ? 1 : (g->S + 63) / 64);      // (sequence, head) units, or wavefronts
     if (nw > 0x7fffffffll) mi_die("at_fa_fwd: %lld wavefronts", nw);
     const float sl2 = 1.4426950408889634f / sqrtf((float)HD);
-    if (shrt) fa16_short_k<<<(unsigned)nw, 128>>>(Qh, Kh, Vh, o, lse, g->S, H, C, Tp, sl2, g->lens);
+    // (a launch has fewer than 2^32 threads: 128 of them per unit, 2^31 per piece)
+    constexpr long long PIECE = 1ll << 24;
+    if (shrt) for (long long u0 = 0; u0 < nw; u0 += PIECE) fa16_short_k<<<(unsigned)(nw - u0 < PIECE ? nw - u0 : PIECE), 128>>>(Qh, Kh, Vh, o, lse, g->S, H, C, Tp, sl2, g->lens, (unsigned)u0);
     else fa16_rows_k<<<nblk_((size_t)nw, 4), 256>>>(Qh, Kh, Vh, o, lse, g->S, H, C, Tp, g->nseq, sl2, g->lens);
     MICK();
 }
