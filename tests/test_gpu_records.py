@@ -5,7 +5,7 @@ import pytest
 from ufsm_amd import lib
 import orc
 from ufsm_amd.lp import DevBuf
-from test_gpu_conv import exact_case, gpu_conv
+from test_gpu_conv import exact_case, rand_case, gpu_conv
 
 pytestmark = pytest.mark.gpu
 
@@ -51,3 +51,26 @@ def test_forward_takes_none_of_the_regrouping_kernels(gpu):
         y.append(lg.to_numpy(np.uint32))
     assert np.array_equal(y[0], y[1])
     assert lib.mi_conv_keep_records(0) == 0                                      # the setting is the forward's, not the thread's afterwards
+
+
+def test_short_walks_keep_the_precision_of_the_row_kernels_sums(gpu):
+    """One block into one channel tile on the small-channel kernel, where the one-block row kernel ran: a record per wavefront of 128 voxels there too, so that no more
+    is summed in fp32. The errors of the sums of squares against 64 bits have the row kernel's size: their root mean squares over 128 groups differ by 9 % by chance (1 / sqrt 128);
+    a record per tile of 512 voxels gives 1.7 times."""
+    err = {}
+    for seed in range(4):
+        rng = np.random.default_rng(40 + seed)
+        N, C, D, H, W, G = 4, 32, 16, 32, 64, 8
+        x, w, b = rand_case(rng, N, C, C, D * H * W)
+        xq = orc.f32_to_mx(8, x, N, C, D * H * W)
+        for thin, kern in ((-1, "conv3_small_k"), (0, "conv3_row1_k")):
+            lib.mi_conv_thin(thin)
+            try:
+                y, s = gpu_conv(xq, 3, N, C, D, H, W, w, b, C, 0, Go=G, stats=True)
+            finally:
+                lib.mi_conv_thin(-1)
+            assert kern in lib.mi_last_kernel().decode()
+            ref = (y.astype(np.float64) ** 2).reshape(N, G, -1).sum(-1)
+            err.setdefault(kern, []).append((s[..., 1] - ref) / ref)
+    rms = {k: np.sqrt(np.mean(np.square(v))) for k, v in err.items()}
+    assert rms["conv3_small_k"] < 1.35 * rms["conv3_row1_k"], rms

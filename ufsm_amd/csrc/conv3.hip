@@ -284,7 +284,7 @@ static void conv_stats_reduce(const char *who, const conv_args &a, int MT, split
         // few records: the pre-pass that follows adds them itself, one launch less (its rule: mi_restage_records)
         const gn_stage_t g = g_stage; g_stage.gamma = nullptr;
         const int xdt = a.ydt; const size_t S = (size_t)a.Do * a.Ho * a.Wo;
-        const gn_records_t rec = {(const float2 *)a.part, (int)(a.ntiles / a.N) * (a.row1 ? 8 : 1) / a.ncs, a.ncs * MT * 8, a.Go, fin.len, fin.eps, fin.mean, fin.rstd};
+        const gn_records_t rec = {(const float2 *)a.part, (int)(a.ntiles / a.N) * a.wrec / a.ncs, a.ncs * MT * 8, a.Go, fin.len, fin.eps, fin.mean, fin.rstd};
         if (!a.stat_ch && mi_restage_records(a.y, xdt, a.N, a.Co, S, g.gamma, g.beta, rec, g.y8, g.y4)) return;
         conv_stats_reduce(who, a, MT, sp, osum);
         gnp_t gp; memset(&gp, 0, sizeof gp); gp.gamma = g.gamma; gp.beta = g.beta; gp.mean = fin.mean; gp.rstd = fin.rstd; gp.G = a.Go;
@@ -296,7 +296,7 @@ static void conv_stats_reduce(const char *who, const conv_args &a, int MT, split
         return;
     }
     if (a.stat_ch) { gn_part_reduce_ch_k<<<a.N * a.Go, 256>>>((const float2 *)a.part, (int)(a.ntiles / a.N), a.ncs, a.Co, a.Go, osum, fin); MICK(); return; }
-    const int tiles_per_n = (int)(a.ntiles / a.N) * (a.row1 ? 8 : 1);      // (row1: eight records per tile)
+    const int tiles_per_n = (int)(a.ntiles / a.N) * a.wrec;      // (records)
     const int Q = a.ncs * MT * 8, nst = tiles_per_n / a.ncs;
     if (mi_records_few(a.Co, a.Go, nst)) {
         const gn_records_t rec = {(const float2 *)a.part, nst, Q, a.Go, fin.len, fin.eps, nullptr, nullptr};
@@ -339,6 +339,7 @@ static int conv_stem(const char *who, const void *x, int xbf, shape5 xs, const f
         mi_die("%s: slab-local GroupNorm geometry (zs %d, zo %d, ns %d, zhw %d) does not fit planes of %d voxels (at most 256 slabs)", who, gp.zs, gp.zo, gp.ns, gp.zhw, H * W);
     const int CP = rows ? 0 : Ci <= 4 ? 4 : Ci <= 8 ? 8 : 16, TPK = rows ? 2 : 32 / CP, NKB = rows ? 18 : (27 + TPK - 1) / TPK, NP = (NKB + 1) / 2;
     conv_args a; memset(&a, 0, sizeof a);
+    a.wrec = 1;
     a.sx = x; a.sxdt = xbf; a.sCi = Ci;
     a.sgam = gp.gamma; a.sbet = gp.beta; a.smean = gp.mean; a.srstd = gp.rstd; a.sG = gp.G;
     if (gp.G && gp.ns) { a.szs = gp.zs; a.szo = gp.zo; a.sns = gp.ns; }      // (each slab's coefficient table in LDS: the staged positions take their plane's)
@@ -376,7 +377,7 @@ static int conv_stem(const char *who, const void *x, int xbf, shape5 xs, const f
     if (!have) conv3_stem_prep(CP, w, wq, wsc, cout, Ci, nmt_all, NP);
     a.wq = wq; a.wsc = wsc;
     a.stat_ch = osum && (cout / Go) % 4 ? 1 : 0;
-    if (osum) a.part = (float *)mi_ws(MI_WS_MISC, (size_t)a.ntiles * (a.stat_ch ? 32 : a.row1 ? 64 : MT * 8) * 2 * sizeof(float));      // (row1: a record per wavefront, eight per tile)
+    if (osum) a.part = (float *)mi_ws(MI_WS_MISC, (size_t)a.ntiles * (a.stat_ch ? 32 : a.wrec * MT * 8) * 2 * sizeof(float));
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     const bool ktime = g_ktime && !mi_ws_arena_on();
     if (ktime) { MIRT(hipEventCreate(&ev0)); MIRT(hipEventCreate(&ev1)); MIRT(hipEventRecord(ev0, 0)); }
@@ -619,19 +620,22 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     if (rowcs_env < 0) rowcs_env = getenv("MI_CONV_ROW_CS") ? atoi(getenv("MI_CONV_ROW_CS")) : 1;
     const bool row_cs = (rowcs_env && nmt_all == 2 && MT == 2) || row_cs4;
     a.row = row_env && !big && !s2d && !(osum && (cout / Go) % 4) && cout > 16 && (nmt_all == 1 || row_cs) && stride == 1 && NT == 4 && a.wide && Wo > 16 && a.nbt >= (row_env > 1 || row1_env ? 1 : 2) && a.nbt <= 64;
-    // ... but one channel tile from one block goes back to the small-channel kernel (two workgroups per CU, 16-wide tiles, an eighth of the statistics records) where the row
-    // kernel has fewer than four tiles per CU to walk (its ring of planes and its half-tile offset need a walk: 1 024 tiles) or where runs of 32 fit the rows worse than tiles
-    // of 16. A call with statistics, us, the row kernel against this one, e4m3: 32^3 17.5 / 14.1, 48^3 23.7 / 17.7, 64^3 (256 row tiles) 26.5 / 24.8, 2 x 64^3 (512) 42.4 / 40.1,
-    // 96^3 (864) 56.5 / 53.3, 64 x 128^2 (1 024) 56.6 / 59.6, 4 x 64^3 (1 024) 55.6 / 57.3, 2 x 96^3 (1 728) 88.7 / 89.0, 2 x 128^3 208 / 224; rows of 104 in 88 planes 68.2 / 60.0, of 72
-    // (128 x 96 x 72) 59.9 / 56.9, of 112 69.1 / 68.4, of 120 (four runs of 32, eight tiles of 16) 88.5 / 90.5. e2m1: 64^3 21.8 / 19.8, 96^3 46.6 / 44.0, 2 x 96^3 68.1 / 70.7. fp16 planes out:
-    // 64^3 29.4 / 25.5, 40^3 22.7 / 16.8. Launches of under 16 384 voxels gain as well (24^3 17.7 / 13.3), but the tests hold two of them on the row kernel
+    // ... but one channel tile from one block goes back to the small-channel kernel (two workgroups per CU, 16-wide tiles; a statistics record per wavefront, as the row kernel's, so that
+    // the sums keep their precision) where the row kernel has fewer than four tiles per CU to walk (its ring of planes and its half-tile offset need a walk: 1 024 tiles) or where runs of 32
+    // fit the rows worse than tiles of 16. A call with statistics, us, the row kernel against this one, e4m3: 16 x 32^2 14.1 / 10.6, 32^3 14.5 / 11.0, 48^3 16.9 / 12.5, 64^3 (256 row tiles)
+    // 17.9 / 16.3, 2 x 64^3 (512) 24.3 / 23.4, 96^3 (864) 35.5 / 33.5; rows of 104 in 88 planes 42.3 / 37.7, of 72 (128 x 96 x 72) 41.9 / 37.0, of 112 (112^3) 52.8 / 46.5, of 80 (80^3)
+    // 30.9 / 26.1. e2m1: 64^3 15.0 / 13.6, 96^3 28.5 / 26.4, 88 x 104^2 33.9 / 29.8. Past 1 024 tiles of whole runs the row kernel is the faster one (with a record per tile here: 64 x 128^2
+    // 56.6 / 59.6, 4 x 64^3 55.6 / 57.3, 2 x 128^3 208 / 224, of a call that prepares its weights; rows of 120 - four runs of 32, eight tiles of 16 - 88.5 / 90.5). fp16 planes out: 64^3
+    // 29.4 / 25.5, 40^3 22.7 / 16.8. Launches of under 16 384 voxels gain as well (24^3 17.7 / 13.3), but the tests hold two of them on the row kernel
     // A conv's fp32 statistics records add up in another order on another kernel, which moves a mean or 1 / std by its last bit now and then; a code of the next conv's rows at a rounding
     // boundary then moves, and with it the rest of a network (e4m3: up to 2 % of the logits, one window size in ten; e2m1 more). Inside a network the three rules that came with the
     // flat kernel (this one, the short 96 -> 32 walks and the flat tiles) therefore leave convs with statistics where they were
     const bool rec = g_records && osum;
     const size_t row_tiles = (size_t)((Wo + 31) / 32) * ((Ho + 7) / 8) * ((Dr + 3) / 4) * N;
-    if (a.row && a.areg && row1_env == 1 && !rec && g_thin < 0 && (size_t)N * Dr * Ho * Wo >= 16384 && (row_tiles < 1024 || 2 * ((Wo + 31) / 32) > (Wo + 15) / 16)) a.row = false;
+    const bool row_small = a.row && a.areg && row1_env == 1 && !rec && g_thin < 0 && (size_t)N * Dr * Ho * Wo >= 16384 && (row_tiles < 1024 || 2 * ((Wo + 31) / 32) > (Wo + 15) / 16);
+    if (row_small) a.row = false;
     a.row1 = a.row && a.nbt == 1 && row1_env && row_env < 2;
+    a.wrec = a.row1 ? 8 : row_small && osum ? 4 : 1;
     if (a.row && nmt_all >= 2) MT = 1;
     if (a.row) { a.areg = false; a.CB = a.nbt; }
     // few output voxels: the K range split over a workgroup's wavefronts (conv3_thin_k). The staged kernels' time hardly depends on how many workgroups a
@@ -681,7 +685,7 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     const size_t frun = ((size_t)Dr * Ho * Wo + 31) / 32, fwg = (frun + 3) / 4 * (size_t)((nmt_all + 1) / 2) * N;
     a.flat = flat_ok && (g_flat > 0 || (g_flat < 0 && flat_env && !rec && g_thin < 0 && g_split < 0 && g_s2d < 0 && thin_tiles > (a.thin && nmt_all <= 4 ? 512u : 256u) &&
                          (fmt == 8 ? a.nbt >= 2 : a.nbt >= 4 && frun <= 512) && fwg <= (a.nbt >= 8 ? 512u : 256u)));
-    if (a.flat) a.thin = a.row = a.row1 = a.areg = false;
+    if (a.flat) { a.thin = a.row = a.row1 = a.areg = false; a.wrec = 1; }
     if (a.thin || a.flat) { big = false; MT = 1; NT = 2; a.CB = a.flat ? 2 : a.nbt; }
     size_t smem = a.flat ? (size_t)(fmt == 8 ? flat_t<8>::LDS : flat_t<4>::LDS) : a.thin ? MI_THIN_LDS : a.row1 ? (size_t)10 * 352 * (RB + 4) : a.row ? (size_t)2 * 2048 * (RB + 4) : a.areg ? (size_t)2 * ((TT + 63) / 64 * 64) * (RB + 4) : big ? (size_t)4 * MT * (WTILE + 256) + (size_t)3 * ((TT + 63) / 64 * 64) * (RB + 4) + (size_t)(((27 * a.nbt + 1) >> 1) + 2) * 32 : lds_bytes(a.CB);
     if (s2d) smem = a.s2row ? conv3s2_row_lds(fmt) : 0;
@@ -754,7 +758,7 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     }
     a.wq = wq; a.wsc = wsc;
     a.stat_ch = osum && (cout / Go) % 4 ? 1 : 0;
-    if (osum) a.part = (float *)mi_ws(MI_WS_MISC, (size_t)a.ntiles * (a.stat_ch ? 32 : a.row1 ? 64 : MT * 8) * 2 * sizeof(float));      // (row1: a record per wavefront, eight per tile)
+    if (osum) a.part = (float *)mi_ws(MI_WS_MISC, (size_t)a.ntiles * (a.stat_ch ? 32 : a.wrec * MT * 8) * 2 * sizeof(float));
     const bool epi = act != 0;
     const int out = ybf == 3 ? 8 : ybf == 4 ? 4 : 0;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;

@@ -121,6 +121,7 @@ struct conv_args {
     bool areg;                         // the persistent small-channel kernel (one channel tile, one input block, weights in registers) takes the launch
     bool row;                          // the row kernel (one channel tile, any number of input blocks, 4 x 8 x 32 voxel tiles) takes the launch
     bool row1;                         // ... its one-input-block form (weights in registers, the two halves of the workgroup half a tile apart)
+    int wrec;                          // statistics records of a tile and channel slice: 1, or one per wavefront (the one-block row kernel 8, the small-channel kernel on that kernel's launches 4)
     bool thin;                         // the K-split kernel of the launches of few output voxels takes the launch
     bool s2row;                        // the stride-2 row kernel takes the launch (one block, one channel tile)
     bool flat;                         // ... the one of about a tile of 128 voxels x 64 channels per CU (flat runs, the taps split over the wavefronts)
@@ -678,12 +679,12 @@ static void launch_mt(int MT, int NT, const conv_args &a, size_t smem) {
     case 11: if constexpr (STRIDE == 2) { launch_conv<FMT, 2, 1, 1, OUT, EPI>(a, smem); break; }
     case 21: if constexpr (STRIDE == 2) { launch_conv<FMT, 2, 2, 1, OUT, EPI>(a, smem); break; }
     case 41: if constexpr (STRIDE == 2) { launch_conv<FMT, 2, 4, 1, OUT, EPI>(a, smem); break; }
-    case 12: if constexpr (STRIDE == 1) { if (a.areg) { launch_small<FMT, 2, OUT, EPI>(a, smem); break; } }
+    case 12: if constexpr (STRIDE == 1) { if (a.areg) { launch_small<FMT, 2, OUT, EPI, false>(a, smem); break; } }
              launch_conv<FMT, STRIDE, 1, 2, OUT, EPI>(a, smem); break;
     case 22: launch_conv<FMT, STRIDE, 2, 2, OUT, EPI>(a, smem); break;
     case 32: launch_conv<FMT, STRIDE, 3, 2, OUT, EPI>(a, smem); break;
     case 42: launch_conv<FMT, STRIDE, 4, 2, OUT, EPI>(a, smem); break;
-    case 14: if constexpr (STRIDE == 1) { if (a.row1) launch_row1<FMT, OUT, EPI>(a, smem); else if (a.row) { if constexpr (FMT == 4) { if (a.wl_o) { launch_row<FMT, OUT, EPI, true>(a, smem); break; } } launch_row<FMT, OUT, EPI, false>(a, smem); } else if (a.areg) launch_small<FMT, 4, OUT, EPI>(a, smem); else launch_conv<FMT, 1, 1, 4, OUT, EPI>(a, smem); break; }
+    case 14: if constexpr (STRIDE == 1) { if (a.row1) launch_row1<FMT, OUT, EPI>(a, smem); else if (a.row) { if constexpr (FMT == 4) { if (a.wl_o) { launch_row<FMT, OUT, EPI, true>(a, smem); break; } } launch_row<FMT, OUT, EPI, false>(a, smem); } else if (a.areg) { if (a.wrec > 1) launch_small<FMT, 4, OUT, EPI, true>(a, smem); else launch_small<FMT, 4, OUT, EPI, false>(a, smem); } else launch_conv<FMT, 1, 1, 4, OUT, EPI>(a, smem); break; }
     case 24: if constexpr (STRIDE == 1) { if (a.big) launch_wide<FMT, OUT, EPI, 2>(a, smem); else launch_conv<FMT, 1, 2, 4, OUT, EPI>(a, smem); break; }
     default: mi_die("conv3: no kernel for MT %d NT %d stride %d", MT, NT, STRIDE);
     }
