@@ -88,7 +88,9 @@ void mi_conv_s2_wkey(unsigned wkey);
  * overridden by UFSM_F8S_ZC (src/lp_f8fwd.cuh:412-416). */
 void mi_conv_stem_zc(int zc);
 /* tuning knob of the calling thread (no counterpart in the reference): stride-1 launches with fewer tiles of 128 output channels than this run as
-   slices of 64 channels, twice the workgroups; 0: never, -1: the default (192, or MI_CONV_SPLIT). The results do not depend on it. */
+   slices of 64 channels, twice the workgroups; 0: never, -1: the default (192, or MI_CONV_SPLIT). A setting (0 or more) also
+   keeps the thread's convs off what the default has beside those slices: the K-split kernel, the flat tiles chosen by size, one channel tile per workgroup on the coarse levels, and the
+   row kernels' slices for 65 .. 128 channels of one input block. The same conv either way, its fp32 sums in another order on those kernels. */
 void mi_conv_split(int tiles);
 /* Extension: which kernel takes the calling thread's 3x3x3 stride-2 convs on 32-channel rows. -1 (default): the kernel that reads the taps' rows
    straight from the stored tensor when the launch has enough output voxels to fill the device, else the general kernel (staged halo); one input block
@@ -96,7 +98,9 @@ void mi_conv_split(int tiles);
    0: always the general kernel; 1: the direct kernel, 2: the row kernel whenever its operands allow it. The results are the same conv either way. */
 void mi_conv_s2_direct(int mode);
 /* Extension: up to how many tiles (64 voxels x 32 output channels, of the whole tensor) the calling thread's 3x3x3 convs may run on the kernel that splits
-   the K range over a workgroup's wavefronts. -1 (default): the measured limits; 0: never. The same conv either way, its fp32 sums in another order. */
+   the K range over a workgroup's wavefronts. -1 (default): the measured limits; 0: never. A setting (0 or more) also
+   switches off the default's other rules for few tiles: flat tiles by size, short 32 -> 32 walks on the small-channel kernel, three input blocks into one channel tile off the row kernel.
+   The same conv either way, its fp32 sums in another order. */
 void mi_conv_thin(int tiles);
 /* Extension: whether the calling thread's 3x3x3 convs run on the kernel of flat 128-voxel tiles whose taps are split over a workgroup's wavefronts: 1 wherever
    that kernel can (stride 1, an even number of input blocks, more than 32 output channels, rows of at most 41 voxels), 0 nowhere, -1 (default) by size. The same

@@ -88,3 +88,19 @@ def test_statistics_of_a_range_of_planes(gpu, bits, N, Ci, Co, D, H, W, kern):
         want = np.stack([u.sum((2, 3, 4)), (u * u).sum((2, 3, 4))], -1)
         # (sums in fp32 within a record of at most 512 voxels x 4 channels, in double between them: 2^-24 per addition, a random walk of them, against the sum of magnitudes)
         assert np.abs(gs - want).max() <= 1e-5 * max(np.abs(u).sum((2, 3, 4)).max(), (u * u).sum((2, 3, 4)).max(), 1e-30), (lo, hi)
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2])
+def test_the_stride_2_choice_leaves_stride_1_alone(gpu, mode):
+    """mi_conv_s2_direct is about stride-2 convs: with it set, stride-1 convs run on the kernels of the default"""
+    for bits, N, Ci, Co, D, H, W, kern in [(8, 1, 64, 64, 4, 5, 7, "conv3_thin_k"), (8, 1, 128, 32, 9, 30, 31, "conv3_thin_k"), (8, 1, 64, 64, 10, 23, 41, "conv3_flat_k")]:
+        rng = np.random.default_rng(Ci + D)
+        x, w, b = exact_case(rng, N, Ci, Co, D * H * W)
+        xq = orc.f32_to_mx(bits, x, N, Ci, D * H * W)
+        lib.mi_conv_s2_direct(mode)
+        try:
+            got, _ = gpu_conv(xq, 3, N, Ci, D, H, W, w, b, Co, 3)
+        finally:
+            lib.mi_conv_s2_direct(-1)
+        assert kern in lib.mi_last_kernel().decode(), lib.mi_last_kernel().decode()
+        assert np.array_equal(got, orc.conv3(xq, 3, N, Ci, D, H, W, w, b, Co, 3, acc64=1)[0])

@@ -663,7 +663,7 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     // 28^3 (343) 23.9 / 16.6, 32^3 (512) 23.2 / 17.5; e2m1 at 24^3 18.5 / 11.3, at 32^3 18.8 / 16.1 and more records to add. (From 129 tiles on and with one channel tile only - 96 -> 64
     // at 24^3 24.4 / 16.4 -: the tests hold launches beyond that on the row kernel)
     // thin_ok: what the K-split kernel can take; a call it cannot - an activation, the thread's own choice of slices - stays on the row kernel
-    const bool thin_ok = !s2d && !act && a.wide && cout > 16 && !(osum && (cout / Go) % 4) && g_split < 0 && g_s2d < 0 && N <= 65535 && (size_t)D * H * W * 32 < ((size_t)1 << 31);
+    const bool thin_ok = !s2d && !act && a.wide && cout > 16 && !(osum && (cout / Go) % 4) && g_split < 0 && (stride == 1 || g_s2d < 0) && N <= 65535 && (size_t)D * H * W * 32 < ((size_t)1 << 31);
     const size_t thin_tiles = ((size_t)Dr * Ho * Wo + 63) / 64 * (size_t)nmt_all * N;
     const bool thin_row = thin_ok && a.row && nmt_all == 1 && a.nbt >= 3 && !rec && g_thin < 0 && thin_tiles > 128 && thin_tiles <= (fmt == 8 ? 2 * (size_t)thin_env : (size_t)thin_env);
     if (thin_row) a.row = false;
@@ -683,7 +683,7 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     if (flat_env < 0) flat_env = getenv("MI_CONV_FLAT") ? atoi(getenv("MI_CONV_FLAT")) : 1;      // tuning knob: 0 never
     const bool flat_ok = stride == 1 && a.wide && !act && nmt_all >= 2 && a.nbt % 2 == 0 && W <= flat_t<8>::WMAX && !(osum && (cout / Go) % 4) && N <= 65535 && (size_t)D * H * W < ((size_t)1 << 24);
     const size_t frun = ((size_t)Dr * Ho * Wo + 31) / 32, fwg = (frun + 3) / 4 * (size_t)((nmt_all + 1) / 2) * N;
-    a.flat = flat_ok && (g_flat > 0 || (g_flat < 0 && flat_env && !rec && g_thin < 0 && g_split < 0 && g_s2d < 0 && thin_tiles > (a.thin && nmt_all <= 4 ? 512u : 256u) &&
+    a.flat = flat_ok && (g_flat > 0 || (g_flat < 0 && flat_env && !rec && g_thin < 0 && g_split < 0 && thin_tiles > (a.thin && nmt_all <= 4 ? 512u : 256u) &&
                          (fmt == 8 ? a.nbt >= 2 : a.nbt >= 4 && frun <= 512) && fwg <= (a.nbt >= 8 ? 512u : 256u)));
     if (a.flat) { a.thin = a.row = a.row1 = a.areg = false; a.wrec = 1; }
     if (a.thin || a.flat) { big = false; MT = 1; NT = 2; a.CB = a.flat ? 2 : a.nbt; }
