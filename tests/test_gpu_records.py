@@ -29,27 +29,72 @@ def test_kernel_alone_and_inside_a_network(gpu, bits, N, Ci, Co, D, H, W, alone,
         finally:
             lib.mi_conv_keep_records(was)
         assert (alone if not keep else inside) in name and (not keep or alone not in name), name
-    assert np.array_equal(out[0][0], out[1][0])                                  # the codes do not depend on it
+    assert np.array_equal(out[0][0], out[1][0])                                  # exact operands: the codes do not depend on it
     assert np.abs(out[0][1] - out[1][1]).max() <= 1e-6 * np.abs(out[1][1]).max()
 
 
-def test_forward_takes_none_of_the_regrouping_kernels(gpu):
+@pytest.mark.parametrize("bits,N,Ci,Co,D,H,W,alone,inside", CASES)
+def test_what_separates_the_two(gpu, bits, N, Ci, Co, D, H, W, alone, inside):
+    """The kernels add the products in another order, too, not only the statistics: on operands of several magnitudes the fp32 outputs themselves differ in their
+    last bits with e4m3 (an order-free sum of the statistics alone would not bring such a network's bits together), and the statistics by as little. (e2m1 products, of
+    four significant bits at most, add up without a rounding here: what separates those two is the statistics' records.)"""
+    rng = np.random.default_rng(2 * Ci + Co + D)
+    x, w, b = rand_case(rng, N, Ci, Co, D * H * W)
+    x *= np.exp(2 * rng.standard_normal(x.shape)).astype(np.float32)
+    xdt = 3 if bits == 8 else 4
+    xq = orc.f32_to_mx(bits, x, N, Ci, D * H * W)
+    out = []
+    for keep in (0, 1):
+        was = lib.mi_conv_keep_records(keep)
+        try:
+            out.append(gpu_conv(xq, xdt, N, Ci, D, H, W, w, b, Co, 0, cbits=bits, Go=8, stats=True))
+        finally:
+            lib.mi_conv_keep_records(was)
+        assert (inside if keep else alone) in lib.mi_last_kernel().decode()
+    d = np.abs(out[0][0] - out[1][0])
+    assert (d.any() or bits == 4) and d.max() <= 2e-4 * np.abs(out[1][0]).max()                 # (the conv tolerance of the other kernels' tests)
+    assert np.abs(out[0][1] - out[1][1]).max() <= 1e-5 * np.abs(out[1][1]).max()
+
+
+def kernels_of(run):
+    """The conv kernels of what run() launches, in order."""
+    import ctypes as C
+    lib.mi_kernel_timing(1)
+    try:
+        run()
+        name = C.create_string_buffer(96)
+        n = lib.mi_kernel_timing_launch(-1, None, None, None, 0)
+        out = []
+        for i in range(n):
+            lib.mi_kernel_timing_launch(i, None, None, name, 96)
+            out.append(name.value.decode())
+    finally:
+        lib.mi_kernel_timing(0)
+    return out
+
+
+# windows whose 32 -> 32, 96 -> 32 and deep convs the three rules would take
+@pytest.mark.parametrize("N,D,W", [(1, 32, 32), (2, 56, 64)])
+def test_forward_takes_none_of_the_regrouping_kernels(gpu, N, D, W):
     from ufsm_amd.unet import UNet, make_cfg
-    N, D, W, cout = 2, 56, 64, 8
+    cout = 8
     net = UNet(make_cfg(4, [32, 64, 128, 256], G=8, head_out=cout, act_dt=8, prec=0), N, D, W, W, seed=5)
     ct = DevBuf.from_numpy(np.random.default_rng(1).integers(1, 255, (N, D, W, W), dtype=np.uint8))
     off = DevBuf.from_numpy(np.full(N * D, 9.0, np.float32))
-    y = []
+    y, names = [], []
     for mode in (-1, 0):                                                         # by size, and the flat kernel nowhere: the same bits
         lib.mi_conv_flat(mode)
         lg = DevBuf(N * cout * D * W * W * 4)
         try:
-            assert net.forward_ct(ct.ptr, 120.0, 0.02, off.ptr, off.ptr, 0, lg.ptr) == 0
+            names.append(kernels_of(lambda: net.forward_ct(ct.ptr, 120.0, 0.02, off.ptr, off.ptr, 0, lg.ptr)))
         finally:
             lib.mi_conv_flat(-1)
         lib.mi_sync()
         y.append(lg.to_numpy(np.uint32))
-    assert np.array_equal(y[0], y[1])
+    assert np.array_equal(y[0], y[1]) and names[0] == names[1]
+    # one block into one channel tile: the two 32 -> 32 convs of level 0 on the one-block row kernel; 96 -> 32 on the row kernel; no flat tiles anywhere
+    assert not any("conv3_flat_k" in k or "conv3_small_k" in k for k in names[0]), names[0]
+    assert sum("conv3_row1_k" in k for k in names[0]) >= 2 and any("conv3_row_k" in k and "blocks 3" in k for k in names[0]), names[0]
     assert lib.mi_conv_keep_records(0) == 0                                      # the setting is the forward's, not the thread's afterwards
 
 

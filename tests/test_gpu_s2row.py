@@ -1,5 +1,6 @@
 """The stride-2 row kernel (one input block, one channel tile; tiles of 4 rows of 32 output voxels, staged whole): exact operands equal the oracle byte for byte
-in every output type at the edges of its tiles and of odd volumes, and random operands give the bytes of the kernel that reads every tap's rows from memory."""
+in every output type at the edges of its tiles and of odd volumes, and random operands give the bytes of the two kernels it
+runs in the place of, in the inputs' format as well: the one that reads every tap's rows from memory and the general one, whose pairs are others."""
 import numpy as np
 import pytest
 
@@ -35,7 +36,11 @@ def test_stride_2_row_kernel(gpu, bits, N, Ci, Co, D, H, W):
         assert np.array_equal(run(2, xq, w, b, ydt), want), ydt
     x, w, b = rand_case(rng, N, Ci, Co, S)
     xq = orc.f32_to_mx(bits, x, N, Ci, S)
-    assert np.array_equal(run(2, xq, w, b, 0), run(1, xq, w, b, 0))            # the same pairs in the same order
+    # (the direct kernel: the same pairs in the same order. The general kernel adds tap by tap; on values of ordinary spread a block's 27 x 32 products are
+    # added without a rounding that depends on the order: these bytes are the network's, which must not move with a window's size)
+    for ydt in (0, xdt):
+        got = run(2, xq, w, b, ydt)
+        assert np.array_equal(got, run(1, xq, w, b, ydt)) and np.array_equal(got, run(0, xq, w, b, ydt)), ydt
 
 
 def test_taps_outside_read_zeros(gpu):
