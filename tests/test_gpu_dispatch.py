@@ -80,7 +80,7 @@ def test_statistics_of_a_range_of_planes(gpu, bits, N, Ci, Co, D, H, W, kern):
     y, _ = gpu_conv(xq, xdt, N, Ci, D, H, W, w, b, Co, 0, cbits=bits, Go=G, stats=True)
     assert kern in lib.mi_last_kernel().decode(), lib.mi_last_kernel().decode()
     v = y.reshape(N, G, Co // G, D, H * W).astype(np.float64)
-    for lo, hi in ((1, 2), (0, D - 1), (4, 0), (D, 0)):
+    for lo, hi in ((1, 2), (0, D - 1), (4, 0), (D, 0), (1 << 28, 0), (0, 1 << 28)):
         got, gs = gpu_conv(xq, xdt, N, Ci, D, H, W, w, b, Co, 0, cbits=bits, Go=G, stats=True, zrange=(lo, hi))
         assert kern in lib.mi_last_kernel().decode(), lib.mi_last_kernel().decode()
         assert np.array_equal(got, y), (lo, hi)

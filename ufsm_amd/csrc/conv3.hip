@@ -493,7 +493,7 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     a.N = N; a.D = D; a.H = H; a.W = W; a.Do = Do; a.Ho = Ho; a.Wo = Wo;
     a.zi0 = sp.Di ? sp.zi0 : 0; a.yD = sp.yD; a.yzo = sp.yD ? sp.yzo : 0;
     a.bias = b; a.Co = cout; a.y = y; a.ydt = ybf;
-    a.osum = osum; a.Go = Go; a.stored_stats = sp.stored_stats && ybf >= 3; a.zs0 = sp.zlo; a.zs1 = Do - sp.zhi;
+    a.osum = osum; a.Go = Go; a.stored_stats = sp.stored_stats && ybf >= 3; a.zs0 = sp.zlo < Do ? sp.zlo : Do; a.zs1 = sp.zhi < Do ? Do - sp.zhi : 0;      // (within the planes there are: some kernels count in voxels)
     a.ep_a = ep_a; a.ep_b = ep_b; a.act = act;
     // ---- tile shape: MT channel tiles of 32 per workgroup, NT voxel tiles of 32 per wavefront, MT * NT <= 8 accumulators ----
     const int nmt_all = (cout + 31) / 32;
@@ -718,9 +718,9 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     a.nmt_all = nmt_all; a.ncs = nmt_all / MT;
     a.ntx = a.row ? (Wo + 31) / 32 : (Wo + 15) / 16; a.nty = (Ho + 7) / 8; a.ntz = (Do + TZ - 1) / TZ;      // (the row kernel: 4 x 8 x 32 voxels per tile)
     a.ntiles = (unsigned)((size_t)a.ntx * a.nty * a.ntz * a.ncs * N);
-    if (a.thin || a.flat) {                                       // (their statistics records)
+    if (a.thin || a.flat) {                                       // (their statistics records; whether they leave planes out rides on the offset, below 32)
         const thin_runs_t t = mi_thin_runs(a.zi0, Do, Ho, Wo);
-        a.zc = t.off; a.ntx = t.step; a.nty = (int)t.recs; a.ntz = (int)t.runs; a.ntiles = (unsigned)(t.recs * nmt_all * N);
+        a.zc = t.off | (a.zs0 > 0 || a.zs1 < Do ? 32 : 0); a.ntx = t.step; a.nty = (int)t.recs; a.ntz = (int)t.runs; a.ntiles = (unsigned)(t.recs * nmt_all * N);
         a.ngrp = (unsigned)((t.runs + 3) / 4);
     }
     if (a.s2row) { a.ntx = (Wo + 31) / 32; a.nty = (Ho + 3) / 4; a.ntz = Do; a.ntiles = (unsigned)((size_t)a.ntx * a.nty * Do * N); }

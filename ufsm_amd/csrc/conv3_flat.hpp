@@ -38,7 +38,7 @@ __global__ void __launch_bounds__(512, 1) conv3_flat_k(const conv_args a) {
     const unsigned per = gridDim.x >> 3;
     const int g = (int)((blockIdx.x & 7u) * per + (blockIdx.x >> 3)), cs2 = (int)blockIdx.y, n = (int)blockIdx.z;
     if (4 * g >= a.ntz) return;
-    const int HW = a.H * a.W, Scol = a.Do * HW, off = a.zc;
+    const int HW = a.H * a.W, Scol = a.Do * HW, off = a.zc & 31;
     const size_t Sin = (size_t)a.D * HW;
     const int f0 = g * 128 - off;                             // first output voxel of the tile (negative: a z-range whose first run starts before it)
     // ---- weights ----
@@ -226,7 +226,7 @@ __global__ void __launch_bounds__(512, 1) conv3_flat_k(const conv_args a) {
     }
     const int col = f0 + j * 32 + r;
     const long long ovx[1] = {(unsigned)col < (unsigned)Scol ? (long long)col + (long long)a.yzo * HW : -1};
-    conv_epilogue<1, 1, OUT, false, false, true, false, true, 1, true, true, true>(a, sum, lds + m * 128, (unsigned)rec, n, cs, 0, 0, 0, 0, 0, j * 64 + lane, ovx, seg, step, col >= a.zs0 * HW && col < a.zs1 * HW);
+    conv_epilogue<1, 1, OUT, false, false, true, false, true, 1, true, true, true>(a, sum, lds + m * 128, (unsigned)rec, n, cs, 0, 0, 0, 0, 0, j * 64 + lane, ovx, seg, step, a.zc > 31, f0 + j * 32);
 }
 template <int FMT, int OUT>
 static void launch_flat(const conv_args &a, size_t smem) {

@@ -116,15 +116,15 @@ struct conv_args {
     const void *sx; int sxdt, sCi;
     const float *sgam, *sbet, *smean, *srstd; int sG;
     int szs, szo, sns;            // slab-local statistics of the few-channel kernels' input (gnp_t zs / zo / ns; sns 0: per sample): plane z reads row n sns + clamp((z + szo) / szs)
-    int zc; unsigned ngrp;             // consecutive z tiles a workgroup walks, workgroups with work
+    int zc; unsigned ngrp;             // consecutive z tiles a workgroup walks, workgroups with work (K-split and flat kernel: zc is the idle voxels of the first run, + 32 for statistics of a range of planes)
     bool big;                          // the wide kernel takes the launch (MT 4, or MT 2 with NT 4)
     bool areg;                         // the persistent small-channel kernel (one channel tile, one input block, weights in registers) takes the launch
     bool row;                          // the row kernel (one channel tile, any number of input blocks, 4 x 8 x 32 voxel tiles) takes the launch
     bool row1;                         // ... its one-input-block form (weights in registers, the two halves of the workgroup half a tile apart)
-    int wrec;                          // statistics records of a tile and channel slice: 1, or one per wavefront (the one-block row kernel 8, the small-channel kernel on that kernel's launches 4)
     bool thin;                         // the K-split kernel of the launches of few output voxels takes the launch
     bool s2row;                        // the stride-2 row kernel takes the launch (one block, one channel tile)
     bool flat;                         // ... the one of about a tile of 128 voxels x 64 channels per CU (flat runs, the taps split over the wavefronts)
+    unsigned char wrec;                // statistics records of a tile and channel slice: 1, or one per wavefront (the one-block row kernel 8, the small-channel kernel on that kernel's launches 4)
 };
 
 template <int FMT> struct fmt_t;
@@ -272,11 +272,11 @@ __device__ __forceinline__ void conv_epi_consts(const conv_args &a, unsigned cha
 // holds voxel (oz0 + lz, oy0 + ly0 + j, ox0 + r) of a 32-voxel run along x
 // WPART: every wavefront writes its own statistics record (record tile NW + wave: the reduce kernel then sees NW records per tile) and the
 // epilogue has no workgroup barrier and touches no LDS scratch, so the wavefronts of a workgroup need not run it at the same time (one channel tile)
-// SEG: the wavefront's record ends before lane seg of the run and another begins (every seg_step lanes from there on; seg past 32: one record); seg_in: the
-// statistics cover the lane's voxel (its plane lies in [zs0, zs1): the caller's voxel mapping knows no planes here)
+// SEG: the wavefront's record ends before lane seg of the run and another begins (every seg_step lanes from there on; seg past 32: one record); rng: the
+// statistics cover the planes [zs0, zs1) only, whose lanes are found by the output voxel f0 of lane 0
 template <int MT, int NT, int OUT, bool EPI, bool PIN = false, bool W32 = false, bool FULL = false, bool NOCH = false, int NW = 4, bool ROW = false, bool WPART = false, bool SEG = false>
 __device__ __forceinline__ void conv_epilogue(const conv_args &a, v16f (&acc)[MT][NT], unsigned char *lds, unsigned tile, int n, int cs,
-                                              int oz0, int oy0, int ox0, int lz, int ly0, int tid, const long long *ovx = nullptr, int seg = 33, int seg_step = 0, bool seg_in = true) {
+                                              int oz0, int oy0, int ox0, int lz, int ly0, int tid, const long long *ovx = nullptr, int seg = 33, int seg_step = 0, bool rng = false, int f0 = 0) {
     const int lane = tid & 63, wave = tid >> 6, r = lane & 31, h = lane >> 5;
     // accumulator layout of the 32x32 MFMA: lane (r = voxel within the tile, h), register i -> row (i & 3) + 4 h + 8 (i >> 2) = channel 16 h + i
     const size_t So = (size_t)(a.yD ? a.yD : a.Do) * a.Ho * a.Wo;      // voxels per channel plane of the output tensor
@@ -418,8 +418,17 @@ __device__ __forceinline__ void conv_epilogue(const conv_args &a, v16f (&acc)[MT
     if constexpr (WPART) {
         static_assert(!WPART || (MT == 1 && NOCH), "per-wavefront statistics records: one channel tile, no per-channel records");
         if (stats) {
+            int s0 = 0, s1 = 32;
+            if (SEG && rng) {
+                // (read here, through the arguments' own address: an argument that is named is loaded with the others at the kernel's start, whose first use then waits for one load more -
+                // 0.12 us of 9.4 in each of the thirteen K-split launches of a 32^3 window's forward, which have no range)
+                typedef const int __attribute__((address_space(4))) *karg_t;
+                karg_t z = (karg_t)__builtin_amdgcn_kernarg_segment_ptr();
+                asm volatile("" : "+s"(z));
+                s0 = z[offsetof(conv_args, zs0) / 4] * a.Ho * a.Wo - f0; s1 = z[offsetof(conv_args, zs1) / 4] * a.Ho * a.Wo - f0;
+            }
             for (int lo = 0, rec = 0;; rec++) {
-                const bool in = !SEG || (seg_in && r >= lo && r < seg);
+                const bool in = !SEG || (r >= max(lo, s0) && r < min(seg, s1));
                 float v[8];
 #pragma unroll
                 for (int q4 = 0; q4 < 4; q4++) { v[q4 * 2] = in ? qs[0][q4] : 0.f; v[q4 * 2 + 1] = in ? qss[0][q4] : 0.f; }
