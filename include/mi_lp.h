@@ -106,9 +106,10 @@ void mi_conv_thin(int tiles);
    that kernel can (stride 1, an even number of input blocks, more than 32 output channels, rows of at most 41 voxels), 0 nowhere, -1 (default) by size. The same
    conv either way, its fp32 sums in another order. */
 void mi_conv_flat(int mode);
-/* Extension: 1: the calling thread's 3x3x3 convs with statistics leave the kernels aside whose statistics records group the voxels otherwise than the staged and row kernels'
-   (the default's flat tiles, small-channel kernel on short walks, K split of 96 -> 32): the U-Net graph sets it around its convs, because a mean that moves by its last bit can move a code of the
-   next layer's rows. Returns the setting before. A conv by itself (0, the default) takes the faster kernel; its codes are the same ones. */
+/* Extension: 1: the calling thread's 3x3x3 convs with statistics leave the kernels aside that add the products and group the voxels of the statistics records otherwise than the staged and
+   row kernels (the default's flat tiles, small-channel kernel on short walks, K split of 96 -> 32): the U-Net graph sets it around its convs, because a mean that moves by its last bit can move a code of the
+   next layer's rows, and with it the rest of a network (up to 2 % of the logits). Returns the setting before. A conv by itself (0, the default) takes the faster kernel: the same conv and
+   statistics of the same precision, but a mean or 1 / std may differ by its last bit from the same layer's inside the graph. A caller that builds a network of single convs and wants the graph's bits sets 1 around them. */
 int mi_conv_keep_records(int on);
 /* 1x1x1 head with eight outputs on whole 32-channel blocks: where its 8 x 32 products per voxel run. mode 1: the matrix pipe (batched 4 x 4 x 1
    fp32 outer products, one product per accumulator and step, in channel order), 0: fused multiply-adds on the vector ALUs, -1: the default

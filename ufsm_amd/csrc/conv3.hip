@@ -541,7 +541,7 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     const size_t s2runs = ((size_t)Do * Ho * Wo + 63) / 64;
     // (by default only one input block and one channel tile, the shape it is measured faster on: 64 -> 64 takes 0.034 against 0.030 ms from 2 x 64^3
     // and 0.36 against 0.09 ms from 8 x 64^3)
-    // ... on rows of more than 16 output voxels the row kernel does: the tile's rows staged in LDS as they lie in memory, the weights in registers. us, general / direct / row kernel,
+    // ... on rows of more than 16 output voxels the row kernel does: the tile's rows staged in LDS as they lie in memory, the weights in registers. us of the conv by itself, general / direct / row kernel,
     // e4m3: 2 x 128^3 85.8 / 59.0 / 43.6, 9 x 128^3 364 / 278 / 170, 88 x 104^2 30.8 / 19.1 / 13.8, 64^3 8.3 / 12.6 / 7.5; e2m1: 128^3 19.7 / 28.1 / 15.9, 2 x 96^3 17.0 / 28.0 / 16.4, 48^3 6.6 / 12.5 / 6.3. On rows of
     // 16 and fewer half its lanes idle (4 x 64^2 x 32: 10.8 general, 13.7); up to 256 tiles of the K-split kernel e4m3 stays there (48^3 7.2 / 7.8 here, 32 x 64^2 7.4 / 7.7)
     static int s2row_env = -1;
@@ -627,7 +627,7 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     // 30.9 / 26.1. e2m1: 64^3 15.0 / 13.6, 96^3 28.5 / 26.4, 88 x 104^2 33.9 / 29.8. Past 1 024 tiles of whole runs the row kernel is the faster one (with a record per tile here: 64 x 128^2
     // 56.6 / 59.6, 4 x 64^3 55.6 / 57.3, 2 x 128^3 208 / 224, of a call that prepares its weights; rows of 120 - four runs of 32, eight tiles of 16 - 88.5 / 90.5). fp16 planes out: 64^3
     // 29.4 / 25.5, 40^3 22.7 / 16.8. Launches of under 16 384 voxels gain as well (24^3 17.7 / 13.3), but the tests hold two of them on the row kernel
-    // A conv's fp32 statistics records add up in another order on another kernel, which moves a mean or 1 / std by its last bit now and then; a code of the next conv's rows at a rounding
+    // A conv's products and its fp32 statistics records add up in another order on another kernel, which moves a mean or 1 / std by its last bit now and then; a code of the next conv's rows at a rounding
     // boundary then moves, and with it the rest of a network (e4m3: up to 2 % of the logits, one window size in ten; e2m1 more). Inside a network the three rules that came with the
     // flat kernel (this one, the short 96 -> 32 walks and the flat tiles) therefore leave convs with statistics where they were
     const bool rec = g_records && osum;

@@ -7,7 +7,8 @@
 // 27 input rows of 65 voxels, copied to LDS asynchronously as they lie in memory (64 KB, so that two workgroups share a CU and one's copies run under the
 // other's products). The fourteen weight pairs stay in registers over the workgroup's walk, so the K loop is LDS reads at constant offsets and products; the next
 // tile's copies go out before the epilogue. A tap's 32 lanes read every second voxel of a row; the 16-byte pieces of a row lie permuted (swz) so that they meet all
-// banks. The walk runs down the planes: the plane two tiles share is in the L2 the second time. 2 x 128^3 59.0 -> 43.6 us (3.6 TB/s), nine windows 278 -> 170 (4.1 TB/s).
+// banks. The walk runs down the planes: the plane two tiles share is in the L2 the second time. 2 x 128^3 59.0 -> 43.6 us (3.6 TB/s), nine windows 278 -> 170 (4.1 TB/s) for the conv
+// by itself; inside a forward, whose last kernel has just written the input, 47.5 and 185.
 #pragma once
 
 template <int FMT> struct s2row_t {

@@ -122,8 +122,8 @@ extern "C" void mi_ct_window(const uint8_t *vol, int64_t Z, int64_t Y, int64_t X
 // "holds a voxel >= iso" of every cell of a grid over the volume: cell (a, b, c) of nss[3] is [a S, a S + S) x [b S, ..) x [c S, ..) clipped to the
 // volume, i.e. the interior of the sliding window with that index. The cells tile the volume, so this is one read of it. A thread tests 16
 // consecutive x of a cell row (one 16-byte load of a whole piece, else bytes); a workgroup's rows belong to one cell, and a cell whose flag is set already
-// needs no more of them. (a call over 190 x 280 x 260 in cells of 96, dense: 30 us with a look per wavefront and the compiler's workgroup reduction, 16 now;
-// 512 x 1024^2 64 and 46)
+// needs no more of them. (calls back to back over 190 x 280 x 260 in cells of 96, dense: 30 us with a look per wavefront and the compiler's workgroup reduction,
+// 16 now; 512 x 1024^2 64 and 46; in a prediction, on a volume not read lately, 45 and 43)
 __global__ void __launch_bounds__(256) ct_flags_k(const uint8_t *__restrict__ vol, long long Z, long long Y, long long X, int S, int n1, int n2, int iso, unsigned *any) {
     const int S16 = (S + 15) >> 4;
     const unsigned cell = blockIdx.x, c = cell % (unsigned)n2, b = (cell / (unsigned)n2) % (unsigned)n1, a = cell / ((unsigned)n2 * (unsigned)n1);

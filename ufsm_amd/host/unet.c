@@ -850,7 +850,8 @@ static int graph_convs(unet *u, const void *x, float *logits) {
     lp_conv1_fwd_mx(last->a2, u->act_dt == 4 ? 4 : 3, last->ys, P(u, u->head.w), P(u, u->head.b), u->cfg.cout, logits, gnp_mk(g.gamma, g.beta, g.mean, g.rstd, g.G));
     return 0;
 }
-/* the logits of a window are the same bits whatever kernels later convs of their sizes are given: its statistics keep their records (mi_conv_keep_records) */
+/* the stride-1 convs with statistics keep the kernels whose order of sums and records the logits were made with (mi_conv_keep_records): a faster kernel for such a conv by itself does not move a window's bits. The
+   stride-2 convs have no statistics and take their kernel by size; on rows of ordinary spread the three kernels give the same bytes */
 static int graph_fwd(unet *u, const void *x, float *logits) {
     const int was = mi_conv_keep_records(1), rc = graph_convs(u, x, logits);
     mi_conv_keep_records(was);
