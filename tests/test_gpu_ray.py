@@ -73,6 +73,26 @@ def test_ray_maps_at_the_edges_of_a_tokens_lanes(gpu, D, Hh, W, mult):
     test_ray_maps(gpu, D, Hh, W, mult)
 
 
+@pytest.mark.parametrize("u0", [-np.inf, np.inf, 1e30])
+def test_a_ray_that_starts_nowhere_touches_no_token_past_its_slots(gpu, u0):
+    """One ray of the table starts at an infinite or far coordinate: its samples clamp to the plane's edge, the tokens list samples of the ray's own length only and the other
+    rays' weights are what they were; the scatter stays finite."""
+    D, Hh, W, mult = 6, 5, 7, 2.0
+    axr = make_axr(1, D, Hh, W, (0,), (0,))
+    t = DevRays(1, D, Hh, W, mult, axr)
+    ws = t.bufs["wsum"].to_numpy(np.float32, (t.Tg,)).reshape(D, Hh, W)
+    q = int(t.R.Nt) * 2                                                            # the first ray of plane 2
+    ray = t.ray_h.copy(); ray[0, q, 0] = u0
+    lib.mi_h2d(t.bufs["ray"].ptr, ray.ctypes.data, ray.nbytes)
+    lib.at_rays_setup(C.byref(t.R)); LP.check()
+    w2 = t.bufs["wsum"].to_numpy(np.float32, (t.Tg,)).reshape(D, Hh, W)
+    assert np.array_equal(np.delete(w2, 2, 0), np.delete(ws, 2, 0)) and np.isfinite(w2).all()
+    y = np.random.default_rng(1).standard_normal((t.Tr, 8)).astype(np.float32)
+    dy, ds = DevBuf.from_numpy(y), DevBuf.from_numpy(np.full((t.Tg, 8), np.nan, np.float32))
+    lib.at_ray_scatter(C.byref(t.R), dy.ptr, ds.ptr, 8, 1); LP.check()
+    assert np.isfinite(ds.to_numpy(np.float32)).all()
+
+
 def test_scroll_pos_on_the_device(gpu):
     D, Hh, W, n, nreg = 5, 6, 4, 3, 2
     axr = make_axr(n, D, Hh, W, (1, 0, 2), (0, 1, 2))

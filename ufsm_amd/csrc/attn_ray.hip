@@ -150,7 +150,7 @@ __global__ void __launch_bounds__(256) ray_inverse_k(ray_geo G, const float *__r
             const int L = min((int)rr[6], G.Nr);
             if (L > 0) {
                 const float ist = ((float)ua - rr[0]) * rr[2] + ((float)vb - rr[1]) * rr[3];      // the token's projection on the ray, in samples
-                const int i0 = max(0, (int)ceilf(ist - 2.2f)), i1 = min(L - 1, (int)floorf(ist + 2.2f));      // (at most five)
+                const int i0 = min(max(0, (int)ceilf(ist - 2.2f)), L), i1 = min(L - 1, (int)floorf(ist + 2.2f));      // (at most five; none for a ray that starts at infinity, and i0 + 4 stays a number)
 #pragma unroll
                 for (int q = 0; q < 5; q++) {
                     if (i0 + q > i1) continue;
