@@ -109,6 +109,30 @@ def test_conv_past_4gib(gpu, name, Ci, Co, dims, N, stride, bits, gn, kpart):
         assert np.allclose(sl[0], wsum[0], rtol=1e-6) and np.array_equal(sl[0], sl[N - 1]) and np.array_equal(sl[0], sl[N // 2])
 
 
+def test_prepared_weights_past_2_gib(gpu):
+    """8192 -> 10240 channels on a handful of voxels: 2.3 GB of prepared weights, past the flat kernel's 32-bit offsets, stay off it (also where it is asked for), and the last
+    channels' taps are read where they lie."""
+    Ci, Co, D, H, W = 8192, 10240, 1, 2, 3
+    S = D * H * W
+    x = np.zeros((1, Ci, S), np.float32); x[0, Ci - 1] = np.arange(1, S + 1)
+    w = DevBuf(Co * Ci * 27 * 4)                                                  # zeros, but for the centre and one neighbour tap of the last channels
+    row = np.zeros(27, np.float32); row[13], row[14] = 0.5, 2.0
+    lib.mi_h2d(w.ptr + ((Co - 1) * Ci + Ci - 1) * 27 * 4, row.ctypes.data, row.nbytes)
+    xq = DevBuf.from_numpy(orc.f32_to_mx(8, x, 1, Ci, S))
+    want = np.zeros((Co, S), np.float32)
+    v = x[0, Ci - 1].reshape(H, W); want[-1] = (0.5 * v + 2.0 * np.pad(v[:, 1:], ((0, 0), (0, 1)))).reshape(-1)
+    for mode in (-1, 1):
+        y = DevBuf(Co * S * 4)
+        lib.mi_conv_flat(mode)
+        try:
+            assert lib.lp_conv_fwd_f8(xq.ptr, 3, shape5(1, Ci, D, H, W), w.ptr, None, Co, y.ptr, 0, gnp_t(), None, 0, split_t()) == 0
+        finally:
+            lib.mi_conv_flat(-1)
+        LP.check()
+        assert "conv3_flat_k" not in lib.mi_last_kernel().decode(), lib.mi_last_kernel().decode()
+        assert np.array_equal(y.to_numpy(np.float32, (Co, S)), want)
+
+
 def test_elementwise_past_4gib(gpu):
     """Converters, GroupNorm + SiLU apply, add, the materialising upsample and the head on tensors past 4 GiB."""
     rng = np.random.default_rng(77)

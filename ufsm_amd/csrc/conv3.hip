@@ -681,7 +681,8 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     // tensor's voxels count, not a z-range's
     static int flat_env = -1;
     if (flat_env < 0) flat_env = getenv("MI_CONV_FLAT") ? atoi(getenv("MI_CONV_FLAT")) : 1;      // tuning knob: 0 never
-    const bool flat_ok = stride == 1 && a.wide && !act && nmt_all >= 2 && a.nbt % 2 == 0 && W <= flat_t<8>::WMAX && !(osum && (cout / Go) % 4) && N <= 65535 && (size_t)D * H * W < ((size_t)1 << 24);
+    const bool flat_ok = stride == 1 && a.wide && !act && nmt_all >= 2 && a.nbt % 2 == 0 && W <= flat_t<8>::WMAX && !(osum && (cout / Go) % 4) && N <= 65535 && (size_t)D * H * W < ((size_t)1 << 24) &&
+                         ((size_t)27 * (a.nbt / 2) + 2) * nmt_all * WTILE < ((size_t)1 << 31);      // (its weight offsets are 32 bits)
     const size_t frun = ((size_t)Dr * Ho * Wo + 31) / 32, fwg = (frun + 3) / 4 * (size_t)((nmt_all + 1) / 2) * N;
     a.flat = flat_ok && (g_flat > 0 || (g_flat < 0 && flat_env && !rec && g_thin < 0 && g_split < 0 && thin_tiles > (a.thin && nmt_all <= 4 ? 512u : 256u) &&
                          (fmt == 8 ? a.nbt >= 2 : a.nbt >= 4 && frun <= 512) && fwg <= (a.nbt >= 8 ? 512u : 256u)));
