@@ -2,7 +2,7 @@
 import numpy as np
 import pytest
 
-from ufsm_amd import lib
+from ufsm_amd import lib, LP, DevBuf, shape5, gnp_t, split_t
 import orc
 from gpuutil import code_mismatch_fraction
 from test_gpu_conv import exact_case, rand_case, gpu_conv
@@ -104,3 +104,33 @@ def test_the_stride_2_choice_leaves_stride_1_alone(gpu, mode):
             lib.mi_conv_s2_direct(-1)
         assert kern in lib.mi_last_kernel().decode(), lib.mi_last_kernel().decode()
         assert np.array_equal(got, orc.conv3(xq, 3, N, Ci, D, H, W, w, b, Co, 3, acc64=1)[0])
+
+
+@pytest.mark.parametrize("bits,Ci,Co,D,H,W,kern", [(8, 64, 64, 13, 5, 7, "conv3_thin_k"), (4, 96, 64, 12, 6, 7, "conv3_thin_k"), (8, 96, 32, 14, 28, 31, "conv3_thin_k"), (8, 128, 64, 15, 21, 33, "conv3_flat_k"),
+                                                   (4, 128, 64, 17, 29, 31, "conv3_flat_k")])
+def test_overlapping_slabs_that_count_their_own_planes(gpu, bits, Ci, Co, D, H, W, kern):
+    """A tensor in slabs of four planes that compute one more plane on either side and leave it out of their statistics: the whole call's outputs, plane by plane,
+    and its sums (planes of odd voxel counts: a slab's runs start inside a run of the whole tensor's)."""
+    rng = np.random.default_rng(Ci + D + W)
+    S, G, xdt = D * H * W, 8, 3 if bits == 8 else 4
+    x, w, b = rand_case(rng, 1, Ci, Co, S)
+    x *= np.exp(2 * rng.standard_normal(x.shape)).astype(np.float32)
+    xq = orc.f32_to_mx(bits, x, 1, Ci, S)
+    y, ws = gpu_conv(xq, xdt, 1, Ci, D, H, W, w, b, Co, 0, cbits=bits, Go=G, stats=True)
+    assert kern in lib.mi_last_kernel().decode(), lib.mi_last_kernel().decode()
+    dx, dw, db = DevBuf.from_numpy(xq), DevBuf.from_numpy(w), DevBuf.from_numpy(b)
+    sums, out = DevBuf(G * 2 * 24), DevBuf(G * 2 * 8)
+    lib.mi_gn_sums_zero(sums.ptr, 2 * G)
+    for z in range(0, D, 4):
+        z0, z1, own = max(z - 1, 0), min(z + 5, D), min(z + 4, D)
+        sp = split_t(); sp.zi0, sp.Di, sp.zlo, sp.zhi = z0, D, z - z0, z1 - own
+        dy = DevBuf(Co * (z1 - z0) * H * W * 4)
+        f = lib.lp_conv_fwd_f8 if bits == 8 else lib.lp_conv_fwd_f4
+        assert f(dx.ptr, xdt, shape5(1, Ci, z1 - z0, H, W), dw.ptr, db.ptr, Co, dy.ptr, 0, gnp_t(), sums.ptr, G, sp) == 0
+        assert kern in lib.mi_last_kernel().decode(), lib.mi_last_kernel().decode()
+        assert np.array_equal(dy.to_numpy(np.float32, (Co, z1 - z0, H * W)), y.reshape(Co, D, H * W)[:, z0:z1]), z
+    lib.mi_gn_sums_get(sums.ptr, 2 * G, out.ptr)
+    LP.check()
+    v = np.abs(y.astype(np.float64)).reshape(G, -1)
+    # (fp32 within records of 32 voxels x 4 channels, cut elsewhere in the slabs)
+    assert np.abs(out.to_numpy(np.float64, (G, 2)) - ws[0]).max() <= 1e-5 * max(v.sum(1).max(), (v * v).sum(1).max())
