@@ -72,6 +72,30 @@ def test_random_operands_within_tolerance(gpu, up, bits, xbits, gn):
     assert err < (3e-2 if gn and bits == 4 else 1e-3 if bits == 8 else 1e-5), err
 
 
+@pytest.mark.parametrize("up", [0, 1])
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("Ci,Co,dims,kind", [
+    (96, 160, (2, 6, 22), 1), (224, 40, (4, 2, 8), 1), (160, 96, (2, 10, 26), 1),      # odd block counts (a K pair without its second block), channel tiles that no slice of 2 or 4 fills, columns past a multiple of 256
+    (256, 32, (2, 2, 2), 1), (64, 256, (8, 8, 16), 1),                                  # the smallest launch; every channel tile a chunk of its own
+    (288, 32, (2, 4, 6), 0), (64, 16, (4, 4, 6), 0)])                                   # past the pairs that the transposed conv holds; 16-channel rows: the general kernel
+def test_row_kernels_at_their_edges(gpu, up, bits, Ci, Co, dims, kind):
+    """The kernels that write MX rows of 32 channels (one wavefront per 32 columns): equal to the oracle byte for byte on exact operands, and not taken outside their range."""
+    rng = np.random.default_rng(7 * Ci + Co + up)
+    D, H, W = dims
+    N, S = 2, D * H * W
+    x = refnp.gen_exact(rng, (N, Ci, S))
+    w = refnp.gen_exact(rng, (Ci, Co, 8), block_axis=0) if up else refnp.gen_exact(rng, (Co, Ci, 8))
+    b = rng.integers(-8, 9, Co).astype(np.float32) * 0.25
+    xdt = 3 if bits == 8 else 4
+    xq = orc.f32_to_mx(bits, x, N, Ci, S)
+    for ydt in (3, 4):
+        want = orc.conv2(xq, xdt, N, Ci, D, H, W, w, b, Co, ydt, up, cbits=bits, acc64=1)
+        got = gpu_conv2(up, xq, xdt, N, Ci, D, H, W, w, b, Co, ydt, bits)
+        assert np.array_equal(got, want), ydt
+        rows = ("conv2_up_k" if up else "conv2_down_k") in lib.mi_last_kernel().decode()
+        assert rows == (kind == 1 or (not up and Co > 16))
+
+
 def test_config2_layers_at_full_size(gpu):
     """BASELINE configs[2]'s stride-2 layers in MX-fp4: the 2x2x2 down conv 128 -> 256 on 64^3 (N 2) and the 2x2x2 transposed conv 256 -> 128 on
     32^3 (N 2), inputs uniform[-3, 3], Kaiming weights, MX-fp4 in and out, against the oracle (fp64 accumulation of the same e2m1 operands: fp32

@@ -75,10 +75,21 @@ static int conv2_dispatch(const char *who, int up, int bits, const void *x, int 
     a.epi_o = 0; a.red_o = (unsigned)((size_t)3 * MT * 32 * sizeof(float));
     const size_t smem = a.red_o + 1024;
     const long long Scol = up ? (long long)S : (long long)a.Do * a.Ho * a.Wo;
+    const int out = ybf == 3 ? 8 : ybf == 4 ? 4 : 0;
+    // the transposed conv into MX rows of 32 channels, its rows' fragments held in registers: up to 256 input channels, and 1 024 output channels (their biases lie in LDS). The
+    // kernel counts voxels in 32 bits and writes 16 bytes of a row and two scale bytes at a time
+    if (up && out && cout > 16 && nbp <= 2 * CU2_NP && nmt_all <= CU2_MT && S < (size_t)1 << 27 && ((size_t)y & 15) == 0) {
+        const size_t sm = conv2_up_lds(a, fmt);
+        if (fmt == 8) conv2_launch_f8(out, up, 0, a, dim3(1), sm); else conv2_launch_f4(out, up, 0, a, dim3(1), sm);
+        return 0;
+    }
+    if (!up && out && cout > 16 && S < (size_t)1 << 27 && a.ncs <= 65535) {
+        if (fmt == 8) conv2_launch_f8(out, up, -MT, a, dim3(1), 0); else conv2_launch_f4(out, up, -MT, a, dim3(1), 0);
+        return 0;
+    }
     const long long gx = ((Scol + 31) / 32 + 7) / 8;         // 4 wavefronts x 2 tiles of 32 columns per workgroup
     if (gx > 0x7fffffffLL || a.ncs > 8191) mi_die("%s: launch grid", who);
     const dim3 grid((unsigned)gx, (unsigned)(up ? 8 * a.ncs : a.ncs), (unsigned)N);      // (up: one tap per workgroup)
-    const int out = ybf == 3 ? 8 : ybf == 4 ? 4 : 0;
     if (fmt == 8) conv2_launch_f8(out, up, MT, a, grid, smem); else conv2_launch_f4(out, up, MT, a, grid, smem);
     return 0;
 }

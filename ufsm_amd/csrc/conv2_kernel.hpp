@@ -279,8 +279,11 @@ static void launch_conv2_mt(const conv_args &a, dim3 grid, size_t smem) {
     MICK();
     snprintf(g_last_kernel, sizeof g_last_kernel, "conv2_mx_k<fmt %d, out %d, up %d, MT %d> blocks %d grid %u x %u x %u", FMT, OUT, (int)UP, MT, a.nbs[0], grid.x, grid.y, grid.z);
 }
+#include "conv2_down.hpp"
 template <int FMT>
 static void launch_conv2(int out, int up, int MT, const conv_args &a, dim3 grid, size_t smem) {
+    if (MT < 0) { if (out == 8) launch_conv2_down_t<FMT, 8>(a, -MT); else launch_conv2_down_t<FMT, 4>(a, -MT); return; }
+    if (MT == 0) { if (out == 8) launch_conv2_up_t<FMT, 8>(a, smem); else launch_conv2_up_t<FMT, 4>(a, smem); return; }      // (the dispatch's word for the kernel that keeps its rows)
 #define C2_MT(OUT, UP) do { if (MT == 4) launch_conv2_mt<FMT, OUT, UP, 4>(a, grid, smem); else if (MT == 2) launch_conv2_mt<FMT, OUT, UP, 2>(a, grid, smem); else launch_conv2_mt<FMT, OUT, UP, 1>(a, grid, smem); } while (0)
 #define C2_UP(OUT) do { if (up) C2_MT(OUT, true); else C2_MT(OUT, false); } while (0)
     if (out == 8) C2_UP(8); else if (out == 4) C2_UP(4); else C2_UP(0);
