@@ -56,6 +56,32 @@ def test_what_separates_the_two(gpu, bits, N, Ci, Co, D, H, W, alone, inside):
     assert np.abs(out[0][1] - out[1][1]).max() <= 1e-5 * np.abs(out[1][1]).max()
 
 
+@pytest.mark.parametrize("xdt", [3, 4])
+@pytest.mark.parametrize("Ci,Co,N", [(192, 192, 6), (64, 96, 12)])
+def test_a_slice_of_three_channel_tiles_in_one_workgroup_or_three(gpu, xdt, Ci, Co, N):
+    """96 and 192 output channels in e2m1: few tiles run a channel tile per workgroup, more run three. A sample's codes and sums are the same bits either way (operands of
+    several magnitudes; the squares' sums are what a differently compiled epilogue would move)."""
+    rng = np.random.default_rng(Ci + Co + xdt)
+    D, H, W = 8, 16, 24                                                         # 16 tiles of 2 x 8 x 16 per sample and slice; past the K-split kernel's launches
+    if Co == 96:
+        D = 16
+    S = D * H * W
+    x, w, b = rand_case(rng, N, Ci, Co, S)
+    x *= np.exp(2 * rng.standard_normal(x.shape)).astype(np.float32)
+    was = lib.mi_conv_keep_records(1)
+    try:
+        xq = orc.f32_to_mx(8 if xdt == 3 else 4, x, N, Ci, S)
+        y, gs = gpu_conv(xq, xdt, N, Ci, D, H, W, w, b, Co, 0, cbits=4, Go=8, stats=True)
+        assert "MT 3" in lib.mi_last_kernel().decode(), lib.mi_last_kernel().decode()
+        for n in (0, N - 1):
+            q1 = orc.f32_to_mx(8 if xdt == 3 else 4, x[n:n + 1], 1, Ci, S)
+            y1, g1 = gpu_conv(q1, xdt, 1, Ci, D, H, W, w, b, Co, 0, cbits=4, Go=8, stats=True)
+            assert "MT 1" in lib.mi_last_kernel().decode(), lib.mi_last_kernel().decode()
+            assert np.array_equal(np.asarray(y1).reshape(-1), np.asarray(y).reshape(N, -1)[n]) and np.array_equal(np.asarray(g1).reshape(-1), np.asarray(gs).reshape(N, -1)[n])
+    finally:
+        lib.mi_conv_keep_records(was)
+
+
 def kernels_of(run):
     """The conv kernels of what run() launches, in order."""
     import ctypes as C

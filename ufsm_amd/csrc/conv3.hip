@@ -590,11 +590,23 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     // LDS of a workgroup holding CB input blocks: weight ring, pair table, halo rows and scale words. Prefer the largest CB that
     // still lets two workgroups share a CU (160 KB): the second one computes while the first stages its halo or runs its epilogue.
     // The wide kernel has a fixed layout: ring of two slots of two pairs, three halo slots of one block, two pair tables.
-    const int PPS = MT == 1 ? 7 : MT == 2 ? 2 : 1;        // pairs per ring stage of the general kernel
-    auto lds_bytes = [&](int cb) { return (size_t)2 * PPS * MT * (WTILE + 256) + (size_t)(((27 * cb + 1) >> 1) + 2) * 32 + (size_t)cb * TT * (RB + 4); };
-    int cb2 = 0, cb1 = 0;
-    for (int cb = 1; cb <= a.nbt; cb++) { if (lds_bytes(cb) <= 80 * 1024 - 2816) cb2 = cb; if (lds_bytes(cb) <= 160 * 1024 - 3072) cb1 = cb; }   // (room for the epilogue's constants and scratch)
-    int cbmax = cb2 ? cb2 : cb1;
+    auto lds_of = [&](int mt, int cb) { return (size_t)2 * (mt == 1 ? 7 : mt == 2 ? 2 : 1) * mt * (WTILE + 256) + (size_t)(((27 * cb + 1) >> 1) + 2) * 32 + (size_t)cb * TT * (RB + 4); };      // (a ring stage of the general kernel: 7, 2 or 1 pairs)
+    int cb1 = 0;
+    auto cb_of = [&](int mt) {
+        int cb2 = 0; cb1 = 0;
+        for (int cb = 1; cb <= a.nbt; cb++) { if (lds_of(mt, cb) <= 80 * 1024 - 2816) cb2 = cb; if (lds_of(mt, cb) <= 160 * 1024 - 3072) cb1 = cb; }   // (room for the epilogue's constants and scratch)
+        return cb2 ? cb2 : cb1;
+    };
+    // Three channel tiles per workgroup (96, 192 channels) on fewer than 192 workgroups: a tile each, three times the workgroups, if its chunks of input blocks - the order of K - stay
+    // what they are (e2m1; the e4m3 ring leaves room for fewer blocks). The records are a tile's, quad by quad, either way. A 192 -> 192 conv by itself, e2m1, us, three tiles / one per
+    // workgroup: 16 x 24 x 26 into 96 channels (32 workgroups of three) 37.3 / 20.7, 32 x 24 x 26 (64) 38.0 / 25.1, 7 x 16^3 (224) 37.3 / 37.9, 9 x 16^3 (288) 40.8 / 42.4, 12 x 16^3 (384)
+    // 41.2 / 55.3; in the two deep convs of a 192-channel network at 2 x 128^3 (64) 45 + 62 -> 16 + 19
+    static int split3_env = -1;
+    if (split3_env < 0) split3_env = getenv("MI_CONV_SPLIT3") ? atoi(getenv("MI_CONV_SPLIT3")) : 192;      // tuning knob: that workgroup count (0: never)
+    a.one3 = stride == 1 && !big && MT == 3 && NT == 2 && !(osum && (cout / Go) % 4) && (size_t)((Wo + 15) / 16) * ((Ho + 7) / 8) * ((Do + 1) / 2) * (nmt_all / 3) * N < (size_t)split3_env && (a.nbt + cb_of(3) - 1) / cb_of(3) == (a.nbt + cb_of(1) - 1) / cb_of(1);
+    if (a.one3) MT = 1;
+    int cbmax = cb_of(MT);
+    auto lds_bytes = [&](int cb) { return lds_of(MT, cb); };
     static int cb_env = -1;
     if (cb_env < 0) cb_env = getenv("MI_CONV_CB") ? atoi(getenv("MI_CONV_CB")) : 0;      // tuning knob: blocks per chunk
     if (cb_env > 0 && cb_env <= cb1) cbmax = cb_env;

@@ -123,6 +123,7 @@ struct conv_args {
     bool row1;                         // ... its one-input-block form (weights in registers, the two halves of the workgroup half a tile apart)
     bool thin;                         // the K-split kernel of the launches of few output voxels takes the launch
     bool s2row;                        // the stride-2 row kernel takes the launch (one block, one channel tile)
+    bool one3;                         // the general kernel takes a slice of three channel tiles one tile per workgroup: its statistics are formed as the slice's are
     bool flat;                         // ... the one of about a tile of 128 voxels x 64 channels per CU (flat runs, the taps split over the wavefronts)
     unsigned char wrec;                // statistics records of a tile and channel slice: 1, or one per wavefront (the one-block row kernel 8, the small-channel kernel on that kernel's launches 4)
 };
@@ -657,6 +658,11 @@ __global__ void __launch_bounds__(256, 2) conv3_mx_k(const conv_args a) {
 
     __syncthreads();                                     // the ring and halo are dead: the epilogue reuses LDS for its statistics scratch
     // (uniform) more than 16 output channels, always so with two or more channel tiles: 32-wide output rows known at compile time
+    if constexpr (STRIDE == 1 && MT == 1 && NT == 2) {
+        // (a workgroup of one channel tile may keep per-channel statistics, and the branch around them makes the squares products of their own; those of a slice are fused into
+        // their sums: the form without the branch gives a divided slice the records of the whole one)
+        if (a.one3) { conv_epilogue<1, 2, OUT, EPI, false, true, false, true>(a, acc, lds, tile, n, cs, oz0, oy0, ox0, lz, ly0, tid); return; }
+    }
     if (MT > 1 || a.Co > 16) conv_epilogue<MT, NT, OUT, EPI, false, true>(a, acc, lds, tile, n, cs, oz0, oy0, ox0, lz, ly0, tid);
     else conv_epilogue<MT, NT, OUT, EPI>(a, acc, lds, tile, n, cs, oz0, oy0, ox0, lz, ly0, tid);
 }
