@@ -295,6 +295,48 @@ def test_block_with_scroll_rope_over_the_grid(gpu):
     assert run_block(P, lay, x, d, g)[0] == -1
 
 
+@pytest.mark.parametrize("D,Hh,W", [(6, 5, 7), (1, 1, 3)])
+def test_block_with_the_scattered_rows_packed_where_they_are_summed(gpu, D, Hh, W):
+    """The scatter also writes the projection's packed operand (and the running maximum is cleared by the pass over the rows): the bits of the separate launches, the
+    attention rows in the scratch record included"""
+    rng = np.random.default_rng(70 + W)
+    Cc, H, F, n = 192, 4, 512, 3; S = D * Hh * W
+    t = DevRays(n, D, Hh, W, 2.0, make_axr(n, D, Hh, W, (0, 1, 2), (0, 1, 2)))
+    P, lay = make_block(rng, Cc, F)
+    x = rng.standard_normal((n * S, Cc)).astype(np.float32)
+    d = at_dims(); d.C, d.H, d.F, d.rope, d.nreg, d.rope_base = Cc, H, F, 2, 0, 100.0
+    g = at_geom(); g.nseq, g.S, g.D, g.Hh, g.W = n, S, D, Hh, W; g.rays = C.addressof(t.R)
+    out = []
+    try:
+        for mode in (0, 1, 2):
+            lib.at_fuse_pack(mode)
+            out.append(run_block(P, lay, x, d, g, t.Tr))
+    finally:
+        lib.at_fuse_pack(2)
+    for r in out:
+        assert r[0] == 0 and np.isfinite(r[1]).all() and all(np.array_equal(a, b) for a, b in zip(r[1:], out[0][1:]))
+
+
+@pytest.mark.parametrize("words", [1, 257, 1 << 18, (1 << 18) + 1])
+@pytest.mark.parametrize("odd", [0, 2])
+def test_copies_from_pinned_memory_in_stream_order(gpu, words, odd):
+    """mi_h2d_async: the kernel that reads the pinned words in place (up to 1 MiB of whole words), past that and at odd places the copy command; memory behind the
+    destination stays as it was"""
+    n = 4 * words
+    pin = lib.mi_host_alloc(n + 8)
+    try:
+        src = (C.c_uint8 * (n + 8)).from_address(pin)
+        want = np.random.default_rng(words).integers(0, 256, n + 8, dtype=np.uint8)
+        np.frombuffer(src, np.uint8)[:] = want
+        d = DevBuf.from_numpy(np.full(n + 8, 7, np.uint8))
+        lib.mi_h2d_async(d.ptr + odd, pin + 4, n); LP.check()
+        lib.mi_sync()
+        got = d.to_numpy(np.uint8)
+        assert np.array_equal(got[odd:odd + n], want[4:4 + n]) and (got[:odd] == 7).all() and (got[odd + n:] == 7).all()
+    finally:
+        lib.mi_host_free(pin)
+
+
 def window_axis_records(N, D, kinds):
     """unet_set_attn_axis records (window voxels, the axis along window z) and the same axes at the bottleneck of a two-level net (F = 2 window planes
     per grid plane; a voxel centre c of the window is (c + 0.5) / F - 0.5 on the grid): kind 0 inside the window, 1 outside, 2 none"""

@@ -10,6 +10,9 @@
 // (attn8.hip)
 int mi_fa8_from_qkv(const float *qkv, const float *qg, const float *kg, float *rq, float *rk, float *amx, float *o, float *lse, const at_geom *g, int nreg, int H, int rope, float base);
 
+// (attn_ray.hip)
+void mi_ray_scatter_pack(const at_rays *R, const float *y, float *x, int Cc, int norm, uint8_t *pq, uint8_t *ps);
+
 #define HD AT_HD
 #define FT 64
 
@@ -272,12 +275,12 @@ __global__ void __launch_bounds__(256) qkv_pack_k(const float *__restrict__ qkv,
     if (threadIdx.x == 0 && bmax > *(volatile unsigned *)((unsigned *)amx + 1)) atomicMax((unsigned *)amx + 1, bmax);
 }
 __global__ void at_zero4_k(float *p) { if (threadIdx.x < 4) p[threadIdx.x] = 0.f; }
-static void fa_pack(const float *qkv, const float *qg, const float *kg, void *qkvh, float *rq, float *rk, float *amx, const at_geom *g, int nreg, int C, int rope, float base, const at_rays *R) {
+static void fa_pack(const float *qkv, const float *qg, const float *kg, void *qkvh, float *rq, float *rk, float *amx, const at_geom *g, int nreg, int C, int rope, float base, const at_rays *R, bool zeroed = false) {      // (zeroed: amx is, by an earlier kernel of the stream)
     if (C % HD || (C & 3)) mi_die("at_fa_pack: C %d is not a whole number of heads of %d", C, HD);
     const long long T = (long long)g->nseq * g->S, Tp = T + FT; const int H = C / HD;
     ray_src rs = {};
     if (R) { rs.G = geo_of(R); rs.ray = R->ray; rs.ad = R->ad; }
-    at_zero4_k<<<1, 64>>>(amx);
+    if (!zeroed) at_zero4_k<<<1, 64>>>(amx);
     const rope_t rp = {rope, g->S, g->Hh, g->W, nreg, log2f(base), rope ? g->pos : nullptr};
 #define QP(MODE) qkv_pack_k<MODE><<<nblk_((size_t)Tp * H * 3 * 8, 256), 256>>>(qkv, qg, kg, (__half *)qkvh, rq, rk, amx, T, H, rp, rs)
     switch (rope_mode(rp)) { case ROPE_TABLE: QP(ROPE_TABLE); break; case ROPE_REAL: QP(ROPE_REAL); break; default: QP(ROPE_EACH); }
@@ -401,10 +404,13 @@ extern "C" int at_block_fwd(const at_dims *d, const float *P, const at_bp *bp, c
     const bool fuse = g_fuse_pack && g_at_mx == 8 && C % 64 == 0 && F % 64 == 0 && !((uintptr_t)x & 15) && !((uintptr_t)w->x1 & 15) && !((uintptr_t)w->h & 15);
     uint8_t *aq = nullptr, *as = nullptr;
     // ... and the full attention's pack writes the core's quantised operands from the projection's rows; the binary16 tensor (qkvh) is not stored
+    bool opk = false;                                              // the attention's rows are packed for the projection where their sums were formed
+    bool amx0 = false;                                             // the pass over the rows has cleared the pack's running maximum
     bool direct = fuse && g_fuse_pack > 1 && !R && !((uintptr_t)w->qkv & 15) && at_fa8_one_pass(g->nseq, g->S, d->H);
     // attention branch
     if (fuse && mi_mx_gemm_abuf(8, (int)T, 3 * C, C, &aq, &as)) {
-        ln_pack_fwd(x, P + bp->ln1g, P + bp->ln1b, w->m1, w->r1, T, C, aq, as, direct ? w->amx : nullptr);
+        ln_pack_fwd(x, P + bp->ln1g, P + bp->ln1b, w->m1, w->r1, T, C, aq, as, direct || R ? w->amx : nullptr);
+        amx0 = true;
         if (int e = mi_mx_gemm_apacked(8, 1, (int)T, 3 * C, C, qkv.w, w->qkv, 0.f, qkv.b, nullptr)) return e;
     } else {
         direct = false;
@@ -418,16 +424,17 @@ extern "C" int at_block_fwd(const at_dims *d, const float *P, const at_bp *bp, c
     }
     if (R) {
         // (the pack reads the grid's rows through the rays' stencils: at_ray_gather's rows without their round trip through w->qkvr, which stays unwritten)
-        fa_pack(w->qkv, P + bp->qg, P + bp->kg, w->qkvh, w->rq, w->rk, w->amx, &ga, 0, C, d->rope, d->rope_base, R);
+        fa_pack(w->qkv, P + bp->qg, P + bp->kg, w->qkvh, w->rq, w->rk, w->amx, &ga, 0, C, d->rope, d->rope_base, R, amx0);
         at_fa_fwd(w->qkvh, w->orr, w->lse, &ga, d->H, C);
-        at_ray_scatter(R, w->orr, w->o, C, 1);
+        opk = fuse && mi_mx_gemm_abuf(8, (int)T, C, C, &aq, &as);
+        mi_ray_scatter_pack(R, w->orr, w->o, C, 1, opk ? aq : nullptr, as);
     } else if (direct) {
         if (int e = mi_fa8_from_qkv(w->qkv, P + bp->qg, P + bp->kg, w->rq, w->rk, w->amx, w->o, w->lse, &ga, d->nreg, d->H, d->rope, d->rope_base)) return e;
     } else {
         at_fa_pack(w->qkv, P + bp->qg, P + bp->kg, w->qkvh, w->rq, w->rk, w->amx, &ga, d->nreg, C, d->rope, d->rope_base);
         if (int e = at_fa8_fwd(w->qkvh, w->o, w->lse, &ga, d->H, C)) return e;
     }
-    if (int e = linear(proj, T, w->o, w->x1, x)) return e;
+    if (int e = opk ? mi_mx_gemm_apacked(8, 1, (int)T, C, C, proj.w, w->x1, 0.f, proj.b, x) : linear(proj, T, w->o, w->x1, x)) return e;
     // MLP branch
     if (fuse && mi_mx_gemm_abuf(8, (int)T, 2 * F, C, &aq, &as)) {
         ln_pack_fwd(w->x1, P + bp->ln2g, P + bp->ln2b, w->m2, w->r2, T, C, aq, as);

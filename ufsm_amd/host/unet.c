@@ -68,6 +68,7 @@ struct unet {
     /* cfg.attn_axis 1 / attn_pe 3: the scroll geometry (src/unet.c:280-282). One device buffer tb_rb holds the ray table, lengths, axis dims, ray
        positions, stencil weight sums, the grid tokens' scroll coordinates and the per-plane frames; the host side of a plan; the axis records */
     at_rays tbr; float *tb_rb, *tb_gpos, *tb_cen, *tb_rayh, *tb_cenh, *tb_axb, *tb_axh; int *tb_lensh, *tb_adh;
+    size_t tb_cen_o;                                               /* floats in front of the planes' centres in the tables, on either side */
     void *tb_pin[2], *tb_fence[2]; int tb_set;                     /* the plan's host tables: two pinned sets copied in stream order, each rewritten only after its copy ran */
     int tb_Q, tb_Nt, tb_Nr, tb_axn, tb_axs, tb_axdirty, tb_axwarn, tb_noax;
 };
@@ -345,14 +346,16 @@ static int build_acts(unet *u, shape5 in) {
             Tr = u->cfg.attn_axis == 1 ? (long)ys.n * u->tb_Q * u->tb_Nr : 0;
             const size_t nq = (size_t)ys.n * u->tb_Q, al = 64;
 #define UP(v) (((size_t)(v) + al - 1) / al * al)
-            const size_t o_ray = 0, o_len = o_ray + UP(nq * AT_RAY_F), o_ad = o_len + UP(nq), o_pos = o_ad + UP(ys.n), o_ws = o_pos + UP((size_t)Tr * 3),
-                         o_gp = o_ws + UP((size_t)ys.n * Sg), o_cen = o_gp + UP((size_t)T * 3), o_end = o_cen + UP((size_t)ys.n * Pm * 4);
+            /* (the host's tables first, one after the other as the pinned sets hold them: one copy) */
+            const size_t o_ray = 0, o_len = nq * AT_RAY_F, o_ad = o_len + nq, o_cen = UP(o_ad + (size_t)ys.n), o_pos = o_cen + UP((size_t)ys.n * Pm * 4), o_ws = o_pos + UP((size_t)Tr * 3),
+                         o_gp = o_ws + UP((size_t)ys.n * Sg), o_end = o_gp + UP((size_t)T * 3);
+            u->tb_cen_o = o_cen;
 #undef UP
             u->tb_rb = f32_new(o_end);
             u->tbr = (at_rays){.n = ys.n, .Q = u->tb_Q, .Nt = u->tb_Nt, .Nr = u->tb_Nr, .D = ys.d, .Hh = ys.h, .W = ys.w, .ad = (const int *)(u->tb_rb + o_ad), .ray = u->tb_rb + o_ray,
                                .lens = (const int *)(u->tb_rb + o_len), .pos = u->tb_rb + o_pos, .wsum = u->tb_rb + o_ws};
             u->tb_gpos = u->tb_rb + o_gp; u->tb_cen = u->tb_rb + o_cen;
-            for (int k = 0; k < 2; k++) { u->tb_pin[k] = mi_host_alloc((nq * AT_RAY_F + nq + (size_t)ys.n + (size_t)ys.n * Pm * 4) * 4); u->tb_fence[k] = mi_fence_new(); mi_fence_set(u->tb_fence[k]); }
+            for (int k = 0; k < 2; k++) { u->tb_pin[k] = mi_host_alloc((o_cen + (size_t)ys.n * Pm * 4) * 4); u->tb_fence[k] = mi_fence_new(); mi_fence_set(u->tb_fence[k]); }
             u->tb_set = 0;
             u->tb_axb = malloc((size_t)ys.n * AT_AXR(Pm) * sizeof(float));
             if (!u->tb_axb) { fprintf(stderr, "unet: no host memory for the ray plan\n"); abort(); }
@@ -720,12 +723,9 @@ static void tb_geom(unet *u) {
        would, and the device would then idle while the next forward is enqueued); a set is rewritten only once its own copy has run */
     const size_t nq = (size_t)n * u->tb_Q; const int set = u->tb_set; u->tb_set ^= 1;
     mi_fence_wait(u->tb_fence[set]);
-    u->tb_rayh = u->tb_pin[set]; u->tb_lensh = (int *)(u->tb_rayh + nq * AT_RAY_F); u->tb_adh = u->tb_lensh + nq; u->tb_cenh = (float *)(u->tb_adh + n);
+    u->tb_rayh = u->tb_pin[set]; u->tb_lensh = (int *)(u->tb_rayh + nq * AT_RAY_F); u->tb_adh = u->tb_lensh + nq; u->tb_cenh = u->tb_rayh + u->tb_cen_o;
     at_rays_plan(n, D, Hh, W, attn_ray_mult(), u->tb_axb, u->tb_rayh, u->tb_lensh, u->tb_adh, u->tb_cenh);
-    mi_h2d_async((void *)u->tbr.ray, u->tb_rayh, nq * AT_RAY_F * sizeof(float));
-    mi_h2d_async((void *)u->tbr.lens, u->tb_lensh, nq * sizeof(int));
-    mi_h2d_async((void *)u->tbr.ad, u->tb_adh, (size_t)n * sizeof(int));
-    mi_h2d_async(u->tb_cen, u->tb_cenh, (size_t)n * Pm * 4 * sizeof(float));
+    mi_h2d_async((void *)u->tbr.ray, u->tb_rayh, (u->tb_cen_o + (size_t)n * Pm * 4) * sizeof(float));
     mi_fence_set(u->tb_fence[set]);
     if (u->cfg.attn_axis == 1) at_rays_setup(&u->tbr);
     else at_scroll_pos(n, u->tbd.nreg, D, Hh, W, u->tbr.ad, u->tb_cen, u->tb_gpos);
