@@ -108,6 +108,22 @@ def test_wide_kernel_persistent_walk_few_blocks(gpu, Ci, Co, split):
     assert np.allclose(gsum, wsum, rtol=1e-6)
 
 
+@pytest.mark.parametrize("Ci,Co,dims,wgs", [(128, 64, (20, 70, 66), 456), (192, 64, (40, 40, 90), 512), (384, 64, (24, 40, 72), 304), (160, 64, (12, 57, 130), 432)])
+def test_wide_kernel_two_workgroups_per_cu(gpu, Ci, Co, dims, wgs):
+    """e2m1 slices of 64 channels on more tiles than CUs: two workgroups share a CU, a walk of one or two tiles each, borders cut in every direction, and a table of twelve input blocks (the largest LDS)."""
+    rng = np.random.default_rng(Ci + dims[0])
+    N, (D, H, W) = 2, dims
+    x, w, b = exact_case(rng, N, Ci, Co, D * H * W)
+    xq = orc.f32_to_mx(4, x, N, Ci, D * H * W)
+    for ydt in (3, 4):
+        got, gsum = gpu_conv(xq, 4, N, Ci, D, H, W, w, b, Co, ydt, cbits=4, Go=8, stats=True)
+        name = lib.mi_last_kernel().decode()
+        assert "conv3_wide_k" in name and "MT 2" in name and ("wgs %d" % wgs) in name, name
+        want, wsum = orc.conv3(xq, 4, N, Ci, D, H, W, w, b, Co, ydt, cbits=4, acc64=1, Go=8, want_stats=True)
+        assert np.array_equal(got, want)
+        assert np.allclose(gsum, wsum, rtol=1e-6)
+
+
 def test_wide_kernel_decoder_conv(gpu):
     """[2x upsampled coarse | skip] -> 128 channels with both GroupNorms: the wide kernel on a split, restaged input (12 blocks)."""
     rng = np.random.default_rng(77)

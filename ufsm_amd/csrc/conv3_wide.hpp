@@ -9,7 +9,7 @@
 //     ahead; input halo blocks of 32 channels live in 3 LDS slots and the K loop walks the blocks one after the other (taps inside), so
 //     while blocks b, b + 1 are multiplied block b + 2 streams into the third slot; the first blocks of the next tile follow the last one of
 //     this tile and land during the epilogue. Positions outside the volume read a zero row / scale byte 1 from a constant page;
-//   * workgroups are persistent (one per CU) and walk their tiles XCD by XCD.
+//   * workgroups are persistent (one per CU; two in e2m1 with 64 channels) and walk their tiles XCD by XCD.
 // The asynchronous copies are tracked with vmcnt: every copying step issues its weight copies first and then a fixed number of halo
 // copies, all unconditionally (nothing in a step branches, or the MFMA / LDS interleave would fall apart), so "all but the last few"
 // is exactly "the weights have landed".
@@ -34,10 +34,15 @@ template <int IMM> __device__ __forceinline__ void dma16si(unsigned off, const v
 }
 template <int N> __device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 
+constexpr int wide_tab_entry(int fmt) { return fmt == 8 ? 16 : 8; }           // bytes of a pair-table entry, one per pair and lane half
+constexpr bool wide_two(int fmt, bool epi, int mt) { return fmt == 4 && mt == 2 && !epi; }      // two workgroups per CU (launch_wide)
+
 // MT: channel tiles of 32 per workgroup: 4 (slices of 128 output channels) or 2 (64-channel layers: 8 accumulators per wavefront)
 template <int FMT, int OUT, bool EPI, int MT = 4>
-__global__ void __launch_bounds__(256, 1) conv3_wide_k(const conv_args a) {
+__global__ void __launch_bounds__(256, wide_two(FMT, EPI, MT) ? 2 : 1) conv3_wide_k(const conv_args a) {
     constexpr int NT = 4, TZ = 4;
+    // two wavefronts per SIMD have half the registers: what a lone one keeps over the K loop and the epilogue is formed anew per tile (halo_pos) or per round
+    constexpr bool LEAN = wide_two(FMT, EPI, MT);
     static_assert(MT == 4 || MT == 2, "channel tiles per workgroup");
     using HL = halo_t<FMT, 1, TZ>;
     constexpr int TT = HL::TT, HY = HL::HY, HX = HL::HX, NH = HL::NH, WTILE = fmt_t<FMT>::WTILE;
@@ -90,8 +95,13 @@ __global__ void __launch_bounds__(256, 1) conv3_wide_k(const conv_args a) {
     //     the rows and scale bytes of request block i: blocks 0 .. nbt - 1 of this tile, then the first blocks of the next one.
     const unsigned junk = a.red_o;                              // the statistics scratch (1 KiB) is idle while the K loop runs
     struct hreq { const uint8_t *row, *sc; unsigned rdst, sdst; };
+    auto halo_pos = [&](int rd, int ln) {                       // px | py << 8 | pz << 16 | (position inside the halo) << 24 of round rd
+        const int g = 4 * rd + wave, pos = g * 64 + ln;
+        const int pz = pos / (HY * HX), rem = pos - pz * (HY * HX), py = rem / HX, px = rem - py * HX;
+        return (unsigned)px | ((unsigned)py << 8) | ((unsigned)pz << 16) | ((g < NG && pos < TT ? 1u : 0u) << 24);
+    };
     static_assert(NRND == 5, "the round ring below has five entries");
-    unsigned pc[NRND];                                          // px | py << 8 | pz << 16 | (position inside the halo) << 24
+    unsigned pc[NRND];                                          // (not kept when LEAN)
     unsigned ring0, ring1, ring2, ring3, ring4;
     {
         unsigned dl[NRND];
@@ -108,6 +118,12 @@ __global__ void __launch_bounds__(256, 1) conv3_wide_k(const conv_args a) {
     auto tile_req = [&](const tile_t &t) {
         treq q; q.mask = 0u;
         const int z0 = t.oz0 - 1 + a.zi0, y0 = t.oy0 - 1, x0 = t.ox0 - 1;
+        if constexpr (LEAN) {
+            int ln = lane;
+            asm volatile("" : "+v"(ln));
+#pragma unroll
+            for (int rd = 0; rd < NRND; rd++) pc[rd] = halo_pos(rd, ln);
+        }
 #pragma unroll
         for (int rd = 0; rd < NRND; rd++) {
             const int gz = z0 + (int)((pc[rd] >> 16) & 255u), gy = y0 + (int)((pc[rd] >> 8) & 255u), gx = x0 + (int)(pc[rd] & 255u);
@@ -121,6 +137,7 @@ __global__ void __launch_bounds__(256, 1) conv3_wide_k(const conv_args a) {
     unsigned long long tb_row = 0, tb_sc = 0; int tb_ok = 0;
     int tb_gate = 0, tb_base = 0, tb_slot = 0, tb_msh = 0;      // also per request block: first pair after which it may be requested, its tile's first-position
                                                                 // voxel offset, its halo slot's byte offset, the shift of its tile's validity bits
+                                                                // (LEAN: tb_ok is tb_slot's sign, whose bits are inverted where the block holds no stored channels; tb_base and tb_msh are selected per round)
     auto block_table = [&](const tile_t &c, const tile_t &x, int fmax, unsigned rot, int bcur, int bnxt) {
         const int i = lane, own = i < a.nbt, blk = own ? i : i - a.nbt, n = own ? c.n : x.n;
         const int seg = blk >= a.nb0p, bl = seg ? blk - a.nb0p : blk;
@@ -128,23 +145,23 @@ __global__ void __launch_bounds__(256, 1) conv3_wide_k(const conv_args a) {
         const uint8_t *xq = seg ? a.xq[1] : a.xq[0], *xsc = seg ? a.xsc[1] : a.xsc[0];
         const size_t plane = ((size_t)n * nbs + min(max(bl, 0), max(nbs - 1, 0))) * Sin;
         tb_row = (unsigned long long)(size_t)(xq + plane * (16 * NH)); tb_sc = (unsigned long long)(size_t)(xsc + plane);
-        tb_ok = blk < a.nbt && bl < nbs;
         tb_gate = i > fmax ? 0x7fffffff : i < 3 ? -1 : (27 * (i - 3) + 26) >> 1;       // block i takes the slot block i - 3 is read from until that pair
-        tb_base = own ? bcur : bnxt;
         tb_slot = (int)((rot + (unsigned)i) % 3u) * HB;
-        tb_msh = own ? 0 : 8;
+        if constexpr (LEAN) tb_slot = blk < a.nbt && bl < nbs ? tb_slot : ~tb_slot;
+        else { tb_ok = blk < a.nbt && bl < nbs; tb_base = own ? bcur : bnxt; tb_msh = own ? 0 : 8; }
     };
     treq rq_cur, rq_nxt;
     auto lane64 = [&](unsigned long long v, int i) {
         const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)v, i), hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(v >> 32), i);
         return (unsigned long long)lo | ((unsigned long long)hi << 32);
     };
-    // the round rd (uniform) of request block ti of the tile whose data is (mask, base), into the halo slot at byte offset sbase; go false: a
+    // the round rd (uniform) of request block ti of the tile whose data is (mask, base), into the halo slot sl (tb_slot's entry); go false: a
     // round into the junk area. d: the lane's offset for that round (the ring's head, or a compile-time pick)
-    auto prepare = [&](hreq &q, unsigned mask, int base, int ti, int rd, unsigned d, unsigned sbase, bool go) {
+    auto prepare = [&](hreq &q, unsigned mask, int base, int ti, int rd, unsigned d, int sl, bool go) {
         const int g = 4 * rd + wave;
         const bool real = go & (g < NG);
-        const bool in = real & (__builtin_amdgcn_readlane(tb_ok, ti) != 0) & (((mask >> rd) & 1u) != 0u);
+        const unsigned sbase = (unsigned)(LEAN ? sl ^ (sl >> 31) : sl);
+        const bool in = real & (LEAN ? sl >= 0 : __builtin_amdgcn_readlane(tb_ok, ti) != 0) & (((mask >> rd) & 1u) != 0u);
         const unsigned vox = (unsigned)base + d;
         const uint8_t *rb = (const uint8_t *)(size_t)lane64(tb_row, ti), *sb = (const uint8_t *)(size_t)lane64(tb_sc, ti);
         q.row = in ? rb + (size_t)vox * (16 * NH) : a.zpage;
@@ -162,7 +179,7 @@ __global__ void __launch_bounds__(256, 1) conv3_wide_k(const conv_args a) {
     // slot: per pair the MT tiles of codes, then per lane its MT scale words. Wave w copies the 1 KiB pieces w, w + 4, ... (NW of them; a wave
     // with fewer repeats its last one: the count per step stays fixed). A copy is one instruction pair: m0 = slot + piece, load.
     constexpr int NW = (NCH + 3) / 4;
-    unsigned wvo[NW];                                           // the lane's byte offset inside a stage for copy k
+    unsigned wvo[NW];                                           // the lane's byte offset inside a stage for copy k (LEAN: the last copy takes the first one's, from a base of its own)
 #pragma unroll
     for (int k = 0; k < NW; k++) { int c = wave + 4 * k; c = c < NCH ? c : c - 4; wvo[k] = (unsigned)c * 1024u + (unsigned)lane * 16u; }
     const unsigned wd0 = lds0 + (unsigned)wave * 1024u;         // LDS address of the wave's first piece in slot 0
@@ -170,6 +187,7 @@ __global__ void __launch_bounds__(256, 1) conv3_wide_k(const conv_args a) {
     auto wcopy = [&](auto K, const uint8_t *src, unsigned so) {
         constexpr int k = decltype(K)::value;
         if constexpr (k < NW - 1) dma16si<k * 4096>(wvo[k], src, wd0 + so);
+        else if constexpr (LEAN) dma16s(wvo[0], src + wdl, wd0 + so + wdl);
         else dma16s(wvo[k], src, wd0 + so + wdl);
     };
     auto wstage = [&](int st, int cs, unsigned so) {            // stage st of slice cs into the ring slot at byte offset so
@@ -191,8 +209,8 @@ __global__ void __launch_bounds__(256, 1) conv3_wide_k(const conv_args a) {
 #pragma unroll
         for (int rd = 0; rd < NRND; rd++) {
             hreq q;
-            prepare(q, rq_nxt.mask, rq_nxt.base, 0, rd, d5[rd], 0, true); issue(q);
-            if (nnext > 1) { prepare(q, rq_nxt.mask, rq_nxt.base, 1, rd, d5[rd], HB, true); issue(q); }
+            prepare(q, rq_nxt.mask, rq_nxt.base, 0, rd, d5[rd], LEAN ? __builtin_amdgcn_readlane(tb_slot, 0) : 0, true); issue(q);
+            if (nnext > 1) { prepare(q, rq_nxt.mask, rq_nxt.base, 1, rd, d5[rd], LEAN ? __builtin_amdgcn_readlane(tb_slot, 1) : HB, true); issue(q); }
         }
     }
     wstage(0, cur.cs, 0); wstage(1, cur.cs, SLOT);
@@ -215,22 +233,25 @@ __global__ void __launch_bounds__(256, 1) conv3_wide_k(const conv_args a) {
             const int oA = (int)((rot + bA) % 3u) * HB + (((tA / 9) * HY + (tA / 3) % 3) * HX + tA % 3) * 16;
             const int oB = (int)((rot + bB) % 3u) * HB + (((tB / 9) * HY + (tB / 3) % 3) * HX + tB % 3) * 16;
             const int oH = hh ? oB : oA, sH = (oH / HB) * HB + ((oH % HB) >> 2);
-            *(v4i *)(lds + tab_o + i * 16) = (v4i){NH == 2 ? oA : oH, oB, sH, 0};
+            if constexpr (NH == 2) *(v4i *)(lds + tab_o + i * 16) = (v4i){oA, oB, sH, 0};
+            else *(int2 *)(lds + tab_o + i * 8) = make_int2(oH, sH);
         }
         v16f acc[MT][NT];                                       // (not cleared: the tile's first pair multiplies onto a zero operand)
         __syncthreads();
 
         v8i fb[2][NT], fa[2][MT]; int sb[2][NT]; int sav[2][MT];
         v4i T;
-        unsigned tabp = tab_o + h * 16;
-        T = *(const v4i *)(lds + tabp);
+        constexpr unsigned TE = wide_tab_entry(FMT);
+        unsigned tabp = tab_o + h * TE;
+        auto entry = [&](unsigned o) { if constexpr (NH == 2) T = *(const v4i *)(lds + tabp + o); else { const int2 t2 = *(const int2 *)(lds + tabp + o); T = (v4i){t2.x, 0, t2.y, 0}; } };
+        entry(0);
         // one LDS load of the fetch of a pair: index i = 3 f + part over the NT input fragments, then the MT weight fragments; the last
         // index reads the table entry of the pair after
         v4i lo[NT + MT], hi[NT + MT];
         auto ld = [&](auto I, auto NXT, const v4i tt2, unsigned wbase) {
             constexpr int i = decltype(I)::value, nx = decltype(NXT)::value;
             constexpr int f = i / 3, part = i % 3;
-            if constexpr (i == 3 * (NT + MT)) { T = *(const v4i *)(lds + tabp + 32); tabp += 32; }
+            if constexpr (i == 3 * (NT + MT)) { entry(2 * TE); tabp += 2 * TE; }
             else if constexpr (f < NT) {
                 if constexpr (part == 0) lo[f] = *(const v4i *)(lds + (abr0 + tt2[0]) + f * ABJ);
                 else if constexpr (part == 1) { if constexpr (FMT == 8) hi[f] = *(const v4i *)(lds + (abr0 + tt2[1]) + f * ABJ); }
@@ -268,7 +289,8 @@ __global__ void __launch_bounds__(256, 1) conv3_wide_k(const conv_args a) {
         int fbi = nnext, frd = 0;                             // (blocks 0 .. nnext - 1 of this tile were requested during the tile before, or ahead of the first)
         auto prep_next = [&](hreq &q, int upto_pair) {          // prepare one copy round; pairs <= upto_pair will have been fetched by every wavefront when it is issued
             const bool go = __builtin_amdgcn_readlane(tb_gate, fbi) <= upto_pair;
-            prepare(q, mask2 >> __builtin_amdgcn_readlane(tb_msh, fbi), __builtin_amdgcn_readlane(tb_base, fbi), fbi, frd, ring0, (unsigned)__builtin_amdgcn_readlane(tb_slot, fbi), go);
+            if constexpr (LEAN) prepare(q, mask2 >> (fbi < a.nbt ? 0 : 8), fbi < a.nbt ? rq_cur.base : rq_nxt.base, fbi, frd, ring0, __builtin_amdgcn_readlane(tb_slot, fbi), go);
+            else prepare(q, mask2 >> __builtin_amdgcn_readlane(tb_msh, fbi), __builtin_amdgcn_readlane(tb_base, fbi), fbi, frd, ring0, __builtin_amdgcn_readlane(tb_slot, fbi), go);
             const unsigned t0 = ring0;                          // a consumed round turns the ring
             ring0 = go ? ring1 : ring0; ring1 = go ? ring2 : ring1; ring2 = go ? ring3 : ring2; ring3 = go ? ring4 : ring3; ring4 = go ? t0 : ring4;
             frd += go ? 1 : 0;
@@ -347,8 +369,12 @@ static void launch_wide(const conv_args &a, size_t smem) {
         ncu[d] = pr.multiProcessorCount > 8 ? pr.multiProcessorCount & ~7 : 8;
         attr[d] = true;
     }
-    const unsigned per = (a.ntiles + 7u) / 8u;            // tiles per XCD; one persistent workgroup per CU, a multiple of 8 in all
-    const unsigned nwg = per * 8u < (unsigned)ncu[d] ? per * 8u : (unsigned)ncu[d];
+    // tiles per XCD; one persistent workgroup per CU, a multiple of 8 in all. The e2m1 slices of 64 channels: two, whose registers (128 and 128, none spilled) and LDS (79 936 bytes at the
+    // most, twelve input blocks) fit beside each other: a stage's sixteen products are then no longer than the 150 other instructions of its wavefront, and the second wavefront of a SIMD
+    // multiplies while the first issues them or converts its accumulators. us, one / two per CU: 192 -> 64 at 2 x 64^3 125.6 / 100.5, at 2 x 48^3 61.3 / 46.9, 128 -> 64 there 46.3 / 38.8,
+    // 256 -> 256 at 2 x 24^3 69.7 / 53.5. (Slices of 128 as eight wavefronts of one workgroup, two per SIMD, which meet at every stage's barrier: 66.0 / 68.6 at 256 -> 256, 2 x 32^3)
+    const unsigned per = (a.ntiles + 7u) / 8u, wgs = (unsigned)ncu[d] * (wide_two(FMT, EPI, MT) && smem <= 80 * 1024 ? 2u : 1u);
+    const unsigned nwg = per * 8u < wgs ? per * 8u : wgs;
     conv3_wide_k<FMT, OUT, EPI, MT><<<nwg, 256, smem>>>(a);
     MICK();
     snprintf(g_last_kernel, sizeof g_last_kernel, "conv3_wide_k<fmt %d, out %d, epi %d%s> tiles %u wgs %u", FMT, OUT, (int)EPI, MT == 2 ? ", MT 2" : "", a.ntiles, nwg);
