@@ -700,7 +700,18 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
                          (fmt == 8 ? a.nbt >= 2 : a.nbt >= 4 && frun <= 512) && fwg <= (a.nbt >= 8 ? 512u : 256u)));
     if (a.flat) { a.thin = a.row = a.row1 = a.areg = false; a.wrec = 1; }
     if (a.thin || a.flat) { big = false; MT = 1; NT = 2; a.CB = a.flat ? 2 : a.nbt; }
-    size_t smem = a.flat ? (size_t)(fmt == 8 ? flat_t<8>::LDS : flat_t<4>::LDS) : a.thin ? MI_THIN_LDS : a.row1 ? (size_t)10 * 352 * (RB + 4) : a.row ? (size_t)2 * 2048 * (RB + 4) : a.areg ? (size_t)2 * ((TT + 63) / 64 * 64) * (RB + 4) : big ? (size_t)4 * MT * (WTILE + 256) + (size_t)3 * ((TT + 63) / 64 * 64) * (RB + 4) + (size_t)(((27 * a.nbt + 1) >> 1) + 2) * 2 * wide_tab_entry(fmt) : lds_bytes(a.CB);
+    // the general kernel's one-tile, two-plane launches, pipelined (conv3_pipe.hpp), up to 512 workgroups (what the coarse form and the divided slices of three launch at the most): a workgroup
+    // has a CU's LDS to itself, or half of it where its stages shrink to three pairs (conv3_pipe_pps). A conv with its statistics, us, conv3_mx_k / this. e4m3: 256 -> 256 at 2 x 16^3 (256 workgroups)
+    // 38.9 / 25.3, 128 -> 256 23.4 / 16.7, at 3 x 16^3 (384) 256 -> 256 45.2 / 33.4, at 22 x 26^2 (352) 384 -> 128 66.3 / 48.1, 128 -> 128 27.9 / 22.0, 64 -> 128 18.9 / 16.0; e2m1: 256 -> 256 at 2 x 12^3
+    // (192) 24.7 / 17.0, 192 -> 192 at 2 x 16^3 (192) 20.7 / 14.6, 384 -> 128 there (128) 32.9 / 20.8. Past one round of CUs in chunks of three or four blocks two or more chunks still gain - 384 -> 128
+    // at 22 x 26^2 40.9 / 37.8, 192 -> 192 at 5 x 16^3 (480) 25.4 / 24.3 -, one does not: 128 -> 128 at 22 x 26^2 20.3 / 21.2
+    static int pipe_env = -1;
+    if (pipe_env < 0) pipe_env = getenv("MI_CONV_PIPE") ? atoi(getenv("MI_CONV_PIPE")) : 512;      // tuning knob: that workgroup count (0: never)
+    const size_t pipe_tiles = (size_t)((Wo + 15) / 16) * ((Ho + 7) / 8) * ((Do + 1) / 2) * nmt_all * N;
+    const int pipe_pps = conv3_pipe_pps(fmt, a.CB, pipe_tiles);
+    a.pipe = stride == 1 && !act && MT == 1 && NT == 2 && a.wide && !big && !a.areg && !a.row && !a.thin && !a.flat && (fmt == 8 ? a.CB == 1 : a.CB <= 4) && a.nbt % a.CB == 0 && S < ((size_t)1 << 31) &&
+             pipe_tiles <= (size_t)pipe_env && (pipe_tiles <= 256 || pipe_pps == 3 || a.nbt > a.CB);
+    size_t smem = a.pipe ? conv3_pipe_lds(fmt, a.CB, pipe_pps) : a.flat ? (size_t)(fmt == 8 ? flat_t<8>::LDS : flat_t<4>::LDS) : a.thin ? MI_THIN_LDS : a.row1 ? (size_t)10 * 352 * (RB + 4) : a.row ? (size_t)2 * 2048 * (RB + 4) : a.areg ? (size_t)2 * ((TT + 63) / 64 * 64) * (RB + 4) : big ? (size_t)4 * MT * (WTILE + 256) + (size_t)3 * ((TT + 63) / 64 * 64) * (RB + 4) + (size_t)(((27 * a.nbt + 1) >> 1) + 2) * 2 * wide_tab_entry(fmt) : lds_bytes(a.CB);
     if (s2d) smem = a.s2row ? conv3s2_row_lds(fmt) : 0;
     smem = (smem + 15) & ~(size_t)15;
     a.epi_o = (unsigned)smem; smem += (size_t)3 * (a.flat ? 2 : MT) * 32 * sizeof(float);      // bias, affine a, b of the workgroup's channels
@@ -712,7 +723,7 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     a.wl_o = 0;
     if (a.row && !a.row1 && fmt == 4 && wl_env && smem + (size_t)a.nbt * 15 * 1280 <= 160 * 1024) { a.wl_o = (unsigned)smem; smem += (size_t)a.nbt * 15 * 1280; }
     if (smem > 160 * 1024) mi_die("%s: %zu bytes of LDS for %d input blocks in chunks of %d", who, smem, a.nbt, a.CB);      // (every form above sizes its chunks to fit)
-    if (big || a.areg || a.row || a.s2row) {
+    if (big || a.areg || a.row || a.s2row || a.pipe) {
         // rows and scale bytes of positions outside the volume: 64 zero bytes, then 64 bytes of value 1; one page per device, kept for the process
         // (the entry point that must not allocate keeps its own at the head of its fixed scratch)
         static uint8_t *zpage[8];

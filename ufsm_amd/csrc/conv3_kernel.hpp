@@ -124,6 +124,7 @@ struct conv_args {
     bool thin;                         // the K-split kernel of the launches of few output voxels takes the launch
     bool s2row;                        // the stride-2 row kernel takes the launch (one block, one channel tile)
     bool one3;                         // the general kernel takes a slice of three channel tiles one tile per workgroup: its statistics are formed as the slice's are
+    bool pipe;                         // the pipelined form of the general kernel's one-tile, two-plane launches takes the launch
     bool flat;                         // ... the one of about a tile of 128 voxels x 64 channels per CU (flat runs, the taps split over the wavefronts)
     unsigned char wrec;                // statistics records of a tile and channel slice: 1, or one per wavefront (the one-block row kernel 8, the small-channel kernel on that kernel's launches 4)
 };
@@ -684,10 +685,11 @@ static void launch_conv(const conv_args &a, size_t smem) {
 #include "conv3_row1.hpp"
 #include "conv3_thin.hpp"
 #include "conv3_flat.hpp"
+#include "conv3_pipe.hpp"
 template <int FMT, int STRIDE, int OUT, bool EPI>
 static void launch_mt(int MT, int NT, const conv_args &a, size_t smem) {
     if constexpr (!EPI) { if (a.thin) { launch_thin<FMT, STRIDE, OUT>(a, smem); return; } }
-    if constexpr (!EPI && STRIDE == 1) { if (a.flat) { launch_flat<FMT, OUT>(a, smem); return; } }
+    if constexpr (!EPI && STRIDE == 1) { if (a.flat) { launch_flat<FMT, OUT>(a, smem); return; } if (a.pipe) { launch_pipe<FMT, OUT>(a, smem); return; } }
     switch (MT * 10 + NT) {
     case 44: if constexpr (STRIDE == 1) launch_wide<FMT, OUT, EPI>(a, smem); else mi_die("conv3: the wide kernel is stride 1 only"); break;
     // (one-plane tiles, stride 2 only: its halo is 8 input positions per output, and a 3 x 17 x 33 halo lets two workgroups share a CU)
