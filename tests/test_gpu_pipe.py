@@ -33,7 +33,7 @@ def test_exact_operands(gpu, case):
     x, w, b = exact_case(rng, case[1], case[2], case[3], case[4] * case[5] * case[6])
     for ydt in (3, 4, 0):
         (got, gs), (want, ws), name = _run(case, ydt, True, x, w, b)
-        assert "conv3_pipe_k" in name and "stage %d>" % case[7] in name and "CB %d " % case[8] in name, name
+        assert "conv3_pipe_k" in name and "stage %d CB %d " % case[7:9] in name, name
         assert np.array_equal(got, want), ydt
         assert np.allclose(gs, ws, rtol=1e-6)
 

@@ -236,3 +236,21 @@ def test_edges_of_the_range(gpu, bits, Ci, Co, stride, launches):
             name.append("conv3_thin_k" in lib.mi_last_kernel().decode())
         assert name == [thin, False, True], (N, D, H, W, name)
         assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
+
+
+@pytest.mark.parametrize("bits,N,Ci,Co,dims", [(8, 1, 64, 64, (16, 16, 16)), (8, 1, 64, 64, (17, 16, 16)), (4, 1, 96, 160, (5, 13, 25)), (8, 1, 96, 160, (5, 13, 26)), (8, 1, 33, 17, (1, 1, 1)),
+                                               (8, 1, 1280, 32, (3, 5, 7)), (4, 2, 1216, 32, (4, 4, 5)), (8, 1, 128, 64, (2, 3, 5))])
+def test_one_run_or_two_per_workgroup(gpu, bits, N, Ci, Co, dims):
+    """128 tiles of 64 voxels (a run of 32 per workgroup) and 136, an odd number of runs, one voxel, every length of the walk's tail, and more input blocks than the table of 64 units holds."""
+    rng = np.random.default_rng(Ci + Co + dims[2])
+    D, H, W = dims
+    x, w, b = exact_case(rng, N, Ci, Co, D * H * W)
+    xdt = 3 if bits == 8 else 4
+    xq = orc.f32_to_mx(bits, x, N, Ci, D * H * W)
+    G = 8 if Co % 32 == 0 else 1
+    stats = (Co // G) % 4 == 0
+    got, gs = gpu_conv(xq, xdt, N, Ci, D, H, W, w, b, Co, xdt, cbits=bits, Go=G if stats else 0, stats=stats)
+    assert "conv3_thin_k" in lib.mi_last_kernel().decode(), lib.mi_last_kernel().decode()
+    want, ws = orc.conv3(xq, xdt, N, Ci, D, H, W, w, b, Co, xdt, cbits=bits, acc64=1, Go=G if stats else 0, want_stats=stats)
+    assert np.array_equal(got, want)
+    assert not stats or np.allclose(gs, ws, rtol=1e-6)

@@ -183,7 +183,7 @@ static void launch_pipe_t(const conv_args &a, size_t smem) {
     const unsigned per = (a.ntiles + 7u) / 8u;
     conv3_pipe_k<FMT, OUT, CB, PPS><<<per * 8u, 256, smem>>>(a);
     MICK();
-    snprintf(g_last_kernel, sizeof g_last_kernel, "conv3_pipe_k<fmt %d, out %d, MT 1, NT 2, stage %d> (conv3_mx_k's products) CB %d tiles %u", FMT, OUT, PPS, CB, a.ntiles);
+    snprintf(g_last_kernel, sizeof g_last_kernel, "conv3_pipe_k for conv3_mx_k<fmt %d, stride 1, MT 1, NT 2, out %d, epi 0> stage %d CB %d tiles %u", FMT, OUT, PPS, CB, a.ntiles);
 }
 template <int FMT, int OUT>
 static void launch_pipe(const conv_args &a, size_t smem) {
