@@ -9,10 +9,12 @@ from test_gpu_conv import exact_case, rand_case, gpu_conv
 pytestmark = pytest.mark.gpu
 
 # (bits, N, Ci, Co, D, H, W, pairs of a weight stage, chunk): one block and many; borders cut in every direction; chunks of one to four blocks, one chunk and several; one round of CUs and, with
-# stages of three pairs, two workgroups per CU; chunks of three and four past one round
+# stages of three pairs, two workgroups per CU; chunks of three and four past one round; per-channel
+# statistics records and rows of 16 output channels
 CASES = [(8, 1, 32, 128, 6, 13, 21, 7, 1), (8, 2, 160, 128, 9, 13, 18, 7, 1), (8, 2, 256, 256, 16, 16, 16, 7, 1), (8, 1, 128, 128, 22, 26, 26, 3, 1), (8, 1, 96, 128, 17, 21, 35, 3, 1),
          (4, 2, 32, 128, 9, 14, 18, 7, 1), (4, 1, 64, 128, 14, 15, 20, 7, 2), (4, 2, 192, 192, 10, 16, 16, 7, 3), (4, 1, 96, 192, 9, 11, 33, 7, 3), (4, 2, 128, 256, 12, 12, 12, 7, 4), (4, 1, 384, 128, 15, 16, 19, 7, 4),
-         (4, 1, 64, 128, 22, 26, 26, 3, 2), (4, 1, 32, 128, 22, 26, 26, 3, 1), (4, 3, 192, 192, 16, 16, 16, 7, 3), (4, 1, 256, 128, 22, 26, 26, 7, 4)]
+         (4, 1, 64, 128, 22, 26, 26, 3, 2), (4, 1, 32, 128, 22, 26, 26, 3, 1), (4, 3, 192, 192, 16, 16, 16, 7, 3), (4, 1, 256, 128, 22, 26, 26, 7, 4),
+         (8, 2, 64, 40, 3, 20, 24, 7, 1), (8, 1, 96, 16, 3, 40, 40, 7, 1), (4, 1, 64, 16, 2, 17, 50, 7, 2)]
 
 
 def _run(case, ydt, stats, x, w, b):

@@ -666,6 +666,8 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     // kernels' and the one-block, one-tile kernel's launches stay theirs. The tiles counted are the whole tensor's (Dr planes), not a z-range's: a slab
     // adds in the order of the whole tensor's conv and takes its statistics over the same runs, so that inference in slabs gives its bytes (a slab whose statistics
     // leave planes at its ends out, zlo and zhi, too)
+    // (These figures are of the kernels as they were when the line was drawn. Both sides are faster since - the K-split kernel by 1 - 5 us a launch, the other one as conv3_pipe_k by a third, a call of
+    // 384 -> 128 at 1 x 8^3 18.3 -> 12.8 and of 256 -> 256 at 2 x 16^3 38.9 -> 25.3 -, and the line stays: a conv on the other side of it adds its products in another order, which a network would notice)
     static int thin_env = -1;
     if (thin_env < 0) thin_env = getenv("MI_CONV_THIN") ? atoi(getenv("MI_CONV_THIN")) : 256;      // tuning knob: that tile count (0: never)
     const int kb = a.nbt * (fmt == 8 ? 2 : 1);                 // (K in bytes: halves of 16 per tap)
