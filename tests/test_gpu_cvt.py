@@ -305,6 +305,31 @@ def test_gn_sums_and_finalize(gpu, bits, Cc, G):
     assert (dd.to_numpy(np.float64) == 0).all()
 
 
+@pytest.mark.parametrize("bits,Cc,G,dims", [(8, 192, 8, (16, 16, 16)), (4, 96, 8, (12, 12, 12)), (8, 32, 8, (24, 24, 24)), (8, 40, 4, (3, 5, 33)), (4, 256, 8, (8, 13, 13)), (8, 64, 8, (32, 32, 40))])
+def test_gn_sums_do_not_depend_on_the_batch(gpu, bits, Cc, G, dims):
+    """A sample's slots are the same bits alone and among 2, 8 or 16 samples, whichever calls sum them: row scales spread over 24 powers of two, so that the sums of a slab are rounded
+    and any other division of the voxels would show."""
+    rng = np.random.default_rng(Cc + dims[2])
+    N, S = 16, int(np.prod(dims))
+    x = rng.standard_normal((N, Cc, S)).astype(np.float32) * np.exp2(rng.integers(-12, 13, (N, 1, S))).astype(np.float32)
+    dt, dq, tail = 3 if bits == 8 else 4, to_mx(bits, x), S - S // 5      # (tail: a range of voxels)
+
+    def slots(q, n, calls, v1):
+        d = DevBuf(n * G * 2 * 24)
+        for n0, cnt in calls:
+            assert lib.lp_gn_sums_mx_n(q.ptr, dt, n, Cc, G, S, d.ptr, 0, v1, n0, cnt) == 0
+        LP.check()
+        return d.to_numpy(np.uint64, (n, G * 2 * 3))
+
+    for v1 in (S, tail):
+        whole = slots(dq, N, [(0, N)], v1)
+        assert whole.any()
+        for cnt in (1, 2, 8):
+            assert np.array_equal(slots(dq, N, [(k, cnt) for k in range(0, N, cnt)], v1), whole), (v1, cnt)
+        for n0, cnt in ((5, 1), (3, 2), (8, 8)):                              # tensors of their own
+            assert np.array_equal(slots(to_mx(bits, x[n0:n0 + cnt]), cnt, [(0, cnt)], v1), whole[n0:n0 + cnt]), (v1, n0, cnt)
+
+
 def test_head_matrix_pipe_gives_the_vector_form_s_bits(gpu):
     """The head's products through the matrix pipe (v_mfma_f32_4x4x1: one product per accumulator and step, in channel order) against the same
     products as fused multiply-adds on the vector ALUs: equal bit for bit, with GroupNorm + SiLU on the input, two channel blocks, denormal

@@ -638,11 +638,13 @@ __global__ void __launch_bounds__(256) gn_sums_mx_k(const uint8_t *x, int N, int
 extern "C" int lp_gn_sums_mx_n(const void *x, int xdt, int N, int C, int G, size_t S, double *sums, size_t v0, size_t v1, int n0, int cnt) {
     if ((xdt != 3 && xdt != 4) || G <= 0 || C % G) return -1;
     if (v1 <= v0 || cnt <= 0) return 0;
-    // few, large slabs (every block ends in atomic adds to the same few slots), but smaller ones while CUs are idle: a thread's chain of rows and fp64 adds is the launch's length.
-    // 192 channels of 2 x 16^3: one slab of 4 096 voxels (12 workgroups) 19.9 us, eight of 512 11.1; the sums are fp64 either way, of products that have at most 53 bits but for
-    // rows many powers of two apart
+    // few, large slabs (every block ends in atomic adds to the same few slots), but smaller ones, of 512 voxels and more, while a sample has fewer than 64 workgroups: a thread's chain of rows
+    // and fp64 adds is the launch's length. Passes back to back, us, slabs of 8 192 / these: 192 channels of 16^3, 2 samples 16.6 / 9.3, 16 samples 16.4 / 15.4, 32 samples 19.0 / 26.9, of 24^3
+    // 22.4 / 11.2, 26.8 / 24.3, 30.7 / 45.2 (up to 32 workgroups a sample: 10.1, 12.1, 20.5 and 14.0, 18.5, 33.3; up to 128: 9.3, 15.4, 26.9 and 9.8, 38.1, 72.5). A matter of one sample's voxels
+    // and channels, never of how many samples a call has: the slots add exactly, but a slab's own sum is rounded to fp64 (the sum of the squares of 4 096 e4m3 rows of one scale spans some 51 bits,
+    // of rows a power of two or two apart more than 53), so that another division of the voxels can move a sample's last bit
     size_t nsl = (v1 - v0 + 8191) / 8192; if (nsl > 512) nsl = 512;
-    const size_t idle = 256 / ((size_t)mx_nb(C) * cnt), fine = (v1 - v0 + 511) / 512;
+    const size_t idle = 64 / (size_t)mx_nb(C), fine = (v1 - v0 + 511) / 512;
     if (nsl < idle && nsl < fine) nsl = idle < fine ? idle : fine;
     const dim3 grid((unsigned)nsl, (unsigned)mx_nb(C), (unsigned)cnt);
     if (xdt == 4) gn_sums_mx_k<4><<<grid, 256>>>((const uint8_t *)x, N, C, G, S, sums, v0, v1, n0);
