@@ -13,6 +13,8 @@ sys.path.insert(0, os.path.join(ROOT, "oracle"))
 import ray_oracle as ro  # noqa: E402
 from gpuutil import DevBuf, LP, lib  # noqa: E402
 from ufsm_amd import at_geom, at_dims, at_bp, at_ws, at_rays  # noqa: E402
+from ufsm_amd.lp import load  # noqa: E402
+import orc  # noqa: E402
 from test_oracle_block import make_block  # noqa: E402
 from test_oracle_ray import make_axr  # noqa: E402
 
@@ -315,6 +317,29 @@ def test_block_with_the_scattered_rows_packed_where_they_are_summed(gpu, D, Hh, 
         lib.at_fuse_pack(2)
     for r in out:
         assert r[0] == 0 and np.isfinite(r[1]).all() and all(np.array_equal(a, b) for a, b in zip(r[1:], out[0][1:]))
+
+
+@pytest.mark.parametrize("Cc,norm", [(64, 1), (192, 1), (96, 1), (32, 1), (4, 1), (64, 0)])
+def test_the_scatter_says_whether_it_packed_its_rows(gpu, Cc, norm):
+    """Rows asked for in packed form are packed (the codes and scale bytes of the storage quantiser) or refused, never left out in silence: a caller reads them on that word."""
+    f = load().mi_ray_scatter_pack
+    f.restype, f.argtypes = C.c_bool, [C.c_void_p] * 3 + [C.c_int] * 2 + [C.c_void_p] * 2
+    n, D, Hh, W = 2, 6, 5, 7
+    t = DevRays(n, D, Hh, W, 2.0, make_axr(n, D, Hh, W, (0, 1), (0, 2)))
+    y = np.random.default_rng(Cc).standard_normal((t.Tr, Cc)).astype(np.float32)
+    dy, dx, dw = DevBuf.from_numpy(y), DevBuf(t.Tg * Cc * 4), DevBuf(t.Tg * Cc * 4)
+    nb = -(-Cc // 32)
+    pq, ps = DevBuf.from_numpy(np.full(t.Tg * Cc, 0xA5, np.uint8)), DevBuf.from_numpy(np.full(t.Tg * nb, 0xA5, np.uint8))
+    lib.at_ray_scatter(C.byref(t.R), dy.ptr, dw.ptr, Cc, norm)
+    packed = f(C.addressof(t.R), dy.ptr, dx.ptr, Cc, norm, pq.ptr, ps.ptr); LP.check()
+    rows = dx.to_numpy(np.float32)
+    assert np.array_equal(rows.view(np.uint32), dw.to_numpy(np.uint32))
+    q, s = pq.to_numpy(np.uint8), ps.to_numpy(np.uint8)
+    assert packed == (norm == 1 and Cc % 64 == 0)
+    if packed:
+        assert np.array_equal(np.concatenate([q, s]), orc.f32_to_mx(8, rows.reshape(t.Tg, Cc, 1), t.Tg, Cc, 1))
+    else:
+        assert (q == 0xA5).all() and (s == 0xA5).all()
 
 
 @pytest.mark.parametrize("words", [1, 257, 1 << 18, (1 << 18) + 1])

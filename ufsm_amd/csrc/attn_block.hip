@@ -11,7 +11,7 @@
 int mi_fa8_from_qkv(const float *qkv, const float *qg, const float *kg, float *rq, float *rk, float *amx, float *o, float *lse, const at_geom *g, int nreg, int H, int rope, float base);
 
 // (attn_ray.hip)
-void mi_ray_scatter_pack(const at_rays *R, const float *y, float *x, int Cc, int norm, uint8_t *pq, uint8_t *ps);
+extern "C" bool mi_ray_scatter_pack(const at_rays *R, const float *y, float *x, int Cc, int norm, uint8_t *pq, uint8_t *ps);
 
 #define HD AT_HD
 #define FT 64
@@ -426,8 +426,8 @@ extern "C" int at_block_fwd(const at_dims *d, const float *P, const at_bp *bp, c
         // (the pack reads the grid's rows through the rays' stencils: at_ray_gather's rows without their round trip through w->qkvr, which stays unwritten)
         fa_pack(w->qkv, P + bp->qg, P + bp->kg, w->qkvh, w->rq, w->rk, w->amx, &ga, 0, C, d->rope, d->rope_base, R, amx0);
         at_fa_fwd(w->qkvh, w->orr, w->lse, &ga, d->H, C);
-        opk = fuse && mi_mx_gemm_abuf(8, (int)T, C, C, &aq, &as);
-        mi_ray_scatter_pack(R, w->orr, w->o, C, 1, opk ? aq : nullptr, as);
+        const bool ab = fuse && mi_mx_gemm_abuf(8, (int)T, C, C, &aq, &as);
+        opk = mi_ray_scatter_pack(R, w->orr, w->o, C, 1, ab ? aq : nullptr, ab ? as : nullptr);
     } else if (direct) {
         if (int e = mi_fa8_from_qkv(w->qkv, P + bp->qg, P + bp->kg, w->rq, w->rk, w->amx, w->o, w->lse, &ga, d->nreg, d->H, d->rope, d->rope_base)) return e;
     } else {

@@ -441,20 +441,23 @@ extern "C" void at_ray_gather(const at_rays *R, const float *x, float *y, int Cc
     else ray_gather_k<false><<<nblk_((size_t)Tr * C4, 256), 256>>>(G, R->ray, R->ad, R->wsum, Tr, C4, (const float4 *)x, (float4 *)y);
     MICK();
 }
-// (pq, ps: the rows also as the packed e4m3 operand of a GEMM, with norm and Cc a multiple of 64)
-void mi_ray_scatter_pack(const at_rays *R, const float *y, float *x, int Cc, int norm, uint8_t *pq, uint8_t *ps) {
+// at_ray_scatter, its rows also as the packed e4m3 operand (pq, ps; null: none asked for) of the GEMM that reads them. Returns whether they are: with norm and Cc a multiple of 64; a caller that
+// reads packed rows asks here and nowhere else
+extern "C" bool mi_ray_scatter_pack(const at_rays *R, const float *y, float *x, int Cc, int norm, uint8_t *pq, uint8_t *ps) {
     rays_check(R, "at_ray_scatter");
     if (Cc <= 0 || Cc % 4 || ((uintptr_t)x & 15) || ((uintptr_t)y & 15) || (norm && !R->wsum)) mi_die("at_ray_scatter: %d channels (a multiple of 4), 16-byte aligned rows", Cc);
     const ray_geo G = geo_of(R); const long long Tr = (long long)R->n * R->Q * R->Nr; const int C4 = Cc / 4;
     const size_t ng = (size_t)R->n * G.Sg * Cc;
-    if (!ng) return;
-    if ((long long)R->n * R->Q * R->Nr > 0x7fffffffll) mi_die("at_ray_scatter: %lld ray slots", (long long)R->n * R->Q * R->Nr);
+    const bool pack = pq && ps && norm && Cc % 64 == 0;
+    if (!ng) return pack;
+    if (Tr > 0x7fffffffll) mi_die("at_ray_scatter: %lld ray slots", Tr);
     const inv_tab it = inverse_table(R, nullptr);
     const ray_ent *tab = it.tab; const int *cnt = it.cnt; const int cap = it.cap;
-    if (pq && norm && Cc % 64 == 0) ray_scatter_k<true, true><<<nblk_(ng / 4, 256), 256>>>(tab, cnt, cap, R->wsum, ng / 4, C4, (const float4 *)y, (float4 *)x, pq, ps);
+    if (pack) ray_scatter_k<true, true><<<nblk_(ng / 4, 256), 256>>>(tab, cnt, cap, R->wsum, ng / 4, C4, (const float4 *)y, (float4 *)x, pq, ps);
     else if (norm) ray_scatter_k<true><<<nblk_(ng / 4, 256), 256>>>(tab, cnt, cap, R->wsum, ng / 4, C4, (const float4 *)y, (float4 *)x);
     else ray_scatter_k<false><<<nblk_(ng / 4, 256), 256>>>(tab, cnt, cap, R->wsum, ng / 4, C4, (const float4 *)y, (float4 *)x);
     MICK();
+    return pack;
 }
 extern "C" void at_ray_scatter(const at_rays *R, const float *y, float *x, int Cc, int norm) { mi_ray_scatter_pack(R, y, x, Cc, norm, nullptr, nullptr); }
 extern "C" void at_scroll_pos(int n, int nreg, int D, int Hh, int W, const int *ad, const float *cen, float *pos) {
