@@ -158,3 +158,108 @@ def test_refusals(gpu):
     assert lib.mi_conv_down2_fwd(6, x.ptr, 3, shape5(1, 32, 4, 4, 4), w.ptr, None, 32, y.ptr, 3, gnp_t()) == -1      # compute format
     assert lib.mi_convt_up2_fwd(8, x.ptr, 0, shape5(1, 32, 4, 4, 4), w.ptr, None, 32, y.ptr, 3, gnp_t()) == -1       # fp32 planes in
     LP.check()
+
+
+def cancelling_case(rng, up, N, Ci, Co, S):
+    """Operands whose fp32 sums are mostly rounding: the second half of the input blocks repeats the first with the weights negated, at row scales of many powers of two, so that
+    another order of the same products gives other codes nearly everywhere."""
+    half = Ci // 64 * 32
+    x = rng.standard_normal((N, Ci // 32, 32, S)) * np.exp2(rng.integers(-9, 10, (N, Ci // 32, 1, S)))
+    x = x.reshape(N, Ci, S).astype(np.float32)
+    w = (rng.standard_normal((Ci, Co, 8)) * 0.1).astype(np.float32)
+    x[:, half:2 * half] = x[:, :half]
+    w[half:2 * half] = -w[:half]
+    return x, w if up else np.ascontiguousarray(w.transpose(1, 0, 2))
+
+
+def both_kernels(up, xq, xdt, N, Ci, dims, w, b, Co, ydt, bits):
+    """The bytes of the kernel for MX rows and of the general one, and the former's name."""
+    out = []
+    for mode in (-1, 0):
+        lib.mi_conv2_rows(mode)
+        try:
+            y = gpu_conv2(up, xq, xdt, N, Ci, *dims, w, b, Co, ydt, bits)
+        finally:
+            lib.mi_conv2_rows(-1)
+        out.append((y, lib.mi_last_kernel().decode()))
+    assert out[0][1].startswith("conv2_up_k<" if up and Ci <= 256 else "conv2_mx_k<" if up else "conv2_down_k<") and out[1][1].startswith("conv2_mx_k<fmt %d, out %d, up %d" % (bits, 8 if ydt == 3 else 4, up)), out
+    return out[0][0], out[1][0], out[0][1]
+
+
+@pytest.mark.parametrize("up", [0, 1])
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("N,Ci,Co,dims", [(1, 128, 64, (8, 12, 20)), (2, 224, 96, (6, 6, 18)), (1, 256, 256, (8, 8, 16)), (1, 64, 40, (12, 20, 14)), (3, 96, 160, (4, 6, 10)), (1, 640, 64, (4, 4, 10))])
+def test_the_row_kernels_keep_the_general_ones_products_and_order(gpu, up, bits, N, Ci, Co, dims):
+    """The same bytes as the general kernel where every sum shows its order: one, two and four channel tiles a workgroup, odd block counts, a partial channel tile."""
+    rng = np.random.default_rng(Ci + 3 * Co + up)
+    S, xdt = int(np.prod(dims)), 3 if bits == 8 else 4
+    x, w = cancelling_case(rng, up, N, Ci, Co, S)
+    xq = orc.f32_to_mx(bits, x, N, Ci, S)
+    for ydt in (3, 4):
+        got, ref, _ = both_kernels(up, xq, xdt, N, Ci, dims, w, None, Co, ydt, bits)
+        assert np.array_equal(got, ref), (ydt, (got != ref).mean())
+        if bits == 8 and Ci % 128 == 0:                                        # (with 64 channels the two halves meet inside one product, which is exact)
+            assert (got != orc.conv2(xq, xdt, N, Ci, *dims, w, None, Co, ydt, up, cbits=bits, acc64=1)).mean() > 0.1      # (the operands do what they are for)
+
+
+@pytest.mark.parametrize("up", [0, 1])
+@pytest.mark.parametrize("bits", [8, 4])
+def test_rows_that_are_not_finite(gpu, up, bits):
+    """NaN and infinite inputs and biases, and sums past the largest fp32 number: the row kernels' own epilogue writes what the general one does."""
+    rng = np.random.default_rng(60 + up + bits)
+    N, Ci, Co, dims, xdt = 2, 128, 96, (4, 6, 18), 3 if bits == 8 else 4
+    S = int(np.prod(dims))
+    x = rng.standard_normal((N, Ci, S)).astype(np.float32)
+    w = (rng.standard_normal((Ci, Co, 8) if up else (Co, Ci, 8)) * 0.1).astype(np.float32)
+    b = rng.standard_normal(Co).astype(np.float32)
+    clean = orc.f32_to_mx(bits, x, N, Ci, S)
+    x[0, 3, 17], x[0, 40, 200], x[1, 127, S - 1], x[1, :, 100] = np.nan, np.inf, -np.inf, 3e38
+    w[..., 0] *= 64                                                           # (tap 0: products of 3e38 and more)
+    xq = orc.f32_to_mx(bits, x, N, Ci, S)
+    for ydt in (3, 4):
+        fin, _, _ = both_kernels(up, clean, xdt, N, Ci, dims, w, b, Co, ydt, bits)
+        for q, bad in ((xq, None), (xq, np.inf), (clean, np.inf), (clean, np.nan)):      # (not a NaN bias on a NaN sum: the sign of what that gives is nobody's)
+            bias = b.copy()
+            if bad is not None:
+                bias[5], bias[40] = bad, -bad
+            got, ref, _ = both_kernels(up, q, xdt, N, Ci, dims, w, bias, Co, ydt, bits)
+            assert np.array_equal(got, ref), (ydt, bad)
+            assert not np.array_equal(got, fin)
+
+
+# (Ci, Co, N, dims, chunks of a workgroup): one to four K pairs, odd block counts, chunk counts that divide neither the channel tiles nor the chunks there are (walks that start between
+# two tap pairs, a shorter last one), up to every chunk in one workgroup
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("Ci,Co,N,dims,cpw", [(32, 96, 180, (2, 2, 3), 4), (96, 160, 180, (2, 2, 3), 7), (160, 160, 130, (1, 3, 5), 5), (224, 136, 260, (1, 2, 3), 10), (256, 96, 520, (1, 1, 2), 12),
+                                              (64, 160, 60, (3, 5, 45), 7), (160, 96, 20, (7, 11, 41), 6)])
+def test_long_walks_of_the_transposed_conv(gpu, bits, Ci, Co, N, dims, cpw):
+    """conv2_up_k's walk over its two weight slots, three chunks and more per workgroup: the oracle's bytes on exact operands in the first and the last sample, and every sample the same
+    bytes where the inputs are."""
+    rng = np.random.default_rng(Ci + Co + N)
+    S, xdt, ydt = int(np.prod(dims)), 3 if bits == 8 else 4, 3 if bits == 8 else 4
+    one = refnp.gen_exact(rng, (2, Ci, S))
+    x = np.concatenate([one[:1]] * (N - 1) + [one[1:]])
+    w = refnp.gen_exact(rng, (Ci, Co, 8), block_axis=0)
+    b = rng.integers(-8, 9, Co).astype(np.float32) * 0.25
+    got, ref, name = both_kernels(1, orc.f32_to_mx(bits, x, N, Ci, S), xdt, N, Ci, dims, w, b, Co, ydt, bits)
+    assert "chunks %d " % cpw in name, name
+    assert np.array_equal(got, ref)
+    want = orc.mx_to_f32(bits, orc.conv2(orc.f32_to_mx(bits, one, 2, Ci, S), xdt, 2, Ci, *dims, w, b, Co, ydt, 1, cbits=bits, acc64=1), 2, Co, 8 * S)
+    dec = orc.mx_to_f32(bits, got, N, Co, 8 * S).reshape(N, Co, 8 * S)
+    assert np.array_equal(dec[:-1], np.broadcast_to(want.reshape(2, Co, 8 * S)[0], dec[:-1].shape)) and np.array_equal(dec[-1], want.reshape(2, Co, 8 * S)[1])
+
+
+@pytest.mark.parametrize("up", [0, 1])
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("Ci,Co,dims", [(96, 32, (4, 6, 10)), (64, 48, (6, 10, 14)), (128, 256, (8, 8, 8))])
+def test_the_general_kernel_still_writes_rows(gpu, up, bits, Ci, Co, dims):
+    """conv2_mx_k into MX rows of 32 channels, which tensors of 2^27 voxels a sample and more run on: one, two and four channel tiles, the oracle's bytes."""
+    rng = np.random.default_rng(Ci + Co + up)
+    N, S, xdt = 2, int(np.prod(dims)), 3 if bits == 8 else 4
+    x = refnp.gen_exact(rng, (N, Ci, S))
+    w = refnp.gen_exact(rng, (Ci, Co, 8), block_axis=0) if up else refnp.gen_exact(rng, (Co, Ci, 8))
+    xq = orc.f32_to_mx(bits, x, N, Ci, S)
+    for ydt in (3, 4):
+        got, ref, _ = both_kernels(up, xq, xdt, N, Ci, dims, w, None, Co, ydt, bits)
+        want = orc.conv2(xq, xdt, N, Ci, *dims, w, None, Co, ydt, up, cbits=bits, acc64=1)
+        assert np.array_equal(ref, want) and np.array_equal(got, want)

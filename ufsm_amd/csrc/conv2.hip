@@ -32,6 +32,8 @@ __global__ void __launch_bounds__(128) prep_w2_k(const float *__restrict__ w, ui
     }
 }
 
+static thread_local int g_rows2 = -1;       // mi_conv2_rows: whether the calling thread's convs may run on conv2_up_k and conv2_down_k (-1: wherever those can, 0: nowhere)
+extern "C" void mi_conv2_rows(int mode) { g_rows2 = mode; }
 static int conv2_dispatch(const char *who, int up, int bits, const void *x, int xbf, shape5 xs, const float *w, const float *b, int cout, void *y, int ybf, gnp_t gp) {
     const unsigned wkey = mi_take_s2_wkey();                 // (consumed by this call, whatever becomes of it)
     if (bits != 8 && bits != 4) { fprintf(stderr, "%s: compute format %d (8 or 4)\n", who, bits); return -1; }
@@ -78,12 +80,12 @@ static int conv2_dispatch(const char *who, int up, int bits, const void *x, int 
     const int out = ybf == 3 ? 8 : ybf == 4 ? 4 : 0;
     // the transposed conv into MX rows of 32 channels, its rows' fragments held in registers: up to 256 input channels, and 1 024 output channels (their biases lie in LDS). The
     // kernel counts voxels in 32 bits and writes 16 bytes of a row and two scale bytes at a time
-    if (up && out && cout > 16 && nbp <= 2 * CU2_NP && nmt_all <= CU2_MT && S < (size_t)1 << 27 && ((size_t)y & 15) == 0) {
+    if (g_rows2 && up && out && cout > 16 && nbp <= 2 * CU2_NP && nmt_all <= CU2_MT && S < (size_t)1 << 27 && ((size_t)y & 15) == 0) {
         const size_t sm = conv2_up_lds(a, fmt);
         if (fmt == 8) conv2_launch_f8(out, up, 0, a, dim3(1), sm); else conv2_launch_f4(out, up, 0, a, dim3(1), sm);
         return 0;
     }
-    if (!up && out && cout > 16 && S < (size_t)1 << 27 && a.ncs <= 65535) {
+    if (g_rows2 && !up && out && cout > 16 && S < (size_t)1 << 27 && a.ncs <= 65535) {
         if (fmt == 8) conv2_launch_f8(out, up, -MT, a, dim3(1), 0); else conv2_launch_f4(out, up, -MT, a, dim3(1), 0);
         return 0;
     }

@@ -46,6 +46,7 @@ _PROTOS = {
     "mi_conv_stem_zc": (None, [C.c_int]),
     "mi_conv_split": (None, [C.c_int]),
     "mi_conv_s2_direct": (None, [C.c_int]),
+    "mi_conv2_rows": (None, [C.c_int]),
     "mi_conv_thin": (None, [C.c_int]),
     "mi_conv_flat": (None, [C.c_int]),
     "mi_conv_keep_records": (C.c_int, [C.c_int]),
