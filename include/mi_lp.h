@@ -98,7 +98,8 @@ void mi_conv_split(int tiles);
    0: always the general kernel; 1: the direct kernel, 2: the row kernel whenever its operands allow it. The results are the same conv either way. */
 void mi_conv_s2_direct(int mode);
 /* Extension: whether the calling thread's 2x2x2 stride-2 and transposed convs into MX rows of 32 channels run on the kernels for those rows wherever they can (-1, the
-   default: 17 and more output channels, fewer than 2^27 input voxels per sample; transposed: up to 256 input channels) or on the general kernel (0). The same bytes either way. */
+   default: 17 and more output channels, fewer than 2^27 input voxels per sample; transposed: up to 256 input channels; stride 2: not e4m3 from one or two blocks into three and more slices
+   of a large launch) or on the general kernel (0). The same bytes either way. */
 void mi_conv2_rows(int mode);
 /* Extension: up to how many tiles (64 voxels x 32 output channels, of the whole tensor) the calling thread's 3x3x3 convs may run on the kernel that splits
    the K range over a workgroup's wavefronts. -1 (default): the measured limits; 0: never. A setting (0 or more) also

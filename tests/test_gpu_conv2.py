@@ -263,3 +263,21 @@ def test_the_general_kernel_still_writes_rows(gpu, up, bits, Ci, Co, dims):
         got, ref, _ = both_kernels(up, xq, xdt, N, Ci, dims, w, None, Co, ydt, bits)
         want = orc.conv2(xq, xdt, N, Ci, *dims, w, None, Co, ydt, up, cbits=bits, acc64=1)
         assert np.array_equal(ref, want) and np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("bits,Ci,Co,W,rows", [(8, 32, 96, 48, False), (8, 32, 96, 36, True), (8, 64, 96, 48, False), (8, 32, 192, 48, False), (8, 64, 192, 48, True), (8, 96, 96, 48, True), (4, 32, 96, 48, True),
+                                               (8, 32, 64, 64, True), (8, 32, 128, 64, True)])
+def test_short_sums_into_many_slices(gpu, bits, Ci, Co, W, rows):
+    """e4m3 down convs of one and two blocks into three and more slices of their channel tiles, past one round of CUs, run on the general kernel; beside the line, and either side of it: the
+    oracle's bytes on exact operands."""
+    rng = np.random.default_rng(Ci + Co + W)
+    N, D, H, xdt = 2, 48, 48, 3 if bits == 8 else 4                            # (54 workgroups of 256 columns per sample and slice at W 48, 41 at 36)
+    S = D * H * W
+    one = refnp.gen_exact(rng, (1, Ci, S))
+    w = refnp.gen_exact(rng, (Co, Ci, 8))
+    xq = orc.f32_to_mx(bits, np.concatenate([one, one]), N, Ci, S)
+    got = gpu_conv2(0, xq, xdt, N, Ci, D, H, W, w, None, Co, xdt, bits)
+    assert lib.mi_last_kernel().decode().startswith("conv2_down_k<" if rows else "conv2_mx_k<")
+    want = orc.mx_to_f32(bits, orc.conv2(orc.f32_to_mx(bits, one, 1, Ci, S), xdt, 1, Ci, D, H, W, w, None, Co, xdt, 0, cbits=bits, acc64=1), 1, Co, S // 8).reshape(Co, -1)
+    dec = orc.mx_to_f32(bits, got, N, Co, S // 8).reshape(N, Co, -1)
+    assert np.array_equal(dec[0], want) and np.array_equal(dec[1], want)

@@ -85,7 +85,12 @@ static int conv2_dispatch(const char *who, int up, int bits, const void *x, int 
         if (fmt == 8) conv2_launch_f8(out, up, 0, a, dim3(1), sm); else conv2_launch_f4(out, up, 0, a, dim3(1), sm);
         return 0;
     }
-    if (g_rows2 && !up && out && cout > 16 && S < (size_t)1 << 27 && a.ncs <= 65535) {
+    // the down conv into MX rows of 32 channels, but for e4m3 launches past one round of CUs with one or two K pairs per tap class and three and more slices of its channel tiles: the rows are read once
+    // per slice there and little is multiplied. General kernel / conv2_down_k, us: 32 -> 96 from 2 x 64^3 8.7 / 10.2, 32 -> 160 12.1 / 15.2, 32 -> 192 11.5 / 12.3, 64 -> 160 22.0 / 23.7; but
+    // 64 -> 192 19.9 / 18.9, 128 -> 160 49.3 / 44.6, and 32 -> 160 from 32^3 (20 workgroups) 5.1 / 5.2, e2m1 32 -> 160 10.0 / 9.4
+    const size_t dwg = (size_t)((Scol + 255) / 256) * a.ncs * N;
+    const bool thin2 = fmt == 8 && MT * nbp <= 2 && a.ncs >= 3 && dwg > 256;
+    if (g_rows2 && !up && out && cout > 16 && S < (size_t)1 << 27 && a.ncs <= 65535 && !thin2) {
         if (fmt == 8) conv2_launch_f8(out, up, -MT, a, dim3(1), 0); else conv2_launch_f4(out, up, -MT, a, dim3(1), 0);
         return 0;
     }
