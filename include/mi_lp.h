@@ -257,7 +257,8 @@ long mi_alloc_count(void);                     /* device allocations made by thi
    inside the domain the kernels use the instruction on (e4m3: |x 2^-e| <= 464 and not NaN; e2m1: not NaN), out[1]: mismatches among them (0
    expected), out[2] / out[3]: inputs outside it and their mismatches (those blocks take the software encoder). Synchronises. 0, or -1 for bad arguments */
 int mi_cvt_sweep(int bits, int e, unsigned long long out[4]);
-/* name of the conv kernel variant the last conv call on this thread launched (diagnostics / tests), "" if none */
+/* the conv kernel the last conv call on this thread launched (diagnostics / tests), "" if none: its name is the first word; what follows are its template arguments and launch or, after
+   "for" or in parentheses, the kernel whose products, order and records it has - compare the first word to tell the two apart */
 const char *mi_last_kernel(void);
 #ifdef __cplusplus
 }

@@ -134,3 +134,28 @@ def test_overlapping_slabs_that_count_their_own_planes(gpu, bits, Ci, Co, D, H, 
     v = np.abs(y.astype(np.float64)).reshape(G, -1)
     # (fp32 within records of 32 voxels x 4 channels, cut elsewhere in the slabs)
     assert np.abs(out.to_numpy(np.float64, (G, 2)) - ws[0]).max() <= 1e-5 * max(v.sum(1).max(), (v * v).sum(1).max())
+
+
+def first_word():
+    """The kernel that ran. (A name goes on with the form whose products and records the kernel has, which may be another kernel's: `in` does not tell the two apart.)"""
+    return lib.mi_last_kernel().decode().split("<")[0].split(" ")[0]
+
+
+# the calls that other tests look for conv3_mx_k in, with what runs there: few tiles by the staged kernels' rule (thin 0), the general kernel's three-tile slices, a last chunk of fewer blocks, more tiles than the pipelined form takes
+@pytest.mark.parametrize("bits,N,Ci,Co,D,H,W,thin,kern", [
+    (8, 1, 96, 128, 5, 9, 18, 0, "conv3_pipe_k"), (8, 1, 32, 128, 3, 8, 16, 0, "conv3_pipe_k"), (8, 2, 128, 256, 6, 10, 33, 0, "conv3_pipe_k"), (4, 1, 160, 128, 7, 8, 16, 0, "conv3_mx_k"),
+    (4, 2, 64, 256, 4, 16, 16, 0, "conv3_pipe_k"), (8, 1, 384, 128, 4, 8, 16, 0, "conv3_pipe_k"), (8, 1, 96, 96, 16, 16, 24, -1, "conv3_mx_k"), (8, 1, 64, 128, 18, 32, 32, -1, "conv3_pipe_k"),
+    (8, 1, 416, 128, 16, 64, 128, -1, "conv3_mx_k"), (8, 1, 64, 40, 3, 96, 96, 0, "conv3_pipe_k"), (8, 1, 64, 40, 4, 128, 128, 0, "conv3_mx_k"), (8, 2, 64, 40, 3, 96, 96, 0, "conv3_mx_k")])
+def test_the_kernel_that_ran_is_the_first_word(gpu, bits, N, Ci, Co, D, H, W, thin, kern):
+    rng = np.random.default_rng(Ci + Co + W)
+    S, xdt = D * H * W, 3 if bits == 8 else 4
+    dx, dw = DevBuf.from_numpy(orc.f32_to_mx(bits, rng.standard_normal((N, Ci, S)).astype(np.float32), N, Ci, S)), DevBuf.from_numpy(rng.standard_normal((Co, Ci, 27)).astype(np.float32))
+    dy, sums = DevBuf((lib.lp_mx8_bytes if bits == 8 else lib.lp_mx4_bytes)(N, Co, S)), DevBuf(N * Co * 2 * 24)
+    f, G = lib.lp_conv_fwd_f8 if bits == 8 else lib.lp_conv_fwd_f4, 8 if Co % 32 == 0 else Co
+    lib.mi_conv_thin(thin)
+    try:
+        assert f(dx.ptr, xdt, shape5(N, Ci, D, H, W), dw.ptr, None, Co, dy.ptr, xdt, gnp_t(), sums.ptr, G, split_t()) == 0
+    finally:
+        lib.mi_conv_thin(-1)
+    LP.check()
+    assert first_word() == kern, lib.mi_last_kernel().decode()
