@@ -254,3 +254,26 @@ def test_one_run_or_two_per_workgroup(gpu, bits, N, Ci, Co, dims):
     want, ws = orc.conv3(xq, xdt, N, Ci, D, H, W, w, b, Co, xdt, cbits=bits, acc64=1, Go=G if stats else 0, want_stats=stats)
     assert np.array_equal(got, want)
     assert not stats or np.allclose(gs, ws, rtol=1e-6)
+
+
+@pytest.mark.parametrize("bits,Ci,Co,dims,stride", [(8, 64, 64, (4, 4, 8), 1), (8, 256, 96, (3, 5, 7), 1), (4, 96, 64, (4, 4, 8), 1), (4, 384, 64, (3, 5, 9), 1), (8, 128, 64, (6, 7, 9), 2), (4, 96, 64, (8, 8, 8), 2)])
+def test_one_run_or_two_per_workgroup_give_the_same_bits(gpu, bits, Ci, Co, dims, stride):
+    """Up to 128 tiles of 64 voxels a workgroup takes one run of 32, beyond that two: a sample's fp32 outputs and statistics are the same bits, on operands of several magnitudes, whose sums
+    depend on their order."""
+    rng = np.random.default_rng(Ci + Co + stride)
+    N, G, xdt = 70, 8, 3 if bits == 8 else 4
+    D, H, W = dims
+    x, w, b = rand_case(rng, N, Ci, Co, D * H * W)
+    x *= np.exp(2 * rng.standard_normal(x.shape)).astype(np.float32)
+    out = []
+    for n in (N, 9, 1):
+        lib.mi_conv_thin(4096)
+        try:
+            y, g = gpu_conv(orc.f32_to_mx(bits, x[:n], n, Ci, D * H * W), xdt, n, Ci, D, H, W, w, b, Co, 0, cbits=bits, stride=stride, **(dict(Go=G, stats=True) if stride == 1 else {}))
+        finally:
+            lib.mi_conv_thin(-1)
+        name = lib.mi_last_kernel().decode()
+        assert name.startswith("conv3_thin_k<") and (int(name.split("tiles ")[1]) > 128) == (n == N), name
+        out.append((y, g))
+    for n, (y, g) in zip((9, 1), out[1:]):
+        assert np.array_equal(y.view(np.uint32), out[0][0][:n].view(np.uint32)) and (g is None or np.array_equal(g, out[0][1][:n]))
