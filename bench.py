@@ -252,8 +252,8 @@ def hbm_leg(np, lib, LP, DevBuf):
     yd = DevBuf(lib.lp_mx4_bytes(N, 256, 32 ** 3)); yu = DevBuf(lib.lp_mx4_bytes(N, 128, 64 ** 3))
     wd = DevBuf.from_numpy((rng.standard_normal((256, 128, 8)) * 0.04).astype(np.float32))
     cases += [
-        ("conv2_mx_k (2x2x2 stride-2 down conv 128 -> 256, 64^3 in, MX-fp4)", mx4(128, 64 ** 3) + mx4(256, 32 ** 3), lambda: (lib.mi_conv_s2_wkey(902), lib.mi_conv_down2_fwd(4, qd.ptr, 4, shape5(N, 128, 64, 64, 64), wd.ptr, None, 256, yd.ptr, 4, gnp_t()))),
-        ("conv2_mx_k (2x2x2 stride-2 transposed conv 256 -> 128, 32^3 in, MX-fp4)", mx4(256, 32 ** 3) + mx4(128, 64 ** 3), lambda: (lib.mi_conv_s2_wkey(903), lib.mi_convt_up2_fwd(4, yd.ptr, 4, shape5(N, 256, 32, 32, 32), wd.ptr, None, 128, yu.ptr, 4, gnp_t()))),
+        ("conv2_down_k (2x2x2 stride-2 down conv 128 -> 256, 64^3 in, MX-fp4)", mx4(128, 64 ** 3) + mx4(256, 32 ** 3), lambda: (lib.mi_conv_s2_wkey(902), lib.mi_conv_down2_fwd(4, qd.ptr, 4, shape5(N, 128, 64, 64, 64), wd.ptr, None, 256, yd.ptr, 4, gnp_t()))),
+        ("conv2_up_k (2x2x2 stride-2 transposed conv 256 -> 128, 32^3 in, MX-fp4)", mx4(256, 32 ** 3) + mx4(128, 64 ** 3), lambda: (lib.mi_conv_s2_wkey(903), lib.mi_convt_up2_fwd(4, yd.ptr, 4, shape5(N, 256, 32, 32, 32), wd.ptr, None, 128, yu.ptr, 4, gnp_t()))),
     ]
     rows = []
     for name, nbytes, call in cases:

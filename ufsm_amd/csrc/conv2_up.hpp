@@ -6,14 +6,16 @@
 // SIMD, each of which spends a third of its life in front of its first product (64-bit divisions for the lane's voxel, then the rows, then the weights) and
 // writes every second 16-byte row of its output lines. Here
 //   * a wavefront owns 32 consecutive input voxels whose fragments of all K pairs stay in registers; a workgroup of eight walks CHUNKS: chunk (dz, dy, m) is the
-//     two dx taps into channel tile m, two accumulator tiles, 32 registers. Four wavefronts per SIMD fit, and one's epilogue runs beside another's products;
+//     two dx taps into channel tile m, two accumulator tiles, 32 registers. Four wavefronts per SIMD fit (e4m3 with four K pairs by five spilled registers into
+//     e4m3 rows and three into e2m1 ones, stored once and read back once a chunk), and one's epilogue runs beside another's products;
 //   * a chunk's weights (2 taps x K pairs) come by LDS-DMA into the second of two slots while the chunk before is multiplied: the workgroup's 256 voxels share
 //     them. One barrier per chunk, in front of its stores, so that waiting for the copies waits for stores a chunk old;
 //   * the two voxels of a chunk are neighbours in memory: e2m1 rows change halves between the lanes of a voxel (one lane gets a whole row of each), so that a
 //     wavefront's store covers 1 KiB without holes, and the two scale bytes leave as one 16-bit store.
 // The launch splits the chunks over blockIdx.y until two workgroups per CU are there (the rows are then read once per split, from the L2).
-// The products and their order are those of conv2_mx_k: the same bytes. Measured, e2m1 256 -> 128 from 2 x 32^3 (44.6 MB, 8.6 GFLOP): 31.6 -> 21.0 us
-// under the kernel trace (2.1 TB/s); with the down conv in front of it, passes back to back, 48.7 -> 36.3 us. e4m3, 128 -> 128 down and up at 38 x 50 x 20: 29.5 -> 18.1.
+// The products and their order are those of conv2_mx_k: the same bytes. Measured, passes back to back, us, conv2_mx_k / this: e2m1 256 -> 128 from 2 x 32^3 (44.6 MB, 8.6 GFLOP) 27.8 / 20.9
+// (2.1 TB/s); e4m3 the same 104.3 / 32.2, 224 -> 128 there 103.2 / 31.7, 128 -> 128 from 2 x 38 x 50 x 20 90.9 / 28.9. With the down conv in front of it (conv2_down.hpp), e2m1 128 -> 256 -> 128 at
+// 2 x 64^3: 48.8 -> 35.5.
 // What is left is the start (rows and the first weights, about 3 us, which every workgroup of the single round waits for) and the epilogues.
 #pragma once
 #include "conv3_kernel.hpp"

@@ -692,7 +692,10 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     // 256 -> 256 at 4 x 16^3 50.1 and 38.1 (512), 384 -> 128 at 28^3 63.6 and 44.8 (344), 128 -> 128 at 28^3 28.0 and 27.3; e2m1 384 -> 128 at 2 x 24^3 48.5 and 34.5 (432), 128 -> 128 25.1
     // and 23.4; in four it does not: 384 -> 128 at 2 x 32^3 75.4 and 90.9 (1024). A record per run of 32 voxels is four to eight times the staged kernels': past 512 a sample their
     // sums take a launch more (3 - 5 us), which e2m1's shorter products do not always win back: 256 -> 128 at 28^3 (686 runs) 33.1 against 37.7 with it. As above, the whole
-    // tensor's voxels count, not a z-range's
+    // tensor's voxels count, not a z-range's.
+    // (Where the other kernel was the general one, that is of before conv3_pipe_k, which has closed much of the gap; a call with its statistics, us, conv3_pipe_k / this: e4m3 256 -> 256 at 2 x 16^3
+    // 24.0 / 21.9, 64 -> 128 at 22 x 26^2 16.1 / 16.5, 128 -> 128 22.6 / 19.3, 384 -> 128 46.3 / 28.7, at 28^3 46.0 / 48.5; e2m1 128 -> 192 at 2 x 16^3 12.9 / 14.5, 192 -> 192 15.3 / 16.1, 384 -> 128
+    // 21.6 / 19.7. The line stays where it was: the two add their products in different orders)
     static int flat_env = -1;
     if (flat_env < 0) flat_env = getenv("MI_CONV_FLAT") ? atoi(getenv("MI_CONV_FLAT")) : 1;      // tuning knob: 0 never
     const bool flat_ok = stride == 1 && a.wide && !act && nmt_all >= 2 && a.nbt % 2 == 0 && W <= flat_t<8>::WMAX && !(osum && (cout / Go) % 4) && N <= 65535 && (size_t)D * H * W < ((size_t)1 << 24) &&
@@ -705,7 +708,7 @@ static int conv_dispatch(const char *who, int fmt, int stride, const void *x, in
     // the general kernel's one-tile, two-plane launches, pipelined (conv3_pipe.hpp), up to 512 workgroups (what the coarse form and the divided slices of three launch at the most): a workgroup
     // has a CU's LDS to itself, or half of it where its stages shrink to three pairs (conv3_pipe_pps). A conv with its statistics, us, conv3_mx_k / this. e4m3: 256 -> 256 at 2 x 16^3 (256 workgroups)
     // 38.9 / 25.3, 128 -> 256 23.4 / 16.7, at 3 x 16^3 (384) 256 -> 256 45.2 / 33.4, at 22 x 26^2 (352) 384 -> 128 66.3 / 48.1, 128 -> 128 27.9 / 22.0, 64 -> 128 18.9 / 16.0; e2m1: 256 -> 256 at 2 x 12^3
-    // (192) 24.7 / 17.0, 192 -> 192 at 2 x 16^3 (192) 20.7 / 14.6, 384 -> 128 there (128) 32.9 / 20.8. Past one round of CUs in chunks of three or four blocks two or more chunks still gain - 384 -> 128
+    // (192) 24.7 / 17.0, in stages of three pairs 64 -> 128 at 22 x 26^2 (352) 15.8 / 13.4, 32 -> 128 13.2 / 11.8, 64 -> 256 at 3 x 11 x 16^2 (288) 14.5 / 12.3, 192 -> 192 at 2 x 16^3 (192) 20.7 / 14.6, 384 -> 128 there (128) 32.9 / 20.8. Past one round of CUs in chunks of three or four blocks two or more chunks still gain - 384 -> 128
     // at 22 x 26^2 40.9 / 37.8, 192 -> 192 at 5 x 16^3 (480) 25.4 / 24.3 -, one does not: 128 -> 128 at 22 x 26^2 20.3 / 21.2
     static int pipe_env = -1;
     if (pipe_env < 0) pipe_env = getenv("MI_CONV_PIPE") ? atoi(getenv("MI_CONV_PIPE")) : 512;      // tuning knob: that workgroup count (0: never)

@@ -369,8 +369,8 @@ static void launch_wide(const conv_args &a, size_t smem) {
         ncu[d] = pr.multiProcessorCount > 8 ? pr.multiProcessorCount & ~7 : 8;
         attr[d] = true;
     }
-    // tiles per XCD; one persistent workgroup per CU, a multiple of 8 in all. The e2m1 slices of 64 channels: two, whose registers (128 and 128, none spilled) and LDS (79 936 bytes at the
-    // most, twelve input blocks) fit beside each other: a stage's sixteen products are then no longer than the 150 other instructions of its wavefront, and the second wavefront of a SIMD
+    // tiles per XCD; one persistent workgroup per CU, a multiple of 8 in all. The e2m1 slices of 64 channels: two, whose registers (128 and 128; into e2m1 rows three more are
+    // spilled, stored once in front of the walk and read back once a tile, by the statistics) and LDS (79 936 bytes at the most, twelve input blocks) fit beside each other: a stage's sixteen products are then no longer than the 150 other instructions of its wavefront, and the second wavefront of a SIMD
     // multiplies while the first issues them or converts its accumulators. us, one / two per CU: 192 -> 64 at 2 x 64^3 125.6 / 100.5, at 2 x 48^3 61.3 / 46.9, 128 -> 64 there 46.3 / 38.8,
     // 256 -> 256 at 2 x 24^3 69.7 / 53.5. (Slices of 128 as eight wavefronts of one workgroup, two per SIMD, which meet at every stage's barrier: 66.0 / 68.6 at 256 -> 256, 2 x 32^3)
     const unsigned per = (a.ntiles + 7u) / 8u, wgs = (unsigned)ncu[d] * (wide_two(FMT, EPI, MT) && smem <= 80 * 1024 ? 2u : 1u);
